@@ -1,5 +1,6 @@
 // C ABI of libqmm_hip.so: argument validation and regime dispatch.
 // See include/qmm_hip.h for the contract of every entry point.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -40,7 +41,9 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
                     int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
                     const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N,
                     int64_t K, int gs, int bits, int mode, int row_tile, void* workspace,
-                    hipStream_t st);
+                    size_t workspace_bytes, hipStream_t st);
+double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits);
+size_t gemm2_split_workspace_bytes(int64_t R, int64_t N, int64_t K);
 bool mxfp4_mfma_supported(int64_t R, int64_t N, int64_t K);
 size_t mxfp4_workspace_bytes(int64_t R, int64_t K);
 void mxfp4_geometry(int64_t R, int64_t N, int64_t K, int* grid, int* block);
@@ -229,6 +232,14 @@ size_t dense_scratch(int64_t rows, int64_t N, int64_t K, int mode, bool exact) {
   return 0;
 }
 
+// ... with room for the sums of a split K, which the dense prefill product takes where it is there
+size_t dense_scratch_split(int64_t rows, int64_t N, int64_t K, int mode, bool exact) {
+  const size_t least = dense_scratch(rows, N, K, mode, exact);
+  const bool mx = mode == QMM_MODE_MXFP4 && !exact && mxfp4_mfma_supported(rows, N, K);
+  if (rows <= kGemvMaxM || N <= 0 || mx || !gemm2_supported(rows, N, K)) return least;
+  return std::max(least, gemm2_split_workspace_bytes(rows, N, K));
+}
+
 size_t gather_scratch(int64_t P, int64_t E, int64_t N, int64_t K, bool exact) {
   if (P < kGroupedDecodeMinPairs) return 0;
   const size_t decode = grouped_decode_pairs(P, E) ? route_bytes_segments(P, E) : 0;
@@ -284,11 +295,11 @@ const char* qmm_last_error(void) { return g_err; }
 size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int, int, int mode,
                            int x_dtype) {
   const int terms = act_terms(x_dtype);
-  if (terms == 1) return dense_scratch(M, N, K, mode, false);
+  if (terms == 1) return dense_scratch_split(M, N, K, mode, false);
   // terms as bf16 rows, their float32 products, then the scratch of the bf16
   // product: over terms x M stacked rows (dense) or over M rows (grouped)
   if (batch < 1) batch = 1;
-  const size_t stacked = dense_scratch(terms * M, N, K, mode, true), plain = dense_scratch(M, N, K, mode, true);
+  const size_t stacked = dense_scratch_split(terms * M, N, K, mode, true), plain = dense_scratch(M, N, K, mode, true);
   return align256((size_t)(batch * terms * M * K) * 2) + align256((size_t)(batch * terms * M * N) * 4) +
          (stacked > plain ? stacked : plain);
 }
@@ -341,11 +352,12 @@ int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode
     if (kernel) *kernel = QMM_KERNEL_GEMV;
     if (grid) *grid = (int)ceil_div(N, 16 * t);
     if (block) *block = 64 * waves;
-  } else if (K % 256 == 0 && (mode == QMM_MODE_MXFP4 || bits == 4 || bits == 8)) {
-    // the split-role kernel (bf16 tables assumed): 256-row tiles, four
-    // multiplying and four dequantizing wavefronts
+  } else if (gemm2_supported(M, N, K) && (mode == QMM_MODE_MXFP4 || bits == 4 || bits == 8)) {
+    // the split-role kernel (bf16 tables assumed): four multiplying and four dequantizing wavefronts
+    int rows, splits;
+    gemm2s_plan(M, 1, N, K, ~(size_t)0, &rows, &splits);
     if (kernel) *kernel = QMM_KERNEL_GEMM;
-    if (grid) *grid = (int)(ceil_div(N, 128) * ceil_div(M, 256));
+    if (grid) *grid = (int)(ceil_div(N, 128) * ceil_div(M, rows) * splits);
     if (block) *block = 512;
   } else {
     const int64_t bm = gemm_row_tile(M, 1);
@@ -415,7 +427,7 @@ static int dense_bf16(const void* x, int x_dtype, const void* w, const void* sca
                      static_cast<const char*>(scales) + z * N * ng * tabsz,
                      biases ? static_cast<const char*>(biases) + z * N * ng * tabsz : nullptr,
                      table_dtype, static_cast<char*>(y) + z * M * N * ysz, y_dtype, nullptr, nullptr,
-                     nullptr, M, M, 1, N, K, group_size, bits, mode, bm, workspace, st);
+                     nullptr, M, M, 1, N, K, group_size, bits, mode, bm, workspace, workspace_bytes, st);
       rc = check_launch("gemm launch");
       if (rc) return rc;
     }
@@ -458,7 +470,7 @@ static int grouped_bf16(const void* x, int x_dtype, const void* w, const void* s
   if (gemm2_supported(R, N, K) && workspace && workspace_bytes >= gemm2_workspace_bytes(R, K) &&
       aligned16(workspace)) {
     gemm2_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, row_offsets, nullptr, nullptr, R,
-                   R, E, N, K, group_size, bits, mode, (int)gemm_row_tile(R, E), workspace,
+                   R, E, N, K, group_size, bits, mode, (int)gemm_row_tile(R, E), workspace, workspace_bytes,
                    static_cast<hipStream_t>(stream));
     return check_launch("grouped gemm launch");
   }
@@ -555,7 +567,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     // rows gathered in expert order into the re-laid copy, results scattered back to pair order
     gemm2_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K,
                    group_size, bits, mode, (int)gemm_row_tile(P, E),
-                   static_cast<char*>(workspace) + need, st);
+                   static_cast<char*>(workspace) + need, workspace_bytes - need, st);
     return check_launch("gather gemm launch");
   }
   gemm_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K,
@@ -588,7 +600,7 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
   int rc = check_launch("activation split launch");
   if (rc) return rc;
   rc = dense_bf16(ws, QMM_BF16, w, scales, biases, table_dtype, ws + xs, QMM_F32, batch, terms * M, N, K,
-                  group_size, bits, mode, inner ? ws + xs + ps : nullptr, inner, stream, true);
+                  group_size, bits, mode, inner ? ws + xs + ps : nullptr, workspace_bytes - xs - ps, stream, true);
   if (rc) return rc;
   if (!y) return fail(QMM_ERR_BAD_ARGUMENT, "null output pointer");
   sum_terms_dispatch(ws + xs, terms, y, y_dtype, batch, M, N, nullptr, nullptr, 0, st);

@@ -33,8 +33,9 @@
 
 namespace qmm {
 
-// the grouped kernel for short row groups (qmm_gemm2s.hip)
+// the split-role kernel (qmm_gemm2s.hip)
 bool gemm2s_wanted(const g2::Gemm2Args& a, int mode, int bits);
+double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits);
 void gemm2s_launch(const g2::Gemm2Args& a, int mode, int bits, hipStream_t st);
 
 namespace {
@@ -81,19 +82,15 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const uint16_t* __restri
 // rows end in its first half leaves every wavefront's second block empty and
 // runs a main loop without it.
 //
-// TF selects how scales / biases are fetched.  1..3: as 16-byte windows (four
-// K-tiles of a row at once), with the entry type fixed at compile time --
-// 1 = two-byte bf16 (one-byte E8M0 for MXFP4), 2 = float32, 3 = float16 -- so
-// that picking an entry is a handful of selects and the K loop has no branch
-// in it (a branch would end the region the MFMAs are interleaved in).
-// 0: any layout, one load per entry, types read at run time (unaligned or
-// short tables).
-//
-// G64 (bf16 tables, groups of 64): a K-tile is one group, so the entry of
-// K-tile t' of a window is its t'-th, the same for every thread: no selects.
-template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG, int TF, bool G64>
+// What comes here is what the split-role kernel does not take.  WIN: float32
+// tables of groups of 32, fetched as 32-byte windows (four K-tiles of a row at
+// once), so that picking an entry is a handful of selects and the K loop has no
+// branch in it (a branch would end the region the MFMAs are interleaved in).
+// Otherwise any layout, one load per entry, types read at run time (tables that
+// do not start on dwords, and experts' tables that do not).
+template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG, bool WIN>
 __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
-  static_assert(!G64 || (TF == 1 && MODE == 0), "the one-group-a-K-tile form reads bf16 windows");
+  static_assert(!WIN || MODE == 0, "windows of float32 tables");
   constexpr int WNW = NWAVES / WMW;
   static_assert(WNW * NT * 32 == BN, "the wavefronts must span the weight tile");
   constexpr int WM = MT * 32;                      // rows per wavefront
@@ -145,7 +142,7 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
   const int64_t wpr = (int64_t)a.K * WBITS / 32;
   const int gs = (MODE == 1) ? 32 : a.gs;
   const int64_t ng = a.K / gs;
-  const int tabsz = (MODE == 1) ? 1 : (TF == 2 ? 4 : TF != 0 ? 2 : (a.tab == QMM_F32 ? 4 : 2));
+  const int tabsz = (MODE == 1) ? 1 : (WIN || a.tab == QMM_F32 ? 4 : 2);
   const uint32_t* wb = a.w + (int64_t)e * a.N * wpr;
   const char* sb = static_cast<const char*>(a.s) + (int64_t)e * a.N * ng * tabsz;
   const char* bb = (MODE == 1) ? nullptr : static_cast<const char*>(a.b) + (int64_t)e * a.N * ng * tabsz;
@@ -208,11 +205,10 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
   const int gshift = gs == 32 ? 5 : (gs == 64 ? 6 : 7);
   auto load_win = [&](int quad, TabWin& tw) {
     const uint32_t so = (uint32_t)(((quad * 4 * BK) >> gshift) * tabsz);
-    tw.s[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, tvo, so, 0);
-    if constexpr (TF == 2) tw.s[1] = __builtin_amdgcn_raw_buffer_load_b128(rs, tvo + 16, so, 0);
-    if constexpr (MODE == 0) {
-      tw.b[0] = __builtin_amdgcn_raw_buffer_load_b128(rb, tvo, so, 0);
-      if constexpr (TF == 2) tw.b[1] = __builtin_amdgcn_raw_buffer_load_b128(rb, tvo + 16, so, 0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      tw.s[h] = __builtin_amdgcn_raw_buffer_load_b128(rs, tvo + 16 * h, so, 0);
+      tw.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rb, tvo + 16 * h, so, 0);
     }
   };
   // entry index of K-tile t' inside its window, for this thread's k-half
@@ -220,37 +216,18 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
 #pragma unroll
   for (int t = 0; t < 4; ++t) eidx[t] = (uint32_t)((t * BK + whalf * CPT) >> gshift);
   auto pick = [&](const u32x4 (&w)[2], uint32_t e) -> float {
-    // entry e (0..7) of a window of 1-, 2- or 4-byte entries (TF != 0 only)
-    constexpr uint32_t TS = (MODE == 1) ? 1u : (TF == 2 ? 4u : 2u);
-    const uint32_t byte = e * TS;
-    const uint32_t d = byte >> 2;
-    uint32_t v = w[0][0];
-    v = d == 1 ? w[0][1] : v;
-    v = d == 2 ? w[0][2] : v;
-    v = d == 3 ? w[0][3] : v;
-    if constexpr (TF == 2) {
-      v = d == 4 ? w[1][0] : v;
-      v = d == 5 ? w[1][1] : v;
-      v = d == 6 ? w[1][2] : v;
-      v = d == 7 ? w[1][3] : v;
-      return __uint_as_float(v);
-    }
-    v >>= (byte & 3u) * 8u;
-    if constexpr (MODE == 1) return e8m0_to_f32(v & 255u);
-    if constexpr (TF == 3) return f16_bits_to_f32(v & 0xFFFFu);
-    return __uint_as_float(v << 16);
+    uint32_t v = w[0][0];                          // (WIN only)
+#pragma unroll
+    for (uint32_t d = 1; d < 8; ++d) v = e == d ? w[d >> 2][d & 3] : v;
+    return __uint_as_float(v);
   };
   // (scale, bias) of K-tile kt for this thread; tq = kt & 3 at compile time
   // (a clamped kt past the last tile only feeds a stage that nobody reads)
   auto entry = [&](int kt, auto tqc, const TabWin& tw, float& sc, float& bi) {
     constexpr int tq = decltype(tqc)::value;
-    if constexpr (G64) {
-      const uint32_t vs = tw.s[0][tq >> 1], vb = tw.b[0][tq >> 1];
-      sc = __uint_as_float((tq & 1) ? (vs & 0xFFFF0000u) : (vs << 16));
-      bi = __uint_as_float((tq & 1) ? (vb & 0xFFFF0000u) : (vb << 16));
-    } else if constexpr (TF != 0) {
+    if constexpr (WIN) {
       sc = pick(tw.s, eidx[tq]);
-      bi = MODE == 1 ? 0.f : pick(tw.b, eidx[tq]);
+      bi = pick(tw.b, eidx[tq]);
     } else {
       const int64_t ti = trow + ((kt * BK + whalf * CPT) >> gshift);
       if constexpr (MODE == 1) {
@@ -283,7 +260,7 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
   // prologue: tile 0 dequantized, tiles 0..1 of the activations and the words
   // of tiles 1..3 in flight
   TabWin tw_cur, tw_nxt;
-  if constexpr (TF != 0) load_win(0, tw_cur);
+  if constexpr (WIN) load_win(0, tw_cur);
   // Issue order matters: a wait counts the loads issued after the one it needs,
   // and the waits inside the loop must also hold on its first pass.  The words
   // that the loop dequantizes first (tiles 1, 2, 3) therefore go out before the
@@ -349,7 +326,7 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
       }
       load_a_part(kt2, af[(t + 2) & 3], ks, na);
       if (ks == 0) load_w(kt4, wr[t & 3]);          // three K-tiles ahead of its dequantization
-      if (TF != 0 && ks == 1 && t == 0) {          // next quad's table window (clamped at the end)
+      if (WIN && ks == 1 && t == 0) {          // next quad's table window (clamped at the end)
         const int q = (kt >> 2) + 1;
         load_win(q * 4 < KT ? q : (kt >> 2), tw_nxt);
       }
@@ -467,7 +444,7 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
   }
 }
 
-template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG, int TF, bool G64 = false>
+template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG, bool WIN>
 void launch2_k(const Gemm2Args& a0, hipStream_t st) {
   constexpr int BM = WMW * MT * 32;
   Gemm2Args a = a0;
@@ -479,22 +456,17 @@ void launch2_k(const Gemm2Args& a0, hipStream_t st) {
   // three weight stages; the epilogue transposes 32 x NT*32 sixteen-bit results per wavefront there
   const size_t epi = (size_t)NWAVES * 32 * NT * 32 * 2;
   const size_t lds = epi > (size_t)(kStages * kStage) ? epi : (size_t)(kStages * kStage);
-  constexpr auto kern = gemm2_kernel<MODE, BITS, MT, NT, WMW, NWAVES, RAG, TF, G64>;
+  constexpr auto kern = gemm2_kernel<MODE, BITS, MT, NT, WMW, NWAVES, RAG, WIN>;
   if (!lds_limit<kern>(lds)) return;
   hipLaunchKernelGGL(kern, grid, dim3(64 * NWAVES), lds, st, a);
 }
 
 template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG>
 void launch2_tf(const Gemm2Args& a, hipStream_t st) {
-  if (!a.tabfast) return launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 0>(a, st);
-  if constexpr (MODE == 1) {
-    launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 1>(a, st);
-  } else {
-    if (a.tab == QMM_BF16 && a.gs == 64) launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 1, true>(a, st);
-    else if (a.tab == QMM_BF16) launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 1>(a, st);
-    else if (a.tab == QMM_F32) launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 2>(a, st);
-    else launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, 3>(a, st);
+  if constexpr (MODE == 0) {
+    if (a.tabfast) return launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, true>(a, st);
   }
+  launch2_k<MODE, BITS, MT, NT, WMW, NWAVES, RAG, false>(a, st);
 }
 
 template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES>
@@ -520,12 +492,25 @@ bool gemm2_supported(int64_t R, int64_t N, int64_t K) {
 
 size_t gemm2_workspace_bytes(int64_t R, int64_t K) { return (size_t)(prep_rows(R) * K * 2); }
 
+// ... with the sums of as many splits of K as a dense product would take
+size_t gemm2_split_workspace_bytes(int64_t R, int64_t N, int64_t K) {
+  int rows, splits;
+  gemm2s_plan(R, 1, N, K, ~(size_t)0, &rows, &splits);
+  return gemm2_workspace_bytes(R, K) + (splits > 1 ? (size_t)splits * R * N * 4 : 0);
+}
+
+// About how long the product takes, in microseconds.
+double gemm2_us(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes) {
+  int rows, splits;
+  return gemm2s_plan(R, E, N, K, part_bytes, &rows, &splits);
+}
+
 // x bf16 [x_rows, K] (rows gathered through lhs_idx when given); the rest as gemm_dispatch.
 void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                     int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
                     const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N,
                     int64_t K, int gs, int bits, int mode, int row_tile, void* workspace,
-                    hipStream_t st) {
+                    size_t workspace_bytes, hipStream_t st) {
   if (R == 0 || N == 0) return;
   const int64_t rp = prep_rows(R);
   const int64_t prep_blocks = ceil_div(R, 8) * ceil_div(K / 8, 32);
@@ -544,13 +529,21 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
   a.gs = gs; a.tab = tab; a.y_dtype = y_dtype;
   a.m_tiles = 0;
   {
-    const int esz = mode == QMM_MODE_MXFP4 ? 1 : (tab == QMM_F32 ? 4 : 2);
-    const int g = mode == QMM_MODE_MXFP4 ? 32 : gs;
-    const bool aligned = ((K / g) * esz) % 4 == 0 && (reinterpret_cast<uintptr_t>(s) & 3u) == 0 &&
-                         (mode == QMM_MODE_MXFP4 || (reinterpret_cast<uintptr_t>(b) & 3u) == 0);
-    a.tabfast = aligned && K % 256 == 0 && N * (K / g) * esz < (1ll << 31) && !experiment_env("QMM_G2_NOTABFAST");
+    const int64_t esz = mode == QMM_MODE_MXFP4 ? 1 : (tab == QMM_F32 ? 4 : 2);
+    const int64_t row = K / (mode == QMM_MODE_MXFP4 ? 32 : gs) * esz;            // bytes of a table row
+    const bool dword = (reinterpret_cast<uintptr_t>(s) & 3u) == 0 && (mode == QMM_MODE_MXFP4 || (reinterpret_cast<uintptr_t>(b) & 3u) == 0);
+    a.tab_odd = row % 4 != 0;
+    a.tab_ok = dword && (E <= 1 || N * row % 4 == 0) && N * row < (1ll << 31);
+    a.tabfast = a.tab_ok && tab == QMM_F32 && gs == 32 && K % 256 == 0;
   }
-  if (gemm2s_wanted(a, mode, bits)) return gemm2s_launch(a, mode, bits, st);
+  if (gemm2s_wanted(a, mode, bits)) {
+    const size_t prep = gemm2_workspace_bytes(R, K);
+    a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + prep);
+    gemm2s_plan(R, row_offsets ? E : 1, N, K, workspace_bytes > prep ? workspace_bytes - prep : 0, &a.tile_rows, &a.splits);
+    gemm2s_launch(a, mode, bits, st);
+    if (a.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, a.splits, nullptr, 1, out_idx, st);
+    return;
+  }
   const int mt = row_tile >= 256 ? 2 : 1;
   if (mode == QMM_MODE_MXFP4) launch2_mt<1, 4>(a, mt, st);
   else if (bits == 4) launch2_mt<0, 4>(a, mt, st);

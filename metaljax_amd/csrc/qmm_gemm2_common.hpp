@@ -6,6 +6,7 @@
 #include "qmm_common.hpp"
 
 namespace qmm {
+
 namespace g2 {
 
 constexpr int BN = 128, BK = 64;
@@ -43,7 +44,11 @@ struct Gemm2Args {
   int R, N, K, E, Rp;
   int gs, tab, y_dtype;
   int m_tiles;
-  int tabfast;           // table rows are dword-aligned: fetch them as 16-byte windows
+  int tabfast;           // general kernel: float32 tables of groups of 32, fetched as windows
+  int tab_ok, tab_odd;   // split-role kernel: tables start on dwords; their rows may start inside one
+  int tile_rows;         // split-role kernel: rows a tile may hold (128 or 256)
+  int splits;            // split-role kernel, dense: workgroups that share a tile's K ...
+  float* part;           // ... and leave their float32 sums here, [splits][R][N]
 };
 
 // How the tiles of a grouped product are dealt to the eight XCDs (workgroup
@@ -65,10 +70,34 @@ __device__ __forceinline__ void deal_grouped_tile(int n_tiles, int xcd, int l, i
   }
 }
 
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+
+// fma(scale, q, bias) of small integer codes without converting them: a code in
+// the low bits of a half word is the float16 denormal q * 2^-24 (a nibble
+// further up q * 2^-20), v_fma_mix_f32 takes that as an operand, and with the
+// scale times 2^24 (2^20) -- exact -- it is the same product with the same one
+// rounding, one instruction a code.  Eight four-bit codes take 17 vector
+// instructions this way instead of 23, four eight-bit ones 9 instead of 10.
+__device__ __forceinline__ u32x4 dequant_nibbles(uint32_t w, float s24, float s20, float bi) {
+  const uint32_t w8 = w >> 8;
+  const f16x2 a = __builtin_bit_cast(f16x2, w & 0x000F000Fu), b = __builtin_bit_cast(f16x2, w & 0x00F000F0u);
+  const f16x2 c = __builtin_bit_cast(f16x2, w8 & 0x000F000Fu), d = __builtin_bit_cast(f16x2, w8 & 0x00F000F0u);
+  const float f0 = fmaf((float)a[0], s24, bi), f4 = fmaf((float)a[1], s24, bi);
+  const float f1 = fmaf((float)b[0], s20, bi), f5 = fmaf((float)b[1], s20, bi);
+  const float f2 = fmaf((float)c[0], s24, bi), f6 = fmaf((float)c[1], s24, bi);
+  const float f3 = fmaf((float)d[0], s20, bi), f7 = fmaf((float)d[1], s20, bi);
+  return u32x4{pack_bf16x2(f0, f1), pack_bf16x2(f2, f3), pack_bf16x2(f4, f5), pack_bf16x2(f6, f7)};
+}
+__device__ __forceinline__ u32x2 dequant_bytes(uint32_t w, float s24, float bi) {
+  const f16x2 a = __builtin_bit_cast(f16x2, w & 0x00FF00FFu), b = __builtin_bit_cast(f16x2, (w >> 8) & 0x00FF00FFu);
+  const float f0 = fmaf((float)a[0], s24, bi), f2 = fmaf((float)a[1], s24, bi);
+  const float f1 = fmaf((float)b[0], s24, bi), f3 = fmaf((float)b[1], s24, bi);
+  return u32x2{pack_bf16x2(f0, f1), pack_bf16x2(f2, f3)};
+}
+
 // 32 codes (one row, one 32-group) -> four 16-byte pieces of bf16 weights
 template <int MODE, int BITS>
 __device__ __forceinline__ u32x4 dequant_piece(const uint32_t* q, int pc, float sc, float bi) {
-  float f[8];
   if constexpr (MODE == 1) {
     // exact: the converter widens the two codes of a byte and applies the power-of-two scale
     const uint32_t w = q[pc];
@@ -77,27 +106,11 @@ __device__ __forceinline__ u32x4 dequant_piece(const uint32_t* q, int pc, float 
                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 2)),
                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3))};
   } else if constexpr (BITS == 8) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t w = q[2 * pc + h];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) f[4 * h + j] = fmaf(sc, (float)((w >> (8 * j)) & 255u), bi);
-    }
+    const u32x2 lo = dequant_bytes(q[2 * pc], sc * 16777216.f, bi), hi = dequant_bytes(q[2 * pc + 1], sc * 16777216.f, bi);
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
   } else {
-    const uint32_t w = q[pc];
-    uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;           // even / odd codes as bytes
-    // kept opaque, so that each code is one byte-to-float conversion of lo / hi
-    // (merged with the masks above they become a bit-field extract plus a conversion)
-    asm("" : "+v"(lo));
-    asm("" : "+v"(hi));
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f[2 * j] = fmaf(sc, (float)((lo >> (8 * j)) & 255u), bi);
-      f[2 * j + 1] = fmaf(sc, (float)((hi >> (8 * j)) & 255u), bi);
-    }
+    return dequant_nibbles(q[pc], sc * 16777216.f, sc * 1048576.f, bi);
   }
-  return u32x4{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]),
-               pack_bf16x2(f[6], f[7])};
 }
 
 }  // namespace g2

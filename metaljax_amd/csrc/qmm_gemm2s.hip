@@ -42,7 +42,6 @@ namespace {
 using namespace g2;
 
 constexpr int kS = 3;                 // LDS stages: K-tile t lives in stage t % 3
-constexpr int kTileRows = 256;        // eight row blocks, two a consumer
 constexpr int kAR = 3;                // activation fragments: K-tile t lives in ring slot t % 3 (t % 2 on full tiles)
 
 // Table rows staged in LDS (a row's scales / biases of the whole K when they
@@ -53,7 +52,8 @@ constexpr int kTabKind = BN * kTabRow;
 // TLDS: a tile's table rows are fetched once, into LDS (each row's line comes
 // in once instead of once per four K-tiles); otherwise 16-byte windows per
 // four K-tiles in registers.
-template <int MODE, int BITS, bool G64, bool TLDS>
+// TAB: the tables' type (MXFP4: QMM_BF16, unused).
+template <int MODE, int BITS, int TAB, bool G64, bool TLDS>
 __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
   static_assert(!G64 || MODE == 0, "one group a K-tile is an affine layout");
   constexpr int WBITS = (MODE == 1) ? 4 : BITS;
@@ -71,28 +71,35 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
   const int xcd = blockIdx.x & 7, l = blockIdx.x >> 3;
   int tile_m, tile_n;
   deal_grouped_tile(n_tiles, xcd, l, tile_m, tile_n);
-  int e = 0, row_lo = 0, row_hi = a.R, mt_idx = 0;
+  int e = 0, row_lo = 0, row_hi = a.R, mt_idx = 0, split = 0;
   if (!a.row_offsets) {
     // one expert of all rows: an eighth of the grid takes a contiguous run of
     // tiles, column tile fastest, so its workgroups share few activation rows
-    const int m_tiles = (a.R + kTileRows - 1) / kTileRows;
-    const int total = n_tiles * m_tiles, per = (total + 7) / 8;
+    // (and the workgroups that share a tile's K come one K range after the other)
+    const int m_tiles = (a.R + a.tile_rows - 1) / a.tile_rows;
+    const int tiles = n_tiles * m_tiles, total = tiles * a.splits, per = (total + 7) / 8;
     const int t = xcd * per + l;
     if (l >= per || t >= total) return;
-    tile_m = t / n_tiles;
-    tile_n = t % n_tiles;
+    split = t / tiles;
+    tile_m = (t - split * tiles) / n_tiles;
+    tile_n = (t - split * tiles) % n_tiles;
     mt_idx = tile_m;
   } else {
     if (tile_n >= n_tiles) return;
-    const RowTile rt = find_row_tile(a.row_offsets, a.E, a.R, kTileRows, tile_m);
+    const RowTile rt = find_row_tile(a.row_offsets, a.E, a.R, a.tile_rows, tile_m);
     if (!rt.found) return;
     e = rt.e; row_lo = rt.lo; row_hi = rt.hi; mt_idx = rt.idx;
   }
-  const int m0 = row_lo + mt_idx * kTileRows;
+  const int m0 = row_lo + mt_idx * a.tile_rows;
   if (m0 >= row_hi) return;
-  const int m_end = row_hi < m0 + kTileRows ? row_hi : m0 + kTileRows;
+  const int m_end = row_hi < m0 + a.tile_rows ? row_hi : m0 + a.tile_rows;
   const int n0 = tile_n * BN;
-  const int KT = a.K / BK;
+  // This workgroup's K-tiles: KT of them from kb on, a multiple of four (whole
+  // quads); K-tile numbers below count from kb.
+  const int KA = a.K / BK, quads = (KA + 3) / 4;
+  const int kb = a.splits == 1 ? 0 : quads * split / a.splits * 4;
+  const int ke = a.splits == 1 ? KA : quads * (split + 1) / a.splits * 4;
+  const int KT = (ke < KA ? ke : KA) - kb;
   auto clampk = [&](int kt) { return kt < KT ? kt : KT - 1; };
 
   if (wave >= 4) {
@@ -102,7 +109,7 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     const int64_t wpr = (int64_t)a.K * WBITS / 32;
     const int gs = (MODE == 1) ? 32 : a.gs;
     const int64_t ng = a.K / gs;
-    constexpr int tabsz = (MODE == 1) ? 1 : 2;     // E8M0 bytes | bf16
+    constexpr int tabsz = (MODE == 1) ? 1 : (TAB == QMM_F32 ? 4 : 2);     // E8M0 bytes | float32 | 16-bit
     const uint32_t* wb = a.w + (int64_t)e * a.N * wpr;
     const char* sb = static_cast<const char*>(a.s) + (int64_t)e * a.N * ng * tabsz;
     const char* bb = (MODE == 1) ? sb : static_cast<const char*>(a.b) + (int64_t)e * a.N * ng * tabsz;
@@ -112,7 +119,7 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     const uint32_t wvo = (uint32_t)((wn_row * wpr + whalf * WPT) * 4);
     struct WRegs { uint32_t q[WPT]; };
     auto load_w = [&](int kt, WRegs& r) {
-      const uint32_t so = (uint32_t)kt * (BK * WBITS / 8);
+      const uint32_t so = (uint32_t)(kb + kt) * (BK * WBITS / 8);
 #pragma unroll
       for (int j = 0; j < WPT; j += 4) {
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo + j * 4, so, 0);
@@ -120,20 +127,48 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
       }
     };
     // scale / bias window: the entries of four K-tiles of this thread's row
-    // (at most 16 bytes a table), fetched once per four K-tiles
+    // (at most 16 bytes a table), fetched once per four K-tiles.  Where rows may
+    // start inside a dword (tab_odd) a dword more is fetched and the window is
+    // shifted into place.
     struct TabWin { u32x4 s, b; };
-    const auto rs = make_rsrc(sb, (int64_t)a.N * ng * tabsz);
-    const auto rb = make_rsrc(bb, (int64_t)a.N * ng * tabsz);
+    const int64_t tbytes = ((int64_t)a.N * ng * tabsz + 3) / 4 * 4;
+    const auto rs = make_rsrc(sb, tbytes);
+    const auto rb = make_rsrc(bb, tbytes);
     const uint32_t tvo = (uint32_t)(wn_row * ng * tabsz);
     const int gshift = gs == 32 ? 5 : (gs == 64 ? 6 : 7);
-    auto load_win = [&](int quad, TabWin& tw) {
-      const uint32_t so = (uint32_t)(((quad * 4 * BK) >> gshift) * tabsz);
-      tw.s = __builtin_amdgcn_raw_buffer_load_b128(rs, tvo, so, 0);
-      if constexpr (MODE == 0) tw.b = __builtin_amdgcn_raw_buffer_load_b128(rb, tvo, so, 0);
+    struct RawWin { u32x4 s, b; uint32_t xs, xb, mis; } rawn;
+    auto load_win = [&](int quad, RawWin& r) {
+      const uint32_t so = (uint32_t)((((kb + quad * 4) * BK) >> gshift) * tabsz);
+      const uint32_t at = tvo + so, al = at & ~3u;
+      r.s = __builtin_amdgcn_raw_buffer_load_b128(rs, al, 0, 0);
+      if constexpr (MODE == 0) r.b = __builtin_amdgcn_raw_buffer_load_b128(rb, al, 0, 0);
+      if constexpr (tabsz < 4) {
+        if (a.tab_odd) {
+          r.mis = (at & 3u) * 8;
+          r.xs = __builtin_amdgcn_raw_buffer_load_b32(rs, al + 16, 0, 0);
+          if constexpr (MODE == 0) r.xb = __builtin_amdgcn_raw_buffer_load_b32(rb, al + 16, 0, 0);
+        }
+      }
+    };
+    auto settle_win = [&](const RawWin& r, TabWin& tw) {
+      tw.s = r.s;
+      if constexpr (MODE == 0) tw.b = r.b;
+      if constexpr (tabsz < 4) {
+        if (a.tab_odd) {
+          tw.s = u32x4{__builtin_amdgcn_alignbit(r.s[1], r.s[0], r.mis), __builtin_amdgcn_alignbit(r.s[2], r.s[1], r.mis),
+                       __builtin_amdgcn_alignbit(r.s[3], r.s[2], r.mis), __builtin_amdgcn_alignbit(r.xs, r.s[3], r.mis)};
+          if constexpr (MODE == 0)
+            tw.b = u32x4{__builtin_amdgcn_alignbit(r.b[1], r.b[0], r.mis), __builtin_amdgcn_alignbit(r.b[2], r.b[1], r.mis),
+                         __builtin_amdgcn_alignbit(r.b[3], r.b[2], r.mis), __builtin_amdgcn_alignbit(r.xb, r.b[3], r.mis)};
+        }
+      }
     };
     uint32_t eidx[4];                              // entry of K-tile t' inside its window, for this thread's half
 #pragma unroll
     for (int t = 0; t < 4; ++t) eidx[t] = (uint32_t)((t * BK + whalf * 32) >> gshift);
+    auto widen = [&](uint32_t v) -> float {        // a 16-bit entry (in the low half)
+      return TAB == QMM_F16 ? f16_bits_to_f32(v & 0xFFFFu) : __uint_as_float(v << 16);
+    };
     auto pick = [&](const u32x4& w, uint32_t ei) -> float {
       const uint32_t byte = ei * (uint32_t)tabsz;
       const uint32_t d = byte >> 2;
@@ -141,26 +176,35 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
       v = d == 1 ? w[1] : v;
       v = d == 2 ? w[2] : v;
       v = d == 3 ? w[3] : v;
+      if constexpr (tabsz == 4) return __uint_as_float(v);
       v >>= (byte & 3u) * 8u;
       if constexpr (MODE == 1) return e8m0_to_f32(v & 255u);
-      return __uint_as_float(v << 16);
+      return widen(v);
     };
     unsigned char* tabs = smem + kS * kStage + wrow * kTabRow;
+    const uint32_t tmis = tvo & 3u;                // staged rows start on a dword as well
     auto entry = [&](int kt, auto tqc, const TabWin& tw, float& sc, float& bi) {
       constexpr int tq = decltype(tqc)::value;
       if constexpr (TLDS) {
-        const int ei = (kt * BK + whalf * 32) >> gshift;
+        const unsigned char* p = tabs + tmis + (((kb + kt) * BK + whalf * 32) >> gshift) * tabsz;
         if constexpr (MODE == 1) {
-          sc = e8m0_to_f32(tabs[ei]);
+          sc = e8m0_to_f32(*p);
           bi = 0.f;
+        } else if constexpr (tabsz == 4) {
+          sc = *reinterpret_cast<const float*>(p);
+          bi = *reinterpret_cast<const float*>(p + kTabKind);
         } else {
-          sc = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(tabs)[ei]);
-          bi = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(tabs + kTabKind)[ei]);
+          sc = widen(*reinterpret_cast<const uint16_t*>(p));
+          bi = widen(*reinterpret_cast<const uint16_t*>(p + kTabKind));
         }
       } else if constexpr (G64) {                          // one group a K-tile: entry tq for every thread
-        const uint32_t vs = tw.s[tq >> 1], vb = tw.b[tq >> 1];
-        sc = __uint_as_float((tq & 1) ? (vs & 0xFFFF0000u) : (vs << 16));
-        bi = __uint_as_float((tq & 1) ? (vb & 0xFFFF0000u) : (vb << 16));
+        if constexpr (tabsz == 4) {
+          sc = __uint_as_float(tw.s[tq]);
+          bi = __uint_as_float(tw.b[tq]);
+        } else {
+          sc = widen((tq & 1) ? tw.s[tq >> 1] >> 16 : tw.s[tq >> 1]);
+          bi = widen((tq & 1) ? tw.b[tq >> 1] >> 16 : tw.b[tq >> 1]);
+        }
       } else {
         sc = pick(tw.s, eidx[tq]);
         bi = MODE == 1 ? 0.f : pick(tw.b, eidx[tq]);
@@ -200,12 +244,13 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t o = (uint32_t)(whalf * 64 + i * 16);
-        *reinterpret_cast<u32x4*>(tabs + o) = __builtin_amdgcn_raw_buffer_load_b128(rs, tvo + o, 0, 0);
+        *reinterpret_cast<u32x4*>(tabs + o) = __builtin_amdgcn_raw_buffer_load_b128(rs, (tvo & ~3u) + o, 0, 0);
         if constexpr (MODE == 0)
-          *reinterpret_cast<u32x4*>(tabs + kTabKind + o) = __builtin_amdgcn_raw_buffer_load_b128(rb, tvo + o, 0, 0);
+          *reinterpret_cast<u32x4*>(tabs + kTabKind + o) = __builtin_amdgcn_raw_buffer_load_b128(rb, (tvo & ~3u) + o, 0, 0);
       }
     } else {
-      load_win(0, tw_cur);
+      load_win(0, rawn);
+      settle_win(rawn, tw_cur);
     }
     load_quad(0, std::integral_constant<int, 0>{});
     load_quad(4, std::integral_constant<int, 4>{});
@@ -233,9 +278,10 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
         load_quad(kt + 8, std::integral_constant<int, (t12 + 8) % 12>{});
         if constexpr (!TLDS) {
           const int q = (kt >> 2) + 1;              // next quad's windows (clamped at the end)
-          load_win(q * 4 < KT ? q : (kt >> 2), tw_nxt);
+          load_win(q * 4 < KT ? q : (kt >> 2), rawn);
         }
       }
+      if constexpr (!TLDS && t == 2) settle_win(rawn, tw_nxt);
       float sc, bi;
       entry(clampk(kt + 2), std::integral_constant<int, (t + 2) & 3>{}, t >= 2 ? tw_nxt : tw_cur, sc, bi);
       // the step's barrier as soon as the write has landed (the consumers reach
@@ -291,7 +337,7 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
   const uint32_t avo1 = avo + (uint32_t)(five ? (4 - wm) * 512 : 128 * 16);
   typedef u32x4 AFrag[4][2];
   auto load_a_part = [&](int kt, AFrag& dst, int ks, auto nac) __attribute__((always_inline)) {
-    const uint32_t so = (uint32_t)((kt * 8 + ks * 2) * 16) * (uint32_t)a.Rp;
+    const uint32_t so = (uint32_t)(((kb + kt) * 8 + ks * 2) * 16) * (uint32_t)a.Rp;
     dst[ks][0] = __builtin_amdgcn_raw_buffer_load_b128(ra, avo, so, 0);
     if constexpr (decltype(nac)::value == 2) dst[ks][1] = __builtin_amdgcn_raw_buffer_load_b128(ra, avo1, so, 0);
   };
@@ -411,7 +457,7 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
   // (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5), r = 0..15.  Block 0 is row block
   // w over all columns; block 1 the fifth block's column block w, or row
   // block w + 4 over all columns.
-  const bool wide = a.y_dtype != QMM_F32 && (a.N & 7) == 0 &&
+  const bool wide = a.y_dtype != QMM_F32 && (a.N & 7) == 0 && a.splits == 1 &&
                     (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0;
   if (wide) {
     // 16-bit outputs: transpose each 32-row block through this wavefront's
@@ -463,6 +509,10 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
         for (int r = 0; r < 16; ++r) {
           const int m = m0 + (i == 0 ? wm : (two ? wm + 4 : 4)) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh;
           if (m < m_end && n < a.N) {
+            if (a.splits > 1) {
+              a.part[((int64_t)split * a.R + m) * a.N + n] = i == 0 ? acc[j][r] : acc2[j][r];
+              continue;
+            }
             const int64_t orow = a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m;
             store_out(a.y, orow * a.N + n, i == 0 ? acc[j][r] : acc2[j][r], a.y_dtype);
           }
@@ -472,47 +522,91 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
   }
 }
 
-template <int MODE, int BITS, bool G64, bool TLDS>
+template <int MODE, int BITS, int TAB, bool G64, bool TLDS>
 void launch_k(const Gemm2Args& a, hipStream_t st) {
-  const int64_t m_tiles = ceil_div(a.R, kTileRows) + a.E;      // provisioned: a tile never straddles an expert
+  const int64_t m_tiles = ceil_div(a.R, a.tile_rows) + a.E;    // provisioned: a tile never straddles an expert
   int64_t total = ceil_div(ceil_div(a.N, BN), 8) * 8 * m_tiles;
-  if (!a.row_offsets) total = ceil_div(ceil_div(a.N, BN) * ceil_div(a.R, kTileRows), 8) * 8;
+  if (!a.row_offsets) total = ceil_div(ceil_div(a.N, BN) * ceil_div(a.R, a.tile_rows) * a.splits, 8) * 8;
   const size_t epi = (size_t)4 * 32 * BN * 2;
   const size_t need = (size_t)(kS * kStage) + (TLDS ? 2 * kTabKind : 0);
   const size_t lds = epi > need ? epi : need;
-  constexpr auto kern = gemm2s_kernel<MODE, BITS, G64, TLDS>;
+  constexpr auto kern = gemm2s_kernel<MODE, BITS, TAB, G64, TLDS>;
   if (!lds_limit<kern>(lds)) return;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(512), lds, st, a);
 }
 
-template <int MODE, int BITS, bool G64>
+template <int MODE, int BITS, int TAB, bool G64>
 void launch_s(const Gemm2Args& a, hipStream_t st) {
-  // a row's table of the whole K in one 128-byte line per kind?
-  const int64_t row_bytes = MODE == 1 ? a.K / 32 : (int64_t)(a.K / a.gs) * 2;
+  // a row's table of the whole K (and the up to three bytes a row may start into
+  // its first dword) in one 128-byte line per kind?
+  const int64_t row_bytes = (MODE == 1 ? a.K / 32 : (int64_t)(a.K / a.gs) * (TAB == QMM_F32 ? 4 : 2)) + (a.tab_odd ? 3 : 0);
   static const bool no_tlds = experiment_env("QMM_GEMM2S_NOTLDS") != nullptr;
-  if (row_bytes <= 128 && !no_tlds) launch_k<MODE, BITS, G64, true>(a, st);
-  else launch_k<MODE, BITS, G64, false>(a, st);
+  if (row_bytes <= 128 && !no_tlds) launch_k<MODE, BITS, TAB, G64, true>(a, st);
+  else launch_k<MODE, BITS, TAB, G64, false>(a, st);
+}
+
+template <int BITS, int TAB>
+void launch_a(const Gemm2Args& a, hipStream_t st) {
+  if (a.gs == 64) launch_s<0, BITS, TAB, true>(a, st);
+  else launch_s<0, BITS, TAB, false>(a, st);
+}
+
+template <int BITS>
+void launch_b(const Gemm2Args& a, hipStream_t st) {
+  if (a.tab == QMM_BF16) launch_a<BITS, QMM_BF16>(a, st);
+  else if (a.tab == QMM_F16) launch_a<BITS, QMM_F16>(a, st);
+  else launch_a<BITS, QMM_F32>(a, st);
 }
 
 }  // namespace
 
-// Products whose tables can be fetched as 16-byte windows of bf16 (E8M0 for
-// MXFP4) entries and whose K is a multiple of four K-tiles; everything else
-// stays on the general kernel.
+// Every product whose tables can be fetched as 16-byte windows (four K-tiles'
+// entries of a row: not float32 ones of groups of 32) from dword-aligned tables;
+// the rest stays on the general kernel.
 bool gemm2s_wanted(const g2::Gemm2Args& a, int mode, int bits) {
-  static const char* env = experiment_env("QMM_GEMM2S");   // "0": never, "2": short experts only
-  if (env && env[0] == '0') return false;
-  const bool can = (a.row_offsets ? a.E > 0 : a.E == 1) && a.tabfast && a.K % 256 == 0 &&
-                   (mode == QMM_MODE_MXFP4 || (a.tab == QMM_BF16 && (bits == 4 || bits == 8)));
-  if (!can) return false;
-  if (env && env[0] == '2') return a.row_offsets && a.R / a.E <= 144;
-  return true;
+  if (experiment_env("QMM_GEMM2S") && experiment_env("QMM_GEMM2S")[0] == '0') return false;
+  return (a.row_offsets ? a.E > 0 : a.E == 1) && a.tab_ok &&
+         (mode == QMM_MODE_MXFP4 || ((bits == 4 || bits == 8) && !(a.tab == QMM_F32 && a.gs == 32)));
+}
+
+// Rows a tile may hold and workgroups that share its K: those that make the
+// product shortest.  Returns that time in microseconds, from a fit (within 7%
+// on average) to 700 measured products of 17 to 2048 rows, N and K 1024 to
+// 14336: the launches, a round for every 256 tiles (one workgroup fills a
+// compute unit), a K-tile of up to 128 or up to 256 rows, the re-laid
+// activations, the result, and a split K's sums.  The grouped product keeps
+// 256-row tiles (every expert in one, and the short loop where it fits) and its
+// whole K.
+double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits) {
+  const char* er = experiment_env("QMM_G2S_ROWS");
+  const char* es = experiment_env("QMM_G2S_SPLITS");
+  const int64_t kt = ceil_div(K, BK), quads = ceil_div(kt, 4), nt = ceil_div(N, BN), group = E > 1 ? ceil_div(R, E) : R;
+  double best = 1e30, least = 1e30;
+  *tile_rows = 256;
+  *splits = 1;
+  for (int rows = E > 1 ? 256 : 128; rows <= 256; rows += 128) {
+    // (ragged groups: a quarter more rows than their mean to be expected in one)
+    const int64_t mt = E > 1 ? E * ceil_div(group * 5 / 4, rows) : ceil_div(R, rows);
+    const bool half = rows == 128 || (E > 1 ? group * 5 / 4 : R) <= 128;
+    for (int s = 1; s <= (E > 1 ? 1 : 12); s = s < 6 ? s + 1 : s < 8 ? 8 : s + 4) {
+      if (s > 1 && (s > quads || (double)s * R * N * 4 > (double)part_bytes)) break;
+      const int64_t tiles = nt * mt * s;
+      const double step = (half ? 0.41 : 0.60) + 0.105 * (tiles < 256 ? tiles / 256.0 : 1.0);
+      const double us = 5.9 + (double)ceil_div(tiles, 256) * (2.5 + (s == 1 ? kt : 4 * ceil_div(quads, s)) * step) +
+                        (double)R * K * 0.54e-6 + (double)R * N * 0.5e-6 + (s > 1 ? 4.6 + (double)s * R * N * 1.4e-6 : 0.0);
+      double cost = us * (1.0 + 0.01 * s);       // (of two alike the one with fewer splits)
+      if (er && E <= 1 && atoi(er) != rows) cost += 1e9;
+      if (es && E <= 1 && atoi(es) != s) cost += 1e9;
+      if (cost < best) { best = cost; least = us; *tile_rows = rows; *splits = s; }
+    }
+  }
+  return least;
 }
 
 void gemm2s_launch(const g2::Gemm2Args& a, int mode, int bits, hipStream_t st) {
-  if (mode == QMM_MODE_MXFP4) launch_s<1, 4, false>(a, st);
-  else if (bits == 4) { if (a.gs == 64) launch_s<0, 4, true>(a, st); else launch_s<0, 4, false>(a, st); }
-  else { if (a.gs == 64) launch_s<0, 8, true>(a, st); else launch_s<0, 8, false>(a, st); }
+  if (mode == QMM_MODE_MXFP4) launch_s<1, 4, QMM_BF16, false>(a, st);
+  else if (bits == 4) launch_b<4>(a, st);
+  else launch_b<8>(a, st);
 }
 
 }  // namespace qmm

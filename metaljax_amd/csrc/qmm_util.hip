@@ -165,6 +165,47 @@ __global__ void sum_terms_kernel(const float* __restrict__ part, void* __restric
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)ceil_div(n, kBlock); }
 
+// y = the splits' sums, added in order and rounded once.  Rows that no expert
+// covers hold nothing and are left alone.  Four columns a thread (V = 4: N a
+// multiple of four), else one.
+template <int V>
+__global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ part, void* __restrict__ y,
+                                                        int y_dtype, int R, int N, int splits,
+                                                        const int32_t* __restrict__ row_offsets, int E,
+                                                        const int32_t* __restrict__ out_idx) {
+  const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * V;    // (R * N < 2^31: a K is only split where tiles are few)
+  if (i >= (uint32_t)R * (uint32_t)N) return;
+  const int m = (int)(i / (uint32_t)N);
+  if (row_offsets && (m < row_offsets[0] || m >= row_offsets[E])) return;
+  const int64_t at = (out_idx ? (int64_t)out_idx[m] : (int64_t)m) * N + (i - (uint32_t)m * (uint32_t)N);
+  float v[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = 0.f;
+#pragma unroll 4
+  for (int z = 0; z < splits; ++z) {
+    const float* p = part + (int64_t)z * R * N + i;
+    if constexpr (V == 4) {
+      const f32x4 q = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += q[j];
+    } else {
+      v[0] += p[0];
+    }
+  }
+  if constexpr (V == 4) {
+    if (y_dtype == QMM_F32) {
+      *reinterpret_cast<f32x4*>(static_cast<float*>(y) + at) = f32x4{v[0], v[1], v[2], v[3]};
+    } else {
+      u32x2 h;
+      if (y_dtype == QMM_BF16) h = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      else h = u32x2{f32_to_f16_bits(v[0]) | (f32_to_f16_bits(v[1]) << 16), f32_to_f16_bits(v[2]) | (f32_to_f16_bits(v[3]) << 16)};
+      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(y) + at) = h;
+    }
+  } else {
+    store_out(y, at, v[0], y_dtype);
+  }
+}
+
 }  // namespace
 
 void unpack_dispatch(const void* w, void* codes, int64_t rows, int64_t K, int bits,
@@ -245,6 +286,14 @@ void take_dispatch(const void* x, int x_dtype, const int32_t* perm, void* out, i
     hipLaunchKernelGGL(take_kernel<uint32_t>, dim3(blocks_for(n)), dim3(kBlock), 0, st, static_cast<const uint32_t*>(x), perm, static_cast<uint32_t*>(out), rows, K);
   else
     hipLaunchKernelGGL(take_kernel<uint16_t>, dim3(blocks_for(n)), dim3(kBlock), 0, st, static_cast<const uint16_t*>(x), perm, static_cast<uint16_t*>(out), rows, K);
+}
+
+void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,
+                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, hipStream_t st) {
+  const bool v4 = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+  const dim3 grid((unsigned)ceil_div(R * N, 256 * (v4 ? 4 : 1)));
+  if (v4) hipLaunchKernelGGL(split_sum_kernel<4>, grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
+  else hipLaunchKernelGGL(split_sum_kernel<1>, grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
 }
 
 }  // namespace qmm

@@ -1,0 +1,75 @@
+"""The prefill products that split K over workgroups or take short row groups,
+at the edges of their tiles: rows round the sixteens and the 128 / 256 of a
+row tile, columns that end inside a tile, a K that ends inside a step, table
+rows that start inside a dword, groups without rows.  The reference is a plain
+product of the bf16 weight tile in double precision (MXFP4 tiles are exact)."""
+
+import pytest
+import torch
+
+from metaljax_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+ACT = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
+# (bits, group_size, mode, tables)
+KINDS = [(4, 64, "affine", "bf16"), (4, 32, "affine", "f16"), (4, 128, "affine", "f32"), (8, 64, "affine", "bf16"),
+         (8, 32, "affine", "f32"), (4, 32, "mxfp4", None)]
+
+
+def weight(g, lead, n, k, bits, gs, mode, tab):
+    w = torch.randint(-2**31, 2**31 - 1, lead + (n, k * bits // 32), dtype=torch.int32, device=DEV, generator=g)
+    if mode == "mxfp4":
+        return w, torch.randint(118, 130, lead + (n, k // 32), dtype=torch.uint8, device=DEV, generator=g), None
+    s = torch.rand(lead + (n, k // gs), device=DEV, generator=g) * 0.02 + 0.005
+    b = -s * torch.rand(s.shape, device=DEV, generator=g) * (1 << bits)
+    return w, s.to(ACT[tab]), b.to(ACT[tab])
+
+
+def tile(w, s, b, how):
+    return K.dequantize(w, s, b, out_dtype=torch.float32, **how).bfloat16().double()
+
+
+def close(y, want):
+    err = ((y.double() - want).norm() / want.norm()).item()
+    assert err <= 2e-5, err
+
+
+# few rows or few columns: the short-group kernel; many: the prefill kernel with 128- and 256-row tiles, its K split
+@pytest.mark.parametrize("m,n,k", [(17, 64, 64), (33, 130, 320), (65, 65, 448), (48, 1000, 2112), (128, 333, 4096),
+                                   (200, 4104, 8192), (300, 9208, 2944), (513, 2056, 1088)])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("act", ["bf16", "f16", "f32"])
+def test_dense(m, n, k, kind, act):
+    bits, gs, mode, tab = kind
+    if k % gs or (mode == "mxfp4" and k % 512 == 0 and act == "bf16"):     # (the latter: the FP6 kernel's tolerance)
+        pytest.skip("not a shape of these kernels")
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (), n, k, bits, gs, mode, tab)
+    x = torch.randn((m, k), device=DEV, generator=g).to(ACT[act])
+    close(K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how), x.double() @ tile(w, s, b, how).T)
+
+
+@pytest.mark.parametrize("counts", [(0, 1, 16, 0, 17), (40, 0, 3, 70, 64), (90, 129, 0, 161, 300)])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_groups(counts, kind, act, gathered):
+    bits, gs, mode, tab = kind
+    n, k = 520, 1088 if gs < 128 else 1152
+    g = torch.Generator(device=DEV).manual_seed(sum(counts))
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (len(counts),), n, k, bits, gs, mode, tab)
+    x = torch.randn((sum(counts), k), device=DEV, generator=g).to(ACT[act])
+    owner = torch.repeat_interleave(torch.arange(len(counts), device=DEV), torch.tensor(counts, device=DEV))
+    want = torch.cat([x[owner == e].double() @ tile(w[e], s[e], None if b is None else b[e], how).T for e in range(len(counts))])
+    if not gathered:
+        ro = torch.tensor([sum(counts[:e]) for e in range(len(counts) + 1)], dtype=torch.int32, device=DEV)
+        close(K.grouped_qmm(x, w, s, b, ro, out_dtype=torch.float32, **how), want)
+    elif sum(counts) > 64:                                              # (fewer pairs: decode kernels, exact weights)
+        mix = torch.randperm(sum(counts), device=DEV, generator=g)
+        y = K.gather_qmm(x, w, s, b, mix.int(), owner[mix].int(), out_dtype=torch.float32, **how)
+        if sum(counts) > 16 * len(counts):
+            close(y, want[mix])
