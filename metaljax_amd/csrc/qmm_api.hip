@@ -43,9 +43,21 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
                     int64_t K, int gs, int bits, int mode, int row_tile, void* workspace,
                     size_t workspace_bytes, hipStream_t st);
 double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits);
+double gemm2_us(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes);
 size_t gemm2_split_workspace_bytes(int64_t R, int64_t N, int64_t K);
+bool short_supported(int64_t R, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab, int terms,
+                     const void* s, const void* b);
+double short_us(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, size_t part_bytes);
+void short_geometry(int64_t R, int64_t N, int64_t K, int bits, int mode, int* grid);
+size_t short_prep_bytes(int64_t R, int64_t K, int terms);
+size_t short_workspace_bytes(int64_t R, int64_t N, int64_t K, int bits, int mode, int terms);
+void short_dispatch(const void* x, int x_dtype, const void* w, const void* s, const void* b, int tab, void* y,
+                    int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx, const int32_t* out_idx, int64_t R,
+                    int64_t x_rows, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, void* workspace,
+                    size_t workspace_bytes, hipStream_t st);
 bool mxfp4_mfma_supported(int64_t R, int64_t N, int64_t K);
 size_t mxfp4_workspace_bytes(int64_t R, int64_t K);
+double mxfp4_us(int64_t R, int64_t E, int64_t N, int64_t K);
 void mxfp4_geometry(int64_t R, int64_t N, int64_t K, int* grid, int* block);
 void mxfp4_mfma_dispatch(const void* x, const void* w, const void* s, void* y, int y_dtype,
                          const int32_t* row_offsets, const int32_t* lhs_idx,
@@ -240,6 +252,30 @@ size_t dense_scratch_split(int64_t rows, int64_t N, int64_t K, int mode, bool ex
   return std::max(least, gemm2_split_workspace_bytes(rows, N, K));
 }
 
+// Is the short-group kernel the one to take?  `E` experts share the R rows (1:
+// dense), the activations are `terms` bf16 terms.  All kernels' times have been
+// fitted over the shapes they serve; where they come close the choice matters
+// little.  (4096 x 4096, four-bit codes: 17 rows 13 against 20 us of the
+// prefill kernel, 128 rows 19 against 23, 512 rows 32 against 36; 14336 x 4096:
+// 19 against 29, 32 against 33, 108 against 59.)
+bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms) {
+  if (K % 64 || N <= 0) return false;
+  if (const char* env = experiment_env("QMM_SHORT")) return env[0] != '0';
+  double other;
+  if (mode == QMM_MODE_MXFP4 && terms == 1 && mxfp4_mfma_supported(R, N, K)) {
+    if (N < 512) return false;                   // (a few column tiles: not measured, left as it is)
+    other = mxfp4_us(R, E, N, K);
+  }
+  else if (E > 1) other = terms * gemm2_us(R, E, N, K, 0) + (terms > 1 ? 5.2 + (double)terms * R * N * 1.4e-6 : 0.0);
+  else other = gemm2_us(terms * R, 1, N, K, ~(size_t)0) + (terms > 1 ? 5.2 + (double)terms * R * N * 1.4e-6 : 0.0);
+  return short_us(R, E, N, K, bits, mode, terms, ~(size_t)0) < other;
+}
+
+// Scratch that lets a short-group product over R rows run as it would best.
+size_t short_scratch(int64_t R, int64_t N, int64_t K, int bits, int mode, int terms) {
+  return R > 0 && R <= 4096 && N > 0 && K > 0 && K % 64 == 0 && terms * R > kGemvMaxM ? short_workspace_bytes(R, N, K, bits, mode, terms) : 0;
+}
+
 size_t gather_scratch(int64_t P, int64_t E, int64_t N, int64_t K, bool exact) {
   if (P < kGroupedDecodeMinPairs) return 0;
   const size_t decode = grouped_decode_pairs(P, E) ? route_bytes_segments(P, E) : 0;
@@ -292,19 +328,22 @@ int qmm_abi_version(void) { return 2; }
 
 const char* qmm_last_error(void) { return g_err; }
 
-size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int, int, int mode,
+size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int, int bits, int mode,
                            int x_dtype) {
   const int terms = act_terms(x_dtype);
-  if (terms == 1) return dense_scratch_split(M, N, K, mode, false);
+  const size_t sh = short_scratch(M, N, K, bits, mode, terms);
+  if (terms == 1) return std::max(sh, dense_scratch_split(M, N, K, mode, false));
   // terms as bf16 rows, their float32 products, then the scratch of the bf16
   // product: over terms x M stacked rows (dense) or over M rows (grouped)
   if (batch < 1) batch = 1;
   const size_t stacked = dense_scratch_split(terms * M, N, K, mode, true), plain = dense_scratch(M, N, K, mode, true);
-  return align256((size_t)(batch * terms * M * K) * 2) + align256((size_t)(batch * terms * M * N) * 4) +
-         (stacked > plain ? stacked : plain);
+  return std::max(sh, align256((size_t)(batch * terms * M * K) * 2) + align256((size_t)(batch * terms * M * N) * 4) +
+                          std::max(stacked, plain));
 }
 
-size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, int x_dtype) {
+// What a gathered product needs to run at all on its preferred kernels, without
+// the sums of a split K (those it takes only where there is room).
+static size_t gather_minimum(int64_t P, int64_t E, int64_t N, int64_t K, int x_dtype) {
   const int terms = act_terms(x_dtype);
   if (terms == 1) return gather_scratch(P, E, N, K, false);
   // the gathered rows' terms, their float32 products, the bf16 product's scratch
@@ -312,8 +351,23 @@ size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, in
          gather_scratch(P, E, N, K, true);
 }
 
+size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, int x_dtype) {
+  const int terms = act_terms(x_dtype);
+  const size_t sh = P > kGatherGemvMaxPairs ? route_bytes(P, E) + 
+                                                                  std::max(short_scratch(P, N, K, 4, QMM_MODE_AFFINE, terms), short_scratch(P, N, K, 8, QMM_MODE_AFFINE, terms)) : 0;
+  return std::max(sh, gather_minimum(P, E, N, K, x_dtype));
+}
+
 int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode, int* kernel,
              int* grid, int* block) {
+  if (M > kGemvMaxM && short_wins(M, 1, N, K, bits, mode, 1)) {     // (bf16 activations and tables assumed)
+    int g;
+    short_geometry(M, N, K, bits, mode, &g);
+    if (kernel) *kernel = QMM_KERNEL_GEMM;
+    if (grid) *grid = g;
+    if (block) *block = 512;
+    return QMM_OK;
+  }
   if (mode == QMM_MODE_MXFP4 && M > kGemvMaxM && mxfp4_mfma_supported(M, N, K)) {
     int g, b;
     mxfp4_geometry(M, N, K, &g, &b);
@@ -366,6 +420,29 @@ int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode
     if (block) *block = 256;
   }
   return QMM_OK;
+}
+
+// One product on the short-group kernel if it serves it, arguments and scratch
+// included: true when it was launched (*rc: the launches' status), false when
+// the other kernels are to take it (or to say what is wrong with it).
+static bool ran_short(const void* x, int x_dtype, const void* w, const void* scales, const void* biases,
+                      int table_dtype, void* y, int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
+                      const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N, int64_t K,
+                      int group_size, int bits, int mode, void* workspace, size_t workspace_bytes, void* stream,
+                      int* rc) {
+  const int terms = act_terms(x_dtype);
+  if (R <= 0 || E <= 0 || N <= 0 || K <= 0 || terms * R <= kGemvMaxM || R > INT32_MAX / 2 || N > INT32_MAX ||
+      K > INT32_MAX || E > 65535 || !short_wins(R, E, N, K, bits, mode, terms))
+    return false;
+  if (check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases) || check_io(x, x_dtype, y, y_dtype) ||
+      !workspace || !aligned16(workspace) || workspace_bytes < short_prep_bytes(R, K, terms) ||
+      !short_supported(R, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : group_size, bits, mode, table_dtype, terms, scales, biases))
+    return false;
+  short_dispatch(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, lhs_idx, out_idx, R, x_rows, E, N,
+                 K, mode == QMM_MODE_MXFP4 ? 32 : group_size, bits, mode, workspace, workspace_bytes,
+                 static_cast<hipStream_t>(stream));
+  *rc = check_launch("short-group product launch");
+  return true;
 }
 
 // The three products on bf16 activations.  `exact`: the activations are exact
@@ -555,6 +632,9 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
                      ro, cursor, src_row, out_row, static_cast<int32_t*>(nullptr));
   rc = check_launch("route launch");
   if (rc) return rc;
+  if (ran_short(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K, group_size,
+                bits, mode, static_cast<char*>(workspace) + need, workspace_bytes - need, stream, &rc))
+    return rc;
   if (mode == QMM_MODE_MXFP4 && !exact && mxfp4_mfma_supported(P, N, K) &&
       workspace_bytes >= need + mxfp4_workspace_bytes(P, K) && aligned16(workspace) &&
       aligned16(scales)) {
@@ -581,6 +661,21 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
                          int bits, int mode, void* workspace, size_t workspace_bytes,
                          void* stream) {
   const int terms = act_terms(x_dtype);
+  if (batch > 0 && batch <= 65535 && M > 0 && N > 0 && K > 0 && terms * M > kGemvMaxM && x && w && scales && y) {
+    const size_t xb = (size_t)M * K * (x_dtype == QMM_F32 ? 4 : 2), yb = (size_t)M * N * (y_dtype == QMM_F32 ? 4 : 2);
+    const size_t wb = (size_t)N * (K * (mode == QMM_MODE_MXFP4 ? 4 : bits) / 8);
+    const size_t tb = mode == QMM_MODE_MXFP4 ? (size_t)N * (K / 32) : (size_t)N * (K / std::max(group_size, 1)) * (table_dtype == QMM_F32 ? 4 : 2);
+    int rc = QMM_OK;
+    int64_t z = 0;
+    for (; z < batch; ++z)
+      if (!ran_short(static_cast<const char*>(x) + z * xb, x_dtype, static_cast<const char*>(w) + z * wb,
+                     static_cast<const char*>(scales) + z * tb, biases ? static_cast<const char*>(biases) + z * tb : nullptr,
+                     table_dtype, static_cast<char*>(y) + z * yb, y_dtype, nullptr, nullptr, nullptr, M, M, 1, N, K,
+                     group_size, bits, mode, workspace, workspace_bytes, stream, &rc) || rc)
+        break;
+    if (z == batch || rc) return rc;
+    // (batch entries differ in their tables' alignment alone: the ones that ran are computed again below)
+  }
   if (terms == 1 || batch <= 0 || M <= 0 || N <= 0 || K <= 0 || !x)
     return dense_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, batch, M, N, K,
                       group_size, bits, mode, workspace, workspace_bytes, stream, false);
@@ -613,6 +708,10 @@ int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scale
                     int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
                     void* stream) {
   const int terms = act_terms(x_dtype);
+  int rs = QMM_OK;
+  if (row_offsets && ran_short(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, nullptr, nullptr, R,
+                               R, E, N, K, group_size, bits, mode, workspace, workspace_bytes, stream, &rs))
+    return rs;
   if (terms == 1 || R <= 0 || E <= 0 || N <= 0 || K <= 0 || !x || !row_offsets || !y)
     return grouped_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, R, E, N, K,
                         group_size, bits, mode, workspace, workspace_bytes, stream, false);
@@ -645,6 +744,27 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   if (terms == 1 || P <= 0 || T < 0 || E < 0 || N <= 0 || K <= 0 || !x || !rhs_idx || !y)
     return gather_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, lhs_idx, rhs_idx, P, T, E,
                        N, K, group_size, bits, mode, workspace, workspace_bytes, stream, false);
+  // more pairs than the decode kernels take: short groups read float16 / float32
+  // activations as they are
+  if (P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
+      short_wins(P, E, N, K, bits, mode, terms) && workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
+      short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, terms, scales, biases)) {
+    const size_t need = route_bytes(P, E);
+    int32_t* ro = static_cast<int32_t*>(workspace);
+    int32_t* cursor = ro + E + 1;
+    int32_t* src_row = cursor + E;
+    int32_t* out_row = src_row + P;
+    int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
+    if (!rc) rc = check_io(x, x_dtype, y, y_dtype);
+    if (rc) return rc;
+    hipLaunchKernelGGL(route_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), lhs_idx, rhs_idx, (int)P,
+                       (int)E, ro, cursor, src_row, out_row, static_cast<int32_t*>(nullptr));
+    rc = check_launch("route launch");
+    if (rc) return rc;
+    if (ran_short(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K, group_size,
+                  bits, mode, static_cast<char*>(workspace) + need, workspace_bytes - need, stream, &rc))
+      return rc;
+  }
   // the pairs' rows are gathered while they are split; every term is then a
   // gathered product over rows already in pair order
   const size_t xs = align256((size_t)(terms * P * K) * 2), ps = align256((size_t)(terms * P * N) * 4);
@@ -672,7 +792,7 @@ int qmm_gather_qmm_static(const void* x, int x_dtype, const void* w, const void*
                           int64_t E, int64_t N, int64_t K, int group_size, int bits, int mode,
                           void* stream) {
   if (P < 0 || T < 0 || E < 0 || N < 0 || K < 0) return fail(QMM_ERR_BAD_ARGUMENT, "negative shape");
-  const size_t need = qmm_gather_workspace_bytes(P, E, N, K, x_dtype);
+  const size_t need = gather_minimum(P, E, N, K, x_dtype);
   if (need > (size_t)QMM_STATIC_SCRATCH_BYTES)
     return fail(QMM_ERR_WORKSPACE,
                 "gather_qmm_static: %lld pairs over %lld experts of [%lld, %lld] need %zu scratch "
