@@ -17,6 +17,9 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
 void gemv_geometry(int64_t M, int64_t N, int64_t K, int* t, int* waves);
 void skinny_geometry(int64_t N, int64_t K, int bits, int* waves, int* rows_per_wg);
 bool skinny2_plan(int64_t M, int64_t N, int64_t K, int bits, int* rows_per_wg);
+bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
+                              int64_t products);
+int64_t skinny2_ragged_rows(int64_t N, int64_t K, int64_t products);
 bool skinny2_mx_plan(int64_t N, int64_t K, int* rows_per_wg);
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                                const void* s, const void* b, int64_t E);
@@ -30,7 +33,8 @@ void gemm_dispatch(const void* x, const void* w, const void* s, const void* b, i
                    const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N,
                    int64_t K, int gs, int bits, int mode, hipStream_t st);
 int64_t gemm_row_tile(int64_t R, int64_t E);
-bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b);
+bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b,
+                       int64_t products);
 void gemv_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                            int y_dtype, const int32_t* segments, const int32_t* src_row,
                            const int32_t* out_row, int64_t max_segments, int64_t x_rows, int64_t N,
@@ -400,6 +404,12 @@ int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode
     if (block) *block = loaders ? 64 * 12 : 64 * waves;
     return QMM_OK;
   }
+  if (M <= kGemvMaxM && mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, group_size, bits, QMM_BF16, nullptr, nullptr, 1)) {
+    if (kernel) *kernel = QMM_KERNEL_GEMV;
+    if (grid) *grid = (int)ceil_div(N, skinny2_ragged_rows(N, K, 1));
+    if (block) *block = 64 * 12;
+    return QMM_OK;
+  }
   if (M <= kGemvMaxM) {
     int t, waves;
     gemv_geometry(M, N, K, &t, &waves);
@@ -601,7 +611,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     // codes: 16 pairs 108 against 206 us, 32 pairs 110 against 397.)
     if (P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace &&
         workspace_bytes >= route_bytes_segments(P, E) &&
-        gemv_runs_general(N, K, group_size, bits, mode, table_dtype, scales, biases) &&
+        gemv_runs_general(N, K, group_size, bits, mode, table_dtype, scales, biases, E) &&
         !experiment_env("QMM_NO_GROUPED_GEMV")) {
       int32_t* ro = static_cast<int32_t*>(workspace);
       int32_t* cursor = ro + E + 1;

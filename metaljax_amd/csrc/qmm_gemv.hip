@@ -26,6 +26,7 @@
 // 4-bit codes are widened as the bf16 value 128+q (one and-or per pair), the
 // 128 is folded into the bias; their pairs come out as (k, k+4), so the
 // activation registers are byte-permuted to the same order.
+#include <algorithm>
 #include <type_traits>
 
 #include "qmm_gemv_common.hpp"
@@ -424,7 +425,10 @@ bool skinny2_plan(int64_t M, int64_t N, int64_t K, int bits, int* rows_per_wg);
 void skinny2_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int rows, hipStream_t st,
                       int tab, bool force_direct);
 int skinny2_direct_rows(int64_t N);
-bool skinny2_mx_supported(int64_t N, int64_t K, const void* s);
+bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products);
+bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
+                              int64_t products);
+void skinny2_ragged_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int tab, hipStream_t st);
 void skinny2_mx_dispatch(const GemvArgs& a0, int64_t batch, hipStream_t st);
 
 // Tile / slice / unroll choice; QMM_GEMV_T, QMM_GEMV_WAVES and QMM_GEMV_U
@@ -488,13 +492,16 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
     skinny2_dispatch(a, batch, gs, bits, rows, st, tab, !planned);
     return;
   }
+  const int64_t weights = std::max(batch, n_experts);
+  if (!no_skinny && mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, weights))
+    return skinny2_ragged_dispatch(a, batch, gs, bits, tab, st);
   Geometry g;
   gemv_geometry(M, N, K, &g.t, &g.waves);
   g.u = env_u ? env_u : 8;
   if (mode == QMM_MODE_MXFP4) {
     a.gshift = 0;
     // big weights: the loader-wavefront kernel (activations fetched directly)
-    if (!no_skinny && skinny2_mx_supported(N, K, s)) return skinny2_mx_dispatch(a, batch, st);
+    if (!no_skinny && skinny2_mx_supported(N, K, s, weights)) return skinny2_mx_dispatch(a, batch, st);
     if (!env_u) g.u = 4;
     launch_mxfp4(a, batch, g, st);
     return;
@@ -511,12 +518,14 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
 }
 
 // The general kernels would serve this shape (no staged decode kernel does).
-bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b) {
+bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b,
+                       int64_t products) {
   if (skinny_supported(N, K, gs, bits, mode, tab, s, b)) return false;
+  if (mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, products)) return false;
   if ((tab == QMM_F16 || tab == QMM_F32) && K * bits / 8 / 256 >= 8 &&
       skinny_supported(N, K, gs, bits, mode, QMM_BF16, s, b))
     return false;
-  if (mode == QMM_MODE_MXFP4 && skinny2_mx_supported(N, K, s)) return false;
+  if (mode == QMM_MODE_MXFP4 && skinny2_mx_supported(N, K, s, products)) return false;
   return true;
 }
 

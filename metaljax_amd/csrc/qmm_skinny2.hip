@@ -190,21 +190,32 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // (E2M1 codes, one E8M0 byte per 32 codes); 3 / 4 = float16 tables; 5 / 6 =
   // float32 tables.  A row's table share of a slice is 16 bytes, except for
   // float32 tables with groups of 64 (eight 4-byte entries: 32 bytes, WIDE).
-  constexpr bool WIDE = GSHIFT == 5;
+  // From 7 on K is any multiple of 64 (a RAGGED last slice): 7 = MXFP4, 8 + kind
+  // = the affine kinds above.
+  constexpr bool RAG = GSHIFT >= 7;
+  constexpr int GK = GSHIFT >= 8 ? GSHIFT - 8 : GSHIFT;
+  constexpr bool WIDE = GK == 5;
   constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (WIDE ? 2 : 1);   // scale rows | bias rows of one tile
   constexpr int kTab = 2 * kTabKind;
   constexpr int NTAB = 2 * (CW >= 4 ? CW / 4 : 1) * (WIDE ? 2 : 1);        // table load instructions per tile
   static_assert((CW * 4) % NL == 0 && NTAB % NL == 0, "loader shares must be whole");
   constexpr int QI = CW * 4 / NL;                 // code / activation loads per loader wavefront per item
   constexpr int QT = NTAB / NL;                   // table loads per loader wavefront per tile
-  constexpr int LX = QI, LT = QI + QT;            // loads per loader wavefront: activation item | tile item
+  // A ragged four-bit row of 16-bit entries may start inside a dword, and the
+  // eight entries of a slice then end in the dword after its sixteen bytes: that
+  // is the first one of the next slice's, which for a pass's last slice is
+  // fetched apart (XD = 1: that slice is the ragged one and does not need it).
+  constexpr bool EXTRA = XD == 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11);
+  constexpr int LX = QI, LT = QI + QT + (EXTRA ? 1 : 0);      // loads per loader wavefront: activation item | tile item
   typedef Sched<XR, TMAX, LX, LT> S;
+  static_assert(!EXTRA || NL == 4, "four requests of eight rows");
   extern __shared__ __align__(16) unsigned char smem[];
   unsigned char* ring = smem;
   unsigned char* tabs = smem + S::B * kItem;
   // Direct variants: behind the ring and the tables, a 1 KB patch a compute
   // wavefront (staging of activations that come in with whole-line loads).
   unsigned char* patches = smem + 4 * (kItem + kTab);
+  unsigned char* extras = patches + CW * 1024;    // EXTRA: 512 bytes a slot, scale | bias rows
 
   const int lane = threadIdx.x & 63;
   // (Wavefronts start in the order of their hardware index, a whole workgroup
@@ -221,25 +232,29 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   const int64_t wpr = (int64_t)a.K * BITS / 8;                  // bytes per weight row
   // float16 / float32 entries are split into two / three bf16 terms, exactly,
   // where they have to be matrix operands.
-  // GSHIFT = 7: MXFP4 whose K is any multiple of 64 up to one pass (the hidden
-  // size 2880 of gpt-oss: five and a half slices a row, 90 scale bytes a row):
-  // the last slice is ragged -- the code pieces and activation chunks past K are
-  // requested out of range and read as zeros -- and a tile's scale rows, which
-  // are not dword-aligned one by one, come in as the one contiguous run they
-  // are in memory and are picked apart by byte offset.
+  // RAG: K is any multiple of 64 (the hidden size 2880 of gpt-oss: five and a
+  // half slices a row; the 11008 of a 7B model's down projection: 21.5).  The code
+  // pieces and activation chunks of the last slice past K are requested out of
+  // range and read as zeros, and the table entries there (the next row's) are
+  // masked off.  Table rows may start inside a dword: a row's share is fetched
+  // from the dword it starts in and shifted into place; for MXFP4, whose sixteen
+  // scale bytes then need eighteen, the second table request fetches the same row
+  // a dword further.  One-pass MXFP4: a tile's scale rows come in as the one
+  // contiguous run they are in memory and are picked apart by byte offset.
   constexpr bool MXR = GSHIFT == 7;
   constexpr bool MX = GSHIFT == 2 || MXR;
-  constexpr bool F16T = GSHIFT == 3 || GSHIFT == 4;
-  constexpr bool F32T = GSHIFT == 5 || GSHIFT == 6;
-  static_assert(!MXR || XD == 1, "the ragged MXFP4 form is a one-pass direct variant");
+  constexpr bool MXRUN = MXR && XD == 1;
+  constexpr bool F16T = GK == 3 || GK == 4;
+  constexpr bool F32T = GK == 5 || GK == 6;
+  static_assert(!RAG || XD != 0, "ragged forms are direct variants");
   constexpr int ES = F32T ? 4 : 2;                             // bytes per table entry
-  constexpr int GLOG = (GSHIFT == 1 || GSHIFT == 4 || GSHIFT == 6) ? 1 : 0;   // log2(group / 64)
+  constexpr int GLOG = (GK == 1 || GK == 4 || GK == 6) ? 1 : 0;   // log2(group / 64)
   static_assert(!MX || (BITS == 4 && XD != 0), "MXFP4: four-bit codes, direct variants");
   const int64_t ng = MX ? (int64_t)(a.K / 64) : (int64_t)(a.K / 64) >> GLOG;   // table row = ng * ES bytes (MXFP4: K/32 bytes)
-  const int slices = MXR ? (a.K + KS - 1) / KS : a.K / KS;
+  const int slices = RAG ? (a.K + KS - 1) / KS : a.K / KS;
   const int passes = (slices + CW - 1) / CW;
-  const int tail_codes = MXR ? a.K % KS : 0;                   // codes of a ragged last slice (0: it is whole)
-  const int tailp = tail_codes / 32, tailc = tail_codes / 64;  // its 16-byte pieces | its 64-code chunks
+  const int tail_codes = RAG ? a.K % KS : 0;                   // codes of a ragged last slice (0: it is whole)
+  const int tailp = tail_codes * BITS / 128, tailc = tail_codes / 64;  // its 16-byte pieces | its 64-code chunks
   const uint32_t spitch = (uint32_t)(ng * ES);                 // bytes of a table row
 
   int64_t xz = a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
@@ -280,8 +295,10 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     const int lw = wave - CW;
     const auto rx = make_rsrc(a.x + xz * a.M * (int64_t)a.K, x_ok ? (int64_t)a.M * a.K * 2 : 0);
     const auto rw = make_rsrc(reinterpret_cast<const char*>(a.w) + wz * a.N * wpr, a.N * wpr);
-    const auto rs = make_rsrc(static_cast<const char*>(a.s) + wz * a.N * ng * ES, a.N * ng * ES);
-    const auto rb = make_rsrc(static_cast<const char*>(a.b) + wz * a.N * ng * ES, a.N * ng * ES);
+    // (ragged: whole dwords, the last row may end in the middle of one)
+    const int64_t tbytes = RAG ? (a.N * ng * ES + 3) / 4 * 4 : a.N * ng * ES;
+    const auto rs = make_rsrc(static_cast<const char*>(a.s) + wz * a.N * ng * ES, tbytes);
+    const auto rb = make_rsrc(static_cast<const char*>(a.b) + wz * a.N * ng * ES, tbytes);
     const int lrow = lane >> 4, lp = lane & 15;
     // Load q of this wavefront is instruction j = lw + q*NL of the item: slice
     // j / 4, row quad j % 4 = (lw + o) % 4 with o = q*NL % 4 known at compile
@@ -295,7 +312,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
       const uint32_t gp = (uint32_t)(lp ^ (row & 15));
       wrow[o] = row;
       wv[o] = (uint32_t)((n_begin + row) * wpr) + gp * 16;
-      wvt[o] = MXR && tailp != 0 && (int)gp >= tailp ? kOutOfRange : wv[o];   // in a ragged last slice
+      wvt[o] = RAG && tailp != 0 && (int)gp >= tailp ? kOutOfRange : wv[o];   // in a ragged last slice
       xv[o] = row < a.M ? (uint32_t)((int64_t)row * a.K * 2) + gp * 16 : kOutOfRange;
     }
     const int trow = lane & 15, tsl = lane >> 4;  // table loads: lane = (slice within four, row)
@@ -321,7 +338,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 #pragma unroll
       for (int q = 0; q < QT; ++q) {
         const int jt = lw + q * NL;               // uniform
-        if constexpr (MXR) {
+        if constexpr (MXRUN) {
           // the tile's scale rows as the contiguous run they are: request jt covers its bytes [1024 jt, 1024 jt + 1024)
           const int64_t n0t = n_begin + t * 16;
           const int rows_here = n_end - n0t < 16 ? (int)(n_end - n0t) : 16;
@@ -337,14 +354,23 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         const int sl = p * CW + sloc;
         const int64_t n = n_begin + t * 16 + trow;
         const bool ok = sloc < CW && sl < slices && n < n_end;
-        const uint32_t vo = ok ? (uint32_t)(n * ng * ES) + (uint32_t)((sl * CPS) >> (MX ? 0 : GLOG)) * (uint32_t)ES + (uint32_t)h2 * 16u
-                               : kOutOfRange;
+        uint32_t vo = ok ? (uint32_t)(n * ng * ES) + (uint32_t)((sl * CPS) >> (MX ? 0 : GLOG)) * (uint32_t)ES + (uint32_t)h2 * 16u
+                         : kOutOfRange;
+        if constexpr (RAG) vo &= ~3u;
         unsigned char* tdst = tb + kind * kTabKind + (WIDE ? h * 2048 + h2 * 1024 : h * 1024);
         // (MXFP4 has no second table: the load still goes out, fetching nothing,
         // so that every loader wavefront issues the same number per tile -- the
         // waits count loads)
-        if constexpr (MX) dma16<kStream>(rs, tdst, kind == 0 ? vo : kOutOfRange, 0u);
+        if constexpr (MXR) dma16<kStream>(rs, tdst, vo + (uint32_t)kind * 4u, 0u);
+        else if constexpr (MX) dma16<kStream>(rs, tdst, kind == 0 ? vo : kOutOfRange, 0u);
         else dma16<kStream>(kind ? rb : rs, tdst, vo, 0u);
+      }
+      if constexpr (EXTRA) {
+        // one request a loader: the entries that follow this pass's, eight rows of one table
+        const int kind = lw & 1, row = 8 * (lw >> 1) + (lane & 7), sl = (p + 1) * CW;
+        const int64_t n = n_begin + t * 16 + row;
+        const uint32_t vo = sl < slices && n < n_end ? ((uint32_t)(n * ng + sl * CPS) * 2u) & ~3u : kOutOfRange;
+        if (lane < 8) dma16<kStream>(kind ? rb : rs, extras + slot * 512 + kind * 256 + (lw >> 1) * 128, vo, 0u);
       }
       static_for<QI>([&](auto qc) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
@@ -354,7 +380,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         const int sl = p * CW + sloc;
         const bool sok = sl < slices;             // uniform; false for passes past the last
         const uint32_t so = sok ? (uint32_t)sl * 256u + tile_off : 0u;
-        const bool rag = MXR && sl == slices - 1;  // uniform
+        const bool rag = RAG && sl == slices - 1;  // uniform
         dma16<kStream>(rw, base + sloc * 4096 + rq * 1024, sok ? (rag ? vtt[o] : vt[o]) : kOutOfRange, so);
       });
     };
@@ -528,9 +554,11 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     const int sw = XD == 1 ? (wave + (int)(blockIdx.x >> 3)) & (CW - 1) : wave;
     const uint32_t rowb = (uint32_t)(sw * 4096 + r * 256);      // this lane's row inside its slice's 4 KB
     // the operand row r of this lane is row xrow(r) of x (gathered in the grouped form)
-    const int tab_row = MXR ? 0 : (sw >> 2) * (WIDE ? 2048 : 1024) + (sw & 3) * 256 + r * 16;   // this lane's table row inside a kind
-    // chunks of this wavefront's slice that lie inside K (a ragged last slice has fewer)
-    const int vc = MXR && tailc != 0 && sw == slices - 1 ? tailc : CPS;
+    const int tab_row = MXRUN ? 0 : (sw >> 2) * (WIDE ? 2048 : 1024) + (sw & 3) * 256 + r * 16;   // this lane's table row inside a kind
+    // chunks of slice `sl` that lie inside K (a ragged last slice has fewer)
+    auto chunks_of = [&](int sl) __attribute__((always_inline)) { return RAG && sl == slices - 1 ? tailc : CPS; };
+    // bits by which this lane's table row starts inside a dword (tiles are sixteen rows: the same for all)
+    const uint32_t tsh = RAG && !F32T ? (uint32_t)((int)(n_begin + r) & (int)ng & 1) * 16u : 0u;
     const int64_t xrows = src_row ? (int64_t)a.x_rows : (int64_t)a.M;
     const auto rxc = make_rsrc(a.x + xz * a.M * (int64_t)a.K, x_ok ? xrows * a.K * 2 : 0);
     auto xrow = [&](int m) -> int64_t {
@@ -594,14 +622,20 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     };
     // acc + this wavefront's K-slice of one tile: `base` is the lane's row in
     // the slice's 4 KB of codes, `tb` its table row
-    auto tile_math = [&](const unsigned char* base, const unsigned char* tb, f32x4 acc_in) __attribute__((always_inline)) {
+    // (`nv`: chunks of the slice inside K; `slot`: the ring slot)
+    auto tile_math = [&](const unsigned char* base, const unsigned char* tb, f32x4 acc_in, int nv, int slot) __attribute__((always_inline)) {
       if constexpr (MX) {
         // E2M1 codes: the converter widens two codes at a time and multiplies
         // by the 32-block's power-of-two scale (exact in bf16), so the chunks
         // chain straight through the MFMA accumulator.  Lane kg holds codes
         // [16 kg, 16 kg + 16) of the chunk: block 2c + kg/2 of the slice.
         u32x4 sv;
-        if constexpr (MXR) {
+        if constexpr (MXR && !MXRUN) {
+          const u32x4 d = *reinterpret_cast<const u32x4*>(tb);
+          const uint32_t d4 = *reinterpret_cast<const uint32_t*>(tb + kTabKind + 12);
+          sv = u32x4{__builtin_amdgcn_alignbit(d[1], d[0], tsh), __builtin_amdgcn_alignbit(d[2], d[1], tsh),
+                     __builtin_amdgcn_alignbit(d[3], d[2], tsh), __builtin_amdgcn_alignbit(d4, d[3], tsh)};
+        } else if constexpr (MXRUN) {
           // this row's sixteen scale bytes of the slice, at an even byte offset of the tile's run
           const uint32_t off = (uint32_t)r * spitch + 16u * (uint32_t)sw;
           const uint32_t* pw = reinterpret_cast<const uint32_t*>(tb + (off & ~3u));
@@ -618,7 +652,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           const uint32_t pc = (uint32_t)(2 * c + (kg >> 1));
           const u32x2 q = *reinterpret_cast<const u32x2*>(base + ((pc ^ swz) << 4) + (kg & 1) * 8);
           float sc = e8m0_to_f32((sv[c >> 1] >> (16 * (c & 1) + 8 * (kg >> 1))) & 255u);
-          if constexpr (MXR) sc = c < vc ? sc : 1.0f;        // past K: zero codes times a finite scale
+          if constexpr (MXR) sc = c < nv ? sc : 1.0f;        // past K: zero codes times a finite scale
           at = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], widen_e2m1(q[0], sc), at, 0, 0, 0);
           at = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][1], widen_e2m1(q[1], sc), at, 0, 0, 0);
         }
@@ -626,11 +660,33 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
       }
       u32x4 svt = *reinterpret_cast<const u32x4*>(tb);
       u32x4 bvt = *reinterpret_cast<const u32x4*>(tb + kTabKind);
+      if constexpr (RAG && !F32T) {
+        // the row's entries from where they start (four-bit codes in groups of 64 take all
+        // sixteen bytes: the fifth dword is the next slice's first)
+        uint32_t s4 = 0u, b4 = 0u;
+        if constexpr (BITS == 4 && GLOG == 0) {
+          const unsigned char* nx = EXTRA && sw == CW - 1 ? extras + slot * 512 + r * 16 : tb + 256;
+          s4 = *reinterpret_cast<const uint32_t*>(nx);
+          b4 = *reinterpret_cast<const uint32_t*>(EXTRA && sw == CW - 1 ? nx + 256 : nx + kTabKind);
+        }
+        svt = u32x4{__builtin_amdgcn_alignbit(svt[1], svt[0], tsh), __builtin_amdgcn_alignbit(svt[2], svt[1], tsh),
+                    __builtin_amdgcn_alignbit(svt[3], svt[2], tsh), __builtin_amdgcn_alignbit(s4, svt[3], tsh)};
+        bvt = u32x4{__builtin_amdgcn_alignbit(bvt[1], bvt[0], tsh), __builtin_amdgcn_alignbit(bvt[2], bvt[1], tsh),
+                    __builtin_amdgcn_alignbit(bvt[3], bvt[2], tsh), __builtin_amdgcn_alignbit(b4, bvt[3], tsh)};
+      }
       if constexpr (GLOG == 1 && !F32T) {   // group 128: one entry serves two chunks -> duplicate each 16-bit entry
         svt = u32x4{byte_perm(svt[0], svt[0], 0x01000100u), byte_perm(svt[0], svt[0], 0x03020302u),
                     byte_perm(svt[1], svt[1], 0x01000100u), byte_perm(svt[1], svt[1], 0x03020302u)};
         bvt = u32x4{byte_perm(bvt[0], bvt[0], 0x01000100u), byte_perm(bvt[0], bvt[0], 0x03020302u),
                     byte_perm(bvt[1], bvt[1], 0x01000100u), byte_perm(bvt[1], bvt[1], 0x03020302u)};
+      }
+      if constexpr (RAG && !F32T) {         // entries past K: the next row's, whatever they are
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t keep = (2 * i < nv ? 0x0000FFFFu : 0u) | (2 * i + 1 < nv ? 0xFFFF0000u : 0u);
+          svt[i] &= keep;
+          bvt[i] &= keep;
+        }
       }
       // eight table entries as matrix operands over the chunk index: one bf16
       // operand, or for float16 tables two (hi + lo, exact: 11 significant bits)
@@ -664,6 +720,13 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           for (int i = 0; i < 4; ++i) {
             sf[2 * i] = sf[2 * i + 1] = __uint_as_float(svt[i]);
             bfv[2 * i] = bfv[2 * i + 1] = __uint_as_float(bvt[i]);
+          }
+        }
+        if constexpr (RAG) {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            sf[c] = c < nv ? sf[c] : 0.f;
+            bfv[c] = c < nv ? bfv[c] : 0.f;
           }
         }
       }
@@ -729,7 +792,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
       // This wavefront's slice of pass p of the activations straight from
       // global memory (L2 after the first workgroup) into operand layout: lane
       // (r, kg) takes pieces 2*kg and 2*kg + 1 of every chunk of row r.
-      auto fetch_x = [&](int p, bool active, uint32_t lane_off) __attribute__((always_inline)) {
+      // (`nv`: chunks of this lane's slice inside K.)
+      auto fetch_x = [&](int p, bool active, uint32_t lane_off, int nv) __attribute__((always_inline)) {
         u32x4 raw[CPS][2];
         const uint32_t so = active ? (uint32_t)((p * CW + sw) * KS) * 2u : 0u;
 #pragma unroll
@@ -737,7 +801,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 #pragma unroll
           for (int j = 0; j < 2; ++j)
             raw[c][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                rxc, active && (!MXR || c < vc) ? lane_off + (uint32_t)(c * 128 + j * 16) : kOutOfRange, so, 0);
+                rxc, active && (!RAG || c < nv) ? lane_off + (uint32_t)(c * 128 + j * 16) : kOutOfRange, so, 0);
 #pragma unroll
         for (int c = 0; c < CPS; ++c)
 #pragma unroll
@@ -767,6 +831,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         const int srow = lane >> 3, sp = lane & 7;
         u32x4 raw[CPS][2];
         uint32_t lo[2];
+        int nv[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int rr = 8 * h + srow;
@@ -774,10 +839,12 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           uint32_t pass_off = 0u;
           if (pk == 0) {
             xr = active ? xrow(rr) : -1;
+            nv[h] = chunks_of(p * CW + sw);
           } else {
             const int q = pk == 8 ? rr >> 3 : rr >> 2, m = rr - q * pk;
             xr = active && q * CW + wave < slices ? xrow(m) : -1;
             pass_off = (uint32_t)(q * CW * KS) * 2u;
+            nv[h] = chunks_of(q * CW + wave);
           }
           lo[h] = xr >= 0 ? (uint32_t)(xr * a.K * 2) + pass_off + (uint32_t)sp * 16u : kOutOfRange;
         }
@@ -787,7 +854,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 #pragma unroll
           for (int h = 0; h < 2; ++h)
             raw[c][h] = __builtin_amdgcn_raw_buffer_load_b128(
-                rxc, !MXR || (c + ROT) % CPS < vc ? lo[h] : kOutOfRange, so + (uint32_t)(((c + ROT) % CPS) * 128), 0);
+                rxc, !RAG || (c + ROT) % CPS < nv[h] ? lo[h] : kOutOfRange, so + (uint32_t)(((c + ROT) % CPS) * 128), 0);
         const uint32_t wr = (uint32_t)(srow * 128 + ((sp ^ ((srow >> 1) & 3)) << 4));
         const uint32_t rkey = (uint32_t)((r >> 1) & 3);
         const bool upper = r >= 8;
@@ -841,11 +908,12 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         const int64_t xr = active ? xrow(srow) : -1;
         const uint32_t lo = xr >= 0 ? (uint32_t)(xr * a.K * 2) + (uint32_t)sp * 16u : kOutOfRange;
         const uint32_t so = active ? (uint32_t)(sw * KS) * 2u : 0u;
+        const int nv = chunks_of(sw);
         u32x4 raw[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i)
           raw[i] = __builtin_amdgcn_raw_buffer_load_b128(
-              rxc, !MXR || i * CPI + (sp >> 3) < vc ? lo : kOutOfRange, so + (uint32_t)(i * W), 0);
+              rxc, !RAG || i * CPI + (sp >> 3) < nv ? lo : kOutOfRange, so + (uint32_t)(i * W), 0);
         const uint32_t wr = (uint32_t)(srow * W + ((sp ^ key(srow)) << 4));
         const int rr = r % R;
         const uint32_t rd = (uint32_t)(rr * W), rkey = (uint32_t)key(rr);
@@ -874,6 +942,52 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           if (active) chunk_sums();
         }
       };
+      // The pass's slice of up to sixteen rows, eight rows at a time with whole
+      // 128-byte lines: the form for several passes, whose accumulators leave no
+      // registers for both halves' loads at once (MXFP4 at sixteen rows, against
+      // the direct fetch: 8192 x 8192 16.8 -> 14.9 us, 4096 x 11008 16.7 -> 14.6;
+      // four-bit affine codes, with their table operands, spill here and keep it).
+      auto fetch_x_halves = [&](int p, bool active) __attribute__((always_inline)) {
+        unsigned char* stg = patches + wave * 1024;
+        const int srow = lane >> 3, sp = lane & 7;
+        const uint32_t so = active ? (uint32_t)((p * CW + sw) * KS) * 2u : 0u;
+        const int nv = chunks_of(p * CW + sw);
+        const uint32_t wr = (uint32_t)(srow * 128 + ((sp ^ ((srow >> 1) & 3)) << 4));
+        const uint32_t rd = (uint32_t)((r & 7) * 128), rkey = (uint32_t)((r >> 1) & 3);
+#pragma nounroll
+        for (int h = 0; h < 2; ++h) {
+          if (h == 1 && M <= 8) break;
+          const int64_t xr = active ? xrow(8 * h + srow) : -1;
+          const uint32_t lo = xr >= 0 ? (uint32_t)(xr * a.K * 2) + (uint32_t)sp * 16u : kOutOfRange;
+          u32x4 raw[CPS];
+#pragma unroll
+          for (int c = 0; c < CPS; ++c)
+            raw[c] = __builtin_amdgcn_raw_buffer_load_b128(rxc, !RAG || c < nv ? lo : kOutOfRange, so + (uint32_t)(c * 128), 0);
+          const bool mine = (r >> 3) == h;
+#pragma unroll
+          for (int c = 0; c < CPS; ++c) {
+            *reinterpret_cast<u32x4*>(stg + wr) = raw[c];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              const u32x4 v = *reinterpret_cast<const u32x4*>(stg + rd + (((uint32_t)(kg * 2 + j) ^ rkey) << 4));
+              bf16x8 o;
+              if constexpr (BITS == 4 && !MX) o = pair_stride4(v);
+              else o = __builtin_bit_cast(bf16x8, v);
+              if (mine) xa[c][j] = o;
+              else if (h == 0) xa[c][j] = as_bf16x8(0u, 0u, 0u, 0u);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          }
+        }
+        if constexpr (!MX) {
+          if (active) chunk_sums();
+        }
+      };
       if constexpr (XD == 1) {
         // One pass (the host sees to it).  The tiles as a real loop (any number of them): a tile's sums leave
         // for its slot at once, where the loaders add up the slices.
@@ -890,9 +1004,9 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           }
           else if (M > 4) fetch_x_lines(std::integral_constant<int, 8>{}, active);
           else if (M > 2) fetch_x_lines(std::integral_constant<int, 4>{}, active);
-          else fetch_x(0, active, xlane);
+          else fetch_x(0, active, xlane, chunks_of(sw));
         } else {
-          fetch_x(0, active, xlane);
+          fetch_x(0, active, xlane, chunks_of(sw));
         }
         QMM_STAMP(2);
 #pragma nounroll
@@ -901,7 +1015,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           if (g < 4) QMM_STAMP(3 + 2 * g);
           const int slot = g & 3;
           f32x4 at = zero;
-          if (active) at = tile_math(ring + slot * kItem + rowb, tabs + slot * kTab + tab_row, zero);
+          if (active) at = tile_math(ring + slot * kItem + rowb, tabs + slot * kTab + tab_row, zero, chunks_of(sw), slot);
           float* part = reinterpret_cast<float*>(ring + slot * kItem + sw * 4096);
 #pragma unroll
           for (int e = 0; e < 4; ++e) part[e * kWave + lane] = at[e];
@@ -930,13 +1044,16 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           bool staged = false;
           if constexpr (!WIDE) staged = M * passes > 8;
           if (staged) fetch_x_staged(std::integral_constant<int, 0>{}, 0, wave < slices, PK);
-          else fetch_x(0, wave < slices, off);
+          else fetch_x(0, wave < slices, off, chunks_of(q * CW + wave));
         }
         const int my_pass = PK == 8 ? kg >> 1 : kg;   // the pass whose sums this lane's accumulator rows hold
         QMM_STAMP(2);
         for (int p = 0; p < passes; ++p) {
           const bool active = p * CW + wave < slices;   // uniform
-          if (PK == 0) fetch_x(p, active, xlane);
+          if (PK == 0) {
+            if constexpr (!WIDE && (MX || BITS == 8)) fetch_x_halves(p, active);
+            else fetch_x(p, active, xlane, chunks_of(p * CW + sw));
+          }
           static_for<TMAX>([&](auto tc) __attribute__((always_inline)) {
             constexpr int t = decltype(tc)::value;
             if (t < ntiles) {
@@ -944,7 +1061,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
               if (p * ntiles + t < 4) QMM_STAMP(3 + 2 * (p * ntiles + t));
               const int slot = (p * ntiles + t) & 3;
               if (active) {
-                const f32x4 d = tile_math(ring + slot * kItem + rowb, tabs + slot * kTab + tab_row, zero);
+                const f32x4 d = tile_math(ring + slot * kItem + rowb, tabs + slot * kTab + tab_row, zero,
+                                          chunks_of(p * CW + wave), slot);
                 const bool mine = PK == 0 || my_pass == p;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[t][e] += mine ? d[e] : 0.f;
@@ -989,7 +1107,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         } else {
           constexpr int t = i - XR;
           if (active && t < ntiles)
-            acc[t] = tile_math(base, tabs + slot * kTab + tab_row, acc[t]);
+            acc[t] = tile_math(base, tabs + slot * kTab + tab_row, acc[t], CPS, slot);
           // Last pass: this wavefront's partial sums of tile t go where its own
           // slice of the tile was (nobody else reads that region, and a tile's
           // slot is not refilled within a pass); the loaders add the slices up.
@@ -1019,11 +1137,13 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD>
 void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int chunks = 1) {
   dim3 grid((unsigned)ceil_div(a.N, rows_per_wg), (unsigned)batch, (unsigned)chunks);
-  constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (GSHIFT == 5 ? 2 : 1);
+  constexpr bool wide = GSHIFT == 5 || GSHIFT == 13;
+  constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (wide ? 2 : 1);
   constexpr int XR = XD ? 0 : 2048 / BITS / 128;
   // (direct variants: plus a 1 KB patch a compute wavefront for staging activations)
   const size_t lds = (size_t)(XD || XR + TMAX >= 4 ? 4 : XR + TMAX) * (CW * 4096 + 2 * kTabKind) +
-                     (XD != 0 && GSHIFT != 5 ? (size_t)CW * 1024 : 0);
+                     (XD != 0 && !wide ? (size_t)CW * 1024 : 0) +
+                     (XD == 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11) ? 2048 : 0);      // (the kernel's EXTRA)
   constexpr auto kern = skinny2_kernel<BITS, CW, NL, TMAX, GSHIFT, XD>;
   if (!lds_limit<kern>(lds)) return;
   hipLaunchKernelGGL(kern, grid, dim3(kWave * (CW + NL)), lds, st, a, rows_per_wg);
@@ -1034,8 +1154,19 @@ void launch_k(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st,
   if constexpr (BITS == 4 && XD != 0) {
     if (a.gshift == 2) return launch_one<BITS, CW, NL, TMAX, 2, XD>(a, batch, rows_per_wg, st, chunks);
   }
-  if constexpr (BITS == 4 && XD == 1) {
+  if constexpr (BITS == 4 && XD != 0) {
     if (a.gshift == 7) return launch_one<BITS, CW, NL, TMAX, 7, XD>(a, batch, rows_per_wg, st, chunks);
+  }
+  if constexpr (XD != 0) {
+    switch (a.gshift) {
+      case 8: return launch_one<BITS, CW, NL, TMAX, 8, XD>(a, batch, rows_per_wg, st, chunks);
+      case 9: return launch_one<BITS, CW, NL, TMAX, 9, XD>(a, batch, rows_per_wg, st, chunks);
+      case 11: return launch_one<BITS, CW, NL, TMAX, 11, XD>(a, batch, rows_per_wg, st, chunks);
+      case 12: return launch_one<BITS, CW, NL, TMAX, 12, XD>(a, batch, rows_per_wg, st, chunks);
+      case 13: return launch_one<BITS, CW, NL, TMAX, 13, XD>(a, batch, rows_per_wg, st, chunks);
+      case 14: return launch_one<BITS, CW, NL, TMAX, 14, XD>(a, batch, rows_per_wg, st, chunks);
+      default: break;
+    }
   }
   switch (a.gshift) {
     case 1: return launch_one<BITS, CW, NL, TMAX, 1, XD>(a, batch, rows_per_wg, st, chunks);
@@ -1143,12 +1274,17 @@ int skinny2_direct_rows(int64_t N) {
   return (int)(r < 16 ? 16 : r);
 }
 
+// Table kind of the kernel (its GSHIFT) for affine weights, K whole slices.
+static int affine_kind(int gs, int tab) {
+  return (gs == 128 ? 1 : 0) + (tab == QMM_F16 ? 3 : tab == QMM_F32 ? 5 : 0);
+}
+
 // tab: QMM_BF16 or QMM_F16 tables; force_direct: a direct variant even where
 // the ring variant or the self-loading kernel would be chosen
 void skinny2_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int rows, hipStream_t st,
                       int tab, bool force_direct) {
   GemvArgs a = a0;
-  a.gshift = (gs == 128 ? 1 : 0) + (tab == QMM_F16 ? 3 : tab == QMM_F32 ? 5 : 0);
+  a.gshift = affine_kind(gs, tab);
   bool xd = force_direct || direct_x(a.M, a.N, a.K, bits);
   // float32 tables with groups of 64 fill the LDS with table rows: no room for
   // the staging patches, and direct loads of more than eight rows lose to the ring
@@ -1178,14 +1314,17 @@ bool skinny_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
 // segment, provisioned for the most there can be (workgroups past the count
 // leave at once; an empty workgroup still costs about a microsecond of a
 // compute unit, which is why the grid is not expert x chunk).
-bool skinny2_mx_supported(int64_t N, int64_t K, const void* s);
+bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products);
+bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
+                              int64_t products);
 static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products);
 
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                                const void* s, const void* b, int64_t E) {
+  if (mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, E)) return true;
   // (MXFP4 whose K is no whole number of slices has no other staged kernel to go to: its ragged
   // one-pass form takes the grouped decode from three slices on)
-  if (mode == QMM_MODE_MXFP4) return (K / 512 >= 8 || K % 512 != 0) && skinny2_mx_supported(N, K, s);
+  if (mode == QMM_MODE_MXFP4) return (K / 512 >= 8 || K % 512 != 0) && skinny2_mx_supported(N, K, s, E);
   if (!skinny_supported(N, K, gs, bits, mode, QMM_BF16, s, b)) return false;   // bf16, float16 and float32 tables alike
   return K * bits / 8 / 256 >= 8;
 }
@@ -1203,8 +1342,8 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   a.b = b;
   a.y = y;
   a.M = 1; a.N = (int)N; a.K = (int)K;
-  a.gshift = mode == QMM_MODE_MXFP4 ? (K % 512 ? 7 : 2)
-                                    : (gs == 128 ? 1 : 0) + (tab == QMM_F16 ? 3 : tab == QMM_F32 ? 5 : 0);
+  const bool ragged = K * bits / 8 % 256 != 0;
+  a.gshift = mode == QMM_MODE_MXFP4 ? (ragged ? 7 : 2) : (ragged ? 8 : 0) + affine_kind(gs, tab);
   a.y_dtype = y_dtype;
   a.lhs_idx = nullptr;
   a.rhs_idx = nullptr;
@@ -1216,9 +1355,9 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   const int64_t rounds = ceil_div(ceil_div(N, cus), (int64_t)128);
   int64_t rows = ceil_div(N, cus * rounds);
   if (rows < 16) rows = 16;
-  if (mode == QMM_MODE_MXFP4) rows = mx_rows_per_wg(N, K, P < E ? P : E);
+  if (mode == QMM_MODE_MXFP4 || ragged) rows = mx_rows_per_wg(N, K, P < E ? P : E);
   const int64_t segs = skinny2_max_segments(P, E);
-  if (K * bits / 8 / 256 <= 8) {
+  if (K * bits / 8 <= 2048) {
     if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, segs, (int)rows, st);
     else launch_k<8, 8, 4, 4, 1>(a, segs, (int)rows, st);
   } else {
@@ -1232,13 +1371,19 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
 // a launch against the general kernel: 16384 x 3072 8.2 / 16.4, 37888 x 3584
 // 19.4 / 33.3, 32768 x 1536 9.9 / 13.6), scale rows dword-aligned (they are
 // fetched as 16-byte runs).
-bool skinny2_mx_supported(int64_t N, int64_t K, const void* s) {
+// `products`: weights side by side (experts, batch entries), each starting where the last one ends.
+bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products) {
   static const bool off = experiment_env("QMM_NO_SKINNY_MX") != nullptr;
   if (off || N * (K / 2) >= 0x7FFFFFFFll) return false;       // 32-bit lane offsets
   if (K % 512 == 0) return K / 512 >= 3 && (reinterpret_cast<uintptr_t>(s) & 3u) == 0;
+  if ((reinterpret_cast<uintptr_t>(s) & 3u) || K % 64) return false;
+  // the ragged form over several passes: every weight's table starts on a dword (us a launch
+  // against the general kernel, 1 / 16 rows: 4096 x 11008 8.6 / 14.6 and 11.5 / 19.1, 14336 x 4224
+  // 12.6 / 16.2 and 15.2 / 21.7)
+  if (K > 4096) return products <= 1 || N * (K / 32) % 4 == 0;
   // the ragged one-pass form: K any multiple of 64 between three and eight slices, a tile's
   // scale rows a 16-byte-aligned run (every expert's table a multiple of 16 bytes, rows dealt by eights)
-  return K % 64 == 0 && K > 1024 && K < 4096 && (N * (K / 32)) % 16 == 0 &&
+  return K > 1024 && (N * (K / 32)) % 16 == 0 &&
          (reinterpret_cast<uintptr_t>(s) & 15u) == 0;
 }
 
@@ -1260,9 +1405,44 @@ static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products) {
 // For the plan query: whether a dense MXFP4 decode product of this shape runs here (tables taken as
 // aligned), and with how many rows a workgroup.
 bool skinny2_mx_plan(int64_t N, int64_t K, int* rows_per_wg) {
-  if (!skinny2_mx_supported(N, K, nullptr)) return false;
+  if (!skinny2_mx_supported(N, K, nullptr, 1)) return false;
   *rows_per_wg = (int)mx_rows_per_wg(N, K, 1);
   return true;
+}
+
+// Affine decode with a K that is no whole number of slices: the direct variants'
+// ragged forms, from a third slice on (us a launch against the general kernel,
+// four-bit codes in groups of 64, 1 / 5 / 16 rows: 8192 x 2944 6.8 / 7.0 / 7.7
+// against 11.7 / 12.4 / 14.2, 4096 x 11008 9.7 / 14.1 / 19.5 against 17.8 / 19.0 /
+// 24.3, 14336 x 4224 14.2 / 15.3 / 18.4 against 23.6 / 26.1 / 26.3; eight-bit 16384
+// x 1152 7.4 / 7.8 / 7.7 against 13.5 / 14.9 / 15.1; with several passes the
+// activations fetched when a pass begins are what bounds it).  Tables start on a dword (rows need not).
+// With four-bit codes, less than three whole slices (float32 tables: four) and at
+// most one tile a compute unit the general kernel's shorter start wins (4.6-4.9
+// against 4.8-5.1 us on 4096 x 1152).
+bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
+                              int64_t products) {
+  if ((gs != 64 && gs != 128) || K % 64 || K * bits / 8 <= 512 || K * bits / 8 % 256 == 0) return false;
+  if ((reinterpret_cast<uintptr_t>(s) & 3u) || (reinterpret_cast<uintptr_t>(b) & 3u)) return false;
+  if (bits == 4 && K < (tab == QMM_F32 ? 2048 : 1536) && products <= 1 && N <= 16 * device_cus()) return false;
+  const int64_t tbytes = N * (K / gs) * (tab == QMM_F32 ? 4 : 2);
+  if (products > 1 && tbytes % 4) return false;
+  return N * (K * bits / 8) < 0x7FFFFFFFll && tbytes < 0x7FFFFFFCll;   // 32-bit lane offsets
+}
+
+int64_t skinny2_ragged_rows(int64_t N, int64_t K, int64_t products) { return mx_rows_per_wg(N, K, products); }
+
+void skinny2_ragged_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int tab, hipStream_t st) {
+  GemvArgs a = a0;
+  a.gshift = 8 + affine_kind(gs, tab);
+  const int rows = (int)mx_rows_per_wg(a.N, a.K, batch);
+  if (a.K * bits / 8 <= 2048) {
+    if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, batch, rows, st);
+    else launch_k<8, 8, 4, 4, 1>(a, batch, rows, st);
+  } else {
+    if (bits == 4) launch_k<4, 8, 4, 8, 2>(a, batch, rows, st);
+    else launch_k<8, 8, 4, 8, 2>(a, batch, rows, st);
+  }
 }
 
 void skinny2_mx_dispatch(const GemvArgs& a0, int64_t batch, hipStream_t st) {
