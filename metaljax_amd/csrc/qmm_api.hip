@@ -22,11 +22,12 @@ bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, c
 int64_t skinny2_ragged_rows(int64_t N, int64_t K, int64_t products);
 bool skinny2_mx_plan(int64_t N, int64_t K, int* rows_per_wg);
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
-                               const void* s, const void* b, int64_t E);
+                               const void* s, const void* b, int64_t E, int64_t least_slices);
 void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, void* y,
                               int y_dtype, const int32_t* segments, const int32_t* src_row,
                               const int32_t* out_row, int64_t P, int64_t T, int64_t E, int64_t N,
-                              int64_t K, int gs, int bits, int mode, int tab, hipStream_t st);
+                              int64_t K, int gs, int bits, int mode, int tab, const int32_t* lhs_idx,
+                              const int32_t* rhs_idx, hipStream_t st);
 int64_t skinny2_max_segments(int64_t P, int64_t E);
 void gemm_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                    int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
@@ -111,6 +112,25 @@ constexpr int64_t kGatherGemvMaxPairs = 64;
 // by expert and every expert's weight is streamed once (grouped decode); below
 // it the sort's launch costs more than a shared expert saves.
 constexpr int64_t kGroupedDecodeMinPairs = 4;
+
+// Are these few pairs for the grouped decode whose workgroups sort them by
+// themselves (where it serves the shape)?  Otherwise every pair is a decode
+// product of its own.  From four pairs on; four-bit affine weights of
+// whole slices from two, unless the result is narrow (2 pairs over 16 of 2048 x
+// 4032: 6.7 / 7.1); with less than eight whole K-slices the per-pair products
+// are short and it takes more pairs (us, per pair or after a sort's launch /
+// here: four-bit, 8 experts of 4096 x 4096, 2 pairs 10.9 / 8.3, 16 pairs 36.9 /
+// 16.7; 16 of 1024 x 8192, 3 pairs 7.9 / 9.0, 4 pairs 15.4 / 9.3; 32 of 1024 x
+// 2048, 4 pairs 5.6 / 6.1, 6 pairs 8.8 / 7.0; MXFP4, 32 of 5760 x 2880, 3 pairs
+// 11.2 / 11.9, 4 pairs 22.5 / 13.3; 32 of 1024 x 2048, 32 pairs 10.4 / 11.4, 64
+// pairs 19.0 / 14.5).
+bool sorted_here_pairs(int64_t P, int64_t N, int64_t K, int bits, int mode) {
+  if (P > kGatherGemvMaxPairs) return false;
+  const bool mx = mode == QMM_MODE_MXFP4;
+  const int64_t row = K * (mx ? 4 : bits) / 8;
+  if (row % 256 == 0 && row < 8 * 256) return P >= (mx ? 48 : 6);
+  return P >= (!mx && bits == 4 && N >= 2048 && row % 256 == 0 ? 2 : 4);
+}
 
 int check_quant(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* w,
                 const void* s, const void* b) {
@@ -583,9 +603,16 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   hipStream_t st = static_cast<hipStream_t>(stream);
   static const bool no_grouped_decode = experiment_env("QMM_NO_GROUPED_DECODE") != nullptr;
+  // few pairs: the grouped decode whose workgroups sort them by themselves
+  if (sorted_here_pairs(P, N, K, bits, mode) && E > 0 && !(mode == QMM_MODE_AFFINE && table_dtype == QMM_F32 && group_size == 64) &&
+      skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E, 3)) {
+    skinny2_grouped_dispatch(x, w, scales, biases, y, y_dtype, nullptr, nullptr, nullptr, P, T, E, N, K,
+                             group_size, bits, mode, table_dtype, lhs_idx, rhs_idx, st);
+    return check_launch("grouped decode launch");
+  }
   if (grouped_decode_pairs(P, E) && !no_grouped_decode && workspace &&
       workspace_bytes >= route_bytes_segments(P, E) &&
-      skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E)) {
+      skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E, 8)) {
     int32_t* ro = static_cast<int32_t*>(workspace);
     int32_t* cursor = ro + E + 1;
     int32_t* src_row = cursor + E;
@@ -596,7 +623,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     rc = check_launch("route launch");
     if (rc) return rc;
     skinny2_grouped_dispatch(x, w, scales, biases, y, y_dtype, segments, src_row, out_row, P, T, E, N, K,
-                             group_size, bits, mode, table_dtype, st);
+                             group_size, bits, mode, table_dtype, nullptr, nullptr, st);
     return check_launch("grouped decode launch");
   }
   if (P <= kGatherGemvMaxPairs) {

@@ -177,7 +177,14 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD>
+// GRP: the grouped decode of at most 64 pairs that sorts them here.  Pair p of a.M multiplies row
+// lhs_idx[p] (p when null) of x, which has a.x_rows, by w[rhs_idx[p]], into row p of y; the
+// workgroups find the segments themselves and deal themselves over them, rows_per_wg of them to a
+// round of the compute units.  A form of its own, because its prologue costs the plain one 2-5 %.
+// (Workgroups of up to 128 rows a segment behind a sort's launch left the last round nearly empty
+// and paid 10 us for the sort: 16 MXFP4 pairs over 32 experts of 5760 x 2880 51 -> 30 us, 64 pairs
+// 88 -> 58, 16 four-bit pairs over 8 of 14336 x 4096 67 -> 43.)
+template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD, bool GRP>
 __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, int rows_per_wg) {
   load_args_now(a);
   asm volatile("" ::"s"(rows_per_wg));
@@ -216,6 +223,10 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // wavefront (staging of activations that come in with whole-line loads).
   unsigned char* patches = smem + 4 * (kItem + kTab);
   unsigned char* extras = patches + CW * 1024;    // EXTRA: 512 bytes a slot, scale | bias rows
+  // GRP: the rows of this workgroup's segment, 128 bytes a wavefront (each keeps
+  // its own copy): source rows [16] | result rows [16].
+  static_assert(!GRP || (XD != 0 && !WIDE), "a direct variant with LDS to spare");
+  int32_t* rowtab = reinterpret_cast<int32_t*>(extras + (EXTRA ? 2048 : 0)) + (threadIdx.x >> 6) * 32;
 
   const int lane = threadIdx.x & 63;
   // (Wavefronts start in the order of their hardware index, a whole workgroup
@@ -225,8 +236,57 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // 4096 x 14336 measured 10.6 against 9.9 us at one row, 13.3 against 11.4 us
   // at sixteen.)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t bz = blockIdx.y;
-  const int64_t n_begin = (int64_t)blockIdx.x * rows_per_wg;
+  int64_t bz = blockIdx.y;
+  uint32_t bx = blockIdx.x;
+  int M = a.M;
+  int seg_expert = 0;
+  if constexpr (GRP) {
+    // Pair `lane` names an expert; a segment is up to sixteen pairs of one
+    // expert, segments in the order of their first pair.  Lane s keeps the
+    // pairs of segment s.
+    // (One wavefront reads the indices for all: every wavefront has to come to
+    // the same segments, also if the caller were to write to them meanwhile.)
+    int32_t* idx = reinterpret_cast<int32_t*>(extras + (EXTRA ? 2048 : 0)) + (CW + NL) * 32;
+    if (threadIdx.x < kWave) {
+      idx[lane] = lane < a.M ? a.rhs_idx[lane] : -1;
+      idx[kWave + lane] = lane >= a.M ? -1 : a.lhs_idx ? a.lhs_idx[lane] : lane;
+    }
+    __syncthreads();
+    const int ex = idx[lane], src = idx[kWave + lane];
+    uint64_t left = __ballot(ex >= 0 && ex < a.n_experts), mine = 0;
+    int segs = 0;
+    while (left) {                              // (every turn takes a pair out)
+      const int e0 = __builtin_amdgcn_readlane(ex, __builtin_ctzll(left));
+      const uint64_t same = __ballot(ex == e0) & left;
+      const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+      const uint64_t take = same & __ballot(rank < 16u);
+      if (lane == segs) mine = take;
+      left &= ~take;
+      ++segs;
+    }
+    if (segs == 0) return;
+    // Workgroups a segment: as many as fill whole rounds of the compute units,
+    // with at least those that the tiles a workgroup may hold ask for.
+    const int tiles = (a.N + 15) / 16, least = XD == 2 ? (tiles + TMAX - 1) / TMAX : 1;
+    const int round = rows_per_wg, rounds = (segs * least + round - 1) / round;
+    int wgs = rounds * round / segs;
+    if (wgs > tiles) wgs = tiles;
+    const int seg = (int)bx / wgs;
+    if (seg >= segs) return;                    // uniform: before any barrier
+    bx -= (uint32_t)(seg * wgs);
+    rows_per_wg = (tiles + wgs - 1) / wgs * 16;
+    if ((int64_t)bx * rows_per_wg >= a.N) return;
+    const uint64_t take = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, seg) |
+                          (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), seg) << 32;
+    M = __builtin_popcountll(take);
+    seg_expert = __builtin_amdgcn_readlane(ex, __builtin_ctzll(take));
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(take >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)take, 0u));
+    if (take >> lane & 1) {
+      rowtab[rank] = src;
+      rowtab[16 + rank] = lane;
+    }
+  }
+  const int64_t n_begin = (int64_t)bx * rows_per_wg;
   const int64_t n_end = n_begin + rows_per_wg < a.N ? n_begin + rows_per_wg : a.N;
   const int ntiles = (int)((n_end - n_begin + 15) / 16);        // uniform, <= TMAX
   const int64_t wpr = (int64_t)a.K * BITS / 8;                  // bytes per weight row
@@ -257,19 +317,22 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   const int tailp = tail_codes * BITS / 128, tailc = tail_codes / 64;  // its 16-byte pieces | its 64-code chunks
   const uint32_t spitch = (uint32_t)(ng * ES);                 // bytes of a table row
 
-  int64_t xz = a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
-  int64_t wz = a.rhs_idx ? (int64_t)a.rhs_idx[bz] : bz;
+  int64_t xz = !GRP && a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
+  int64_t wz = !GRP && a.rhs_idx ? (int64_t)a.rhs_idx[bz] : bz;
   bool x_ok = true;
-  if (a.rhs_idx) {                                  // gather form: indices are data
+  if (!GRP && a.rhs_idx) {                  // gather form: indices are data
     if (wz < 0 || wz >= a.n_experts) return;        // uniform, before any barrier
     if (xz < 0 || xz >= a.n_xrows) { xz = 0; x_ok = false; }
   }
   // Rows of activations of this workgroup: a.M, or in the grouped form (direct
-  // variants only) those of segment blockIdx.y.
-  int M = a.M;
+  // variants only) those of its segment.
   const int32_t* src_row = nullptr;
   const int32_t* out_row = nullptr;
-  if (XD != 0 && a.segments) {
+  if constexpr (GRP) {
+    xz = 0;
+    wz = seg_expert;
+  }
+  if (XD != 0 && !GRP && a.segments) {
     if (bz >= a.segments[0]) return;              // uniform: before any barrier
     const int lo = a.segments[2 + 3 * bz];
     M = a.segments[3 + 3 * bz];
@@ -426,7 +489,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         const int64_t n = n_begin + t * 16 + (lane & 15);
         const bool row_ok = m < M && (PK == 0 || m < PK);
         int64_t yrow = bz * a.M + m;
-        if (out_row) yrow = row_ok ? (int64_t)out_row[m] : -1;
+        if (GRP) yrow = row_ok ? (int64_t)rowtab[16 + m] : -1;
+        else if (out_row) yrow = row_ok ? (int64_t)out_row[m] : -1;
         if (row_ok && yrow >= 0 && n < n_end) store_out(a.y, yrow * (int64_t)a.N + n, v, a.y_dtype);
       }
     };
@@ -551,7 +615,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     // rotated (measured with a fetch-only kernel).  The slices' sums are added
     // in slice order whoever computed them, so the results do not change.
     static_assert((CW & (CW - 1)) == 0, "slice rotation");
-    const int sw = XD == 1 ? (wave + (int)(blockIdx.x >> 3)) & (CW - 1) : wave;
+    const int sw = XD == 1 ? (wave + (int)(bx >> 3)) & (CW - 1) : wave;
     const uint32_t rowb = (uint32_t)(sw * 4096 + r * 256);      // this lane's row inside its slice's 4 KB
     // the operand row r of this lane is row xrow(r) of x (gathered in the grouped form)
     const int tab_row = MXRUN ? 0 : (sw >> 2) * (WIDE ? 2048 : 1024) + (sw & 3) * 256 + r * 16;   // this lane's table row inside a kind
@@ -559,12 +623,12 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     auto chunks_of = [&](int sl) __attribute__((always_inline)) { return RAG && sl == slices - 1 ? tailc : CPS; };
     // bits by which this lane's table row starts inside a dword (tiles are sixteen rows: the same for all)
     const uint32_t tsh = RAG && !F32T ? (uint32_t)((int)(n_begin + r) & (int)ng & 1) * 16u : 0u;
-    const int64_t xrows = src_row ? (int64_t)a.x_rows : (int64_t)a.M;
+    const int64_t xrows = GRP || src_row ? (int64_t)a.x_rows : (int64_t)a.M;
     const auto rxc = make_rsrc(a.x + xz * a.M * (int64_t)a.K, x_ok ? xrows * a.K * 2 : 0);
     auto xrow = [&](int m) -> int64_t {
       if (m >= M) return -1;
-      if (!src_row) return m;
-      const int64_t sr = src_row[m];
+      if (!GRP && !src_row) return m;
+      const int64_t sr = GRP ? rowtab[m] : src_row[m];
       return sr < xrows ? sr : -1;
     };
     const int64_t xr0 = xrow(r);
@@ -995,7 +1059,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         QMM_STAMP(0);
         if constexpr (!WIDE) {                    // (wide table rows leave no LDS for the staging patches)
           if (M > 8) {
-            switch ((blockIdx.x >> 6) & 3) {
+            switch ((bx >> 6) & 3) {
               case 0: fetch_x_staged(std::integral_constant<int, 0>{}, 0, active, 0); break;
               case 1: fetch_x_staged(std::integral_constant<int, 2>{}, 0, active, 0); break;
               case 2: fetch_x_staged(std::integral_constant<int, 4>{}, 0, active, 0); break;
@@ -1134,47 +1198,50 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   }
 }
 
-template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD>
-void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int chunks = 1) {
-  dim3 grid((unsigned)ceil_div(a.N, rows_per_wg), (unsigned)batch, (unsigned)chunks);
+template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD, bool GRP = false>
+void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int pair_wgs = 0) {
+  if constexpr (XD != 0 && !GRP && GSHIFT != 5 && GSHIFT != 13) {
+    if (pair_wgs) return launch_one<BITS, CW, NL, TMAX, GSHIFT, XD, true>(a, batch, rows_per_wg, st, pair_wgs);
+  }
+  dim3 grid(GRP ? (unsigned)pair_wgs : (unsigned)ceil_div(a.N, rows_per_wg), (unsigned)batch);
   constexpr bool wide = GSHIFT == 5 || GSHIFT == 13;
   constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (wide ? 2 : 1);
   constexpr int XR = XD ? 0 : 2048 / BITS / 128;
   // (direct variants: plus a 1 KB patch a compute wavefront for staging activations)
   const size_t lds = (size_t)(XD || XR + TMAX >= 4 ? 4 : XR + TMAX) * (CW * 4096 + 2 * kTabKind) +
-                     (XD != 0 && !wide ? (size_t)CW * 1024 : 0) +
+                     (XD != 0 && !wide ? (size_t)CW * 1024 : 0) + (GRP ? (CW + NL) * 128 + 512 : 0) +
                      (XD == 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11) ? 2048 : 0);      // (the kernel's EXTRA)
-  constexpr auto kern = skinny2_kernel<BITS, CW, NL, TMAX, GSHIFT, XD>;
+  constexpr auto kern = skinny2_kernel<BITS, CW, NL, TMAX, GSHIFT, XD, GRP>;
   if (!lds_limit<kern>(lds)) return;
   hipLaunchKernelGGL(kern, grid, dim3(kWave * (CW + NL)), lds, st, a, rows_per_wg);
 }
 
 template <int BITS, int CW, int NL, int TMAX, int XD>
-void launch_k(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int chunks = 1) {
+void launch_k(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int pair_wgs = 0) {
   if constexpr (BITS == 4 && XD != 0) {
-    if (a.gshift == 2) return launch_one<BITS, CW, NL, TMAX, 2, XD>(a, batch, rows_per_wg, st, chunks);
+    if (a.gshift == 2) return launch_one<BITS, CW, NL, TMAX, 2, XD>(a, batch, rows_per_wg, st, pair_wgs);
   }
   if constexpr (BITS == 4 && XD != 0) {
-    if (a.gshift == 7) return launch_one<BITS, CW, NL, TMAX, 7, XD>(a, batch, rows_per_wg, st, chunks);
+    if (a.gshift == 7) return launch_one<BITS, CW, NL, TMAX, 7, XD>(a, batch, rows_per_wg, st, pair_wgs);
   }
   if constexpr (XD != 0) {
     switch (a.gshift) {
-      case 8: return launch_one<BITS, CW, NL, TMAX, 8, XD>(a, batch, rows_per_wg, st, chunks);
-      case 9: return launch_one<BITS, CW, NL, TMAX, 9, XD>(a, batch, rows_per_wg, st, chunks);
-      case 11: return launch_one<BITS, CW, NL, TMAX, 11, XD>(a, batch, rows_per_wg, st, chunks);
-      case 12: return launch_one<BITS, CW, NL, TMAX, 12, XD>(a, batch, rows_per_wg, st, chunks);
-      case 13: return launch_one<BITS, CW, NL, TMAX, 13, XD>(a, batch, rows_per_wg, st, chunks);
-      case 14: return launch_one<BITS, CW, NL, TMAX, 14, XD>(a, batch, rows_per_wg, st, chunks);
+      case 8: return launch_one<BITS, CW, NL, TMAX, 8, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 9: return launch_one<BITS, CW, NL, TMAX, 9, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 11: return launch_one<BITS, CW, NL, TMAX, 11, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 12: return launch_one<BITS, CW, NL, TMAX, 12, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 13: return launch_one<BITS, CW, NL, TMAX, 13, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 14: return launch_one<BITS, CW, NL, TMAX, 14, XD>(a, batch, rows_per_wg, st, pair_wgs);
       default: break;
     }
   }
   switch (a.gshift) {
-    case 1: return launch_one<BITS, CW, NL, TMAX, 1, XD>(a, batch, rows_per_wg, st, chunks);
-    case 3: return launch_one<BITS, CW, NL, TMAX, 3, XD>(a, batch, rows_per_wg, st, chunks);
-    case 4: return launch_one<BITS, CW, NL, TMAX, 4, XD>(a, batch, rows_per_wg, st, chunks);
-    case 5: return launch_one<BITS, CW, NL, TMAX, 5, XD>(a, batch, rows_per_wg, st, chunks);
-    case 6: return launch_one<BITS, CW, NL, TMAX, 6, XD>(a, batch, rows_per_wg, st, chunks);
-    default: return launch_one<BITS, CW, NL, TMAX, 0, XD>(a, batch, rows_per_wg, st, chunks);
+    case 1: return launch_one<BITS, CW, NL, TMAX, 1, XD>(a, batch, rows_per_wg, st, pair_wgs);
+    case 3: return launch_one<BITS, CW, NL, TMAX, 3, XD>(a, batch, rows_per_wg, st, pair_wgs);
+    case 4: return launch_one<BITS, CW, NL, TMAX, 4, XD>(a, batch, rows_per_wg, st, pair_wgs);
+    case 5: return launch_one<BITS, CW, NL, TMAX, 5, XD>(a, batch, rows_per_wg, st, pair_wgs);
+    case 6: return launch_one<BITS, CW, NL, TMAX, 6, XD>(a, batch, rows_per_wg, st, pair_wgs);
+    default: return launch_one<BITS, CW, NL, TMAX, 0, XD>(a, batch, rows_per_wg, st, pair_wgs);
   }
 }
 
@@ -1320,13 +1387,13 @@ bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, c
 static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products);
 
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
-                               const void* s, const void* b, int64_t E) {
+                               const void* s, const void* b, int64_t E, int64_t least_slices) {
   if (mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, E)) return true;
   // (MXFP4 whose K is no whole number of slices has no other staged kernel to go to: its ragged
   // one-pass form takes the grouped decode from three slices on)
-  if (mode == QMM_MODE_MXFP4) return (K / 512 >= 8 || K % 512 != 0) && skinny2_mx_supported(N, K, s, E);
+  if (mode == QMM_MODE_MXFP4) return (K / 512 >= least_slices || K % 512 != 0) && skinny2_mx_supported(N, K, s, E);
   if (!skinny_supported(N, K, gs, bits, mode, QMM_BF16, s, b)) return false;   // bf16, float16 and float32 tables alike
-  return K * bits / 8 / 256 >= 8;
+  return K * bits / 8 / 256 >= least_slices;
 }
 
 int64_t skinny2_max_segments(int64_t P, int64_t E) { return (E < P ? E : P) + P / 16; }
@@ -1334,7 +1401,8 @@ int64_t skinny2_max_segments(int64_t P, int64_t E) { return (E < P ? E : P) + P 
 void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, void* y,
                               int y_dtype, const int32_t* segments, const int32_t* src_row,
                               const int32_t* out_row, int64_t P, int64_t T, int64_t E, int64_t N,
-                              int64_t K, int gs, int bits, int mode, int tab, hipStream_t st) {
+                              int64_t K, int gs, int bits, int mode, int tab, const int32_t* lhs_idx,
+                              const int32_t* rhs_idx, hipStream_t st) {
   GemvArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.w = static_cast<const uint32_t*>(w);
@@ -1343,10 +1411,12 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   a.y = y;
   a.M = 1; a.N = (int)N; a.K = (int)K;
   const bool ragged = K * bits / 8 % 256 != 0;
+  const bool sorted_here = rhs_idx != nullptr;
   a.gshift = mode == QMM_MODE_MXFP4 ? (ragged ? 7 : 2) : (ragged ? 8 : 0) + affine_kind(gs, tab);
   a.y_dtype = y_dtype;
-  a.lhs_idx = nullptr;
-  a.rhs_idx = nullptr;
+  a.lhs_idx = lhs_idx;
+  a.rhs_idx = rhs_idx;
+  a.n_experts = (int)E;
   a.segments = segments;
   a.src_row = src_row;
   a.out_row = out_row;
@@ -1357,6 +1427,20 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   if (rows < 16) rows = 16;
   if (mode == QMM_MODE_MXFP4 || ragged) rows = mx_rows_per_wg(N, K, P < E ? P : E);
   const int64_t segs = skinny2_max_segments(P, E);
+  if (sorted_here) {
+    // workgroups dealt over the segments there are: enough for the most there can be
+    const int64_t tiles = ceil_div(N, (int64_t)16), least = K * bits / 8 <= 2048 ? 1 : ceil_div(tiles, (int64_t)8);
+    a.M = (int)P;
+    const int wgs = (int)(ceil_div(std::min(P, segs) * least, cus) * cus);
+    if (K * bits / 8 <= 2048) {
+      if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, 1, (int)cus, st, wgs);
+      else launch_k<8, 8, 4, 4, 1>(a, 1, (int)cus, st, wgs);
+    } else {
+      if (bits == 4) launch_k<4, 8, 4, 8, 2>(a, 1, (int)cus, st, wgs);
+      else launch_k<8, 8, 4, 8, 2>(a, 1, (int)cus, st, wgs);
+    }
+    return;
+  }
   if (K * bits / 8 <= 2048) {
     if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, segs, (int)rows, st);
     else launch_k<8, 8, 4, 4, 1>(a, segs, (int)rows, st);
@@ -1377,6 +1461,9 @@ bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products)
   if (off || N * (K / 2) >= 0x7FFFFFFFll) return false;       // 32-bit lane offsets
   if (K % 512 == 0) return K / 512 >= 3 && (reinterpret_cast<uintptr_t>(s) & 3u) == 0;
   if ((reinterpret_cast<uintptr_t>(s) & 3u) || K % 64) return false;
+  // a second pass for part of a slice, one tile a compute unit: the general kernel (4096 x 4160 at 1 / 5 /
+  // 16 rows 6.5 / 7.2 / 9.4 against 7.0 / 7.1 / 10.1 us)
+  if (K > 4096 && K < 4608 && N <= 16 * device_cus()) return false;
   // the ragged form over several passes: every weight's table starts on a dword (us a launch
   // against the general kernel, 1 / 16 rows: 4096 x 11008 8.6 / 14.6 and 11.5 / 19.1, 14336 x 4224
   // 12.6 / 16.2 and 15.2 / 21.7)

@@ -71,7 +71,7 @@ def test_a_rows_tables_stay_its_own(k, kind):
 
 @pytest.mark.parametrize("k", [1856, 2944, 11072, 11136])
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("pairs,experts", [(3, 5), (40, 6), (90, 7)])
+@pytest.mark.parametrize("pairs,experts", [(3, 5), (40, 6), (64, 2), (90, 7)])
 def test_experts(pairs, experts, k, kind):
     bits, gs, mode, tab = kind
     if k % gs:
