@@ -1422,10 +1422,7 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   a.out_row = out_row;
   a.x_rows = (int)T;
   const int64_t cus = device_cus();
-  const int64_t rounds = ceil_div(ceil_div(N, cus), (int64_t)128);
-  int64_t rows = ceil_div(N, cus * rounds);
-  if (rows < 16) rows = 16;
-  if (mode == QMM_MODE_MXFP4 || ragged) rows = mx_rows_per_wg(N, K, P < E ? P : E);
+  const int64_t rows = mx_rows_per_wg(N, K, P < E ? P : E);
   const int64_t segs = skinny2_max_segments(P, E);
   if (sorted_here) {
     // workgroups dealt over the segments there are: enough for the most there can be
@@ -1474,10 +1471,12 @@ bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products)
          (reinterpret_cast<uintptr_t>(s) & 15u) == 0;
 }
 
-// Rows a workgroup for the MXFP4 decode: `products` decode products run side by side (batch entries,
+// Rows a workgroup for the MXFP4, ragged and grouped decode: `products` decode products run side by side (batch entries,
 // the segments of a grouped product), so each gets its share of the compute units -- a workgroup's
 // fixed cost (its first tile lands about 3.5 us after it starts) is then paid once a compute unit, not
-// once per product.  For the ragged form a multiple of eight (see above).
+// once per product (grouped, four-bit codes, us against a share of all compute units for every
+// segment: 128 pairs over 8 experts of 4096 x 4096 38.6 / 66.8, over 32 of 2048 x 4096 40.8 / 81.7; 256
+// over 32 of 2048 x 4096 44.0 / 96.9).  For the ragged form a multiple of eight (see above).
 static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products) {
   const int64_t cus = device_cus();
   if (products < 1) products = 1;
