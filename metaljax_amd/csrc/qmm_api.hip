@@ -322,9 +322,9 @@ size_t route_bytes_segments(int64_t P, int64_t E) {
 }
 
 // Pairs up to which the grouped decode (one decode product per expert and
-// sixteen pairs) beats the grouped prefill kernel: measured on 8 experts of
-// 14336 x 4096: 128 pairs 151 against 235 us, 256 pairs 239 against 244 us, 512
-// pairs 436 against 237 us.
+// sixteen pairs) is taken: 8 experts of 14336 x 4096, 128 pairs 94 us here, 256
+// pairs 120 us and 512 pairs 163 us on the row-group kernels; 32 experts of 2048 x
+// 4096, 256 pairs 44 us and 512 pairs 63 us here.
 bool grouped_decode_pairs(int64_t P, int64_t E) {
   static const int64_t gd_max = experiment_env("QMM_GD_MAX") ? atoll(experiment_env("QMM_GD_MAX")) : 0;
   if (P < kGroupedDecodeMinPairs) return false;
