@@ -539,9 +539,12 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
   if (gemm2s_wanted(a, mode, bits)) {
     const size_t prep = gemm2_workspace_bytes(R, K);
     a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + prep);
-    gemm2s_plan(R, row_offsets ? E : 1, N, K, workspace_bytes > prep ? workspace_bytes - prep : 0, &a.tile_rows, &a.splits);
+    // (row groups keep their whole K, also those of a single expert: their tiles are
+    // found in the kernel, which deals no K ranges over them)
+    gemm2s_plan(R, row_offsets ? E : 1, N, K, !row_offsets && workspace_bytes > prep ? workspace_bytes - prep : 0, &a.tile_rows,
+                &a.splits);
     gemm2s_launch(a, mode, bits, st);
-    if (a.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, a.splits, nullptr, 1, out_idx, st);
+    if (a.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, a.splits, nullptr, 1, nullptr, st);
     return;
   }
   const int mt = row_tile >= 256 ? 2 : 1;

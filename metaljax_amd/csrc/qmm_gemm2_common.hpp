@@ -47,7 +47,7 @@ struct Gemm2Args {
   int tabfast;           // general kernel: float32 tables of groups of 32, fetched as windows
   int tab_ok, tab_odd;   // split-role kernel: tables start on dwords; their rows may start inside one
   int tile_rows;         // split-role kernel: rows a tile may hold (128 or 256)
-  int splits;            // split-role kernel, dense: workgroups that share a tile's K ...
+  int splits;            // split-role kernel, dense (1 with row_offsets): workgroups that share a tile's K ...
   float* part;           // ... and leave their float32 sums here, [splits][R][N]
 };
 

@@ -574,9 +574,10 @@ bool gemm2s_wanted(const g2::Gemm2Args& a, int mode, int bits) {
 // on average) to 700 measured products of 17 to 2048 rows, N and K 1024 to
 // 14336: the launches, a round for every 256 tiles (one workgroup fills a
 // compute unit), a K-tile of up to 128 or up to 256 rows, the re-laid
-// activations, the result, and a split K's sums.  The grouped product keeps
-// 256-row tiles (every expert in one, and the short loop where it fits) and its
-// whole K.
+// activations, the result, and a split K's sums.  Several experts keep 256-row
+// tiles (every expert in one, and the short loop where it fits) and their whole
+// K; for the row groups of a single expert (`row_offsets` with E = 1) the caller
+// passes no room for sums, so that they keep theirs.
 double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits) {
   const char* er = experiment_env("QMM_G2S_ROWS");
   const char* es = experiment_env("QMM_G2S_SPLITS");

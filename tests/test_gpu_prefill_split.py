@@ -73,3 +73,33 @@ def test_groups(counts, kind, act, gathered):
         y = K.gather_qmm(x, w, s, b, mix.int(), owner[mix].int(), out_dtype=torch.float32, **how)
         if sum(counts) > 16 * len(counts):
             close(y, want[mix])
+
+
+# One expert is a dense product but for its offsets: rows outside them, and pairs
+# that name no expert, are left alone, and nothing is written round the result.
+# The sizes are those for which a dense product of as many rows splits its K on the
+# prefill kernel (two or three ways), and for which no split is still ahead of the
+# short-group kernel.
+@pytest.mark.parametrize("r,n,k", [(650, 3080, 6144), (1000, 2056, 6144), (1250, 1544, 8256)])
+@pytest.mark.parametrize("kind", [KINDS[0], KINDS[3]])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_one_expert(r, n, k, kind, gathered):
+    bits, gs, mode, tab = kind
+    g = torch.Generator(device=DEV).manual_seed(r + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (1,), n, k, bits, gs, mode, tab)
+    x = torch.randn((r, k), device=DEV, generator=g).bfloat16()
+    guarded = torch.full((r + 128, n), 7.0, device=DEV)
+    y = guarded[64:64 + r]
+    want = x.double() @ tile(w[0], s[0], b[0], how).T
+    if gathered:
+        rhs = torch.randint(-1, 2, (r,), dtype=torch.int32, device=DEV, generator=g)
+        lhs = torch.randperm(r, device=DEV, generator=g).int()
+        K.BoundGather(x, w, s, b, lhs, rhs, y, **how).launch()
+        live, want = rhs == 0, want[lhs.long()]
+    else:
+        live = torch.zeros(r, dtype=torch.bool, device=DEV)
+        live[7:r - 13] = True
+        K.BoundGrouped(x, w, s, b, torch.tensor([7, r - 13], dtype=torch.int32, device=DEV), y, **how).launch()
+    close(y[live], want[live])
+    assert bool((y[~live] == 7).all()) and bool((guarded[:64] == 7).all()) and bool((guarded[64 + r:] == 7).all())
