@@ -331,6 +331,15 @@ bool grouped_decode_pairs(int64_t P, int64_t E) {
   return gd_max ? P <= gd_max : P <= 16 * E && P <= 4096;
 }
 
+// Are these pairs for the grouped decode behind a sort's launch?  (`workspace_bytes`
+// hold the sort's arrays and the segment list.)
+bool grouped_decode_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
+                           const void* s, const void* b, size_t workspace_bytes) {
+  static const bool off = experiment_env("QMM_NO_GROUPED_DECODE") != nullptr;
+  return grouped_decode_pairs(P, E) && !off && workspace_bytes >= route_bytes_segments(P, E) &&
+         skinny2_grouped_supported(N, K, gs, bits, mode, tab, s, b, E, 8);
+}
+
 // ---- float16 / float32 activations ---------------------------------------------
 // The kernels multiply bf16 operands.  Wider activations are split, exactly,
 // into bf16 terms (float16: two, float32: three), every term is multiplied
@@ -686,7 +695,6 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
   if (P > INT32_MAX / 2 || N > INT32_MAX || K > INT32_MAX || E > 65535 || T * K >= (1ll << 30))
     return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  static const bool no_grouped_decode = experiment_env("QMM_NO_GROUPED_DECODE") != nullptr;
   // few pairs: the grouped decode whose workgroups sort them by themselves
   if (sorted_here_pairs(P, N, K, bits, mode) && E > 0 && !(mode == QMM_MODE_AFFINE && table_dtype == QMM_F32 && group_size == 64) &&
       skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E, 3)) {
@@ -694,9 +702,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
                              group_size, bits, mode, table_dtype, lhs_idx, rhs_idx, st);
     return check_launch("grouped decode launch");
   }
-  if (grouped_decode_pairs(P, E) && !no_grouped_decode && workspace &&
-      workspace_bytes >= route_bytes_segments(P, E) &&
-      skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E, 8)) {
+  if (workspace && grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, workspace_bytes)) {
     int32_t* ro = static_cast<int32_t*>(workspace);
     int32_t* cursor = ro + E + 1;
     int32_t* src_row = cursor + E;
@@ -862,9 +868,15 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   if (terms == 1 || P <= 0 || T < 0 || E < 0 || N <= 0 || K <= 0 || !x || !rhs_idx || !y)
     return gather_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, lhs_idx, rhs_idx, P, T, E,
                        N, K, group_size, bits, mode, workspace, workspace_bytes, stream, false);
-  // more pairs than the decode kernels take: short groups read float16 / float32
-  // activations as they are
-  if (P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
+  // More pairs than the decode kernels take: short groups read float16 / float32
+  // activations as they are.  Not where the grouped decode multiplies affine weights:
+  // it keeps them exact, the short-group kernel rounds them to bf16 (1e-6 against
+  // 1.6e-3 from the product of the exact weights, 128 pairs over 8 experts of 1024 x
+  // 4096, eight-bit codes).  MXFP4 weights are exact in both.
+  const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
+                            K % group_size == 0 &&
+                            grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
+  if (!exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
       short_wins(P, E, N, K, bits, mode, terms) && workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
       short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, terms, scales, biases)) {
     const size_t need = route_bytes(P, E);

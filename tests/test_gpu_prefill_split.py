@@ -103,3 +103,21 @@ def test_one_expert(r, n, k, kind, gathered):
         K.BoundGrouped(x, w, s, b, torch.tensor([7, r - 13], dtype=torch.int32, device=DEV), y, **how).launch()
     close(y[live], want[live])
     assert bool((y[~live] == 7).all()) and bool((guarded[:64] == 7).all()) and bool((guarded[64 + r:] == 7).all())
+
+
+# Up to sixteen pairs an expert the grouped decode multiplies float16 / float32
+# activations too, term by term: with the exact weights, not their bf16 tile, which
+# is 1.5e-3 away (the sums are float32: the bound of the other products).
+@pytest.mark.parametrize("pairs,experts", [(65, 8), (128, 8), (200, 16)])
+@pytest.mark.parametrize("k,kind", [(4096, KINDS[0]), (4096, KINDS[2]), (2048, KINDS[3]), (2944, KINDS[0])])
+@pytest.mark.parametrize("act", ["f16", "f32"])
+def test_wide_gathers_keep_their_weights(pairs, experts, k, kind, act):
+    bits, gs, mode, tab = kind
+    g = torch.Generator(device=DEV).manual_seed(pairs + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (experts,), 1024, k, bits, gs, mode, tab)
+    x = torch.randn((pairs, k), device=DEV, generator=g).to(ACT[act])
+    rhs = torch.randint(0, experts, (pairs,), dtype=torch.int32, device=DEV, generator=g)
+    full = K.dequantize(w, s, b, out_dtype=torch.float32, **how).double()
+    want = torch.stack([full[rhs[p]] @ x[p].double() for p in range(pairs)])
+    close(K.gather_qmm(x, w, s, b, None, rhs, out_dtype=torch.float32, **how), want)
