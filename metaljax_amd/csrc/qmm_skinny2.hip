@@ -1,9 +1,9 @@
 // Decode-regime affine quantized matmul (M <= 16) with loader wavefronts.
 //
-// Same arithmetic as qmm_skinny.hip (codes exact in bf16, two
+// Arithmetic as in qmm_skinny.hip (codes exact in bf16, two
 // v_mfma_f32_16x16x32_bf16 per 64-code chunk, scale applied to the chunk's
-// dot, the code-independent terms as small MFMAs over the chunk index); what
-// differs is who moves the bytes.
+// dot; the code-independent terms are added closer to what cancels them, see
+// the chunk sums below); what differs is who moves the bytes.
 //
 // A compute unit cannot keep its whole share of the weight (about 130 KB for
 // the 4096 x 14336 case) in flight: vector-memory instructions are accepted at
@@ -641,32 +641,83 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
       sl_cur[S::item_at(j)] = j;
     });
     bf16x8 xa[CPS][2];
-    // The code-independent part of a tile's sums is sum_c t_c * xs_c over the
-    // chunks c of the slice, xs_c = sum_k x over chunk c, for every table entry
-    // t that multiplies a constant: the bias, and for four-bit codes (widened
-    // as 128 + q) the scale times -128.  It runs on the matrix cores with the
-    // chunk index as the K dimension: xs_c is split into three bf16 terms
-    // (24 bits, exact), a float16 / float32 table entry into two / three.  A
-    // slice has eight chunks and the instruction's K is 32, so four (x term,
-    // table term) pairs share one MFMA, one per lane quarter kg: pair g =
-    // (kind, table term, x term) sits in MFMA g / 4, quarter g % 4.  The A
-    // operands depend on the activations only and are built once; bf16 tables
-    // with four-bit codes take two MFMAs a tile this way instead of six.
+    // What a chunk's dot holds besides the codes: the sum of its activations, xs_c,
+    // times the bias, and with four-bit codes, widened as 128 + q, times 128 before
+    // the scale.  Both are larger than what the codes leave (zero points lie inside
+    // the range of the codes), so where they are added decides the error of the
+    // float32 sums.
+    //
+    // The 128 (thirty times what the codes leave): the dot of a chunk starts from
+    // -128 xs_c, and they are gone before the chunk is added to anything.  (As one
+    // more term over the whole slice, beside the biases', they stood in the sums
+    // until the last chunk.  Distance from float64, 4096 x 11008 and 4096 x 1088,
+    // bf16 tables, zero points 6 to 10: 2.3e-6 and 1.7e-6 then, 0.42e-6 and 0.40e-6
+    // now; the general kernel, which multiplies xs_c by bias - 128 scale: 1.0e-6
+    // and 0.89e-6.  One row of 4096 x 4096 5.6 -> 5.5 us, 14336 x 4096 9.5 -> 9.3,
+    // and 17.2 -> 12.8 of 8192 x 8192 with float32 tables, whose scales need no
+    // splitting any more.)  The start values sit in registers (XC_REG) or, where
+    // eight tiles' sums and eight chunks' activations fill those, in the
+    // wavefront's patch, one float a row and chunk (XC_LDS: 8192 x 8192 at one row
+    // 11.4 us, from registers that spill 13.7); float32 tables in groups of 64
+    // leave no room for either and have two more MFMAs a chunk.
+    //
+    // The biases.  Eight-bit codes: behind a chunk's dot, as in the general kernel;
+    // four chunks' sums fit the registers.  (As one term in front of the first
+    // chunk 1984 codes a row with float32 tables were 1.5e-7 from float64, now and
+    // in the general kernel 1.1e-7.)  Four-bit codes: sum_c bias_c * xs_c runs on
+    // the matrix cores with the chunk index as the K dimension.  xs_c is split into
+    // three bf16 terms (24 bits, exact), a float16 / float32 table entry into two /
+    // three.  A slice has eight chunks and the instruction's K is 32, so four
+    // (x term, table term) pairs share one MFMA, one per lane quarter kg: pair g =
+    // (table term, x term) sits in MFMA g / 4, quarter g % 4.  The A operands
+    // depend on the activations only and are built once.
+    //
+    // SCALE_TERM: four-bit codes over several passes of whole slices with bf16 tables
+    // still add -128 scale_c * xs_c beside the biases' term (kind 1 of the table
+    // terms), at the error above: no registers are left there to read a chunk's
+    // start values from LDS ahead of it, and where the last pass has few slices that
+    // shows (11008 x 5120 at one row 10.6 against 11.6 us; at sixteen, in the ring
+    // variant with start values in registers, 15.0 against 15.6).
     constexpr int NT = F32T ? 3 : F16T ? 2 : 1;     // bf16 terms per table entry
-    constexpr int NG = (BITS == 4 ? 2 : 1) * NT * 3;
+    constexpr bool SCALE_TERM = BITS == 4 && XD != 1 && !RAG && NT == 1;
+    constexpr int NG = BITS == 4 ? (SCALE_TERM ? 2 : 1) * NT * 3 : 0;
     constexpr int NA = (NG + 3) / 4;
-    bf16x8 ax[NA];
+    constexpr bool XC_REG = BITS == 8 || XD == 1 || (XD == 0 && !WIDE && !SCALE_TERM);
+    constexpr bool XC_LDS = !XC_REG && !WIDE && !SCALE_TERM;
+    static_assert(!XC_LDS || XD != 0, "the ring variant has no patches");
+    bf16x8 ax[NA ? NA : 1];
+    f32x4 xc[XC_REG ? CPS : 1];
+    float* const xc_lds = reinterpret_cast<float*>(patches + wave * 1024);
+    const uint32_t xf = MX ? 0u : pin_vgpr(BITS == 4 ? 0xC300C300u : kOnesBf16x2);      // -128 | 1
+    auto chunk_sum = [&](int c) __attribute__((always_inline)) {              // in the layout of the results
+      const f32x4 t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], as_bf16x8(xf, xf, xf, xf), zero, 0, 0, 0);
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][1], as_bf16x8(xf, xf, xf, xf), t, 0, 0, 0);
+    };
     auto chunk_sums = [&]() __attribute__((always_inline)) {
-      float xt[3][8];
+      if constexpr (XC_REG) {
+#pragma unroll
+        for (int c = 0; c < CPS; ++c) xc[c] = chunk_sum(c);
+      }
+      if constexpr (BITS == 8) return;
+      float xs[8], xt[3][8];
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
-        float xs = 0.f;
+        xs[c] = 0.f;
         if (c < CPS) {
           f32x4 t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xa[c][0], zero, 0, 0, 0);
           t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xa[c][1], t4, 0, 0, 0);
-          xs = t4[0];                               // every row of the product holds the column's sum
+          xs[c] = t4[0];                            // every row of the product holds the column's sum
         }
-        split3(xs, xt[0][c], xt[1][c], xt[2][c]);
+        split3(xs[c], xt[0][c], xt[1][c], xt[2][c]);
+      }
+      if constexpr (XC_LDS) {
+        // (all four lanes of a row know its sums: each writes two chunks')
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          xc_lds[(2 * kg + h) * 16 + r] = -128.f * (kg == 0 ? xs[h] : kg == 1 ? xs[2 + h] : kg == 2 ? xs[4 + h] : xs[6 + h]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
       static_for<NA>([&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
@@ -676,9 +727,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         static_for<4>([&](auto qc) __attribute__((always_inline)) {
           constexpr int g = 4 * i + decltype(qc)::value;
           if constexpr (g < NG) {
-            constexpr float f = g / (3 * NT) ? -128.f : 1.f;      // exact: a power of two
 #pragma unroll
-            for (int c = 0; c < 8; ++c) v[c] = kg == (g & 3) ? f * xt[g % 3][c] : v[c];
+            for (int c = 0; c < 8; ++c) v[c] = kg == (g & 3) ? (g / 3 == NT ? -128.f : 1.f) * xt[g % 3][c] : v[c];   // exact
           }
         });
         ax[i] = as_bf16x8(hi16_pair(v[0], v[1]), hi16_pair(v[2], v[3]), hi16_pair(v[4], v[5]), hi16_pair(v[6], v[7]));
@@ -752,23 +802,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           bvt[i] &= keep;
         }
       }
-      // eight table entries as matrix operands over the chunk index: one bf16
-      // operand, or for float16 tables two (hi + lo, exact: 11 significant bits)
-      auto split_f16 = [&](const u32x4& t, bf16x8& hi, bf16x8& lo) __attribute__((always_inline)) {
-        uint32_t h[4], l[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float f0 = f16_bits_to_f32(t[i] & 0xFFFFu), f1 = f16_bits_to_f32(t[i] >> 16);
-          const float h0 = __uint_as_float(__float_as_uint(f0) & 0xFFFF0000u);
-          const float h1 = __uint_as_float(__float_as_uint(f1) & 0xFFFF0000u);
-          h[i] = hi16_pair(h0, h1);
-          l[i] = hi16_pair(f0 - h0, f1 - h1);     // at most three significant bits: exact in bf16
-        }
-        hi = as_bf16x8(h[0], h[1], h[2], h[3]);
-        lo = as_bf16x8(l[0], l[1], l[2], l[3]);
-      };
       // float32 tables: the entries of the eight chunks as floats (group 128: one
-      // entry serves two chunks), and as matrix operands three bf16 terms each
+      // entry serves two chunks)
       float sf[8], bfv[8];
       if constexpr (F32T) {
         if constexpr (WIDE) {
@@ -794,26 +829,32 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           }
         }
       }
-      // the bf16 terms of the table entries as matrix operands over the chunk
-      // index: tt[kind * NT + term], kind 0 = bias, 1 = scale
-      bf16x8 tt[2 * NT];
-      if constexpr (F32T) {
-        auto terms = [&](const float (&v)[8], bf16x8* out) __attribute__((always_inline)) {
-          float h[8], m[8], l[8];
+      // four-bit codes: the bf16 terms of the biases (and with SCALE_TERM the scales) as matrix operands over the chunk index
+      bf16x8 tt[NT + SCALE_TERM];
+      if constexpr (BITS == 8) {
+      } else if constexpr (F32T) {
+        float h[8], m[8], l[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) split3(v[i], h[i], m[i], l[i]);
-          out[0] = as_bf16x8(hi16_pair(h[0], h[1]), hi16_pair(h[2], h[3]), hi16_pair(h[4], h[5]), hi16_pair(h[6], h[7]));
-          out[1] = as_bf16x8(hi16_pair(m[0], m[1]), hi16_pair(m[2], m[3]), hi16_pair(m[4], m[5]), hi16_pair(m[6], m[7]));
-          out[2] = as_bf16x8(hi16_pair(l[0], l[1]), hi16_pair(l[2], l[3]), hi16_pair(l[4], l[5]), hi16_pair(l[6], l[7]));
-        };
-        terms(bfv, tt);
-        if constexpr (BITS == 4) terms(sf, tt + NT);
+        for (int i = 0; i < 8; ++i) split3(bfv[i], h[i], m[i], l[i]);
+        tt[0] = as_bf16x8(hi16_pair(h[0], h[1]), hi16_pair(h[2], h[3]), hi16_pair(h[4], h[5]), hi16_pair(h[6], h[7]));
+        tt[1] = as_bf16x8(hi16_pair(m[0], m[1]), hi16_pair(m[2], m[3]), hi16_pair(m[4], m[5]), hi16_pair(m[6], m[7]));
+        tt[2] = as_bf16x8(hi16_pair(l[0], l[1]), hi16_pair(l[2], l[3]), hi16_pair(l[4], l[5]), hi16_pair(l[6], l[7]));
       } else if constexpr (F16T) {
-        split_f16(bvt, tt[0], tt[1]);
-        if constexpr (BITS == 4) split_f16(svt, tt[2], tt[3]);
+        // hi + lo, exact: 11 significant bits
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float f0 = f16_bits_to_f32(bvt[i] & 0xFFFFu), f1 = f16_bits_to_f32(bvt[i] >> 16);
+          const float h0 = __uint_as_float(__float_as_uint(f0) & 0xFFFF0000u);
+          const float h1 = __uint_as_float(__float_as_uint(f1) & 0xFFFF0000u);
+          h[i] = hi16_pair(h0, h1);
+          l[i] = hi16_pair(f0 - h0, f1 - h1);     // at most three significant bits: exact in bf16
+        }
+        tt[0] = as_bf16x8(h[0], h[1], h[2], h[3]);
+        tt[1] = as_bf16x8(l[0], l[1], l[2], l[3]);
       } else {
         tt[0] = __builtin_bit_cast(bf16x8, bvt);
-        if constexpr (BITS == 4) tt[1] = __builtin_bit_cast(bf16x8, svt);
+        if constexpr (SCALE_TERM) tt[1] = __builtin_bit_cast(bf16x8, svt);
       }
       f32x4 at = acc_in;
       static_for<NA>([&](auto ic) __attribute__((always_inline)) {
@@ -834,7 +875,12 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         if constexpr (BITS == 4) {
           const uint32_t pc = (uint32_t)(2 * c + (kg >> 1));
           const u32x2 q = *reinterpret_cast<const u32x2*>(base + ((pc ^ swz) << 4) + (kg & 1) * 8);
-          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], widen_int4(q[0], nib, magic), zero, 0, 0, 0);
+          f32x4 from;
+          if constexpr (SCALE_TERM) from = zero;
+          else if constexpr (XC_REG) from = xc[c];
+          else if constexpr (XC_LDS) from = *reinterpret_cast<const f32x4*>(xc_lds + c * 16 + kg * 4);
+          else from = chunk_sum(c);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], widen_int4(q[0], nib, magic), from, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][1], widen_int4(q[1], nib, magic), d, 0, 0, 0);
         } else {
           const uint32_t pc = (uint32_t)(4 * c + kg);
@@ -842,13 +888,19 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], widen_int8(q[0], q[1]), zero, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][1], widen_int8(q[2], q[3]), d, 0, 0, 0);
         }
-        const uint32_t sw = svt[c >> 1];
-        float sc;
-        if constexpr (F32T) sc = sf[c];
-        else if constexpr (F16T) sc = f16_bits_to_f32((c & 1) ? sw >> 16 : sw & 0xFFFFu);
-        else sc = __uint_as_float((c & 1) ? (sw & 0xFFFF0000u) : (sw << 16));
+        auto entry = [&](const u32x4& t) __attribute__((always_inline)) {     // chunk c's of a 16-bit table
+          const uint32_t v = t[c >> 1];
+          if constexpr (F16T) return f16_bits_to_f32((c & 1) ? v >> 16 : v & 0xFFFFu);
+          else return __uint_as_float((c & 1) ? (v & 0xFFFF0000u) : (v << 16));
+        };
+        const float sc = F32T ? sf[c] : entry(svt);
 #pragma unroll
         for (int e = 0; e < 4; ++e) at[e] = fmaf(sc, d[e], at[e]);
+        if constexpr (BITS == 8) {
+          const float bi = F32T ? bfv[c] : entry(bvt);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) at[e] = fmaf(bi, xc[c][e], at[e]);
+        }
       }
       return at;
     };

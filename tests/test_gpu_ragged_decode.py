@@ -86,3 +86,29 @@ def test_experts(pairs, experts, k, kind):
     full = exact(w, s, b, how)
     want = torch.stack([full[rhs[p]] @ x[lhs[p]].double() for p in range(pairs)])
     close(K.gather_qmm(x, w, s, b, lhs, rhs, out_dtype=torch.float32, **how), want)
+
+
+# How far float32 results are from the product in double precision where zero points
+# lie in the middle of the codes' range, as a checkpoint's do: what cancels must be
+# gone before a chunk of 64 is added to the others.  In units of scale times the
+# activations' deviation, a rounding being 2.5e-8 of the value (2^-23 / sqrt 12,
+# averaged over a binade): four-bit codes leave 4.6 * 8 a chunk and one rounding of
+# half a chunk's 128 * sqrt 32, together 4.9e-7; eight-bit codes leave 74 * 8 a chunk
+# of sums of 148 * 8, rounded four times a chunk, together 1.1e-7.  (Added over a
+# slice before the codes are: 1.7e-6 to 2.9e-6, and 1.2e-7 to 1.6e-7 with float32
+# tables.)
+@pytest.mark.parametrize("m,n,k", [(1, 4104, 1984), (5, 4104, 1088), (3, 4104, 4160), (16, 1032, 11008), (5, 2056, 4096)])
+@pytest.mark.parametrize("kind", [kind for kind in KINDS if kind[2] == "affine"])
+def test_what_cancels_cancels_early(m, n, k, kind):
+    bits, gs, mode, tab = kind
+    if k % gs or (bits == 8 and k > 4160):
+        pytest.skip("not a whole number of groups, or more chunks than the bound counts")
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, _ = weight(g, (), n, k, bits, gs, mode, tab)
+    zero = torch.randint(6, 11, s.shape, device=DEV, generator=g) * (1 if bits == 4 else 16)
+    b = (-zero * s.float()).to(s.dtype)
+    x = torch.randn((m, k), device=DEV, generator=g).bfloat16()
+    want = x.double() @ exact(w, s, b, how).T
+    err = ((K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how).double() - want).norm() / want.norm()).item()
+    assert err <= (7e-7 if bits == 4 else 1.3e-7), err
