@@ -215,9 +215,18 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     // registers two K-tiles before, and written to LDS at the start of the
     // step before (the write then has the whole step to finish before the
     // barrier that publishes it).
-    auto dequant_tile = [&](u32x4 (&dst)[4], const WRegs& r, float sc, float bi) {
+    // (The scales are looked at tile by tile, here: at most 1 % on large products.
+    // Once in the prologue, with the answer in a scalar register, 1-2 %; in front
+    // of the barrier up to 6 %.)
+    auto dequant_tile = [&](u32x4 (&dst)[4], const WRegs& r, float sc, float bi) __attribute__((always_inline)) {
+      const bool small = MODE == 1 || TAB == QMM_F16 || __ballot(!(fabsf(sc) < kSmallScale)) == 0ull;      // uniform
+      if (__builtin_expect(small, 1)) {
 #pragma unroll
-      for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece<MODE, BITS>(r.q, pc, sc, bi);
+        for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece_small<MODE, BITS>(r.q, pc, sc, bi);
+      } else {
+#pragma unroll
+        for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece<MODE, BITS>(r.q, pc, sc, bi);
+      }
     };
     auto write_tile = [&](int stage, const u32x4 (&src)[4]) {
 #pragma unroll

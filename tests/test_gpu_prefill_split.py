@@ -121,3 +121,28 @@ def test_wide_gathers_keep_their_weights(pairs, experts, k, kind, act):
     full = K.dequantize(w, s, b, out_dtype=torch.float32, **how).double()
     want = torch.stack([full[rhs[p]] @ x[p].double() for p in range(pairs)])
     close(K.gather_qmm(x, w, s, b, None, rhs, out_dtype=torch.float32, **how), want)
+
+
+# Scales up to the top of bfloat16 / float32: a weight is scale times code plus bias
+# whatever the scale's size, and the bias where the code is 0.  (The activations are
+# small, so that sums stay in range; one group in five is large, every third column
+# has none, and each column is judged by its own size.)
+@pytest.mark.parametrize("m,n,k", [(33, 130, 320), (128, 333, 4096), (300, 9208, 2944)])
+@pytest.mark.parametrize("kind", [(4, 64, "affine", "bf16"), (4, 32, "affine", "bf16"), (4, 128, "affine", "f32"),
+                                  (8, 64, "affine", "bf16"), (8, 32, "affine", "f32"), (4, 32, "affine", "f32")])
+def test_large_scales(m, n, k, kind):
+    bits, gs, mode, tab = kind
+    if k % gs:
+        pytest.skip("not a whole number of groups")
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (), n, k, bits, gs, mode, tab)
+    grow = torch.rand(s.shape, device=DEV, generator=g) < 0.2
+    grow[::3] = False
+    power = torch.randint(110, 122, s.shape, device=DEV, generator=g).float()        # scales of 2^103 .. 2^116
+    s = torch.where(grow, s.float() * torch.exp2(power), s.float()).to(s.dtype)
+    x = (torch.randn((m, k), device=DEV, generator=g) * 2.0 ** -20).bfloat16()
+    want = x.double() @ tile(w, s, b, how).T
+    y = K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how).double()
+    err = (y - want).norm(dim=0) / want.norm(dim=0)
+    assert bool((err <= 2e-5).all()), err.max().item()
