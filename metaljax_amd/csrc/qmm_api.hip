@@ -369,6 +369,11 @@ size_t dense_scratch_split(int64_t rows, int64_t N, int64_t K, int mode, bool ex
   return std::max(least, gemm2_split_workspace_bytes(rows, N, K));
 }
 
+// Float16 / float32 activations: their terms as bf16 rows and the terms' float32 products.
+size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
+  return align256((size_t)(terms * rows * K) * 2) + align256((size_t)(terms * rows * N) * 4);
+}
+
 // Is the short-group kernel the one to take?  `E` experts share the R rows (1:
 // dense), the activations are `terms` bf16 terms.  All kernels' times have been
 // fitted over the shapes they serve; where they come close the choice matters
@@ -454,8 +459,7 @@ size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int, 
   // product: over terms x M stacked rows (dense) or over M rows (grouped)
   if (batch < 1) batch = 1;
   const size_t stacked = dense_scratch_split(terms * M, N, K, mode, true), plain = dense_scratch(M, N, K, mode, true);
-  return std::max(sh, align256((size_t)(batch * terms * M * K) * 2) + align256((size_t)(batch * terms * M * N) * 4) +
-                          std::max(stacked, plain));
+  return std::max(sh, term_bytes(terms, batch * M, N, K) + std::max(stacked, plain));
 }
 
 // What a gathered product needs to run at all on its preferred kernels, without
@@ -464,8 +468,7 @@ static size_t gather_minimum(int64_t P, int64_t E, int64_t N, int64_t K, int x_d
   const int terms = act_terms(x_dtype);
   if (terms == 1) return gather_scratch(P, E, N, K, false);
   // the gathered rows' terms, their float32 products, the bf16 product's scratch
-  return align256((size_t)(terms * P * K) * 2) + align256((size_t)(terms * P * N) * 4) +
-         gather_scratch(P, E, N, K, true);
+  return term_bytes(terms, P, N, K) + gather_scratch(P, E, N, K, true);
 }
 
 size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, int x_dtype) {
@@ -545,9 +548,11 @@ int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode
   return QMM_OK;
 }
 
-// One product on the short-group kernel if it serves it, arguments and scratch
-// included: true when it was launched (*rc: the launches' status), false when
-// the other kernels are to take it (or to say what is wrong with it).
+// One product on the short-group kernel if it serves it, arguments included: true
+// when it was launched (*rc: the launches' status), false when the other kernels
+// are to take it (or to say what is wrong with it).  It needs less scratch and less
+// alignment than they do: the callers see to it that a call is refused whichever
+// kernel would have run.
 static bool ran_short(const void* x, int x_dtype, const void* w, const void* scales, const void* biases,
                       int table_dtype, void* y, int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
                       const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N, int64_t K,
@@ -791,7 +796,11 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
     const size_t tb = mode == QMM_MODE_MXFP4 ? (size_t)N * (K / 32) : (size_t)N * (K / std::max(group_size, 1)) * (table_dtype == QMM_F32 ? 4 : 2);
     int rc = QMM_OK;
     int64_t z = 0;
-    for (; z < batch; ++z)
+    // (what dense_bf16 and the terms below would refuse)
+    const size_t inner = dense_scratch(terms * M, N, K, mode, terms > 1);
+    const bool taken = workspace_bytes >= inner + (terms > 1 ? term_bytes(terms, batch * M, N, K) : 0) &&
+                       (inner == 0 || aligned16(scales)) && (terms == 1 || batch * terms * M * K < (1ll << 30));
+    for (; taken && z < batch; ++z)
       if (!ran_short(static_cast<const char*>(x) + z * xb, x_dtype, static_cast<const char*>(w) + z * wb,
                      static_cast<const char*>(scales) + z * tb, biases ? static_cast<const char*>(biases) + z * tb : nullptr,
                      table_dtype, static_cast<char*>(y) + z * yb, y_dtype, nullptr, nullptr, nullptr, M, M, 1, N, K,
@@ -833,8 +842,12 @@ int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scale
                     void* stream) {
   const int terms = act_terms(x_dtype);
   int rs = QMM_OK;
-  if (row_offsets && ran_short(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, nullptr, nullptr, R,
-                               R, E, N, K, group_size, bits, mode, workspace, workspace_bytes, stream, &rs))
+  // (wider activations are refused without room for their terms and the terms' products)
+  const bool taken = terms == 1 || (R > 0 && N > 0 && K > 0 &&
+                                    workspace_bytes >= term_bytes(terms, R, N, K) + dense_scratch(R, N, K, mode, true));
+  if (row_offsets && taken &&
+      ran_short(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, nullptr, nullptr, R, R, E, N, K,
+                group_size, bits, mode, workspace, workspace_bytes, stream, &rs))
     return rs;
   if (terms == 1 || R <= 0 || E <= 0 || N <= 0 || K <= 0 || !x || !row_offsets || !y)
     return grouped_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, R, E, N, K,
@@ -878,6 +891,7 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
   if (!exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
       short_wins(P, E, N, K, bits, mode, terms) && workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
+      workspace_bytes >= term_bytes(terms, P, N, K) + gather_scratch(P, E, N, K, true) &&
       short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, terms, scales, biases)) {
     const size_t need = route_bytes(P, E);
     int32_t* ro = static_cast<int32_t*>(workspace);

@@ -164,3 +164,33 @@ def test_static_scratch_entry_point_rejects_what_does_not_fit(lib):
     rc = lib.qmm_gather_qmm_static(None, _lib.BF16, None, None, None, _lib.BF16, None, _lib.BF16,
                                    None, None, p, p, e, n, k, 64, 4, 0, None)
     assert rc == 4 and b"static scratch" in lib.qmm_last_error()
+
+
+def _no_gpu():
+    import torch
+    return not torch.cuda.is_available()
+
+
+@pytest.mark.skipif(not _no_gpu(), reason="made-up pointers: only where nothing can be launched with them")
+def test_what_is_refused_does_not_depend_on_the_kernel(lib):
+    """Too little scratch, or tables that do not start on sixteen bytes, are refused at
+    every size, also where the kernel that would run needs less."""
+    at = 0x100000
+
+    def dense(m, n, k, act, mode, scratch, scales=at, batch=1):
+        return lib.qmm_quantized_matmul(at, act, at, scales, None if mode else at, _lib.BF16, at, _lib.BF16, batch, m, n,
+                                        k, 32 if mode else 64, 4, mode, at, scratch, None)
+    for m, n, k in ((17, 4096, 4096), (48, 4096, 14336), (77, 1024, 2048), (300, 9216, 2944)):
+        for mode in (0, 1):
+            for act in (_lib.BF16, _lib.F16, _lib.F32):
+                need = lib.qmm_workspace_bytes(1, m, n, k, 64, 4, mode, act)
+                assert dense(m, n, k, act, mode, 256) == 4
+                if act == _lib.BF16:                                  # (wider ones are told behind a first launch)
+                    assert dense(m, n, k, act, mode, need, scales=at + 4) == 1
+                assert dense(m, n, k, act, mode, need) == 5           # (nothing wrong with it: the launch fails)
+        terms = 2 * m * k * 2 + 256                                   # room for float16 terms, not for their products
+        assert dense(m, n, k, _lib.F16, 0, terms) == 4
+        assert lib.qmm_grouped_qmm(at, _lib.F16, at, at, at, _lib.BF16, at, _lib.BF16, at, m, 4, n, k, 64, 4, 0, at,
+                                   terms, None) == 4
+        assert lib.qmm_gather_qmm(at, _lib.F16, at, at, at, _lib.BF16, at, _lib.BF16, at, at, 5 * m, 5 * m, 4, n, k, 64,
+                                  4, 0, at, 5 * terms + 8192, None) == 4
