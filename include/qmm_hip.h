@@ -69,8 +69,13 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
                          int bits, int mode, void* workspace, size_t workspace_bytes,
                          void* stream);
 
-/* Scratch bytes qmm_quantized_matmul / qmm_grouped_qmm need for these
- * arguments (M = total rows for the grouped form). */
+/* Scratch bytes qmm_quantized_matmul / qmm_grouped_qmm run best with for these
+ * arguments (M = total rows for the grouped form); always enough.  The float32
+ * sums of a K that is split over workgroups are part of it: a call with less
+ * runs with fewer splits, and is refused (QMM_ERR_WORKSPACE) only where the
+ * rest -- the re-laid activations, the terms of float16 / float32 ones and
+ * their products -- does not fit.  (bf16 rows of the grouped form run with any
+ * workspace, on a slower kernel.) */
 size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int group_size,
                            int bits, int mode, int x_dtype);
 
@@ -78,9 +83,12 @@ size_t qmm_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, int g
  * weights (0 below four pairs, which run as independent decode products): the
  * expert sort's arrays, plus the segment list of the grouped decode (up to
  * 16 pairs an expert on average: one decode product per expert and sixteen
- * pairs) or the re-laid activation copy of the prefill kernel (more pairs).
- * With less the call still runs, on a slower kernel (bf16 activations; float16
- * and float32 activations need the whole of it). */
+ * pairs) or the re-laid activation copy of the prefill kernel (more pairs), for
+ * float16 / float32 activations also their terms and the terms' products; and
+ * the sums of a split K, as far as they fit QMM_STATIC_SCRATCH_BYTES.
+ * With less the call still runs, on a slower kernel or with fewer splits; bf16
+ * activations need the expert sort's arrays above 64 pairs, float16 and float32
+ * ones everything but the sums. */
 size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, int x_dtype);
 
 /* The kernel family and launch geometry the dispatcher would choose. */

@@ -194,3 +194,17 @@ def test_what_is_refused_does_not_depend_on_the_kernel(lib):
                                    terms, None) == 4
         assert lib.qmm_gather_qmm(at, _lib.F16, at, at, at, _lib.BF16, at, _lib.BF16, at, at, 5 * m, 5 * m, 4, n, k, 64,
                                   4, 0, at, 5 * terms + 8192, None) == 4
+
+
+@pytest.mark.skipif(not _no_gpu(), reason="made-up pointers: only where nothing can be launched with them")
+@pytest.mark.parametrize("act", [_lib.BF16, _lib.F16, _lib.F32])
+def test_the_gather_query_tells_what_the_static_entry_takes(lib, act):
+    """At sizes round the array's: products that fit it without the sums of a split K
+    (and with them would not), that fall a little short, and that do not fit."""
+    at = 0x100000
+    for p, e, n, k in ((260, 8, 9200, 6848), (672, 16, 4168, 7808), (494, 16, 4808, 6848), (100, 8, 14336, 4096),
+                       (1700, 8, 1024, 4096), (2000, 8, 4096, 4096), (512, 32, 2048, 2880), (64, 8, 14336, 14336),
+                       (80, 8, 16384, 14336), (4096, 8, 256, 1024)):
+        rc = lib.qmm_gather_qmm_static(at, act, at, at, at, _lib.BF16, at, _lib.BF16, at, at, p, p, e, n, k, 64, 4, 0, None)
+        want = 4 if lib.qmm_gather_workspace_bytes(p, e, n, k, act) > _lib.STATIC_SCRATCH_BYTES else 5
+        assert rc == want, (p, e, n, k)
