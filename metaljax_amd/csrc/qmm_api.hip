@@ -374,23 +374,28 @@ size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
   return align256((size_t)(terms * rows * K) * 2) + align256((size_t)(terms * rows * N) * 4);
 }
 
-// Is the short-group kernel the one to take?  `E` experts share the R rows (1:
-// dense), the activations are `terms` bf16 terms.  All kernels' times have been
+// Is the short-group kernel the one to take?  `E` experts share the R rows
+// (`grouped`; else a dense product and E = 1), the activations are `terms` bf16
+// terms, and each kernel has what `scratch` leaves it for a split K's sums.  All kernels' times have been
 // fitted over the shapes they serve; where they come close the choice matters
 // little.  (4096 x 4096, four-bit codes: 17 rows 13 against 20 us of the
 // prefill kernel, 128 rows 19 against 23, 512 rows 32 against 36; 14336 x 4096:
 // 19 against 29, 32 against 33, 108 against 59.)
-bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms) {
+bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, bool grouped, size_t scratch) {
   if (K % 64 || N <= 0) return false;
   if (const char* env = experiment_env("QMM_SHORT")) return env[0] != '0';
   double other;
   if (mode == QMM_MODE_MXFP4 && terms == 1 && mxfp4_mfma_supported(R, N, K)) {
     if (N < 512) return false;                   // (a few column tiles: not measured, left as it is)
     other = mxfp4_us(R, E, N, K);
+  } else {
+    // (row groups keep their whole K there, one product a term; dense, the terms are rows of one product)
+    const size_t held = gemm2_workspace_bytes(terms * R, K) + (terms > 1 ? term_bytes(terms, R, N, K) : 0);
+    other = grouped ? terms * gemm2_us(R, E, N, K, 0) : gemm2_us(terms * R, 1, N, K, scratch > held ? scratch - held : 0);
+    if (terms > 1) other += 5.2 + (double)terms * R * N * 1.4e-6;
   }
-  else if (E > 1) other = terms * gemm2_us(R, E, N, K, 0) + (terms > 1 ? 5.2 + (double)terms * R * N * 1.4e-6 : 0.0);
-  else other = gemm2_us(terms * R, 1, N, K, ~(size_t)0) + (terms > 1 ? 5.2 + (double)terms * R * N * 1.4e-6 : 0.0);
-  return short_us(R, E, N, K, bits, mode, terms, ~(size_t)0) < other;
+  const size_t prep = short_prep_bytes(R, K, terms);
+  return short_us(R, E, N, K, bits, mode, terms, scratch > prep ? scratch - prep : 0) < other;
 }
 
 // Scratch that lets a short-group product over R rows run as it would best.
@@ -486,7 +491,7 @@ size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, in
 
 int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode, int* kernel,
              int* grid, int* block) {
-  if (M > kGemvMaxM && short_wins(M, 1, N, K, bits, mode, 1)) {     // (bf16 activations and tables assumed)
+  if (M > kGemvMaxM && short_wins(M, 1, N, K, bits, mode, 1, false, ~(size_t)0)) {     // (bf16 activations and tables, ample scratch assumed)
     int g;
     short_geometry(M, N, K, bits, mode, &g);
     if (kernel) *kernel = QMM_KERNEL_GEMM;
@@ -566,7 +571,7 @@ static bool ran_short(const void* x, int x_dtype, const void* w, const void* sca
                       int* rc) {
   const int terms = act_terms(x_dtype);
   if (R <= 0 || E <= 0 || N <= 0 || K <= 0 || terms * R <= kGemvMaxM || R > INT32_MAX / 2 || N > INT32_MAX ||
-      K > INT32_MAX || E > 65535 || !short_wins(R, E, N, K, bits, mode, terms))
+      K > INT32_MAX || E > 65535 || !short_wins(R, E, N, K, bits, mode, terms, row_offsets != nullptr, workspace_bytes))
     return false;
   if (check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases) || check_io(x, x_dtype, y, y_dtype) ||
       !workspace || !aligned16(workspace) || workspace_bytes < short_prep_bytes(R, K, terms) ||
@@ -896,8 +901,9 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
   if (!exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
-      short_wins(P, E, N, K, bits, mode, terms) && workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
+      workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
       workspace_bytes >= term_bytes(terms, P, N, K) + gather_scratch(P, E, N, K, true) &&
+      short_wins(P, E, N, K, bits, mode, terms, true, workspace_bytes - route_bytes(P, E)) &&
       short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, terms, scales, biases)) {
     const size_t need = route_bytes(P, E);
     int32_t* ro = static_cast<int32_t*>(workspace);

@@ -146,3 +146,32 @@ def test_large_scales(m, n, k, kind):
     y = K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how).double()
     err = (y - want).norm(dim=0) / want.norm(dim=0)
     assert bool((err <= 2e-5).all()), err.max().item()
+
+
+# With no room for the sums of a split K -- the least scratch that is taken -- and with
+# some of it: fewer splits, or the other kernel, and the same product.
+@pytest.mark.parametrize("m,n,k", [(17, 1024, 4096), (48, 4096, 14336), (300, 1000, 8256), (650, 3080, 6144)])
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+@pytest.mark.parametrize("part", [0.0, 0.3])
+def test_scratch_limits(m, n, k, act, part):
+    from metaljax_amd import _lib
+    lib, code = _lib.load(), {"bf16": _lib.BF16, "f16": _lib.F16}[act]
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    how = dict(group_size=64, bits=4, mode="affine")
+    w, s, b = weight(g, (), n, k, 4, 64, "affine", "bf16")
+    x = torch.randn((m, k), device=DEV, generator=g).to(ACT[act])
+    y = torch.empty((m, n), device=DEV)
+
+    def relaid(rows):
+        return (rows + 256 + 63) // 64 * 64 * k * 2
+    least = relaid(m) if act == "bf16" else sum(-(-v // 256) * 256 for v in (2 * m * k * 2, 2 * m * n * 4)) + relaid(2 * m)
+    most = int(lib.qmm_workspace_bytes(1, m, n, k, 64, 4, 0, code))
+    room = least + int(part * (most - least))
+    ws = torch.empty(room, dtype=torch.uint8, device=DEV)
+
+    def call(scratch):
+        return lib.qmm_quantized_matmul(x.data_ptr(), code, w.data_ptr(), s.data_ptr(), b.data_ptr(), _lib.BF16, y.data_ptr(),
+                                        _lib.F32, 1, m, n, k, 64, 4, 0, ws.data_ptr(), scratch, torch.cuda.current_stream().cuda_stream)
+    assert call(least - 1) == 4
+    assert call(room) == 0
+    close(y, x.double() @ tile(w, s, b, how).T)
