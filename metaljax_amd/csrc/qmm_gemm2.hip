@@ -442,6 +442,23 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
         }
       }
   }
+  if constexpr (MODE == 0) {
+    // a scale too large for the short form of the dequantization: its column's results are not finite
+    float probe = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) probe = fmaf(acc[0][j][0], 0.f, probe);      // NaN if one is not
+    if (__builtin_expect(__ballot(probe != probe && kh == 0 && m0 + wm * (RB0 * 32) < row_hi) != 0ull, 0)) {
+      __builtin_amdgcn_s_waitcnt(0);
+#pragma nounroll
+      for (int at = 0; at < MT * NT; ++at) {       // row block at / NT of this wavefront's, column block at % NT
+        const int i = at / NT, j = at % NT;
+        const bool fifth = i == 1 && five_tile;
+        if (fifth && j != wm) continue;
+        const int lo = m0 + (fifth ? WMW : wm * RB0 + i * RBI) * 32 + 16 * kh, hi = lo + 16 < row_hi ? lo + 16 : row_hi;
+        redo_column<BITS>(a, e, n0 + wn * (NT * 32) + j * 32 + li, lo, hi, 0, a.K, 0);
+      }
+    }
+  }
 }
 
 template <int MODE, int BITS, int MT, int NT, int WMW, int NWAVES, bool RAG, bool WIN>
@@ -528,6 +545,8 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
   a.R = (int)R; a.N = (int)N; a.K = (int)K; a.E = (int)E; a.Rp = (int)rp;
   a.gs = gs; a.tab = tab; a.y_dtype = y_dtype;
   a.m_tiles = 0;
+  a.splits = 1;
+  a.part = nullptr;
   {
     const int64_t esz = mode == QMM_MODE_MXFP4 ? 1 : (tab == QMM_F32 ? 4 : 2);
     const int64_t row = K / (mode == QMM_MODE_MXFP4 ? 32 : gs) * esz;            // bytes of a table row

@@ -47,7 +47,7 @@ struct Gemm2Args {
   int tabfast;           // general kernel: float32 tables of groups of 32, fetched as windows
   int tab_ok, tab_odd;   // split-role kernel: tables start on dwords; their rows may start inside one
   int tile_rows;         // split-role kernel: rows a tile may hold (128 or 256)
-  int splits;            // split-role kernel, dense (1 with row_offsets): workgroups that share a tile's K ...
+  int splits;            // split-role kernel, dense (else 1): workgroups that share a tile's K ...
   float* part;           // ... and leave their float32 sums here, [splits][R][N]
 };
 
@@ -72,63 +72,20 @@ __device__ __forceinline__ void deal_grouped_tile(int n_tiles, int xcd, int l, i
 
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 
-// 32 codes (one row, one 32-group) -> four 16-byte pieces of bf16 weights
-template <int MODE, int BITS>
-__device__ __forceinline__ u32x4 dequant_piece(const uint32_t* q, int pc, float sc, float bi) {
-  float f[8];
-  if constexpr (MODE == 1) {
-    // exact: the converter widens the two codes of a byte and applies the power-of-two scale
-    const uint32_t w = q[pc];
-    return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 0)),
-                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 1)),
-                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 2)),
-                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3))};
-  } else if constexpr (BITS == 8) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = fmaf(sc, (float)((q[2 * pc + j / 4] >> (8 * (j % 4))) & 255u), bi);
-  } else {
-    uint32_t lo = q[pc] & 0x0F0F0F0Fu, hi = (q[pc] >> 4) & 0x0F0F0F0Fu;    // even / odd codes as bytes
-    // kept opaque, so that each code is one byte-to-float conversion of lo / hi
-    // (merged with the masks above they become a bit-field extract plus a conversion)
-    asm("" : "+v"(lo));
-    asm("" : "+v"(hi));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = fmaf(sc, (float)(((j % 2 ? hi : lo) >> (8 * (j / 2))) & 255u), bi);
-  }
-  return u32x4{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};
-}
-
-// The same without converting the codes, for scales below kSmallScale in
-// magnitude (and NaN): a code in the low bits of a half word is the float16 denormal q * 2^-24 (a nibble
+// fma(scale, q, bias) of small integer codes without converting them: a code in
+// the low bits of a half word is the float16 denormal q * 2^-24 (a nibble
 // further up q * 2^-20), v_fma_mix_f32 takes that as an operand, and with the
-// scale times 2^24 (2^20) -- exact, where it does not overflow -- it is the same
-// product with the same one rounding, one instruction a code.  Eight four-bit
-// codes take 17 vector instructions this way instead of 23, four eight-bit ones 9
-// instead of 10.  The kernels look at the scales and take the form above where one
-// is larger (float16 tables cannot hold such a one).
+// scale times 2^24 (2^20) -- exact below kSmallScale -- it is the same product
+// with the same one rounding, one instruction a code.  Eight four-bit codes take
+// 17 vector instructions this way instead of 23, four eight-bit ones 9 instead of
+// 10.
+//
+// A larger scale (float16 tables cannot hold one) becomes infinite, its weights
+// infinite or NaN, and so every result of its column: the kernels look at one
+// result a column when they are done and multiply such a column again
+// (redo_column).  Over 160 products of 17 to 2048 rows that is 0.3 % in all; asked
+// of the scales as they come by it was 1 %, up to 4 %.
 constexpr float kSmallScale = 0x1p104f;
-
-// The largest magnitudes of four dwords of bf16 (the two halves apart) or float32
-// scales, as integers that compare like them, joined to `most`; and whether those
-// hold one that is not small.
-template <int TAB>
-__device__ __forceinline__ uint32_t largest_scales(uint32_t most, const u32x4& v) {
-  typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t m = v[j] & (TAB == QMM_F32 ? 0x7FFFFFFFu : 0x7FFF7FFFu);
-    if constexpr (TAB == QMM_F32) most = most > m ? most : m;
-    else most = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, most), __builtin_bit_cast(u16x2, m)));
-  }
-  return most;
-}
-template <int TAB>
-__device__ __forceinline__ bool not_small(uint32_t most) {
-  if constexpr (TAB == QMM_F32) return most >= __builtin_bit_cast(uint32_t, kSmallScale);
-  const uint32_t least = __builtin_bit_cast(uint32_t, kSmallScale) >> 16;
-  return (most & 0xFFFFu) >= least || (most >> 16) >= least;
-}
-
 __device__ __forceinline__ u32x4 dequant_nibbles(uint32_t w, float s24, float s20, float bi) {
   const uint32_t w8 = w >> 8;
   const f16x2 a = __builtin_bit_cast(f16x2, w & 0x000F000Fu), b = __builtin_bit_cast(f16x2, w & 0x00F000F0u);
@@ -145,15 +102,66 @@ __device__ __forceinline__ u32x2 dequant_bytes(uint32_t w, float s24, float bi) 
   const float f1 = fmaf((float)b[0], s24, bi), f3 = fmaf((float)b[1], s24, bi);
   return u32x2{pack_bf16x2(f0, f1), pack_bf16x2(f2, f3)};
 }
+
+// 32 codes (one row, one 32-group) -> four 16-byte pieces of bf16 weights
 template <int MODE, int BITS>
-__device__ __forceinline__ u32x4 dequant_piece_small(const uint32_t* q, int pc, float sc, float bi) {
+__device__ __forceinline__ u32x4 dequant_piece(const uint32_t* q, int pc, float sc, float bi) {
   if constexpr (MODE == 1) {
-    return dequant_piece<MODE, BITS>(q, pc, sc, bi);
+    // exact: the converter widens the two codes of a byte and applies the power-of-two scale
+    const uint32_t w = q[pc];
+    return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 0)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 1)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 2)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3))};
   } else if constexpr (BITS == 8) {
     const u32x2 lo = dequant_bytes(q[2 * pc], sc * 0x1p24f, bi), hi = dequant_bytes(q[2 * pc + 1], sc * 0x1p24f, bi);
     return u32x4{lo[0], lo[1], hi[0], hi[1]};
   } else {
     return dequant_nibbles(q[pc], sc * 0x1p24f, sc * 0x1p20f, bi);
+  }
+}
+
+// The weight row [n] of expert `e` as the long way reads it: without regard to time.
+template <int BITS>
+struct LongRow {
+  const uint8_t* codes;
+  const void *s, *b;
+  int64_t entry;         // of the row's first group
+  int tab, gshift;
+
+  __device__ __forceinline__ LongRow(const uint32_t* w, const void* s_, const void* b_, int64_t e, int64_t n, int64_t N, int64_t K, int gshift_, int tab_)
+      : codes(reinterpret_cast<const uint8_t*>(w) + (e * N + n) * (K * BITS / 8)), s(s_), b(b_), entry((e * N + n) * (K >> gshift_)), tab(tab_),
+        gshift(gshift_) {}
+  // Has it a scale that is not small in [k0, k1)?
+  __device__ __forceinline__ bool large(int k0, int k1) const {
+    bool l = false;
+#pragma nounroll
+    for (int g = k0 >> gshift; g << gshift < k1; ++g) l |= !(fabsf(load_table_rt(s, entry + g, tab)) < kSmallScale);
+    return l;
+  }
+  __device__ __forceinline__ double weight(int k) const {             // the bf16 tile's
+    const uint32_t code = BITS == 8 ? codes[k] : (uint32_t)codes[k >> 1] >> (4 * (k & 1)) & 15u;
+    const int64_t g = entry + (k >> gshift);
+    return (double)bf16_bits_to_f32(f32_to_bf16_bits(fmaf(load_table_rt(s, g, tab), (float)code, load_table_rt(b, g, tab))));
+  }
+};
+
+// Column n of rows [lo, hi) over [k0, k1) again where its scales ask for it (the
+// prefill kernels: activations re-laid, results in y, or in a split's part).  The
+// kernel's own stores have to have landed.
+template <int BITS>
+__device__ __forceinline__ void redo_column(const Gemm2Args& a, int e, int n, int lo, int hi, int k0, int k1, int split) {
+  if (n >= a.N || lo >= hi) return;
+  const LongRow<BITS> row(a.w, a.s, a.b, e, n, a.N, a.K, a.gs == 32 ? 5 : a.gs == 64 ? 6 : 7, a.tab);
+  if (!row.large(k0, k1)) return;                // an activation, or a sum that is out of range
+#pragma nounroll
+  for (int m = lo; m < hi; ++m) {
+    double sum = 0.0;
+#pragma nounroll
+    for (int k = k0; k < k1; ++k)
+      sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.ax)[((int64_t)(k >> 3) * a.Rp + m) * 8 + (k & 7)]), row.weight(k), sum);
+    if (a.splits > 1) a.part[((int64_t)split * a.R + m) * a.N + n] = (float)sum;
+    else store_out(a.y, (a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m) * a.N + n, (float)sum, a.y_dtype);
   }
 }
 

@@ -215,18 +215,9 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     // registers two K-tiles before, and written to LDS at the start of the
     // step before (the write then has the whole step to finish before the
     // barrier that publishes it).
-    // (The scales are looked at tile by tile, here: at most 1 % on large products.
-    // Once in the prologue, with the answer in a scalar register, 1-2 %; in front
-    // of the barrier up to 6 %.)
-    auto dequant_tile = [&](u32x4 (&dst)[4], const WRegs& r, float sc, float bi) __attribute__((always_inline)) {
-      const bool small = MODE == 1 || TAB == QMM_F16 || __ballot(!(fabsf(sc) < kSmallScale)) == 0ull;      // uniform
-      if (__builtin_expect(small, 1)) {
+    auto dequant_tile = [&](u32x4 (&dst)[4], const WRegs& r, float sc, float bi) {
 #pragma unroll
-        for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece_small<MODE, BITS>(r.q, pc, sc, bi);
-      } else {
-#pragma unroll
-        for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece<MODE, BITS>(r.q, pc, sc, bi);
-      }
+      for (int pc = 0; pc < 4; ++pc) dst[pc] = dequant_piece<MODE, BITS>(r.q, pc, sc, bi);
     };
     auto write_tile = [&](int stage, const u32x4 (&src)[4]) {
 #pragma unroll
@@ -526,6 +517,22 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
             store_out(a.y, orow * a.N + n, i == 0 ? acc[j][r] : acc2[j][r], a.y_dtype);
           }
         }
+      }
+    }
+  }
+  if constexpr (MODE == 0 && TAB != QMM_F16) {
+    // a scale too large for the short form of the dequantization: its column's results are not finite
+    float probe = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) probe = fmaf(acc[j][0], 0.f, probe);          // NaN if one is not
+    if (__builtin_expect(__ballot(probe != probe && kh == 0 && m0 + wm * 32 < m_end) != 0ull, 0)) {
+      __builtin_amdgcn_s_waitcnt(0);
+      const int k0 = kb * BK, k1 = (kb + KT) * BK;
+#pragma nounroll
+      for (int at = 0; at < 8; ++at) {             // row block at / 4 of this wavefront's, column block at % 4
+        if (at >= 4 && !two && !(five && (at & 3) == wm)) continue;
+        const int lo = m0 + (at < 4 ? wm : two ? wm + 4 : 4) * 32 + 16 * kh, hi = lo + 16 < m_end ? lo + 16 : m_end;
+        redo_column<BITS>(a, e, n0 + (at & 3) * 32 + li, lo, hi, k0, k1, split);
       }
     }
   }

@@ -115,8 +115,7 @@ struct ShortShape {
   static constexpr int kFit = (163840 - kTabs) / kStage;
   static constexpr int kDepth = kFit < 5 ? kFit : 5;           // stages in the ring
   static constexpr int kSums = kWaves * 4 * MB * 4 * 64 * 4;   // the wavefronts' sums, after the run
-  static constexpr int kNotes = kWaves * 4;                    // behind the sums
-  static constexpr int kLds = kDepth * kStage + kTabs > kSums + kNotes ? kDepth * kStage + kTabs : kSums + kNotes;
+  static constexpr int kLds = kDepth * kStage + kTabs > kSums ? kDepth * kStage + kTabs : kSums;
   static_assert(kDepth >= 3 && kLds <= 163840, "three stages fit");
 };
 
@@ -213,8 +212,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   const uint32_t tvo = n0 + tcol < a.N ? (uint32_t)(n0 + tcol) * tpitch : kOutOfRange;
   const auto rs = make_rsrc(sp, tbytes);
   const auto rb = make_rsrc(bp, tbytes);
-  constexpr bool LARGE = MODE == 0 && TAB != QMM_F16;   // scales that dequant_piece_small does not serve can occur
-  uint32_t most = 0;                             // of the scales that this lane has put into windows
   u32x4 tw_s, tw_b;
   uint32_t tx_s = 0, tx_b = 0, tmis = 0;         // a row that starts inside a dword: one dword more, and how far in
   auto fetch_window = [&](int st) __attribute__((always_inline)) {      // the window that starts at step st
@@ -238,7 +235,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
         vb = u32x4{__builtin_amdgcn_alignbit(tw_b[1], tw_b[0], sh), __builtin_amdgcn_alignbit(tw_b[2], tw_b[1], sh),
                    __builtin_amdgcn_alignbit(tw_b[3], tw_b[2], sh), __builtin_amdgcn_alignbit(tx_b, tw_b[3], sh)};
     }
-    if constexpr (LARGE) most = g2::largest_scales<TAB>(most, vs);
     if constexpr (MODE == 1) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -289,6 +285,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   };
 
   f32x4 acc[4][MB];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < MB; ++i) acc[c][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // ---- where this lane's operands lie in a stage
   const uint32_t ao = (uint32_t)kStageW + (uint32_t)r16 * S::kRowA +
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   };
   // Weight fragment b = (column block b / STEPS, MFMA step b % STEPS), widened
   // while the matrix core works on the fragment before it.
-  auto widen = [&](const Ops& o, auto bc, auto smallc) __attribute__((always_inline)) -> bf16x8 {
+  auto widen = [&](const Ops& o, auto bc) __attribute__((always_inline)) -> bf16x8 {
     constexpr int c = decltype(bc)::value / STEPS, j = decltype(bc)::value % STEPS;
     if constexpr (MODE == 1) {
       return widen_e2m1(o.q[c][j], __uint_as_float(kg >= 2 ? o.t0[c] & 0xFFFF0000u : o.t0[c] << 16));
@@ -336,17 +336,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
         bi = __uint_as_float(o.t0[c] & 0xFFFF0000u);
       }
       const uint32_t q[2] = {o.q[c][BITS == 4 ? j : 0], o.q[c][1]};
-      if constexpr (decltype(smallc)::value) return __builtin_bit_cast(bf16x8, g2::dequant_piece_small<0, BITS>(q, 0, sc, bi));
-      else return __builtin_bit_cast(bf16x8, g2::dequant_piece<0, BITS>(q, 0, sc, bi));
+      return __builtin_bit_cast(bf16x8, g2::dequant_piece<0, BITS>(q, 0, sc, bi));
     }
   };
-  auto math = [&](const Ops& o, auto smallc) __attribute__((always_inline)) {
+  auto math = [&](const Ops& o) __attribute__((always_inline)) {
     constexpr int NB = 4 * STEPS;
-    bf16x8 wq = widen(o, std::integral_constant<int, 0>{}, smallc);
+    bf16x8 wq = widen(o, std::integral_constant<int, 0>{});
     static_for<NB>([&](auto bc) __attribute__((always_inline)) {
       constexpr int b = decltype(bc)::value, c = b / STEPS, j = b % STEPS;
       bf16x8 wn8 = wq;
-      if constexpr (b + 1 < NB) wn8 = widen(o, std::integral_constant<int, b + 1>{}, smallc);
+      if constexpr (b + 1 < NB) wn8 = widen(o, std::integral_constant<int, b + 1>{});
 #pragma unroll
       for (int i = 0; i < MB; ++i) acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.xa[j][i], wq, acc[c][i], 0, 0, 0);
 #pragma unroll
@@ -367,123 +366,125 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
     const int i = st - s0, n = i >> win_shift;
     return st < s1 && (i & ((1 << win_shift) - 1)) == 0 && (n & 3) == duty ? n : -1;
   };
-  auto run = [&](auto smallc) __attribute__((always_inline)) {
+  {
+    int mine = -1;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int d = 0; d < 4; ++d)
+      if (window_at(s0 + d) >= 0) mine = d;      // (at most one: four windows are dealt over four pairs of wavefronts)
+    if (mine >= 0) fetch_window(s0 + mine);
 #pragma unroll
-      for (int i = 0; i < MB; ++i) acc[c][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    {
-      int mine = -1;
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-        if (window_at(s0 + d) >= 0) mine = d;      // (at most one: four windows are dealt over four pairs of wavefronts)
-      if (mine >= 0) fetch_window(s0 + mine);
-#pragma unroll
-      for (int d = 0; d < D; ++d) issue(s0 + d, d);
-      if (mine == 0 || mine == 1) write_window(window_at(s0 + mine));
-    }
-    if (UNEVEN && wave < kWaves / 2) wait_loads<(D - 1) * (LLO + 1)>();
-    else wait_loads<(D - 1) * LLO>();
+    for (int d = 0; d < D; ++d) issue(s0 + d, d);
+    if (mine == 0 || mine == 1) write_window(window_at(s0 + mine));
+  }
+  if (UNEVEN && wave < kWaves / 2) wait_loads<(D - 1) * (LLO + 1)>();
+  else wait_loads<(D - 1) * LLO>();
+  __builtin_amdgcn_s_barrier();
+  Ops even, odd;
+  read_ops(s0, 0, even);
+  int slot = 0;
+  auto step = [&](int st, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
+    if (UNEVEN && wave < kWaves / 2) wait_loads<(D - 2) * (LLO + 1)>();
+    else wait_loads<(D - 2) * LLO>();
     __builtin_amdgcn_s_barrier();
-    Ops even, odd;
-    read_ops(s0, 0, even);
-    int slot = 0;
-    auto step = [&](int st, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
-      if (UNEVEN && wave < kWaves / 2) wait_loads<(D - 2) * (LLO + 1)>();
-      else wait_loads<(D - 2) * LLO>();
-      __builtin_amdgcn_s_barrier();
-      const int next = slot + 1 == D ? 0 : slot + 1;
-      read_ops(st + 1, next, nxt);                 // (past the run: whatever the ring holds, never used)
-      const int put = window_at(st + 2);
-      if (put >= 0) write_window(put);
-      if (window_at(st + 4) >= 0) fetch_window(st + 4);
-      issue(st + D, slot);
-      // (K is a multiple of 64: a quarter lies inside K or past it)
-      if (st * S::kStep + wk * SUB < a.K) math(cur, smallc);
-      slot = next;
-    };
-    for (int st = s0; st < s1; st += 2) {
-      step(st, even, odd);
-      if (st + 1 < s1) step(st + 1, odd, even);
-    }
+    const int next = slot + 1 == D ? 0 : slot + 1;
+    read_ops(st + 1, next, nxt);                 // (past the run: whatever the ring holds, never used)
+    const int put = window_at(st + 2);
+    if (put >= 0) write_window(put);
+    if (window_at(st + 4) >= 0) fetch_window(st + 4);
+    issue(st + D, slot);
+    // (K is a multiple of 64: a quarter lies inside K or past it)
+    if (st * S::kStep + wk * SUB < a.K) math(cur);
+    slot = next;
   };
+  for (int st = s0; st < s1; st += 2) {
+    step(st, even, odd);
+    if (st + 1 < s1) step(st + 1, odd, even);
+  }
+  wait_loads<0>();                               // nothing may still land in the ring: it becomes the summing area
+  __syncthreads();
+
   // ---- the four quarters' sums meet in LDS, four columns of a row a lane; the
   // terms of a row are added up
   f32x4* sums = reinterpret_cast<f32x4*>(smem);
-  uint32_t* notes = reinterpret_cast<uint32_t*>(smem + S::kSums);      // behind them, a word a wavefront: saw a large scale
-  auto meet = [&]() __attribute__((always_inline)) {
-    wait_loads<0>();                             // nothing may still land in the ring: it becomes the summing area
-    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        sums[((wk * 2 + wn) * (MB * 4) + i * 4 + v) * 64 + lane] = f32x4{acc[0][i][v], acc[1][i][v], acc[2][i][v], acc[3][i][v]};
-    if constexpr (LARGE) {
-      const bool large = __ballot(g2::not_small<TAB>(most)) != 0ull;
-      if (lane == 0) notes[wave] = large;
-    }
-    __syncthreads();
-  };
+    for (int v = 0; v < 4; ++v)
+      sums[((wk * 2 + wn) * (MB * 4) + i * 4 + v) * 64 + lane] = f32x4{acc[0][i][v], acc[1][i][v], acc[2][i][v], acc[3][i][v]};
+  __syncthreads();
   // wavefront (h = wn, v = wk) takes component v of every row block of half h
-  auto give_out = [&]() __attribute__((always_inline)) {
-    f32x4 r[MB];
+  f32x4* const own = sums + (wn * (MB * 4) + wk) * 64 + lane;           // ... and i * 4 * 64: nobody else reads them
+  f32x4 r[MB];
 #pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const f32x4* p = sums + (wn * (MB * 4) + i * 4 + wk) * 64 + lane;
-      r[i] = p[0];
+  for (int i = 0; i < MB; ++i) {
+    const f32x4* p = own + i * 4 * 64;
+    r[i] = p[0];
 #pragma unroll
-      for (int k = 1; k < 4; ++k) r[i] += p[k * (2 * MB * 4 * 64)];
+    for (int k = 1; k < 4; ++k) r[i] += p[k * (2 * MB * 4 * 64)];
+  }
+  if constexpr (MB >= 2) {
+    if (a.terms == 2) {
+#pragma unroll
+      for (int i = 0; i < MB / 2; ++i) r[i] += r[i + MB / 2];
     }
-    const int n = n0 + 64 * wn + 4 * r16;
-    const bool v4 = (a.N & 3) == 0 && (a.splits > 1 || (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0);
+  }
+  if constexpr (MB == 3) {
+    if (a.terms == 3) r[0] += r[1] + r[2];
+  }
+  const int n = n0 + 64 * wn + 4 * r16;
+  if constexpr (MODE == 0 && TAB != QMM_F16) {
+    // a scale too large for the short form of the dequantization: its column's results
+    // are not finite, in rows of zeros either
+    float probe = 0.f;
 #pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const int m = m0 + i * 16 + 4 * kg + wk;
-      if (i >= a.blocks || m >= row_hi || n >= a.N) continue;
-      f32x4 v = r[i];
-      if constexpr (MB >= 2) {
-        if (a.terms == 2) v += r[MB >= 2 ? (i + MB / 2 < MB ? i + MB / 2 : i) : 0];
+    for (int j = 0; j < 4; ++j) probe = fmaf(r[0][j], 0.f, probe);        // NaN if one is not
+    if (__builtin_expect(__ballot(probe != probe) != 0ull, 0)) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) own[i * 4 * 64] = r[i];
+      const int k0 = s0 * S::kStep, k1 = s1 * S::kStep < a.K ? s1 * S::kStep : a.K;
+#pragma nounroll
+      for (int at = 0; at < a.blocks * 4; ++at) {
+        const int m = m0 + (at >> 2) * 16 + 4 * kg + wk, c = n + (at & 3);
+        if (m >= row_hi || c >= a.N) continue;
+        const g2::LongRow<BITS> row(a.w, a.s, a.b, e, c, a.N, a.K, a.gshift, TAB);
+        if (!row.large(k0, k1)) continue;        // an activation, or a sum that is out of range
+        const int src = a.src_row ? a.src_row[m] : m;
+        double sum = 0.0;
+        if (src >= 0 && src < a.x_rows)
+#pragma nounroll
+          for (int t = 0; t < a.terms; ++t)
+#pragma nounroll
+            for (int k = k0; k < k1; ++k)
+              sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.x)[((int64_t)t * a.x_rows + src) * a.K + k]), row.weight(k), sum);
+        reinterpret_cast<float*>(own + (at >> 2) * 4 * 64)[at & 3] = (float)sum;
       }
-      if constexpr (MB == 3) {
-        if (a.terms == 3 && i == 0) v += r[1] + r[2];
-      }
-      if (a.splits > 1) {
-        float* p = a.part + ((int64_t)z * a.R + m) * a.N + n;
-        if (v4) *reinterpret_cast<f32x4*>(p) = v;
-        else
-          for (int j = 0; j < 4; ++j) if (n + j < a.N) p[j] = v[j];
-        continue;
-      }
-      const int64_t at = (a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m) * a.N + n;
-      if (!v4) {
-        for (int j = 0; j < 4; ++j) if (n + j < a.N) store_out(a.y, at + j, v[j], a.y_dtype);
-      } else if (a.y_dtype == QMM_F32) {
-        *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
-      } else {
-        u32x2 h;
-        if (a.y_dtype == QMM_BF16) h = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        else h = u32x2{f32_to_f16_bits(v[0]) | (f32_to_f16_bits(v[1]) << 16), f32_to_f16_bits(v[2]) | (f32_to_f16_bits(v[3]) << 16)};
-        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at) = h;
-      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i) r[i] = own[i * 4 * 64];
     }
-  };
-  run(std::true_type{});
-  meet();
-  give_out();
-  if constexpr (LARGE) {
-    // A scale too large for the short form of the dequantization (there never is one
-    // in earnest): everything again, the long way.  Asked behind the results, which
-    // would wait for the answer.  (Having the question costs about 1 %: 48 rows of
-    // 4096 x 14336 20.5 -> 20.6 us, 77 rows of 1024 x 2048 9.3 -> 9.5; asked step by
-    // step it made the compiler spill.)
-    const u32x4 p = *reinterpret_cast<const u32x4*>(notes), q = *reinterpret_cast<const u32x4*>(notes + 4);
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(p[0] | p[1] | p[2] | p[3] | q[0] | q[1] | q[2] | q[3]) != 0, 0)) {
-      wait_loads<0>();                           // (the stores too: the run counts what is under way)
-      __syncthreads();                           // every wavefront has read what it reads: the ring may be filled again
-      run(std::false_type{});
-      meet();
-      give_out();
+  }
+  const bool v4 = (a.N & 3) == 0 && (a.splits > 1 || (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0);
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int m = m0 + i * 16 + 4 * kg + wk;
+    if (i >= a.blocks || m >= row_hi || n >= a.N) continue;
+    const f32x4 v = r[i];
+    if (a.splits > 1) {
+      float* p = a.part + ((int64_t)z * a.R + m) * a.N + n;
+      if (v4) *reinterpret_cast<f32x4*>(p) = v;
+      else
+        for (int j = 0; j < 4; ++j) if (n + j < a.N) p[j] = v[j];
+      continue;
+    }
+    const int64_t at = (a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m) * a.N + n;
+    if (!v4) {
+      for (int j = 0; j < 4; ++j) if (n + j < a.N) store_out(a.y, at + j, v[j], a.y_dtype);
+    } else if (a.y_dtype == QMM_F32) {
+      *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
+    } else {
+      u32x2 h;
+      if (a.y_dtype == QMM_BF16) h = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      else h = u32x2{f32_to_f16_bits(v[0]) | (f32_to_f16_bits(v[1]) << 16), f32_to_f16_bits(v[2]) | (f32_to_f16_bits(v[3]) << 16)};
+      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at) = h;
     }
   }
 }

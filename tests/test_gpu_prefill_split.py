@@ -127,25 +127,49 @@ def test_wide_gathers_keep_their_weights(pairs, experts, k, kind, act):
 # whatever the scale's size, and the bias where the code is 0.  (The activations are
 # small, so that sums stay in range; one group in five is large, every third column
 # has none, and each column is judged by its own size.)
-@pytest.mark.parametrize("m,n,k", [(33, 130, 320), (128, 333, 4096), (300, 9208, 2944)])
+def large_weight(g, lead, n, k, kind):
+    bits, gs, mode, tab = kind
+    w, s, b = weight(g, lead, n, k, bits, gs, mode, tab)
+    grow = torch.rand(s.shape, device=DEV, generator=g) < 0.2
+    grow[..., ::3, :] = False
+    power = torch.randint(110, 122, s.shape, device=DEV, generator=g).float()        # scales of 2^103 .. 2^116
+    return w, torch.where(grow, s.float() * torch.exp2(power), s.float()).to(s.dtype), b
+
+
+def columns_close(y, want):
+    err = (y.double() - want).norm(dim=0) / want.norm(dim=0)
+    assert bool((err <= 2e-5).all()), err.max().item()
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 130, 320), (128, 333, 4096), (300, 2056, 2944), (650, 3080, 6144)])
 @pytest.mark.parametrize("kind", [(4, 64, "affine", "bf16"), (4, 32, "affine", "bf16"), (4, 128, "affine", "f32"),
                                   (8, 64, "affine", "bf16"), (8, 32, "affine", "f32"), (4, 32, "affine", "f32")])
 def test_large_scales(m, n, k, kind):
-    bits, gs, mode, tab = kind
+    bits, gs, mode, _ = kind
     if k % gs:
         pytest.skip("not a whole number of groups")
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     how = dict(group_size=gs, bits=bits, mode=mode)
-    w, s, b = weight(g, (), n, k, bits, gs, mode, tab)
-    grow = torch.rand(s.shape, device=DEV, generator=g) < 0.2
-    grow[::3] = False
-    power = torch.randint(110, 122, s.shape, device=DEV, generator=g).float()        # scales of 2^103 .. 2^116
-    s = torch.where(grow, s.float() * torch.exp2(power), s.float()).to(s.dtype)
+    w, s, b = large_weight(g, (), n, k, kind)
     x = (torch.randn((m, k), device=DEV, generator=g) * 2.0 ** -20).bfloat16()
-    want = x.double() @ tile(w, s, b, how).T
-    y = K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how).double()
-    err = (y - want).norm(dim=0) / want.norm(dim=0)
-    assert bool((err <= 2e-5).all()), err.max().item()
+    columns_close(K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how), x.double() @ tile(w, s, b, how).T)
+
+
+@pytest.mark.parametrize("pairs,n,k", [(100, 130, 576), (700, 1544, 1088)])
+@pytest.mark.parametrize("kind", [(4, 32, "affine", "bf16"), (8, 64, "affine", "f32"), (4, 32, "affine", "f32")])
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+def test_large_scales_of_experts(pairs, n, k, kind, act):
+    bits, gs, mode, _ = kind
+    g = torch.Generator(device=DEV).manual_seed(pairs + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = large_weight(g, (3,), n, k, kind)
+    x = (torch.randn((50, k), device=DEV, generator=g) * 2.0 ** -10).to(ACT[act])
+    lhs = torch.randint(-1, 51, (pairs,), dtype=torch.int32, device=DEV, generator=g)      # (outside [0, 50): a zero row)
+    rhs = torch.randint(0, 3, (pairs,), dtype=torch.int32, device=DEV, generator=g)
+    y = K.gather_qmm(x, w, s, b, lhs, rhs, out_dtype=torch.float32, **how)
+    rows = torch.where(((lhs >= 0) & (lhs < 50))[:, None], x[lhs.clamp(0, 49).long()], torch.zeros((), dtype=x.dtype, device=DEV))
+    for e in range(3):
+        columns_close(y[rhs == e], rows[rhs == e].double() @ tile(w[e], s[e], b[e], how).T)
 
 
 # With no room for the sums of a split K -- the least scratch that is taken -- and with
