@@ -449,14 +449,25 @@ __global__ __launch_bounds__(64 * NWAVES) void gemm2_kernel(Gemm2Args a) {
     for (int j = 0; j < NT; ++j) probe = fmaf(acc[0][j][0], 0.f, probe);      // NaN if one is not
     if (__builtin_expect(__ballot(probe != probe && kh == 0 && m0 + wm * (RB0 * 32) < row_hi) != 0ull, 0)) {
       __builtin_amdgcn_s_waitcnt(0);
-#pragma nounroll
-      for (int at = 0; at < MT * NT; ++at) {       // row block at / NT of this wavefront's, column block at % NT
-        const int i = at / NT, j = at % NT;
-        const bool fifth = i == 1 && five_tile;
-        if (fifth && j != wm) continue;
-        const int lo = m0 + (fifth ? WMW : wm * RB0 + i * RBI) * 32 + 16 * kh, hi = lo + 16 < row_hi ? lo + 16 : row_hi;
-        redo_column<BITS>(a, e, n0 + wn * (NT * 32) + j * 32 + li, lo, hi, 0, a.K, 0);
+      // this wavefront's rows, a half of every block a lane
+      int lo[2], hi[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        lo[i] = m0 + (i == 1 && five_tile ? WMW : wm * RB0 + i * RBI) * 32 + 16 * kh;
+        hi[i] = lo[i] + 16 < row_hi ? lo[i] + 16 : row_hi;
       }
+      // (a column with a finite result in any row has no such scale: it is an activation)
+      uint32_t fin = 0;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (m0 + wm * (RB0 * 32) + (r & 3) + 8 * (r >> 2) + 4 * kh < row_hi && acc[0][j][r] * 0.f == 0.f) fin |= 1u << j;
+      fin |= __shfl_xor(fin, 32);
+#pragma nounroll
+      for (int j = 0; j < NT; ++j)
+        if (!(fin >> j & 1))
+          redo_column<BITS>(a, e, n0 + wn * (NT * 32) + j * 32 + li, lo, hi, MT == 2 && (!five_tile || j == wm) ? 2 : 1, 0, a.K, 0);
     }
   }
 }

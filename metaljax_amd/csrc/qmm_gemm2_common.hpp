@@ -132,11 +132,14 @@ struct LongRow {
   __device__ __forceinline__ LongRow(const uint32_t* w, const void* s_, const void* b_, int64_t e, int64_t n, int64_t N, int64_t K, int gshift_, int tab_)
       : codes(reinterpret_cast<const uint8_t*>(w) + (e * N + n) * (K * BITS / 8)), s(s_), b(b_), entry((e * N + n) * (K >> gshift_)), tab(tab_),
         gshift(gshift_) {}
-  // Has it a scale that is not small in [k0, k1)?
+  // Has it a scale that is not small in [k0, k1)?  (Eight at a time: rows of NaN lead here too.)
   __device__ __forceinline__ bool large(int k0, int k1) const {
+    const int last = (k1 - 1) >> gshift;
     bool l = false;
 #pragma nounroll
-    for (int g = k0 >> gshift; g << gshift < k1; ++g) l |= !(fabsf(load_table_rt(s, entry + g, tab)) < kSmallScale);
+    for (int g = k0 >> gshift; g <= last; g += 8)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) l |= !(fabsf(load_table_rt(s, entry + (g + i < last ? g + i : last), tab)) < kSmallScale);
     return l;
   }
   __device__ __forceinline__ double weight(int k) const {             // the bf16 tile's
@@ -146,22 +149,26 @@ struct LongRow {
   }
 };
 
-// Column n of rows [lo, hi) over [k0, k1) again where its scales ask for it (the
-// prefill kernels: activations re-laid, results in y, or in a split's part).  The
-// kernel's own stores have to have landed.
+// Column n of the `blocks` row ranges [lo[i], hi[i]) over [k0, k1) again if its scales
+// ask for it (the prefill kernels: activations re-laid, results in y, or in a split's
+// part).  The kernel's own stores have to have landed.
 template <int BITS>
-__device__ __forceinline__ void redo_column(const Gemm2Args& a, int e, int n, int lo, int hi, int k0, int k1, int split) {
-  if (n >= a.N || lo >= hi) return;
+__device__ __forceinline__ void redo_column(const Gemm2Args& a, int e, int n, const int (&lo)[2], const int (&hi)[2], int blocks, int k0, int k1,
+                                            int split) {
+  if (n >= a.N) return;
   const LongRow<BITS> row(a.w, a.s, a.b, e, n, a.N, a.K, a.gs == 32 ? 5 : a.gs == 64 ? 6 : 7, a.tab);
   if (!row.large(k0, k1)) return;                // an activation, or a sum that is out of range
 #pragma nounroll
-  for (int m = lo; m < hi; ++m) {
-    double sum = 0.0;
+  for (int i = 0; i < blocks; ++i) {
 #pragma nounroll
-    for (int k = k0; k < k1; ++k)
-      sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.ax)[((int64_t)(k >> 3) * a.Rp + m) * 8 + (k & 7)]), row.weight(k), sum);
-    if (a.splits > 1) a.part[((int64_t)split * a.R + m) * a.N + n] = (float)sum;
-    else store_out(a.y, (a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m) * a.N + n, (float)sum, a.y_dtype);
+    for (int m = i ? lo[1] : lo[0]; m < (i ? hi[1] : hi[0]); ++m) {
+      double sum = 0.0;
+#pragma nounroll
+      for (int k = k0; k < k1; ++k)
+        sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.ax)[((int64_t)(k >> 3) * a.Rp + m) * 8 + (k & 7)]), row.weight(k), sum);
+      if (a.splits > 1) a.part[((int64_t)split * a.R + m) * a.N + n] = (float)sum;
+      else store_out(a.y, (a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m) * a.N + n, (float)sum, a.y_dtype);
+    }
   }
 }
 

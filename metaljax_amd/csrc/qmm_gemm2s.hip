@@ -527,13 +527,25 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     for (int j = 0; j < 4; ++j) probe = fmaf(acc[j][0], 0.f, probe);          // NaN if one is not
     if (__builtin_expect(__ballot(probe != probe && kh == 0 && m0 + wm * 32 < m_end) != 0ull, 0)) {
       __builtin_amdgcn_s_waitcnt(0);
-      const int k0 = kb * BK, k1 = (kb + KT) * BK;
-#pragma nounroll
-      for (int at = 0; at < 8; ++at) {             // row block at / 4 of this wavefront's, column block at % 4
-        if (at >= 4 && !two && !(five && (at & 3) == wm)) continue;
-        const int lo = m0 + (at < 4 ? wm : two ? wm + 4 : 4) * 32 + 16 * kh, hi = lo + 16 < m_end ? lo + 16 : m_end;
-        redo_column<BITS>(a, e, n0 + (at & 3) * 32 + li, lo, hi, k0, k1, split);
+      // this wavefront's rows, a half of every block a lane: block w, and w + 4 or the fifth
+      int lo[2], hi[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        lo[i] = m0 + (i == 0 ? wm : two ? wm + 4 : 4) * 32 + 16 * kh;
+        hi[i] = lo[i] + 16 < m_end ? lo[i] + 16 : m_end;
       }
+      // (a column with a finite result in any row has no such scale: it is an activation)
+      uint32_t fin = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (m0 + wm * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh < m_end && acc[j][r] * 0.f == 0.f) fin |= 1u << j;
+      fin |= __shfl_xor(fin, 32);
+#pragma nounroll
+      for (int j = 0; j < 4; ++j)
+        if (!(fin >> j & 1))
+          redo_column<BITS>(a, e, n0 + j * 32 + li, lo, hi, two || (five && j == wm) ? 2 : 1, kb * BK, (kb + KT) * BK, split);
     }
   }
 }

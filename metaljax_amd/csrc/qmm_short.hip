@@ -442,21 +442,34 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
 #pragma unroll
       for (int i = 0; i < MB; ++i) own[i * 4 * 64] = r[i];
       const int k0 = s0 * S::kStep, k1 = s1 * S::kStep < a.K ? s1 * S::kStep : a.K;
+      // (a column with a finite result in any row has no such scale: it is an activation)
+      uint32_t fin = 0;
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (i < a.blocks && r[i][j] * 0.f == 0.f) fin |= 1u << j;
+      fin |= __shfl_xor(fin, 16);
+      fin |= __shfl_xor(fin, 32);
 #pragma nounroll
-      for (int at = 0; at < a.blocks * 4; ++at) {
-        const int m = m0 + (at >> 2) * 16 + 4 * kg + wk, c = n + (at & 3);
-        if (m >= row_hi || c >= a.N) continue;
-        const g2::LongRow<BITS> row(a.w, a.s, a.b, e, c, a.N, a.K, a.gshift, TAB);
+      for (int j = 0; j < 4; ++j) {
+        if (n + j >= a.N) break;
+        if (fin >> j & 1) continue;
+        const g2::LongRow<BITS> row(a.w, a.s, a.b, e, n + j, a.N, a.K, a.gshift, TAB);
         if (!row.large(k0, k1)) continue;        // an activation, or a sum that is out of range
-        const int src = a.src_row ? a.src_row[m] : m;
-        double sum = 0.0;
-        if (src >= 0 && src < a.x_rows)
 #pragma nounroll
-          for (int t = 0; t < a.terms; ++t)
+        for (int i = 0; i < a.blocks; ++i) {
+          const int m = m0 + i * 16 + 4 * kg + wk;
+          const int src = m >= row_hi ? -1 : a.src_row ? a.src_row[m] : m;
+          double sum = 0.0;
+          if (src >= 0 && src < a.x_rows)
 #pragma nounroll
-            for (int k = k0; k < k1; ++k)
-              sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.x)[((int64_t)t * a.x_rows + src) * a.K + k]), row.weight(k), sum);
-        reinterpret_cast<float*>(own + (at >> 2) * 4 * 64)[at & 3] = (float)sum;
+            for (int t = 0; t < a.terms; ++t)
+#pragma nounroll
+              for (int k = k0; k < k1; ++k)
+                sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.x)[((int64_t)t * a.x_rows + src) * a.K + k]), row.weight(k), sum);
+          reinterpret_cast<float*>(own + i * 4 * 64)[j] = (float)sum;
+        }
       }
 #pragma unroll
       for (int i = 0; i < MB; ++i) r[i] = own[i * 4 * 64];

@@ -172,6 +172,23 @@ def test_large_scales_of_experts(pairs, n, k, kind, act):
         columns_close(y[rhs == e], rows[rhs == e].double() @ tile(w[e], s[e], b[e], how).T)
 
 
+# A result that is not finite makes a kernel look at its column's scales: where an
+# activation is the cause, only its row is touched.
+@pytest.mark.parametrize("m,n,k", [(33, 130, 320), (300, 2056, 2944), (650, 3080, 6144)])
+@pytest.mark.parametrize("kind", [(4, 64, "affine", "bf16"), (8, 64, "affine", "bf16"), (4, 32, "affine", "f32")])
+def test_activations_that_are_not_finite_stay_in_their_rows(m, n, k, kind):
+    bits, gs, mode, tab = kind
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (), n, k, bits, gs, mode, tab)
+    x = torch.randn((m, k), device=DEV, generator=g).bfloat16()
+    clean = K.quantized_matmul(x, w, s, b, **how)
+    x[::16, 5], x[1::16, k - 1] = float("nan"), float("inf")
+    y = K.quantized_matmul(x, w, s, b, **how)
+    odd = torch.arange(m, device=DEV) % 16 < 2
+    assert torch.equal(y[~odd], clean[~odd]) and not bool(y[odd].isfinite().any())
+
+
 # With no room for the sums of a split K -- the least scratch that is taken -- and with
 # some of it: fewer splits, or the other kernel, and the same product.
 @pytest.mark.parametrize("m,n,k", [(17, 1024, 4096), (48, 4096, 14336), (300, 1000, 8256), (650, 3080, 6144)])
