@@ -52,7 +52,7 @@ def test_dense(m, n, k, kind, act):
     close(K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how), x.double() @ tile(w, s, b, how).T)
 
 
-@pytest.mark.parametrize("counts", [(0, 1, 16, 0, 17), (40, 0, 3, 70, 64), (90, 129, 0, 161, 300)])
+@pytest.mark.parametrize("counts", [(0, 1, 16, 0, 17), (22, 0, 3, 31, 17), (40, 0, 3, 70, 64), (90, 129, 0, 161, 300)])
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("act", ["bf16", "f16"])
 @pytest.mark.parametrize("gathered", [False, True])
@@ -64,15 +64,16 @@ def test_groups(counts, kind, act, gathered):
     w, s, b = weight(g, (len(counts),), n, k, bits, gs, mode, tab)
     x = torch.randn((sum(counts), k), device=DEV, generator=g).to(ACT[act])
     owner = torch.repeat_interleave(torch.arange(len(counts), device=DEV), torch.tensor(counts, device=DEV))
-    want = torch.cat([x[owner == e].double() @ tile(w[e], s[e], None if b is None else b[e], how).T for e in range(len(counts))])
+    # up to 64 pairs, and (but for groups of 32) up to sixteen an expert, gathers are decode products: exact weights
+    exact = gathered and (sum(counts) <= 64 or (sum(counts) <= 16 * len(counts) and gs > 32))
+    full = [K.dequantize(w[e], s[e], None if b is None else b[e], out_dtype=torch.float32, **how) for e in range(len(counts))]
+    want = torch.cat([x[owner == e].double() @ (full[e] if exact else full[e].bfloat16()).double().T for e in range(len(counts))])
     if not gathered:
         ro = torch.tensor([sum(counts[:e]) for e in range(len(counts) + 1)], dtype=torch.int32, device=DEV)
         close(K.grouped_qmm(x, w, s, b, ro, out_dtype=torch.float32, **how), want)
-    elif sum(counts) > 64:                                              # (fewer pairs: decode kernels, exact weights)
+    else:
         mix = torch.randperm(sum(counts), device=DEV, generator=g)
-        y = K.gather_qmm(x, w, s, b, mix.int(), owner[mix].int(), out_dtype=torch.float32, **how)
-        if sum(counts) > 16 * len(counts):
-            close(y, want[mix])
+        close(K.gather_qmm(x, w, s, b, mix.int(), owner[mix].int(), out_dtype=torch.float32, **how), want[mix])
 
 
 # One expert is a dense product but for its offsets: rows outside them, and pairs
