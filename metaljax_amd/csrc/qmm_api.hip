@@ -376,11 +376,14 @@ size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
 
 // Is the short-group kernel the one to take?  `E` experts share the R rows
 // (`grouped`; else a dense product and E = 1), the activations are `terms` bf16
-// terms, and each kernel has what `scratch` leaves it for a split K's sums.  All kernels' times have been
-// fitted over the shapes they serve; where they come close the choice matters
-// little.  (4096 x 4096, four-bit codes: 17 rows 13 against 20 us of the
-// prefill kernel, 128 rows 19 against 23, 512 rows 32 against 36; 14336 x 4096:
-// 19 against 29, 32 against 33, 108 against 59.)
+// terms, and each kernel has what `scratch` leaves it for a split K's sums.  All
+// kernels' times have been fitted over the shapes they serve; where they come close
+// the choice matters little.  (4096 x 4096, four-bit codes: 17 rows 12 against 17 us of the
+// prefill kernel, 128 rows 19 against 22, 512 rows 32 against 36; 14336 x 4096:
+// 20 against 29, 31 against 34, 114 against 61.  Of 208 affine products, 48 of them
+// groups, the slower kernel is taken in a few, 11 % slower at worst; MXFP4's
+// block-scaled kernel is taken for faster than it is, for groups up to 1.35 times:
+// profiles/prefill_plan_fits.txt.)
 bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, bool grouped, size_t scratch) {
   if (K % 64 || N <= 0) return false;
   if (const char* env = experiment_env("QMM_SHORT")) return env[0] != '0';
@@ -894,9 +897,9 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
                        N, K, group_size, bits, mode, workspace, workspace_bytes, stream, false);
   // More pairs than the decode kernels take: short groups read float16 / float32
   // activations as they are.  Not where the grouped decode multiplies affine weights:
-  // it keeps them exact, the short-group kernel rounds them to bf16 (1e-6 against
+  // it keeps them exact, the short-group kernel rounds them to bf16 (1e-7 against
   // 1.6e-3 from the product of the exact weights, 128 pairs over 8 experts of 1024 x
-  // 4096, eight-bit codes).  MXFP4 weights are exact in both.
+  // 4096, eight-bit codes; four-bit ones 4e-7).  MXFP4 weights are exact in both.
   const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);

@@ -598,11 +598,13 @@ bool gemm2s_wanted(const g2::Gemm2Args& a, int mode, int bits) {
 }
 
 // Rows a tile may hold and workgroups that share its K: those that make the
-// product shortest.  Returns that time in microseconds, from a fit (within 7%
-// on average) to 700 measured products of 17 to 2048 rows, N and K 1024 to
-// 14336: the launches, a round for every 256 tiles (one workgroup fills a
-// compute unit), a K-tile of up to 128 or up to 256 rows, the re-laid
-// activations, the result, and a split K's sums.  Several experts keep 256-row
+// product shortest.  Returns that time in microseconds, from a fit to dense
+// products of 17 to 2048 rows, N and K 1024 to 14336: the launches, a round for
+// every 256 tiles (one workgroup fills a compute unit), a K-tile of up to 128 or
+// up to 256 rows, the re-laid activations, the result, and a split K's sums.
+// Checked against 68 four-bit and 68 eight-bit products it is 5 and 9 % off on
+// average; for groups it comes out 7 and 18 % too short (without the launches of a
+// caller that clears the result; profiles/prefill_plan_fits.txt).  Several experts keep 256-row
 // tiles (every expert in one, and the short loop where it fits) and their whole
 // K; for the row groups of a single expert (`row_offsets` with E = 1) the caller
 // passes no room for sums, so that they keep theirs.

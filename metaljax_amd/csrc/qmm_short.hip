@@ -26,9 +26,9 @@
 // weight through that path and sat in issue most of the time.)
 //
 // Measured, bf16 activations and four-bit codes in groups of 64, against the
-// prefill kernel on whole K: 48 rows of 4096 x 14336 104 -> 23 us, 17 rows of
-// 4096 x 4096 35 -> 13, 48 rows of 14336 x 4096 37 -> 23; float16 activations, 77
-// rows of 4096 x 4096 46 -> 25.  Of the 23 us about 10 are fixed (launch, first
+// prefill kernel on whole K: 48 rows of 4096 x 14336 104 -> 22 us, 17 rows of
+// 4096 x 4096 35 -> 12, 48 rows of 14336 x 4096 37 -> 22; float16 activations and
+// tables, 77 rows of 4096 x 4096 46 -> 21.  Of the 22 us about 10 are fixed (launch, first
 // data, the sums' second launch); a step takes 0.76 us and 0.14 more per row
 // block, the vector ALU's instructions about half of it.
 //
@@ -545,10 +545,11 @@ struct ShortPlan { int mb, blocks, m_tiles, splits; double us; };
 
 // Rows a tile: at most four row blocks of sixteen, terms included, dealt evenly.
 // Splits: as many workgroups as make the product shortest.  `us` is that time,
-// from a fit (within 7% on average) to 460 measured products of 17 to 512 rows,
-// N and K 1024 to 14336: launch, a round of tiles over the compute units for
-// every 256 workgroups, a step of 256 four-bit (128 eight-bit) codes, the
-// second launch and its traffic.
+// from a fit to products of 17 to 2048 rows, N and K 1024 to 14336: launch, a
+// round of tiles over the compute units for every 256 workgroups, a step of 256
+// four-bit (128 eight-bit) codes, the second launch and its traffic.  Checked
+// against 228 dense products it is 5 % off on average; for groups, whose sizes
+// differ, it comes out 11 to 19 % too short (profiles/prefill_plan_fits.txt).
 ShortPlan short_plan(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, size_t part_bytes) {
   ShortPlan p;
   const int64_t most = terms == 1 ? 4 : terms == 2 ? 2 : 1;      // row blocks a tile can hold
