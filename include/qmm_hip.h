@@ -139,6 +139,15 @@ int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scale
                     int group_size, int bits, int mode, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/* qmm_grouped_qmm into fresh memory: the rows of y outside the offsets, which
+ * qmm_grouped_qmm leaves as they are, are set to zero.  y may hold anything.
+ * Serves the per-expert product of reference src/metaljax/moe.py:1283-1340. */
+int qmm_grouped_qmm_zeroed(const void* x, int x_dtype, const void* w, const void* scales,
+                           const void* biases, int table_dtype, void* y, int y_dtype,
+                           const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
+                           int group_size, int bits, int mode, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
 /* Replaces mx.dequantize(w, scales, biases, group_size, bits[, mode]) --
  * used by the reference's layout tests (tests/test_qmm.py:121;
  * tests/test_qmm_mxfp4.py:192).  rows = product of the leading dims; out

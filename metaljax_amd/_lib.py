@@ -25,7 +25,7 @@ KERNEL_GEMV, KERNEL_GEMM, KERNEL_MXFP4_MFMA = 1, 2, 3
 SYMBOLS = (
     "qmm_abi_version", "qmm_last_error", "qmm_quantized_matmul", "qmm_workspace_bytes",
     "qmm_gather_workspace_bytes", "qmm_plan", "qmm_gather_qmm", "qmm_grouped_qmm",
-    "qmm_gather_qmm_static", "qmm_dequantize", "qmm_unpack_codes", "qmm_pack_codes", "qmm_take_k",
+    "qmm_grouped_qmm_zeroed", "qmm_gather_qmm_static", "qmm_dequantize", "qmm_unpack_codes", "qmm_pack_codes", "qmm_take_k",
 )
 
 
@@ -76,6 +76,7 @@ def load():
                                           i64, i64, ci, ci, ci, vp]
     lib.qmm_grouped_qmm.argtypes = [vp, ci, vp, vp, vp, ci, vp, ci, vp, i64, i64, i64, i64, ci,
                                     ci, ci, vp, sz, vp]
+    lib.qmm_grouped_qmm_zeroed.argtypes = lib.qmm_grouped_qmm.argtypes
     lib.qmm_dequantize.argtypes = [vp, vp, vp, ci, vp, ci, i64, i64, ci, ci, ci, vp]
     lib.qmm_unpack_codes.argtypes = [vp, vp, i64, i64, ci, vp]
     lib.qmm_pack_codes.argtypes = [vp, vp, i64, i64, ci, vp]

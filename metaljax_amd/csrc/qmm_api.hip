@@ -46,7 +46,7 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
                     int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
                     const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N,
                     int64_t K, int gs, int bits, int mode, int row_tile, void* workspace,
-                    size_t workspace_bytes, hipStream_t st);
+                    size_t workspace_bytes, const ClearArgs& clear, hipStream_t st);
 double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits);
 double gemm2_us(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes);
 size_t gemm2_split_workspace_bytes(int64_t R, int64_t N, int64_t K);
@@ -646,7 +646,7 @@ static int dense_bf16(const void* x, int x_dtype, const void* w, const void* sca
                      static_cast<const char*>(scales) + z * N * ng * tabsz,
                      biases ? static_cast<const char*>(biases) + z * N * ng * tabsz : nullptr,
                      table_dtype, static_cast<char*>(y) + z * M * N * ysz, y_dtype, nullptr, nullptr,
-                     nullptr, M, M, 1, N, K, group_size, bits, mode, bm, workspace, workspace_bytes, st);
+                     nullptr, M, M, 1, N, K, group_size, bits, mode, bm, workspace, workspace_bytes, ClearArgs{}, st);
       rc = check_launch("gemm launch");
       if (rc) return rc;
     }
@@ -669,7 +669,7 @@ static int grouped_bf16(const void* x, int x_dtype, const void* w, const void* s
                         const void* biases, int table_dtype, void* y, int y_dtype,
                         const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
                         int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
-                        void* stream, bool exact) {
+                        void* stream, bool exact, ClearArgs* clear) {
   if (R < 0 || E < 0) return fail(QMM_ERR_BAD_ARGUMENT, "negative shape");
   if (R == 0 || N == 0 || E == 0) return QMM_OK;
   if (!row_offsets) return fail(QMM_ERR_BAD_ARGUMENT, "null row_offsets");
@@ -690,7 +690,8 @@ static int grouped_bf16(const void* x, int x_dtype, const void* w, const void* s
       aligned16(workspace)) {
     gemm2_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, row_offsets, nullptr, nullptr, R,
                    R, E, N, K, group_size, bits, mode, (int)gemm_row_tile(R, E), workspace, workspace_bytes,
-                   static_cast<hipStream_t>(stream));
+                   *clear, static_cast<hipStream_t>(stream));
+    clear->y = nullptr;                            // done beside the re-laying
     return check_launch("grouped gemm launch");
   }
   // without a workspace the grouped product runs on the LDS-staged kernel
@@ -790,7 +791,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     // rows gathered in expert order into the re-laid copy, results scattered back to pair order
     gemm2_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K,
                    group_size, bits, mode, (int)gemm_row_tile(P, E),
-                   static_cast<char*>(workspace) + need, workspace_bytes - need, st);
+                   static_cast<char*>(workspace) + need, workspace_bytes - need, ClearArgs{}, st);
     return check_launch("gather gemm launch");
   }
   gemm_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, ro, src_row, out_row, P, T, E, N, K,
@@ -849,11 +850,13 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
   return check_launch("term sum launch");
 }
 
-int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scales,
-                    const void* biases, int table_dtype, void* y, int y_dtype,
-                    const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
-                    int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
-                    void* stream) {
+// The sorted-rows product.  A kernel that clears the rows `clear` asks for on the
+// way takes its y away.
+static int grouped_product(const void* x, int x_dtype, const void* w, const void* scales,
+                           const void* biases, int table_dtype, void* y, int y_dtype,
+                           const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
+                           int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
+                           void* stream, ClearArgs* clear) {
   const int terms = act_terms(x_dtype);
   int rs = QMM_OK;
   // (wider activations are refused without room for their terms and the terms' products)
@@ -865,7 +868,7 @@ int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scale
     return rs;
   if (terms == 1 || R <= 0 || E <= 0 || N <= 0 || K <= 0 || !x || !row_offsets || !y)
     return grouped_bf16(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, R, E, N, K,
-                        group_size, bits, mode, workspace, workspace_bytes, stream, false);
+                        group_size, bits, mode, workspace, workspace_bytes, stream, false, clear);
   // one grouped product per bf16 term (the rows keep their expert order)
   if (!aligned16(x)) return fail(QMM_ERR_BAD_ARGUMENT, "activation pointer not 16-byte aligned");
   const size_t xs = align256((size_t)(terms * R * K) * 2), ps = align256((size_t)(terms * R * N) * 4);
@@ -877,13 +880,39 @@ int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scale
   hipStream_t st = static_cast<hipStream_t>(stream);
   split_terms_dispatch(x, x_dtype, ws, 1, R, K, nullptr, -1, st);
   int rc = check_launch("activation split launch");
+  ClearArgs none{};
   for (int t = 0; t < terms && !rc; ++t)
     rc = grouped_bf16(ws + (size_t)t * R * K * 2, QMM_BF16, w, scales, biases, table_dtype,
                       ws + xs + (size_t)t * R * N * 4, QMM_F32, row_offsets, R, E, N, K, group_size, bits,
-                      mode, inner ? ws + xs + ps : nullptr, inner, stream, true);
+                      mode, inner ? ws + xs + ps : nullptr, inner, stream, true, &none);
   if (rc) return rc;
   sum_terms_dispatch(ws + xs, terms, y, y_dtype, 1, R, N, row_offsets, nullptr, E, st);
   return check_launch("term sum launch");
+}
+
+int qmm_grouped_qmm(const void* x, int x_dtype, const void* w, const void* scales,
+                    const void* biases, int table_dtype, void* y, int y_dtype,
+                    const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
+                    int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
+                    void* stream) {
+  ClearArgs none{};
+  return grouped_product(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, R, E, N, K,
+                         group_size, bits, mode, workspace, workspace_bytes, stream, &none);
+}
+
+int qmm_grouped_qmm_zeroed(const void* x, int x_dtype, const void* w, const void* scales,
+                           const void* biases, int table_dtype, void* y, int y_dtype,
+                           const int32_t* row_offsets, int64_t R, int64_t E, int64_t N, int64_t K,
+                           int group_size, int bits, int mode, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+  const bool rows = y && row_offsets && R > 0 && R <= INT32_MAX && E >= 0 && E <= 65535 && N > 0 && N <= INT32_MAX;
+  ClearArgs clear{};
+  if (rows) clear = ClearArgs{y, row_offsets, (int)R, (int)E, N * (y_dtype == QMM_F32 ? 4 : 2)};
+  const int rc = grouped_product(x, x_dtype, w, scales, biases, table_dtype, y, y_dtype, row_offsets, R, E, N, K,
+                                 group_size, bits, mode, workspace, workspace_bytes, stream, &clear);
+  if (rc || !clear.y) return rc;
+  clear_rows_dispatch(clear, static_cast<hipStream_t>(stream));
+  return check_launch("row clearing launch");
 }
 
 int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales,

@@ -159,6 +159,43 @@ __device__ __forceinline__ RowTile find_row_tile(const int32_t* offsets, int E, 
   return r;
 }
 
+// ---- rows that no expert covers ------------------------------------------------
+// A grouped product leaves the rows outside its offsets alone.  For a caller that
+// hands over fresh memory they are set to zero here, a wavefront a row, by
+// workgroups beside those that re-lay the activations, or by a launch of its own
+// where a product has no such launch.  (Every row was zeroed ahead of the product
+// before, none of which stayed: a launch of 7.3 us for 1024 x 14336 bf16 results,
+// whose product over eight experts takes 172 us with it and 170 without -- the
+// matrix cores, short of power, run a little slower for not having had the pause.)
+struct ClearArgs {
+  void* y;                      // [R][N], null: nothing is cleared
+  const int32_t* row_offsets;   // [E+1]
+  int R, E;
+  int64_t row_bytes;
+};
+
+// Row `row` (the same for the wavefront, every lane active): the offsets are read as find_row_tile reads them.
+__device__ __forceinline__ void clear_row_outside(const ClearArgs& c, int row) {
+  const int lane = (int)(threadIdx.x & 63);
+  for (int e0 = 0; e0 < c.E; e0 += 64) {
+    const int i = e0 + lane;
+    bool in = false;
+    if (i < c.E) {
+      int lo = c.row_offsets[i], hi = c.row_offsets[i + 1];
+      lo = lo < 0 ? 0 : lo;
+      hi = hi < lo ? lo : hi;
+      in = row >= lo && row < hi;
+    }
+    if (__ballot(in)) return;
+  }
+  char* p = static_cast<char*>(c.y) + (int64_t)row * c.row_bytes;
+  if (((reinterpret_cast<uintptr_t>(p) | (uintptr_t)c.row_bytes) & 15u) == 0) {
+    for (int64_t i = lane; i < c.row_bytes / 16; i += 64) reinterpret_cast<u32x4*>(p)[i] = u32x4{0u, 0u, 0u, 0u};
+  } else {
+    for (int64_t i = lane; i < c.row_bytes / 2; i += 64) reinterpret_cast<uint16_t*>(p)[i] = 0;
+  }
+}
+
 // ---- host-side helpers ------------------------------------------------------
 
 // Experiment switches (kernel overrides used while measuring).  The shipped
@@ -196,6 +233,9 @@ inline bool lds_limit(size_t bytes) {
   if (r != hipSuccess) setup_error() = r;
   return r == hipSuccess;
 }
+
+// zeroes in the rows that no expert covers, in a launch of its own (qmm_util.hip)
+void clear_rows_dispatch(const ClearArgs& c, hipStream_t st);
 
 // y = the splits' float32 sums [splits][R][N], added in order and rounded once (qmm_util.hip)
 void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,

@@ -50,10 +50,8 @@ constexpr int kStages = 4;                        // stage of K-tile t = t & 3: 
 // that both sides move whole 128-byte lines: 8 lanes read one row's line, and
 // the 8 rows of one piece are written as one 128-byte run.  A workgroup is
 // four such wavefronts side by side along K (512 contiguous bytes a row).
-__global__ __launch_bounds__(256) void gemm_prep_kernel(const uint16_t* __restrict__ x,
-                                                        const int32_t* __restrict__ lhs_idx,
-                                                        u32x4* __restrict__ ax, int R, int x_rows,
-                                                        int K, int Rp) {
+__device__ __forceinline__ void relay_rows(const uint16_t* __restrict__ x, const int32_t* __restrict__ lhs_idx,
+                                           u32x4* __restrict__ ax, int R, int x_rows, int K, int Rp) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int pieces = K / 8;
   const int pblocks = (pieces + 31) / 32;
@@ -66,6 +64,25 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const uint16_t* __restri
   u32x4 v = {0u, 0u, 0u, 0u};
   if (ok) v = reinterpret_cast<const u32x4*>(x + src * K)[piece];
   ax[(int64_t)piece * Rp + row] = v;
+}
+
+__global__ __launch_bounds__(256) void gemm_prep_kernel(const uint16_t* __restrict__ x,
+                                                        const int32_t* __restrict__ lhs_idx,
+                                                        u32x4* __restrict__ ax, int R, int x_rows,
+                                                        int K, int Rp) {
+  relay_rows(x, lhs_idx, ax, R, x_rows, K, Rp);
+}
+
+// ... and the rows of the result that no expert covers, four a workgroup past the
+// `blocks` that re-lay.  (A kernel of its own: with the further arguments the plain
+// one took 0.5 us more, 333 x 3072.)
+__global__ __launch_bounds__(256) void gemm_prep_clear_kernel(const uint16_t* __restrict__ x,
+                                                              const int32_t* __restrict__ lhs_idx,
+                                                              u32x4* __restrict__ ax, int R, int x_rows,
+                                                              int K, int Rp, int blocks, ClearArgs clear) {
+  if ((int)blockIdx.x < blocks) return relay_rows(x, lhs_idx, ax, R, x_rows, K, Rp);
+  const int row = ((int)blockIdx.x - blocks) * 4 + (threadIdx.x >> 6);
+  if (row < clear.R) clear_row_outside(clear, row);
 }
 
 // MT x NT MFMA tiles (32 x 32) per wavefront; WMW wavefronts stacked in M and
@@ -533,18 +550,24 @@ double gemm2_us(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes) {
   return gemm2s_plan(R, E, N, K, part_bytes, &rows, &splits);
 }
 
-// x bf16 [x_rows, K] (rows gathered through lhs_idx when given); the rest as gemm_dispatch.
+// x bf16 [x_rows, K] (rows gathered through lhs_idx when given); the rest as
+// gemm_dispatch.  `clear`: rows to set to zero beside the re-laying.
 void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                     int y_dtype, const int32_t* row_offsets, const int32_t* lhs_idx,
                     const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N,
                     int64_t K, int gs, int bits, int mode, int row_tile, void* workspace,
-                    size_t workspace_bytes, hipStream_t st) {
+                    size_t workspace_bytes, const ClearArgs& clear, hipStream_t st) {
   if (R == 0 || N == 0) return;
   const int64_t rp = prep_rows(R);
   const int64_t prep_blocks = ceil_div(R, 8) * ceil_div(K / 8, 32);
-  hipLaunchKernelGGL(gemm_prep_kernel, dim3((unsigned)prep_blocks), dim3(256), 0, st,
-                     static_cast<const uint16_t*>(x), lhs_idx, static_cast<u32x4*>(workspace),
-                     (int)R, (int)x_rows, (int)K, (int)rp);
+  if (clear.y)
+    hipLaunchKernelGGL(gemm_prep_clear_kernel, dim3((unsigned)(prep_blocks + ceil_div(R, 4))), dim3(256), 0, st,
+                       static_cast<const uint16_t*>(x), lhs_idx, static_cast<u32x4*>(workspace),
+                       (int)R, (int)x_rows, (int)K, (int)rp, (int)prep_blocks, clear);
+  else
+    hipLaunchKernelGGL(gemm_prep_kernel, dim3((unsigned)prep_blocks), dim3(256), 0, st,
+                       static_cast<const uint16_t*>(x), lhs_idx, static_cast<u32x4*>(workspace),
+                       (int)R, (int)x_rows, (int)K, (int)rp);
   Gemm2Args a;
   a.ax = workspace;
   a.w = static_cast<const uint32_t*>(w);

@@ -163,6 +163,11 @@ __global__ void sum_terms_kernel(const float* __restrict__ part, void* __restric
   store_out(y, i, v, y_dtype);
 }
 
+__global__ __launch_bounds__(256) void clear_rows_kernel(ClearArgs c) {
+  const int row = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (row < c.R) clear_row_outside(c, row);
+}
+
 inline unsigned blocks_for(int64_t n) { return (unsigned)ceil_div(n, kBlock); }
 
 // y = the splits' sums, added in order and rounded once.  Rows that no expert
@@ -286,6 +291,10 @@ void take_dispatch(const void* x, int x_dtype, const int32_t* perm, void* out, i
     hipLaunchKernelGGL(take_kernel<uint32_t>, dim3(blocks_for(n)), dim3(kBlock), 0, st, static_cast<const uint32_t*>(x), perm, static_cast<uint32_t*>(out), rows, K);
   else
     hipLaunchKernelGGL(take_kernel<uint16_t>, dim3(blocks_for(n)), dim3(kBlock), 0, st, static_cast<const uint16_t*>(x), perm, static_cast<uint16_t*>(out), rows, K);
+}
+
+void clear_rows_dispatch(const ClearArgs& c, hipStream_t st) {
+  if (c.R > 0 && c.row_bytes > 0) hipLaunchKernelGGL(clear_rows_kernel, dim3((unsigned)ceil_div(c.R, 4)), dim3(256), 0, st, c);
 }
 
 void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,

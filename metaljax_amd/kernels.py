@@ -128,19 +128,19 @@ def grouped_qmm(x, w, scales, biases, row_offsets, group_size=64, bits=4, mode="
         out_dtype = out_dtype or out.dtype
         if tuple(out.shape) != (r, n) or out.dtype != out_dtype or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous [{r},{n}] tensor of {out_dtype}")
-        y = out
+        y, product = out, lib.qmm_grouped_qmm
     else:
         out_dtype = out_dtype or x.dtype
-        y = torch.zeros((r, n), dtype=out_dtype, device=x.device)
+        y, product = torch.empty((r, n), dtype=out_dtype, device=x.device), lib.qmm_grouped_qmm_zeroed
     x, w, scales = x.contiguous(), w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
     ro = row_offsets.to(torch.int32).contiguous()
     tab = _dt(scales.dtype) if mode == "affine" else BF16
     need = int(lib.qmm_workspace_bytes(1, r, n, k, group_size, bits, _MODE[mode], _dt(x.dtype)))
     ws = _scratch(need, x)
-    rc = lib.qmm_grouped_qmm(_ptr(x), _dt(x.dtype), _ptr(w), _ptr(scales), _ptr(biases), tab,
-                             _ptr(y), _dt(out_dtype), _ptr(ro), r, e, n, k, group_size, bits,
-                             _MODE[mode], _ptr(ws), need, _stream(x))
+    rc = product(_ptr(x), _dt(x.dtype), _ptr(w), _ptr(scales), _ptr(biases), tab,
+                 _ptr(y), _dt(out_dtype), _ptr(ro), r, e, n, k, group_size, bits,
+                 _MODE[mode], _ptr(ws), need, _stream(x))
     _lib.check(rc)
     return y
 

@@ -217,3 +217,26 @@ def test_scratch_limits(m, n, k, act, part):
     assert call(least - 1) == 4
     assert call(room) == 0
     close(y, x.double() @ tile(w, s, b, how).T)
+
+
+# a row group ahead of the offsets, behind them and past the 64 experts a wavefront reads at once; the short-group,
+# prefill, block-scaled and LDS-staged kernels, terms of wider activations
+@pytest.mark.parametrize("n", [72, 1001])
+@pytest.mark.parametrize("r,e,k,kind,act", [(40, 3, 256, 0, "bf16"), (700, 3, 256, 0, "bf16"), (700, 70, 320, 3, "bf16"),
+                                            (300, 3, 512, 5, "bf16"), (300, 3, 96, 1, "bf16"), (700, 3, 256, 0, "f16")])
+def test_rows_that_no_expert_covers_are_zero(n, r, e, k, kind, act):
+    bits, gs, mode, tab = KINDS[kind]
+    g = torch.Generator(device=DEV).manual_seed(n + r)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (e,), n, k, bits, gs, mode, tab)
+    x = torch.randn((r, k), device=DEV, generator=g).to(ACT[act])
+    for first, last in ((5, r - 3), (0, r), (r // 2, r // 2)):
+        ro = torch.linspace(first, last, e + 1, device=DEV).to(torch.int32)
+        given = torch.full((r, n), 7.0, dtype=x.dtype, device=DEV)
+        K.grouped_qmm(x, w, s, b, ro, out=given, **how)
+        poison = torch.full((r, n), float("nan"), dtype=x.dtype, device=DEV)      # what the next allocation holds
+        del poison
+        y = K.grouped_qmm(x, w, s, b, ro, **how)
+        assert torch.equal(y[first:last], given[first:last])
+        assert not y[:first].any() and not y[last:].any()
+        assert (given[:first] == 7.0).all() and (given[last:] == 7.0).all()
