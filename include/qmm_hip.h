@@ -173,6 +173,78 @@ int qmm_pack_codes(const void* codes, void* w, int64_t rows, int64_t K, int bits
 int qmm_take_k(const void* x, int x_dtype, const int32_t* perm, void* out, int64_t rows,
                int64_t K, void* stream);
 
+/* ---- the tensor work round an expert dispatch's products -----------------------
+ * Short programs over float32 registers; an instruction rounds its result to `el`
+ * (QMM_EL_F32: not at all).  Registers are named by number in a pair map, by their
+ * first float in a row program. */
+#define QMM_EL_F32 0
+#define QMM_EL_BF16 1
+#define QMM_EL_F16 2
+#define QMM_EL_BOOL 3
+#define QMM_EL_I32 4                                   /* outputs of a row program */
+enum {
+  QMM_OP_COPY, QMM_OP_ADD, QMM_OP_SUB, QMM_OP_MUL, QMM_OP_DIV, QMM_OP_MAX, QMM_OP_MIN, QMM_OP_POW, QMM_OP_ABS,
+  QMM_OP_NEG, QMM_OP_EXP, QMM_OP_LOG, QMM_OP_LOGISTIC, QMM_OP_TANH, QMM_OP_SQRT, QMM_OP_RSQRT, QMM_OP_CEIL,
+  QMM_OP_FLOOR, QMM_OP_RINT, QMM_OP_SIGN, QMM_OP_EQ, QMM_OP_NE, QMM_OP_LT, QMM_OP_LE, QMM_OP_GT, QMM_OP_GE,
+  QMM_OP_AND, QMM_OP_OR, QMM_OP_XOR, QMM_OP_NOT,
+  QMM_OP_SELECT,                                       /* a ? b : c */
+  QMM_OP_CLAMP,                                        /* b between a and c */
+  QMM_OP_IMM,
+  QMM_OP_SUM, QMM_OP_ROWMAX, QMM_OP_ROWMIN,            /* row programs only, from here on */
+  QMM_OP_SLICE,                                        /* n elements of a from b on, c apart */
+  QMM_OP_TOPK                                          /* the n largest of a, largest first, equal ones by index: dst; indices: c */
+};
+
+#define QMM_MAP_LEAVES 8
+#define QMM_MAP_CODE 40
+#define QMM_MAP_REGISTERS 32
+typedef struct { uint8_t op, dst, a, b, c, el; float imm; } qmm_instruction;
+/* Element base + pair p * pair + its expert * expert + its token * token + the
+ * output coordinates * coef of p. */
+typedef struct { const void* p; int64_t base; int32_t pair, expert, token, coef[3], el; } qmm_map_leaf;
+/* y[p, i] for the P selected (token, expert) pairs -- pair p is token
+ * p / per_token and expert experts_of[p] -- and the i < inner elements of a pair
+ * (coordinates dims[3 - rank..2]); leaf j starts in register j.  With `weights`
+ * [P]: y[t, i] = sum over a token's pairs of weights[p] * (the result in sum_el). */
+typedef struct {
+  void* y;
+  const void* weights;
+  const int32_t* experts_of;
+  int64_t pairs, inner, dims[3];
+  int32_t per_token, experts, rank, y_el, sum_el, weights_el, leaves, instructions, registers, result;
+  qmm_map_leaf leaf[QMM_MAP_LEAVES];
+  qmm_instruction code[QMM_MAP_CODE];
+} qmm_pair_map;
+
+/* One pair map launch: the array operations between and behind the per-expert
+ * products of a gathered dispatch (reference src/metaljax/moe.py:1425-1461).  An
+ * expert index outside [0, experts) reads the nearest expert's data. */
+int qmm_pair_map_run(const qmm_pair_map* map, void* stream);
+
+#define QMM_ROW_LEAVES 8
+#define QMM_ROW_CODE 48
+#define QMM_ROW_OUTS 2
+#define QMM_ROW_FLOATS 8192
+typedef struct { int32_t op, el, dst, n, a, an, b, bn, c, cn; float imm; } qmm_row_instruction;
+typedef struct { const void* p; int64_t base, token, step; int32_t el, dst, n; } qmm_row_leaf;
+typedef struct { void* p; int32_t el, src, srcn, n; } qmm_row_out;
+/* For every token: optionally a row of a product (dot_x[t] . dot_w, dot_n columns
+ * over dot_k, float32 sums; dot_cols: dot_n rounded up to a power of two) into
+ * register dot_dst, then the leaves, then the program; out[j] is [tokens, n]. */
+typedef struct {
+  const void *dot_x, *dot_w;
+  int64_t dot_x_t, dot_x_k, dot_w_n, dot_w_k, dot_k;
+  int32_t dot_n, dot_cols, dot_dst, dot_x_el, dot_w_el, dot_el;
+  int32_t tokens, reg_floats, leaves, instructions, outs;
+  qmm_row_leaf leaf[QMM_ROW_LEAVES];
+  qmm_row_out out[QMM_ROW_OUTS];
+  qmm_row_instruction code[QMM_ROW_CODE];
+} qmm_row_program;
+
+/* One row program launch: a router from its logits to the selected experts and
+ * their weights (the graph of reference src/metaljax/moe.py:335-442). */
+int qmm_row_program_run(const qmm_row_program* program, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

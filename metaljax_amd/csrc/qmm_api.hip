@@ -101,6 +101,13 @@ int check_launch(const char* what) {
   return QMM_OK;
 }
 
+}  // namespace
+
+int moe_fail(int code, const char* what) { return fail(code, "%s", what); }
+int moe_launched(const char* what) { return check_launch(what); }
+
+namespace {
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Largest M served by the decode kernel.

@@ -1,0 +1,335 @@
+// The small tensor work round an expert dispatch's products on gfx950, a launch a
+// stretch of it: the router (logits, top-k, routing weights) and what lies between
+// and behind the per-expert products (biases gathered by expert, slices,
+// activations, the routing-weighted sum over a token's experts).  Reference
+// src/metaljax/moe.py:335-442 and :1425-1461 run the same as one array operation
+// after another.
+//
+// What bounds it: nothing here is more than a few hundred thousand elements, so a
+// launch is its fixed cost and a few dependent loads: a pair map of 6 x 1024 takes
+// 5.4 us, the row program of 3 tokens over 1024 x 8 router weights 11 (both cold;
+// an empty launch is 2.7).  As array operations a block of 3 tokens over 8 experts
+// of 1024 x 1024 was some thirty launches with their host work and three round
+// trips to the host, 432 us; now it is these three launches and the two products,
+// 89 us, most of it the host's work for nine launches.
+//
+// Both kernels interpret a short program that the planner wrote once: the same
+// instruction for every lane, operands in LDS (column of a lane: its own, so that no
+// barrier is needed between instructions), arithmetic in float32, one rounding to the
+// value's element type an instruction -- what an array operation of that type does.
+#include "../../include/qmm_hip.h"
+#include "qmm_common.hpp"
+
+namespace qmm {
+
+int moe_fail(int code, const char* what);        // qmm_api.hip: sets qmm_last_error
+int moe_launched(const char* what);
+
+namespace {
+
+__device__ __forceinline__ float round_to(float v, int el) {
+  if (el == QMM_EL_BF16) return bf16_bits_to_f32(f32_to_bf16_bits(v));
+  if (el == QMM_EL_F16) return f16_bits_to_f32(f32_to_f16_bits(v));
+  return v;
+}
+
+__device__ __forceinline__ float either_nan(float a, float b, float v) { return a != a ? a : b != b ? b : v; }
+
+__device__ __forceinline__ float apply(int op, float a, float b, float c) {
+  switch (op) {
+    case QMM_OP_ADD: return a + b;
+    case QMM_OP_SUB: return a - b;
+    case QMM_OP_MUL: return a * b;
+    case QMM_OP_DIV: return __fdiv_rn(a, b);
+    case QMM_OP_MAX: return either_nan(a, b, fmaxf(a, b));
+    case QMM_OP_MIN: return either_nan(a, b, fminf(a, b));
+    case QMM_OP_POW: return powf(a, b);
+    case QMM_OP_ABS: return fabsf(a);
+    case QMM_OP_NEG: return -a;
+    case QMM_OP_EXP: return expf(a);
+    case QMM_OP_LOG: return logf(a);
+    case QMM_OP_LOGISTIC: return __fdiv_rn(1.f, 1.f + expf(-a));
+    case QMM_OP_TANH: return tanhf(a);
+    case QMM_OP_SQRT: return __fsqrt_rn(a);
+    case QMM_OP_RSQRT: return __fdiv_rn(1.f, __fsqrt_rn(a));
+    case QMM_OP_CEIL: return ceilf(a);
+    case QMM_OP_FLOOR: return floorf(a);
+    case QMM_OP_RINT: return rintf(a);
+    case QMM_OP_SIGN: return a != a ? a : a > 0.f ? 1.f : a < 0.f ? -1.f : a;
+    case QMM_OP_EQ: return a == b ? 1.f : 0.f;
+    case QMM_OP_NE: return a != b ? 1.f : 0.f;
+    case QMM_OP_LT: return a < b ? 1.f : 0.f;
+    case QMM_OP_LE: return a <= b ? 1.f : 0.f;
+    case QMM_OP_GT: return a > b ? 1.f : 0.f;
+    case QMM_OP_GE: return a >= b ? 1.f : 0.f;
+    case QMM_OP_AND: return a != 0.f && b != 0.f ? 1.f : 0.f;
+    case QMM_OP_OR: return a != 0.f || b != 0.f ? 1.f : 0.f;
+    case QMM_OP_XOR: return (a != 0.f) != (b != 0.f) ? 1.f : 0.f;
+    case QMM_OP_NOT: return a != 0.f ? 0.f : 1.f;
+    case QMM_OP_SELECT: return a != 0.f ? b : c;
+    case QMM_OP_CLAMP: {                           // min(max(b, low a), high c), NaN passed on
+      const float m = either_nan(b, a, fmaxf(b, a));
+      return either_nan(m, c, fminf(m, c));
+    }
+    default: return a;                             // QMM_OP_COPY
+  }
+}
+
+// The dword that holds element i, shifted down to it: the same load whatever the
+// type, so that several can be under way (with a branch on the type round each load
+// they came one after the other).  The dword lies in the allocation that holds the
+// element: those are whole dwords.
+struct Raw { uint32_t word; uint32_t shift; };
+__device__ __forceinline__ Raw load_raw(const void* p, int64_t i, int el) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p) + (uint64_t)i * (el == QMM_EL_F32 ? 4u : el == QMM_EL_BOOL ? 1u : 2u);
+  return Raw{*reinterpret_cast<const uint32_t*>(at & ~(uintptr_t)3), (uint32_t)(at & 3u) * 8u};
+}
+__device__ __forceinline__ float widen_raw(const Raw& r, int el) {
+  if (el == QMM_EL_F32) return __uint_as_float(r.word);
+  const uint32_t v = r.word >> r.shift;
+  if (el == QMM_EL_BF16) return __uint_as_float(v << 16);
+  if (el == QMM_EL_F16) return f16_bits_to_f32(v & 0xFFFFu);
+  return (v & 0xFFu) ? 1.f : 0.f;
+}
+__device__ __forceinline__ void store_el(void* p, int64_t i, float v, int el) {
+  if (el == QMM_EL_F32) static_cast<float*>(p)[i] = v;
+  else if (el == QMM_EL_I32) static_cast<int32_t*>(p)[i] = (int32_t)v;
+  else if (el == QMM_EL_BF16) static_cast<uint16_t*>(p)[i] = (uint16_t)f32_to_bf16_bits(v);
+  else static_cast<uint16_t*>(p)[i] = (uint16_t)f32_to_f16_bits(v);
+}
+
+// An instruction out of LDS, into scalar registers: it is the same for all lanes.
+// (The program is copied there when the kernel starts, a word a lane.  Read from the
+// kernel's arguments one instruction after the other, each was a round trip of its own.)
+template <class T>
+__device__ __forceinline__ T uniform(const T& in) {
+  constexpr int n = sizeof(T) / 4;
+  union { T t; int w[n]; } u;
+  u.t = in;
+#pragma unroll
+  for (int i = 0; i < n; ++i) u.w[i] = __builtin_amdgcn_readfirstlane(u.w[i]);
+  return u.t;
+}
+
+constexpr int kThreads = 256;
+
+// One output element a thread: its leaves are requested together (one round trip
+// for all of them), then the program runs over its column of the register file.
+__global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
+  extern __shared__ float regs[];
+  float* const r = regs + threadIdx.x;
+  qmm_map_leaf* const leaves = reinterpret_cast<qmm_map_leaf*>(regs + a.registers * kThreads);
+  qmm_instruction* const code = reinterpret_cast<qmm_instruction*>(leaves + QMM_MAP_LEAVES);
+  if ((int)threadIdx.x < a.instructions) code[threadIdx.x] = a.code[threadIdx.x];
+  else if (threadIdx.x >= 64 && (int)threadIdx.x - 64 < a.leaves) leaves[threadIdx.x - 64] = a.leaf[threadIdx.x - 64];
+  __syncthreads();
+  const int i = (int)blockIdx.x * kThreads + (int)threadIdx.x;
+  if (i >= (int)a.inner) return;
+  int c[3] = {0, 0, i};
+  if (a.rank > 1) { c[1] = i / (int)a.dims[2]; c[2] = i - c[1] * (int)a.dims[2]; }
+  if (a.rank > 2) { c[0] = c[1] / (int)a.dims[1]; c[1] -= c[0] * (int)a.dims[1]; }
+  const int per = a.weights ? a.per_token : 1;
+  float total = 0.f;
+  for (int k = 0; k < per; ++k) {
+    const int p = (int)blockIdx.y * per + k, t = p / a.per_token;
+    const int e0 = __builtin_amdgcn_readfirstlane(a.experts_of[p]);
+    const int e = e0 < 0 ? 0 : e0 >= a.experts ? a.experts - 1 : e0;
+    Raw raw[QMM_MAP_LEAVES];
+    int el[QMM_MAP_LEAVES];
+#pragma unroll
+    for (int j = 0; j < QMM_MAP_LEAVES; ++j) {
+      if (j < a.leaves) {
+        const qmm_map_leaf l = uniform(leaves[j]);
+        const int64_t row = l.base + (int64_t)p * l.pair + (int64_t)e * l.expert + (int64_t)t * l.token;
+        raw[j] = load_raw(l.p, row + (int64_t)c[0] * l.coef[0] + (int64_t)c[1] * l.coef[1] + (int64_t)c[2] * l.coef[2], l.el);
+        el[j] = l.el;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < QMM_MAP_LEAVES; ++j)
+      if (j < a.leaves) r[j * kThreads] = widen_raw(raw[j], el[j]);
+    for (int n = 0; n < a.instructions; ++n) {
+      const qmm_instruction q = uniform(code[n]);
+      const float v = q.op == QMM_OP_IMM ? q.imm : apply(q.op, r[q.a * kThreads], r[q.b * kThreads], r[q.c * kThreads]);
+      r[q.dst * kThreads] = round_to(v, q.el);
+    }
+    const float v = r[a.result * kThreads];
+    if (!a.weights) {
+      store_el(a.y, (int64_t)blockIdx.y * a.inner + i, v, a.y_el);
+      return;
+    }
+    total += round_to(v, a.sum_el) * widen_raw(load_raw(a.weights, p, a.weights_el), a.weights_el);
+  }
+  store_el(a.y, (int64_t)blockIdx.y * a.inner + i, total, a.y_el);
+}
+
+constexpr int kRowThreads = 1024;
+static_assert(QMM_ROW_CODE * sizeof(qmm_row_instruction) / 4 <= kRowThreads && QMM_MAP_CODE <= kThreads, "the program is copied a word (an instruction) a thread");
+
+__device__ __forceinline__ void wave_lds_fence() {          // one wavefront's LDS accesses, in the order written
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One workgroup a token.  All sixteen wavefronts add up the logits (a thread a
+// column and a share of the contraction, neighbouring threads along the dimension
+// that is contiguous), the first one runs the program: a register is a row of
+// floats in LDS, a lane takes elements lane, lane + 64, ...
+__global__ __launch_bounds__(kRowThreads) void row_program_kernel(qmm_row_program a) {
+  extern __shared__ float regs[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t t = blockIdx.x;
+  int* const code = reinterpret_cast<int*>(regs + a.reg_floats + (a.dot_x ? kRowThreads : 0));
+  constexpr int kWords = sizeof(qmm_row_instruction) / 4;
+  if ((int)threadIdx.x < a.instructions * kWords) code[threadIdx.x] = reinterpret_cast<const int*>(a.code)[threadIdx.x];
+  if (wave < a.leaves) {                           // (eight leaves at most, sixteen wavefronts)
+    const qmm_row_leaf l = a.leaf[wave];
+    for (int i = lane; i < l.n; i += 64)
+      regs[l.dst + i] = widen_raw(load_raw(l.p, l.base + t * l.token + (int64_t)i * l.step, l.el), l.el);
+  }
+  if (a.dot_x) {
+    float* const part = regs + a.reg_floats;
+    const int cols = a.dot_cols, shares = kRowThreads / cols;
+    const bool along_k = a.dot_w_k == 1;
+    const int n = along_k ? (int)threadIdx.x / shares : (int)threadIdx.x % cols;
+    const int s = along_k ? (int)threadIdx.x % shares : (int)threadIdx.x / cols;
+    float sum = 0.f;
+    if (n < a.dot_n) {
+      const int64_t x0 = t * a.dot_x_t, w0 = n * a.dot_w_n;
+#pragma unroll 8
+      for (int64_t k = s; k < a.dot_k; k += shares)
+        sum = fmaf(widen_raw(load_raw(a.dot_x, x0 + k * a.dot_x_k, a.dot_x_el), a.dot_x_el),
+                   widen_raw(load_raw(a.dot_w, w0 + k * a.dot_w_k, a.dot_w_el), a.dot_w_el), sum);
+    }
+    part[s * cols + n] = sum;
+    for (int h = shares / 2; h > 0; h /= 2) {
+      __syncthreads();
+      if (s < h) part[s * cols + n] += part[(s + h) * cols + n];
+    }
+    __syncthreads();
+    if (s == 0 && n < a.dot_n) regs[a.dot_dst + n] = round_to(part[n], a.dot_el);
+  }
+  __syncthreads();
+  if (wave) return;
+  for (int q0 = 0; q0 < a.instructions; ++q0) {
+    wave_lds_fence();
+    const qmm_row_instruction q = uniform(reinterpret_cast<const qmm_row_instruction*>(code)[q0]);
+    if (q.op == QMM_OP_TOPK) {
+      // an element's place is the number of those ahead of it: larger, or equal (NaN last) and of a smaller index
+      for (int i = lane; i < q.an; i += 64) {
+        const float v = regs[q.a + i];
+        int place = 0;
+        for (int j = 0; j < q.an; ++j) {
+          const float u = regs[q.a + j];
+          const bool alike = v == u || (v != v && u != u);
+          place += (alike ? j < i : u > v || (v != v && u == u)) ? 1 : 0;
+        }
+        if (place < q.n) {
+          regs[q.dst + place] = v;
+          regs[q.c + place] = (float)i;
+        }
+      }
+      continue;
+    }
+    if (q.op == QMM_OP_SUM || q.op == QMM_OP_ROWMAX || q.op == QMM_OP_ROWMIN) {
+      const int op = q.op == QMM_OP_SUM ? QMM_OP_ADD : q.op == QMM_OP_ROWMAX ? QMM_OP_MAX : QMM_OP_MIN;
+      float v = q.op == QMM_OP_SUM ? 0.f : q.op == QMM_OP_ROWMAX ? -INFINITY : INFINITY;
+      for (int i = lane; i < q.an; i += 64) v = apply(op, v, regs[q.a + i], 0.f);
+#pragma unroll
+      for (int d = 32; d > 0; d /= 2) v = apply(op, v, __shfl_xor(v, d, 64), 0.f);
+      if (lane == 0) regs[q.dst] = round_to(v, q.el);
+      continue;
+    }
+    for (int i = lane; i < q.n; i += 64) {
+      float v;
+      if (q.op == QMM_OP_IMM) v = q.imm;
+      else if (q.op == QMM_OP_SLICE) v = regs[q.a + q.b + i * q.c];
+      else v = apply(q.op, regs[q.a + (q.an == 1 ? 0 : i)], regs[q.b + (q.bn == 1 ? 0 : i)], regs[q.c + (q.cn == 1 ? 0 : i)]);
+      regs[q.dst + i] = round_to(v, q.el);
+    }
+  }
+  wave_lds_fence();
+  for (int j = 0; j < a.outs; ++j) {
+    const qmm_row_out o = a.out[j];
+    for (int i = lane; i < o.n; i += 64) store_el(o.p, t * o.n + i, regs[o.src + (o.srcn == 1 ? 0 : i)], o.el);
+  }
+}
+
+bool float_el(int el) { return el == QMM_EL_F32 || el == QMM_EL_BF16 || el == QMM_EL_F16; }
+bool map_op(int op) { return op >= QMM_OP_COPY && op <= QMM_OP_IMM; }
+
+}  // namespace
+}  // namespace qmm
+
+using namespace qmm;
+
+extern "C" {
+
+// Every index that the program holds is checked here: what the kernel computes from
+// it then stays inside the register file; addresses are the caller's shapes.
+int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
+  if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
+  if (a->pairs < 0 || a->inner < 0 || a->per_token < 1 || a->pairs % a->per_token || a->experts < 1 || a->rank < 1 || a->rank > 3)
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: shape");
+  if (a->pairs == 0 || a->inner == 0) return QMM_OK;
+  const int64_t rows = a->weights ? a->pairs / a->per_token : a->pairs;
+  if (rows > 65535 || a->inner > INT32_MAX - kThreads) return moe_fail(QMM_ERR_BAD_SHAPE, "pair map: more pairs than a grid takes");
+  int64_t n = 1;
+  for (int i = 0; i < a->rank; ++i) {
+    if (a->dims[2 - i] < 1) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: dimensions");
+    n *= a->dims[2 - i];
+  }
+  if (n != a->inner || !a->experts_of || !a->y || !float_el(a->y_el) || !float_el(a->sum_el) || (a->weights && !float_el(a->weights_el)) || a->pairs > INT32_MAX)
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: pointers or types");
+  if (a->leaves < 0 || a->leaves > QMM_MAP_LEAVES || a->instructions < 0 || a->instructions > QMM_MAP_CODE ||
+      a->registers < 1 || a->registers > QMM_MAP_REGISTERS || a->leaves > a->registers || a->result < 0 || a->result >= a->registers)
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: program size");
+  for (int i = 0; i < a->leaves; ++i)
+    if (!a->leaf[i].p || a->leaf[i].el < 0 || a->leaf[i].el > QMM_EL_BOOL) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: leaf");
+  for (int i = 0; i < a->instructions; ++i) {
+    const qmm_instruction& q = a->code[i];
+    if (!map_op(q.op) || q.dst >= a->registers || q.a >= a->registers || q.b >= a->registers || q.c >= a->registers || !float_el(q.el))
+      return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: instruction");
+  }
+  const dim3 grid((unsigned)ceil_div(a->inner, kThreads), (unsigned)rows);
+  const size_t lds = (size_t)a->registers * kThreads * 4 + sizeof(a->code) + sizeof(a->leaf);
+  hipLaunchKernelGGL(pair_map_kernel, grid, dim3(kThreads), lds, static_cast<hipStream_t>(stream), *a);
+  return moe_launched("pair map launch");
+}
+
+int qmm_row_program_run(const qmm_row_program* a, void* stream) {
+  if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
+  if (a->tokens < 0 || a->tokens > (1 << 30) || a->reg_floats < 1 || a->reg_floats > QMM_ROW_FLOATS || a->leaves < 0 ||
+      a->leaves > QMM_ROW_LEAVES || a->instructions < 0 || a->instructions > QMM_ROW_CODE || a->outs < 0 || a->outs > QMM_ROW_OUTS)
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: size");
+  if (a->tokens == 0) return QMM_OK;
+  auto in = [&](int64_t at, int64_t n) { return at >= 0 && n >= 1 && at + n <= a->reg_floats; };
+  if (a->dot_x && (!a->dot_w || a->dot_k < 1 || a->dot_n < 1 || a->dot_cols < a->dot_n || a->dot_cols > kRowThreads ||
+                   (a->dot_cols & (a->dot_cols - 1)) || !in(a->dot_dst, a->dot_n) || !float_el(a->dot_x_el) ||
+                   !float_el(a->dot_w_el) || !float_el(a->dot_el)))
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: product");
+  for (int i = 0; i < a->leaves; ++i)
+    if (!a->leaf[i].p || !in(a->leaf[i].dst, a->leaf[i].n) || a->leaf[i].el < 0 || a->leaf[i].el > QMM_EL_BOOL)
+      return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: leaf");
+  for (int i = 0; i < a->instructions; ++i) {
+    const qmm_row_instruction& q = a->code[i];
+    bool ok = float_el(q.el) && in(q.dst, q.op == QMM_OP_SUM || q.op == QMM_OP_ROWMAX || q.op == QMM_OP_ROWMIN ? 1 : q.n);
+    if (q.op == QMM_OP_TOPK) ok = ok && in(q.a, q.an) && in(q.c, q.n) && q.n <= q.an;
+    else if (q.op == QMM_OP_SUM || q.op == QMM_OP_ROWMAX || q.op == QMM_OP_ROWMIN) ok = ok && in(q.a, q.an);
+    else if (q.op == QMM_OP_SLICE) ok = ok && in(q.a, q.an) && q.b >= 0 && q.c >= 1 && q.b + (int64_t)(q.n - 1) * q.c < q.an;
+    else if (q.op != QMM_OP_IMM)
+      ok = ok && map_op(q.op) && in(q.a, q.an) && in(q.b, q.bn) && in(q.c, q.cn) && (q.an == 1 || q.an >= q.n) &&
+           (q.bn == 1 || q.bn >= q.n) && (q.cn == 1 || q.cn >= q.n);
+    if (!ok) return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: instruction");
+  }
+  for (int i = 0; i < a->outs; ++i)
+    if (!a->out[i].p || a->out[i].n < 1 || !in(a->out[i].src, a->out[i].srcn) || (a->out[i].srcn != 1 && a->out[i].srcn < a->out[i].n) ||
+        !(float_el(a->out[i].el) || a->out[i].el == QMM_EL_I32))
+      return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: output");
+  const size_t lds = ((size_t)a->reg_floats + (a->dot_x ? kRowThreads : 0)) * 4 + sizeof(a->code);
+  hipLaunchKernelGGL(row_program_kernel, dim3((unsigned)a->tokens), dim3(kRowThreads), lds, static_cast<hipStream_t>(stream), *a);
+  return moe_launched("row program launch");
+}
+
+}  // extern "C"

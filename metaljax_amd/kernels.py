@@ -22,7 +22,7 @@ _MODE = {"affine": MODE_AFFINE, "mxfp4": MODE_MXFP4}
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch.cuda.current_stream(t.device.index).cuda_stream
 
 
 # One scratch allocation per (device, stream), grown to the largest request seen:
@@ -33,10 +33,10 @@ def _stream(t: torch.Tensor) -> int:
 _SCRATCH = {}
 
 
-def _scratch(need: int, like: torch.Tensor):
+def _scratch(need: int, like: torch.Tensor, stream=None):
     if not need:
         return None
-    key = (like.device.index, _stream(like))
+    key = (like.device.index, _stream(like) if stream is None else stream)
     ws = _SCRATCH.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=like.device)
@@ -102,12 +102,12 @@ def quantized_matmul(x, w, scales, biases=None, transpose=True, group_size=64, b
     w, scales = w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
     tab = _dt(scales.dtype) if mode == "affine" else BF16
-    need = int(lib.qmm_workspace_bytes(batch, mrows, n, k, group_size, bits, _MODE[mode],
-                                       _dt(x2.dtype)))
-    ws = _scratch(need, x)
+    stream = _stream(x)
+    need = lib.qmm_workspace_bytes(batch, mrows, n, k, group_size, bits, _MODE[mode], _dt(x2.dtype))
+    ws = _scratch(need, x, stream)
     rc = lib.qmm_quantized_matmul(
         _ptr(x2), _dt(x2.dtype), _ptr(w), _ptr(scales), _ptr(biases), tab, _ptr(y), _dt(out_dtype),
-        batch, mrows, n, k, group_size, bits, _MODE[mode], _ptr(ws), need, _stream(x))
+        batch, mrows, n, k, group_size, bits, _MODE[mode], _ptr(ws), need, stream)
     _lib.check(rc)
     return y
 
@@ -161,8 +161,7 @@ def gather_qmm(x, w, scales, biases=None, lhs_indices=None, rhs_indices=None, tr
     _need_cuda(x, w, scales, biases, lhs_indices, rhs_indices)
     lib = _lib.load()
     (e,), n, k = _weight_dims(w, bits, mode)
-    rhs = rhs_indices.to(torch.int32).contiguous()
-    lhs = None if lhs_indices is None else lhs_indices.to(torch.int32).contiguous()
+    rhs, lhs = _indices(rhs_indices), None if lhs_indices is None else _indices(lhs_indices)
     rows, with_rows = 1, x.dim() == 3
     if with_rows:
         rows = x.shape[1]
@@ -180,14 +179,20 @@ def gather_qmm(x, w, scales, biases=None, lhs_indices=None, rhs_indices=None, tr
     y = torch.empty((p, n), dtype=out_dtype, device=x.device)
     x, w, scales = x.contiguous(), w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
-    nbytes = int(lib.qmm_gather_workspace_bytes(p, e, n, k, _dt(x.dtype)))
-    ws = _scratch(nbytes, x)
+    act, stream = _dt(x.dtype), _stream(x)
+    nbytes = lib.qmm_gather_workspace_bytes(p, e, n, k, act)
+    ws = _scratch(nbytes, x, stream)
     tab = _dt(scales.dtype) if mode == "affine" else BF16
-    rc = lib.qmm_gather_qmm(_ptr(x), _dt(x.dtype), _ptr(w), _ptr(scales), _ptr(biases), tab,
+    rc = lib.qmm_gather_qmm(_ptr(x), act, _ptr(w), _ptr(scales), _ptr(biases), tab,
                             _ptr(y), _dt(out_dtype), _ptr(lhs), _ptr(rhs), p, t, e, n, k,
-                            group_size, bits, _MODE[mode], _ptr(ws), nbytes, _stream(x))
+                            group_size, bits, _MODE[mode], _ptr(ws), nbytes, stream)
     _lib.check(rc)
     return y.reshape(p // rows, rows, n) if with_rows else y
+
+
+def _indices(t):
+    t = t if t.dtype == torch.int32 else t.to(torch.int32)
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def dequantize(w, scales, biases=None, group_size=64, bits=4, mode="affine",

@@ -192,6 +192,9 @@ def split_experts(arrays, e):
     (reference moe.py:1276-1280)."""
     out = []
     for a in arrays:
+        if len(a.shape) == 3 and a.shape[0] == e:
+            out.append(a)
+            continue
         rows = count(a.shape[:-1])
         out.append(a.reshape((e, rows // e, a.shape[-1])))
     return out
@@ -412,6 +415,13 @@ def _rest_pos(e, t, axis):
     return sum(1 for i in range(axis) if i != e and i != t)
 
 
+class DotInfo:
+    """A per-expert product as the plan found it: its match, the activations
+    (`data`, expert axis `data_e`, token axis `t_dim`, contraction axes), rows and
+    columns of a pair, and `columns`: dense result axis -> axis of `nshape`."""
+    __slots__ = ("match", "data", "data_e", "t_dim", "contract", "rows", "k", "nshape", "columns", "direct", "out_el")
+
+
 class PairPlan:
     """The region Y of a dispatch re-planned over the selected pairs.
 
@@ -431,6 +441,7 @@ class PairPlan:
         self.reads = []                 # values read from env at run time
         self.matches = []               # quantized-matmul matches whose packs are read
         self.dots = 0
+        self.dot_info = {}              # (value, e, t) -> DotInfo
 
     def _new_slot(self, fill, paired) -> int:
         self.program.append(fill)
@@ -715,6 +726,10 @@ class PairPlan:
         self.dots += 1
         out_el = elem(op.results[0])
         E, T = self.E, self.T
+        info = self.dot_info[op.results[0], e, t] = DotInfo()
+        info.match, info.data, info.data_e, info.t_dim = m, data, data_e, t_dim
+        info.contract, info.rows, info.k, info.nshape, info.direct, info.out_el = list(dcontract), M, K, nshape, direct, out_el
+        info.columns = {i: n_axes.index(origin(i)[1]) for i in range(len(shape)) if i not in (e, t) and origin(i)[0] == weight_side}
 
         def fill(ctx):
             from . import qmm
@@ -758,6 +773,15 @@ class Dispatch:
         self.disabled = False
         self.verified = not VERIFY
         self._tidx = None
+        self.launches = None            # moe_launch.Launches where a GPU is visible and it serves the plan
+
+    def pair_tokens(self, device):
+        """Token of pair p, p // K, as int32 and int64: the same every call."""
+        import torch
+        if self._tidx is None:
+            t32 = torch.arange(self.T, dtype=torch.int32, device=device).repeat_interleave(self.K)
+            self._tidx = (t32, t32.long())
+        return self._tidx
 
     def run(self, interp, env):
         """The closure list on the device, then the routing-weighted sum over
@@ -767,20 +791,13 @@ class Dispatch:
         from . import qmm
         from .interpreter import HOST_COPIES
         copies = HOST_COPIES[0]
+        if self.launches is not None:
+            return self._finish(self.launches.run(interp, env), copies)
         r, plan = self.router, self.plan
         ctx = _Run()
         ctx.interp, ctx.env, ctx.P = interp, env, self.P
-        iv = env[r.indices]
-        if hasattr(iv, "type_enum") and hasattr(iv, "data"):
-            iv = iv.data
-        if isinstance(iv, torch.Tensor):
-            ctx.eidx32 = qmm.to_device(iv).reshape(-1).to(torch.int32)
-        else:
-            ctx.eidx32 = torch.from_numpy(np.ascontiguousarray(host(iv).a.reshape(-1), np.int32)).to(qmm.DEVICE)
-        if self._tidx is None:                      # token of pair p: p // K, the same every call
-            t32 = torch.arange(self.T, dtype=torch.int32, device=qmm.DEVICE).repeat_interleave(self.K)
-            self._tidx = (t32, t32.long())
-        ctx.tidx32, ctx.tidx_dev = self._tidx
+        ctx.eidx32 = pair_experts(env, r)
+        ctx.tidx32, ctx.tidx_dev = self.pair_tokens(qmm.DEVICE)
         ctx.eidx_dev = ctx.eidx32.long()
         ctx.slots = []
         for fill in plan.program:
@@ -793,7 +810,12 @@ class Dispatch:
         wd = qmm.to_device(env[r.weights]).reshape(self.T, self.K)
         if self.sum_el != out.el:
             yd = yd.to(qmm._torch_dtype(self.sum_el))         # the dense graph converts the products before summing
-        total = combine(yd, wd)
+        return self._finish(combine(yd, wd), copies)
+
+    def _finish(self, total, copies):
+        import torch
+        from . import qmm
+        from .interpreter import HOST_COPIES
         if self.out_axis:
             total = torch.movedim(total, 0, self.out_axis)
         if list(total.shape) != self.out_shape:
@@ -801,6 +823,18 @@ class Dispatch:
         STATS["dispatches"] += 1
         STATS["host_copies"] += HOST_COPIES[0] - copies
         return [total.to(qmm._torch_dtype(self.out_el))]
+
+
+def pair_experts(env, router):
+    """The expert of every pair, int32 on the device, from the program's indices."""
+    import torch
+    from . import qmm
+    iv = env[router.indices]
+    if hasattr(iv, "type_enum") and hasattr(iv, "data"):
+        iv = iv.data
+    if isinstance(iv, torch.Tensor):
+        return qmm.to_device(iv).reshape(-1).to(torch.int32)
+    return torch.from_numpy(np.ascontiguousarray(host(iv).a.reshape(-1), np.int32)).to(qmm.DEVICE)
 
 
 Match = Dispatch            # the reference's name for a gathered dispatch (moe.py; qmm.py:670)
@@ -845,6 +879,7 @@ def plan_root(interp, qst, block, root) -> Dispatch:
     for c in casts:
         plan.region[op_key(c)] = c
     g.out_slot = plan.lower(y, e_axis, t_axis)
+    g.y, g.y_e, g.y_t = y, e_axis, t_axis
     if not plan.dots:
         raise Reject("no per-expert dot in the region")
     # a region op may only vanish if nothing outside the region reads it
@@ -864,16 +899,19 @@ def plan_root(interp, qst, block, root) -> Dispatch:
     g.name = f"E{g.E}/K{g.K}/T{g.T}->" + "x".join(str(d) for d in g.out_shape)
     g.bytes = sum(count(dims_of(op.results[0])) * ir._EL_BYTES[elem(op.results[0])] * g.P // max(1, g.E * g.T)
                   for op in plan.region.values() if op.results)
+    from . import moe_launch
+    if moe_launch.available():
+        g.launches = moe_launch.compile_dispatch(interp, g, block)
     return g
 
 
-def sweep_dead(block, skip, g):
+def sweep_dead(block, skip, g, read=None):
     """Besides the region itself, the dense ops that only the replaced sum
     ever read (the [tokens, experts] scores, the one-hot, their broadcasts)
     need not run.  Definitions precede uses in a block, so one walk from the
     last op to the first sees every reader of an op before the op."""
     keep = set()                          # what the dispatch still reads, and everything that computes it
-    todo = list(g.reads) + [g.router.indices, g.router.weights]
+    todo = list(g.reads) + [g.router.indices, g.router.weights] if read is None else list(read)
     while todo:
         v = todo.pop()
         if v in keep:

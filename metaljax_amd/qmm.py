@@ -95,6 +95,8 @@ class State:
             if not dispatch.disabled:
                 roots[dispatch.key] = dispatch
                 skipped.update(dispatch.skip_keys)
+                if dispatch.launches is not None:
+                    skipped.update(dispatch.launches.skip_keys)
         self.roots, self.skip = roots, frozenset(skipped)
         self.active = bool(roots)
 

@@ -1,0 +1,92 @@
+"""Expert blocks as launches against the same blocks as array operations, on the
+GPU: experts past a wavefront, a router wider than a workgroup's share of it, ties
+and NaN among the logits, and the two kernels against float64."""
+
+import numpy as np
+import pytest
+import stablehlo_text as T
+import torch
+
+from metaljax_amd import engine, interpreter as I, moe, moe_launch as ML, qmm
+from test_moe_launch import gemma_inputs
+from test_recognizer import _moe_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def both(text, args, monkeypatch):
+    """(launches, results as launches, results as array operations)"""
+    out, launches = [], []
+    for on in (True, False):
+        monkeypatch.setattr(ML, "available", lambda on=on: on)
+        moe.reset_stats()
+        ex = engine.compile_program(text)
+        bufs = engine.execute(ex, args)
+        bufs = engine.execute(ex, args)                  # (once more on the packed weights)
+        assert moe.stats()["dispatches"] >= 2 and moe.stats()["fallbacks"] == 0
+        out.append([engine.to_numpy(b)[0] for b in bufs])
+        launches.append([g.launches for g in ex.interp._qmm.moe])
+    assert all(g is None for g in launches[1])
+    return launches[0], out[0], out[1]
+
+
+# float32: sums in another order; bf16: the last place of an intermediate that was rounded from such a sum
+def close(a, b, el):
+    tol = 2e-5 if el == "f32" else 2e-2
+    np.testing.assert_allclose(a, b, rtol=tol, atol=tol * np.abs(b[np.isfinite(b)]).max(initial=1e-6))
+
+
+@pytest.mark.parametrize("el", ["f32", "bf16"])
+@pytest.mark.parametrize("E,Tk,H,Ii,K", [(4, 3, 64, 32, 2), (5, 1, 96, 64, 1), (8, 64, 1536, 288, 4), (70, 9, 512, 64, 8), (130, 2, 64, 32, 3)])
+def test_gpt_oss_block(E, Tk, H, Ii, K, el, monkeypatch):
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    args = [I.from_numpy(a, el) if a.dtype == np.float32 else I.from_numpy(a) for a in raw]
+    (g,), (out,), (plain,) = both(T.moe_block_mxfp4(E, Tk, H, Ii, K, el=el), args, monkeypatch)
+    assert g is not None and g.rows is not None and g.rows.dot_k == H
+    if el == "bf16":                                     # (two logits that round to one choose either expert)
+        same = np.abs(out - plain).max(1) <= 2e-2 * np.abs(plain).max()
+        assert same.mean() >= 0.9
+        out, plain = out[same], plain[same]
+    close(out, plain, el)
+
+
+@pytest.mark.parametrize("el", ["f32", "bf16"])
+@pytest.mark.parametrize("E,Tk,K", [(4, 3, 2), (8, 1, 4), (33, 17, 5)])
+def test_gemma4_block(E, Tk, K, el, monkeypatch):
+    args = gemma_inputs(E, Tk, 64, 32, el)
+    (g,), (out,), (plain,) = both(T.moe_block_gemma4_mxfp4(E, Tk, 64, 32, K, el=el), args, monkeypatch)
+    assert g is not None and g.rows is not None
+    close(out, plain, el)
+
+
+def test_ties_and_nan_among_the_logits(monkeypatch):
+    E, Tk, H, Ii, K = 6, 4, 32, 32, 3
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    x, wr, br = raw[0].copy(), np.zeros_like(raw[1]), np.array([1, 2, 1, 2, 1, 0], np.float32)
+    wr[0, 5] = 1.0
+    x[:, 0] = (0, 1, np.nan, np.inf)                    # expert 5: below the ties, among them, NaN, infinite
+    (g,), (out,), (plain,) = both(T.moe_block_mxfp4(E, Tk, H, Ii, K), [I.from_numpy(a) for a in (x, wr, br) + raw[3:]], monkeypatch)
+    assert g is not None and g.rows is not None
+    finite = np.isfinite(plain)
+    assert np.array_equal(finite, np.isfinite(out)) and finite[:2].all()
+    close(out[finite], plain[finite], "f32")
+
+
+@pytest.mark.parametrize("op,fn", [("exponential", np.exp), ("logistic", lambda v: 1 / (1 + np.exp(-v))), ("tanh", np.tanh), ("log", np.log),
+                                   ("rsqrt", lambda v: 1 / np.sqrt(v)), ("round_nearest_even", np.rint), ("sign", np.sign), ("floor", np.floor)])
+def test_an_elementwise_instruction(op, fn):
+    """One instruction on a 3 x 5 x 300 result read through swapped axes: two
+    float32 places of what numpy gives in float64."""
+    from metaljax_amd.kernels import _stream
+    v = torch.randn((5, 3, 300), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)) * 3
+    if op in ("log", "rsqrt"):
+        v = v.abs() + 0.01
+    y, experts = torch.empty((2, 3, 5, 300), device="cuda"), torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+    m = ML.PairMap(y=y.data_ptr(), experts_of=experts.data_ptr(), pairs=2, inner=4500, dims=(3, 5, 300), per_token=1, experts=2,
+                   rank=3, leaves=1, instructions=1, registers=2, result=1)
+    m.leaf[0] = ML.MapLeaf(v.data_ptr(), 0, 0, 0, 0, (300, 900, 1), 0)
+    m.code[0] = ML.Instruction(ML.OP[op], 1, 0, 0, 0, 0, 0.0)
+    ML.run_map(m, _stream(y))
+    want = fn(v.double().cpu().numpy().transpose(1, 0, 2))
+    for half in y.cpu().numpy():
+        np.testing.assert_allclose(half, want, rtol=4e-7, atol=1e-30)

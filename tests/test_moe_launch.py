@@ -1,0 +1,206 @@
+"""Dispatches compiled to launches (metaljax_amd.moe_launch): the programs that
+the planner writes, run here by a plain reading of their structs on host memory,
+give what the dispatch's array operations give -- every form that is compiled, at
+one token and several, in float32 and bf16; what is not modelled stays with the
+array operations."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import stablehlo_text as T
+import torch
+
+from metaljax_amd import _lib, engine, interpreter as I, moe, moe_launch as ML, qmm
+from test_recognizer import _moe_inputs, _oracle_expert_product, _without_a_gpu
+
+pytestmark = pytest.mark.filterwarnings("ignore")
+NAMES = {v: k for k, v in ML.OP.items()}
+TYPES = {0: (ctypes.c_float, 4), 1: (ctypes.c_uint16, 2), 2: (ctypes.c_uint16, 2), 3: (ctypes.c_uint8, 1), 4: (ctypes.c_int32, 4)}
+
+
+def load(p, i, el):
+    raw = TYPES[el][0].from_address(p + i * TYPES[el][1]).value
+    if el == 1:
+        return np.uint32(raw << 16).view(np.float32)
+    return np.float32(np.uint16(raw).view(np.float16)) if el == 2 else np.float32(raw)
+
+
+def rounded(v, el):
+    v = np.float32(v)
+    return I.round_bf16(v.reshape(1))[0] if el == 1 else np.float32(np.float16(v)) if el == 2 else v
+
+
+def store(p, i, v, el):
+    if el == 1:
+        v = int(I.f32_to_bf16_bits(np.float32(v).reshape(1))[0])
+    elif el == 2:
+        v = int(np.float16(v).view(np.uint16))
+    TYPES[el][0].from_address(p + i * TYPES[el][1]).value = int(v) if el == 4 else v
+
+
+def apply(op, a, b, c):
+    with np.errstate(all="ignore"):
+        one = np.float32(1)
+        return {"copy": lambda: a, "add": lambda: a + b, "subtract": lambda: a - b, "multiply": lambda: a * b,
+                "divide": lambda: a / b, "maximum": lambda: np.maximum(a, b), "minimum": lambda: np.minimum(a, b),
+                "exponential": lambda: np.exp(a), "logistic": lambda: one / (one + np.exp(-a)), "tanh": lambda: np.tanh(a),
+                "clamp": lambda: np.minimum(np.maximum(b, a), c), "negate": lambda: -a, "rsqrt": lambda: one / np.sqrt(a),
+                "LT": lambda: one * (a < b), "select": lambda: b if a != 0 else c}[NAMES[op]]()
+
+
+def run_map(m, _stream):
+    per = m.per_token if m.weights else 1
+    for row in range(m.pairs // per):
+        for i in range(m.inner):
+            c, total = np.unravel_index(i, tuple(m.dims)), np.float32(0)
+            for k in range(per):
+                p = row * per + k
+                e = ctypes.c_int32.from_address(m.experts_of + 4 * p).value
+                regs = [None] * m.registers
+                for j in range(m.leaves):
+                    f = m.leaf[j]
+                    regs[j] = load(f.p, f.base + p * f.pair + e * f.expert + p // m.per_token * f.token +
+                                   sum(int(x) * s for x, s in zip(c, f.coef)), f.el)
+                for q in m.code[:m.instructions]:
+                    v = q.imm if NAMES[q.op] == "imm" else apply(q.op, regs[q.a], regs[q.b], regs[q.c])
+                    regs[q.dst] = rounded(v, q.el)
+                v = regs[m.result]
+                if m.weights:
+                    total += rounded(v, m.sum_el) * load(m.weights, p, m.weights_el)
+            store(m.y, row * m.inner + i, total if m.weights else v, m.y_el)
+
+
+def run_rows(r, _stream):
+    for t in range(r.tokens):
+        regs = np.full(r.reg_floats, np.nan, np.float32)
+        if r.dot_x:
+            for n in range(r.dot_n):
+                regs[r.dot_dst + n] = rounded(sum(
+                    load(r.dot_x, t * r.dot_x_t + k * r.dot_x_k, r.dot_x_el) * load(r.dot_w, n * r.dot_w_n + k * r.dot_w_k, r.dot_w_el)
+                    for k in range(r.dot_k)), r.dot_el)
+        for f in r.leaf[:r.leaves]:
+            for i in range(f.n):
+                regs[f.dst + i] = load(f.p, f.base + t * f.token + i * f.step, f.el)
+        for q in r.code[:r.instructions]:
+            name, a = NAMES[q.op], regs[q.a:q.a + q.an].copy()
+            if name == "top_k":
+                vals, idx = I.top_k(a[None], q.n)
+                regs[q.dst:q.dst + q.n], regs[q.c:q.c + q.n] = vals[0], idx[0]
+            elif name in ("sum", "rowmax", "rowmin"):
+                regs[q.dst] = rounded({"sum": np.sum, "rowmax": np.max, "rowmin": np.min}[name](a), q.el)
+            else:
+                for i in range(q.n):
+                    at = [regs[s + (0 if w == 1 else i)] for s, w in ((q.a, q.an), (q.b, q.bn), (q.c, q.cn))] if name not in ("imm", "slice") else []
+                    regs[q.dst + i] = rounded(q.imm if name == "imm" else regs[q.a + q.b + i * q.c] if name == "slice" else apply(q.op, *at), q.el)
+        for o in r.out[:r.outs]:
+            for i in range(o.n):
+                store(o.p, t * o.n + i, regs[o.src + (0 if o.srcn == 1 else i)], o.el)
+
+
+def both(text, args, monkeypatch):
+    """(launches, results as launches, results as array operations)"""
+    monkeypatch.setattr(qmm, "DEVICE", "cpu")
+    monkeypatch.setattr(moe, "emit_dot", _oracle_expert_product([]))
+    plain = [I.host(b.data).a for b in engine.execute(engine.compile_program(text), args)]
+    monkeypatch.setattr(ML, "available", lambda: True)
+    monkeypatch.setattr(ML, "run_map", run_map)
+    monkeypatch.setattr(ML, "run_rows", run_rows)
+    moe.reset_stats()
+    ex = engine.compile_program(text)
+    out = [I.host(b.data).a for b in engine.execute(ex, args)]
+    assert moe.stats()["dispatches"] >= 1 and moe.stats()["fallbacks"] == 0
+    return [g.launches for g in ex.interp._qmm.moe], out, plain
+
+
+def gemma_inputs(E, Tk, H, Ii, el):
+    rng = np.random.default_rng(E + Tk)
+    packed = [T.make_mxfp4_experts(r, c, E, seed=i)[:2] for i, (r, c) in enumerate(((Ii, H), (Ii, H), (H, Ii)))]
+    raw = [(rng.standard_normal((Tk, H)) / 8).astype(np.float32), rng.standard_normal((H, E)).astype(np.float32),
+           (1 + rng.standard_normal(H) / 8).astype(np.float32), *[a for p in packed for a in p],
+           (1 + rng.standard_normal(E) / 8).astype(np.float32)]
+    return [I.from_numpy(a, el) if a.dtype == np.float32 else I.from_numpy(a) for a in raw]
+
+
+@_without_a_gpu
+@pytest.mark.parametrize("el", ["f32", "bf16"])
+@pytest.mark.parametrize("E,Tk,H,Ii,K,composite", [(4, 3, 64, 32, 2, False), (5, 1, 32, 32, 2, True), (4, 4, 32, 64, 4, True), (3, 2, 32, 32, 1, False)])
+def test_gpt_oss_block(E, Tk, H, Ii, K, composite, el, monkeypatch):
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    args = [I.from_numpy(a, el) if a.dtype == np.float32 else I.from_numpy(a) for a in raw]
+    (g,), (out,), (plain,) = both(T.moe_block_mxfp4(E, Tk, H, Ii, K, el=el, composite=composite), args, monkeypatch)
+    assert g is not None and g.rows is not None and g.rows.dot_k == H      # the router's product is part of it
+    assert [d.feed is None for d in g.dots] == [True, False]
+    # the same roundings in the same places; sums in another order (bf16: a last place of an intermediate)
+    np.testing.assert_allclose(out, plain, rtol=2e-5 if el == "f32" else 2e-2, atol=(1e-6 if el == "f32" else 2e-2) * np.abs(plain).max())
+
+
+@_without_a_gpu
+@pytest.mark.parametrize("el", ["f32", "bf16"])
+@pytest.mark.parametrize("E,Tk,K", [(4, 3, 2), (8, 1, 4)])
+def test_gemma4_block(E, Tk, K, el, monkeypatch):
+    args = gemma_inputs(E, Tk, 64, 32, el)
+    (g,), (out,), (plain,) = both(T.moe_block_gemma4_mxfp4(E, Tk, 64, 32, K, el=el), args, monkeypatch)
+    assert g is not None and g.rows is not None and not g.rows.dot_x       # its product reads computed activations
+    assert len(g.dots) == 3
+    np.testing.assert_allclose(out, plain, rtol=2e-5 if el == "f32" else 2e-2, atol=(1e-6 if el == "f32" else 2e-2) * np.abs(plain).max())
+
+
+@_without_a_gpu
+def test_blocks_before_and_inside_a_loop(monkeypatch):
+    args = gemma_inputs(4, 3, 32, 32, "f32")
+    launches, out, plain = both(T.moe_gemma4_decode_loop(4, 3, 32, 32, 2, 2), args, monkeypatch)
+    assert len(launches) == 2 and all(g is not None for g in launches)
+    for a, b in zip(out, plain):
+        np.testing.assert_allclose(a, b, rtol=2e-5, atol=1e-6)
+
+
+@_without_a_gpu
+def test_a_router_that_is_read_elsewhere_stays_with_the_program(monkeypatch):
+    """The weights are a result of the program too: the router runs as it did,
+    the rest of the dispatch as launches."""
+    E, Tk, H, Ii, K = 4, 3, 32, 32, 2
+    text = T.moe_block_mxfp4(E, Tk, H, Ii, K)
+    text = text.replace(f"return %out : tensor<{Tk}x{H}xf32>", f"return %out, %w : tensor<{Tk}x{H}xf32>, tensor<{Tk}x{K}xf32>")
+    text = text.replace(f"-> tensor<{Tk}x{H}xf32> {{\n", f"-> (tensor<{Tk}x{H}xf32>, tensor<{Tk}x{K}xf32>) {{\n", 1)
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    (g,), out, plain = both(text, [I.from_numpy(a) for a in raw], monkeypatch)
+    assert g is not None and g.rows is None and not g.skip_keys
+    for a, b in zip(out, plain):
+        np.testing.assert_allclose(a, b, rtol=2e-5, atol=1e-6)
+
+
+def test_structs_and_instructions_are_the_headers():
+    """Sizes as a C compiler lays them out, and the instruction numbers in the
+    header's order."""
+    import os
+    import re
+    text = open(os.path.join(os.path.dirname(_lib.__file__), os.pardir, "include", "qmm_hip.h")).read()
+    text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
+    names = re.findall(r"QMM_OP_([A-Z0-9]+)", re.search(r"enum \{(\s*QMM_OP_.*?)\};", text, re.S)[1])
+    mine = {"subtract": "SUB", "multiply": "MUL", "divide": "DIV", "maximum": "MAX", "minimum": "MIN", "power": "POW",
+            "negate": "NEG", "exponential": "EXP", "round_nearest_even": "RINT", "top_k": "TOPK"}
+    assert names == [mine.get(n, n.upper()) for n in ML._OPS]
+    for name, value in (("MAP_LEAVES", ML.LEAVES), ("MAP_CODE", ML.CODE), ("MAP_REGISTERS", ML.REGISTERS), ("ROW_LEAVES", ML.ROW_LEAVES),
+                        ("ROW_CODE", ML.ROW_CODE), ("ROW_OUTS", ML.ROW_OUTS), ("ROW_FLOATS", ML.ROW_FLOATS)):
+        assert int(re.search(rf"#define QMM_{name} (\d+)", text)[1]) == value
+    assert ctypes.sizeof(ML.MapLeaf) == 48 and ctypes.sizeof(ML.Instruction) == 12 and ctypes.sizeof(ML.RowInstruction) == 44
+
+
+def test_programs_that_point_outside_their_registers_are_refused():
+    lib = _lib.load()
+    at = 4096                                           # (never read: the call is refused on the host)
+    m = ML.PairMap(y=at, experts_of=at, pairs=2, inner=4, dims=(1, 1, 4), per_token=1, experts=2, rank=1, registers=1)
+    for field, value in (("result", 1), ("leaves", ML.LEAVES + 1), ("instructions", ML.CODE + 1), ("inner", 5), ("per_token", 0),
+                         ("y_el", 3), ("experts", 0)):
+        bad = ML._copy(m)
+        setattr(bad, field, value)
+        assert lib.qmm_pair_map_run(ctypes.byref(bad), None) == 1, field
+    bad = ML._copy(m)
+    bad.instructions, bad.code[0] = 1, ML.Instruction(ML.OP["add"], 0, 0, 1, 0, 0, 0.0)
+    assert lib.qmm_pair_map_run(ctypes.byref(bad), None) == 1
+    r = ML.RowProgram(tokens=1, reg_floats=8, instructions=1)
+    for q in ((ML.OP["add"], 0, 6, 4, 0, 4, 0, 4, 0, 4, 0.0), (ML.OP["top_k"], 0, 0, 3, 4, 2, 0, 1, 6, 2, 0.0),
+              (ML.OP["slice"], 0, 0, 4, 4, 4, 1, 0, 1, 0, 0.0)):
+        r.code[0] = ML.RowInstruction(*q)
+        assert lib.qmm_row_program_run(ctypes.byref(r), None) == 1, q
