@@ -347,6 +347,28 @@ bool grouped_decode_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, i
          skinny2_grouped_supported(N, K, gs, bits, mode, tab, s, b, E, 8);
 }
 
+// Are these pairs for the grouped decode whose workgroups sort them by themselves?
+bool sorted_here_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
+                        const void* s, const void* b) {
+  return sorted_here_pairs(P, N, K, bits, mode) && E > 0 && !(mode == QMM_MODE_AFFINE && tab == QMM_F32 && gs == 64) &&
+         skinny2_grouped_supported(N, K, gs, bits, mode, tab, s, b, E, 3);
+}
+
+// From sixteen pairs on, and half a pair an expert, shapes that only the
+// general decode kernels serve are grouped by expert as well: an expert's
+// weights are then read once for up to sixteen of its pairs instead of
+// once per pair.  (The sort costs a launch of its own, and with fewer
+// pairs than that few of them share an expert.  Measured on 32 MXFP4
+// experts of [5760, 2880]: 16 pairs 61 against 60 us, 32 pairs 86 against
+// 110, 64 pairs 109 against 216; on 128 experts: 32 pairs 128 against 110,
+// 64 pairs 194 against 217; 8 experts of [4096, 11008] with four-bit
+// codes: 16 pairs 108 against 206 us, 32 pairs 110 against 397.)
+bool grouped_general_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
+                            const void* s, const void* b, size_t workspace_bytes) {
+  return P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace_bytes >= route_bytes_segments(P, E) &&
+         gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E) && !experiment_env("QMM_NO_GROUPED_GEMV");
+}
+
 // ---- float16 / float32 activations ---------------------------------------------
 // The kernels multiply bf16 operands.  Wider activations are split, exactly,
 // into bf16 terms (float16: two, float32: three), every term is multiplied
@@ -723,8 +745,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   hipStream_t st = static_cast<hipStream_t>(stream);
   // few pairs: the grouped decode whose workgroups sort them by themselves
-  if (sorted_here_pairs(P, N, K, bits, mode) && E > 0 && !(mode == QMM_MODE_AFFINE && table_dtype == QMM_F32 && group_size == 64) &&
-      skinny2_grouped_supported(N, K, group_size, bits, mode, table_dtype, scales, biases, E, 3)) {
+  if (sorted_here_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases)) {
     skinny2_grouped_dispatch(x, w, scales, biases, y, y_dtype, nullptr, nullptr, nullptr, P, T, E, N, K,
                              group_size, bits, mode, table_dtype, lhs_idx, rhs_idx, st);
     return check_launch("grouped decode launch");
@@ -743,19 +764,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
     return check_launch("grouped decode launch");
   }
   if (P <= kGatherGemvMaxPairs) {
-    // From sixteen pairs on, and half a pair an expert, shapes that only the
-    // general decode kernels serve are grouped by expert as well: an expert's
-    // weights are then read once for up to sixteen of its pairs instead of
-    // once per pair.  (The sort costs a launch of its own, and with fewer
-    // pairs than that few of them share an expert.  Measured on 32 MXFP4
-    // experts of [5760, 2880]: 16 pairs 61 against 60 us, 32 pairs 86 against
-    // 110, 64 pairs 109 against 216; on 128 experts: 32 pairs 128 against 110,
-    // 64 pairs 194 against 217; 8 experts of [4096, 11008] with four-bit
-    // codes: 16 pairs 108 against 206 us, 32 pairs 110 against 397.)
-    if (P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace &&
-        workspace_bytes >= route_bytes_segments(P, E) &&
-        gemv_runs_general(N, K, group_size, bits, mode, table_dtype, scales, biases, E) &&
-        !experiment_env("QMM_NO_GROUPED_GEMV")) {
+    if (workspace && grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, workspace_bytes)) {
       int32_t* ro = static_cast<int32_t*>(workspace);
       int32_t* cursor = ro + E + 1;
       int32_t* src_row = cursor + E;
@@ -969,6 +978,25 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   if (terms * P * K >= (1ll << 30)) return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // Pairs that are decode products of their own: the terms are the rows of one (terms
+  // <= 16: a pair's weight is streamed once, in one launch instead of one a term).
+  if (P <= kGatherGemvMaxPairs && E <= 65535 && N <= INT32_MAX && K <= INT32_MAX &&
+      !sorted_here_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases) &&
+      !grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner) &&
+      !grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
+    int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
+    if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);
+    if (rc) return rc;
+    split_terms_dispatch(x, x_dtype, ws, P, 1, K, lhs_idx, T, st);    // [P, terms, K]
+    rc = check_launch("activation split launch");
+    if (rc) return rc;
+    gemv_dispatch(ws, w, scales, biases, table_dtype, ws + xs, QMM_F32, P, terms, N, K, group_size, bits, mode, nullptr,
+                  rhs_idx, E, P, st);
+    rc = check_launch("gather gemv launch");
+    if (rc) return rc;
+    sum_terms_dispatch(ws + xs, terms, y, y_dtype, P, 1, N, nullptr, rhs_idx, E, st);
+    return check_launch("term sum launch");
+  }
   split_terms_dispatch(x, x_dtype, ws, 1, P, K, lhs_idx, T, st);      // lhs_idx null: row p of x
   int rc = check_launch("activation split launch");
   for (int t = 0; t < terms && !rc; ++t)

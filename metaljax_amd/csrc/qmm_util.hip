@@ -112,15 +112,15 @@ __global__ void split_terms_kernel(const T* __restrict__ x, uint16_t* __restrict
                                    const int32_t* __restrict__ src_row, int64_t x_rows) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= total) return;
-  const int64_t z = i / rows_k, j = i - z * rows_k;
+  const int64_t z = i / rows_k, j = i - z * rows_k;          // (rows are numbered through all batch entries)
   int64_t src = i;
   bool ok = true;
   if (src_row) {                                   // rows gathered: out row j / k is x row src_row[j / k]
-    const int64_t row = j / k, sr = src_row[row];
+    const int64_t row = i / k, sr = src_row[row];
     ok = sr >= 0 && sr < x_rows;                   // a row outside x gathers zeros
-    src = sr * k + (j - row * k);
+    src = sr * k + (i - row * k);
   } else if (x_rows >= 0) {                        // pair p reads row p of x: rows past the end read as zeros
-    ok = j / k < x_rows;
+    ok = i / k < x_rows;
   }
   float v = 0.f;
   if (ok) {
@@ -152,7 +152,7 @@ __global__ void sum_terms_kernel(const float* __restrict__ part, void* __restric
   if (i >= total) return;
   const int64_t z = i / rows_n, j = i - z * rows_n;
   if (offsets || expert_of_row) {
-    const int64_t row = j / n;
+    const int64_t row = i / n;                     // (numbered through all batch entries)
     if (offsets && (row < offsets[0] || row >= offsets[E])) return;
     if (expert_of_row && (expert_of_row[row] < 0 || expert_of_row[row] >= E)) return;
   }
@@ -251,7 +251,7 @@ void dequant_dispatch(const void* w, const void* s, const void* b, int tab, void
 }
 
 // x (float16 / float32) [batch, rows, K] -> bf16 terms [batch, terms, rows, K];
-// with src_row (batch = 1): out row r = x row src_row[r] of x [x_rows, K]; without it and x_rows >= 0:
+// with src_row: out row r = x row src_row[r] of x [x_rows, K]; without it and x_rows >= 0:
 // out row r = x row r, rows past x_rows read as zeros; x_rows < 0: no gather, rows is what x holds
 void split_terms_dispatch(const void* x, int x_dtype, void* out, int64_t batch, int64_t rows,
                           int64_t K, const int32_t* src_row, int64_t x_rows, hipStream_t st) {

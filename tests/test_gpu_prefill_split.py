@@ -240,3 +240,33 @@ def test_rows_that_no_expert_covers_are_zero(n, r, e, k, kind, act):
         assert torch.equal(y[first:last], given[first:last])
         assert not y[:first].any() and not y[last:].any()
         assert (given[:first] == 7.0).all() and (given[last:] == 7.0).all()
+
+
+# float16 / float32 rows of pairs that are decode products of their own: the terms are the rows of one product a pair
+# (two K-slices or less, a K that is no multiple of 64, groups of 32; one pair to the last before a sort)
+@pytest.mark.parametrize("act", ["f16", "f32"])
+@pytest.mark.parametrize("pairs,e,n,k,kind", [(1, 3, 40, 96, 1), (3, 9, 72, 1024, 5), (15, 40, 33, 416, 5), (5, 2, 130, 512, 0),
+                                              (47, 4, 200, 1024, 5), (9, 30, 48, 160, 4), (2, 4, 64, 256, 3)])
+def test_terms_of_a_pair_are_rows_of_one_product(pairs, e, n, k, kind, act):
+    # float32 sums of exact products.  A four-bit code goes through the matrix core as 128 + q, so a sum is up to 136 over
+    # the codes' spread of 4.6 (16 / sqrt 12) times its result, and the roundings of some ten sums, 2^-24 each, meet in it
+    term_err = 136 / 4.6 * 2.0 ** -24 * 10 ** 0.5
+    bits, gs, mode, tab = KINDS[kind]
+    if k % gs:
+        pytest.skip("no whole groups")
+    g = torch.Generator(device=DEV).manual_seed(pairs + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (e,), n, k, bits, gs, mode, tab)
+    exact = K.dequantize(w, s, b, out_dtype=torch.float32, **how).double()
+    x = torch.randn((7, k), device=DEV, generator=g).to(ACT[act])
+    lhs = torch.randint(0, 7, (pairs,), device=DEV, generator=g, dtype=torch.int32)
+    rhs = torch.randint(0, e, (pairs,), device=DEV, generator=g, dtype=torch.int32)
+    lhs[0] = 7 if pairs > 1 else lhs[0]                    # no row of x: reads as zeros
+    y = K.gather_qmm(x, w, s, b, lhs, rhs, out_dtype=torch.float32, **how)
+    rows = torch.cat([x.double(), x.new_zeros((1, k)).double()])[lhs.long()]
+    want = torch.einsum("pk,pnk->pn", rows.cpu(), exact.cpu()[rhs.cpu().long()]).to(DEV)
+    err = ((y.double() - want).norm() / want.norm()).item()
+    assert err <= term_err, err
+    y = K.gather_qmm(x[:pairs], w, s, b, None, rhs[:min(pairs, 7)], out_dtype=torch.float32, **how)
+    want = torch.einsum("pk,pnk->pn", x[:pairs].double().cpu(), exact.cpu()[rhs[:min(pairs, 7)].cpu().long()]).to(DEV)
+    assert ((y.double() - want).norm() / want.norm()).item() <= term_err
