@@ -50,6 +50,7 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
 double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes, int* tile_rows, int* splits);
 double gemm2_us(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes);
 size_t gemm2_split_workspace_bytes(int64_t R, int64_t N, int64_t K);
+int short_terms(int x_dtype, int tab, int gs, int mode);
 bool short_supported(int64_t R, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab, int terms,
                      const void* s, const void* b);
 double short_us(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, size_t part_bytes);
@@ -405,7 +406,7 @@ size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
 
 // Is the short-group kernel the one to take?  `E` experts share the R rows
 // (`grouped`; else a dense product and E = 1), the activations are `terms` bf16
-// terms, and each kernel has what `scratch` leaves it for a split K's sums.  All
+// terms (`own` of the short-group kernel), and each kernel has what `scratch` leaves it for a split K's sums.  All
 // kernels' times have been fitted over the shapes they serve; where they come close
 // the choice matters little.  (4096 x 4096, four-bit codes: 17 rows 12 against 17 us of the
 // prefill kernel, 128 rows 19 against 22, 512 rows 32 against 36; 14336 x 4096:
@@ -413,7 +414,7 @@ size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
 // groups, the slower kernel is taken in a few, 11 % slower at worst; MXFP4's
 // block-scaled kernel is taken for faster than it is, for groups up to 1.35 times:
 // profiles/prefill_plan_fits.txt.)
-bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, bool grouped, size_t scratch) {
+bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, int own, bool grouped, size_t scratch) {
   if (K % 64 || N <= 0) return false;
   if (const char* env = experiment_env("QMM_SHORT")) return env[0] != '0';
   double other;
@@ -426,13 +427,16 @@ bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, 
     other = grouped ? terms * gemm2_us(R, E, N, K, 0) : gemm2_us(terms * R, 1, N, K, scratch > held ? scratch - held : 0);
     if (terms > 1) other += 5.2 + (double)terms * R * N * 1.4e-6;
   }
-  const size_t prep = short_prep_bytes(R, K, terms);
-  return short_us(R, E, N, K, bits, mode, terms, scratch > prep ? scratch - prep : 0) < other;
+  const size_t prep = short_prep_bytes(R, K, own);
+  return short_us(R, E, N, K, bits, mode, own, scratch > prep ? scratch - prep : 0) < other;
 }
 
 // Scratch that lets a short-group product over R rows run as it would best.
 size_t short_scratch(int64_t R, int64_t N, int64_t K, int bits, int mode, int terms) {
-  return R > 0 && R <= 4096 && N > 0 && K > 0 && K % 64 == 0 && terms * R > kGemvMaxM ? short_workspace_bytes(R, N, K, bits, mode, terms) : 0;
+  if (R <= 0 || R > 4096 || N <= 0 || K <= 0 || K % 64 || terms * R <= kGemvMaxM) return 0;
+  // (float16 rows are one term or two: the tables' type is not known here)
+  const size_t own = terms == 2 && mode == QMM_MODE_AFFINE ? short_workspace_bytes(R, N, K, bits, mode, 1) : 0;
+  return std::max(own, short_workspace_bytes(R, N, K, bits, mode, terms));
 }
 
 size_t gather_scratch(int64_t P, int64_t E, int64_t N, int64_t K, bool exact) {
@@ -523,7 +527,7 @@ size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, in
 
 int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode, int* kernel,
              int* grid, int* block) {
-  if (M > kGemvMaxM && short_wins(M, 1, N, K, bits, mode, 1, false, ~(size_t)0)) {     // (bf16 activations and tables, ample scratch assumed)
+  if (M > kGemvMaxM && short_wins(M, 1, N, K, bits, mode, 1, 1, false, ~(size_t)0)) {     // (bf16 activations and tables, ample scratch assumed)
     int g;
     short_geometry(M, N, K, bits, mode, &g);
     if (kernel) *kernel = QMM_KERNEL_GEMM;
@@ -601,9 +605,10 @@ static bool ran_short(const void* x, int x_dtype, const void* w, const void* sca
                       const int32_t* out_idx, int64_t R, int64_t x_rows, int64_t E, int64_t N, int64_t K,
                       int group_size, int bits, int mode, void* workspace, size_t workspace_bytes, void* stream,
                       int* rc) {
-  const int terms = act_terms(x_dtype);
-  if (R <= 0 || E <= 0 || N <= 0 || K <= 0 || terms * R <= kGemvMaxM || R > INT32_MAX / 2 || N > INT32_MAX ||
-      K > INT32_MAX || E > 65535 || !short_wins(R, E, N, K, bits, mode, terms, row_offsets != nullptr, workspace_bytes))
+  const int terms = short_terms(x_dtype, table_dtype, group_size, mode);
+  if (R <= 0 || E <= 0 || N <= 0 || K <= 0 || act_terms(x_dtype) * R <= kGemvMaxM || R > INT32_MAX / 2 || N > INT32_MAX ||
+      K > INT32_MAX || E > 65535 ||
+      !short_wins(R, E, N, K, bits, mode, act_terms(x_dtype), terms, row_offsets != nullptr, workspace_bytes))
     return false;
   if (check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases) || check_io(x, x_dtype, y, y_dtype) ||
       !workspace || !aligned16(workspace) || workspace_bytes < short_prep_bytes(R, K, terms) ||
@@ -945,14 +950,15 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   // it keeps them exact, the short-group kernel rounds them to bf16 (1e-7 against
   // 1.6e-3 from the product of the exact weights, 128 pairs over 8 experts of 1024 x
   // 4096, eight-bit codes; four-bit ones 4e-7).  MXFP4 weights are exact in both.
+  const int own = short_terms(x_dtype, table_dtype, group_size, mode);
   const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
   if (!exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
-      workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, terms) &&
+      workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, own) &&
       workspace_bytes >= term_bytes(terms, P, N, K) + gather_scratch(P, E, N, K, true) &&
-      short_wins(P, E, N, K, bits, mode, terms, true, workspace_bytes - route_bytes(P, E)) &&
-      short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, terms, scales, biases)) {
+      short_wins(P, E, N, K, bits, mode, terms, own, true, workspace_bytes - route_bytes(P, E)) &&
+      short_supported(P, E, N, K, mode == QMM_MODE_MXFP4 ? 32 : std::max(group_size, 1), bits, mode, table_dtype, own, scales, biases)) {
     const size_t need = route_bytes(P, E);
     int32_t* ro = static_cast<int32_t*>(workspace);
     int32_t* cursor = ro + E + 1;

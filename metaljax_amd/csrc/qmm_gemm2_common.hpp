@@ -86,6 +86,13 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 // (redo_column).  Over 160 products of 17 to 2048 rows that is 0.3 % in all; asked
 // of the scales as they come by it was 1 %, up to 4 %.
 constexpr float kSmallScale = 0x1p104f;
+
+// Float16 weight tiles hold the weight times 2^6, which the results give back: then
+// a weight of the smallest float16 scale, 2^-24, is off by 2^-7 of that at most --
+// a bf16 tile's by up to 2^-9 of the weight, some eight scales -- and weights below
+// 1023 fit.  (Scales of float16 weights lie around 2^-12 to 2^-4.)  A column with a
+// larger one has no finite result and is multiplied again, plainly.
+constexpr int kF16Shift = 6;
 __device__ __forceinline__ u32x4 dequant_nibbles(uint32_t w, float s24, float s20, float bi) {
   const uint32_t w8 = w >> 8;
   const f16x2 a = __builtin_bit_cast(f16x2, w & 0x000F000Fu), b = __builtin_bit_cast(f16x2, w & 0x00F000F0u);
@@ -101,6 +108,27 @@ __device__ __forceinline__ u32x2 dequant_bytes(uint32_t w, float s24, float bi) 
   const float f0 = fmaf((float)a[0], s24, bi), f2 = fmaf((float)a[1], s24, bi);
   const float f1 = fmaf((float)b[0], s24, bi), f3 = fmaf((float)b[1], s24, bi);
   return u32x2{pack_bf16x2(f0, f1), pack_bf16x2(f2, f3)};
+}
+
+// The same to float16 weights (tables times 2^kF16Shift, s24 and s20 as above):
+// v_fma_mixlo / mixhi round to float16 as they go, so that eight four-bit codes
+// take 13 vector instructions, eight eight-bit ones 11.
+__device__ __forceinline__ u32x4 dequant_nibbles_f16(uint32_t w, float s24, float s20, float bi) {
+  const uint32_t w8 = w >> 8;
+  const f16x2 a = __builtin_bit_cast(f16x2, w & 0x000F000Fu), b = __builtin_bit_cast(f16x2, w & 0x00F000F0u);
+  const f16x2 c = __builtin_bit_cast(f16x2, w8 & 0x000F000Fu), d = __builtin_bit_cast(f16x2, w8 & 0x00F000F0u);
+  const f16x2 p0 = {(_Float16)fmaf((float)a[0], s24, bi), (_Float16)fmaf((float)b[0], s20, bi)};
+  const f16x2 p1 = {(_Float16)fmaf((float)c[0], s24, bi), (_Float16)fmaf((float)d[0], s20, bi)};
+  const f16x2 p2 = {(_Float16)fmaf((float)a[1], s24, bi), (_Float16)fmaf((float)b[1], s20, bi)};
+  const f16x2 p3 = {(_Float16)fmaf((float)c[1], s24, bi), (_Float16)fmaf((float)d[1], s20, bi)};
+  return u32x4{__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1), __builtin_bit_cast(uint32_t, p2),
+               __builtin_bit_cast(uint32_t, p3)};
+}
+__device__ __forceinline__ u32x2 dequant_bytes_f16(uint32_t w, float s24, float bi) {
+  const f16x2 a = __builtin_bit_cast(f16x2, w & 0x00FF00FFu), b = __builtin_bit_cast(f16x2, (w >> 8) & 0x00FF00FFu);
+  const f16x2 p0 = {(_Float16)fmaf((float)a[0], s24, bi), (_Float16)fmaf((float)b[0], s24, bi)};
+  const f16x2 p1 = {(_Float16)fmaf((float)a[1], s24, bi), (_Float16)fmaf((float)b[1], s24, bi)};
+  return u32x2{__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1)};
 }
 
 // 32 codes (one row, one 32-group) -> four 16-byte pieces of bf16 weights
@@ -142,10 +170,24 @@ struct LongRow {
       for (int i = 0; i < 8; ++i) l |= !(fabsf(load_table_rt(s, entry + (g + i < last ? g + i : last), tab)) < kSmallScale);
     return l;
   }
-  __device__ __forceinline__ double weight(int k) const {             // the bf16 tile's
+  // ... or a weight that is no finite float16 once it is shifted, whatever its code?
+  __device__ __forceinline__ bool large_f16(int k0, int k1) const {
+    const int last = (k1 - 1) >> gshift;
+    bool l = false;
+#pragma nounroll
+    for (int g = k0 >> gshift; g <= last; ++g) {
+      const float sc = load_table_rt(s, entry + g, tab), bi = load_table_rt(b, entry + g, tab);
+      l |= !(fmaxf(fabsf(bi), fabsf(fmaf(sc, (float)((1 << BITS) - 1), bi))) < 65504.f / (1 << kF16Shift));
+    }
+    return l;
+  }
+  __device__ __forceinline__ float unrounded(int k) const {
     const uint32_t code = BITS == 8 ? codes[k] : (uint32_t)codes[k >> 1] >> (4 * (k & 1)) & 15u;
     const int64_t g = entry + (k >> gshift);
-    return (double)bf16_bits_to_f32(f32_to_bf16_bits(fmaf(load_table_rt(s, g, tab), (float)code, load_table_rt(b, g, tab))));
+    return fmaf(load_table_rt(s, g, tab), (float)code, load_table_rt(b, g, tab));
+  }
+  __device__ __forceinline__ double weight(int k) const {             // the bf16 tile's
+    return (double)bf16_bits_to_f32(f32_to_bf16_bits(unrounded(k)));
   }
 };
 

@@ -28,7 +28,7 @@
 // Measured, bf16 activations and four-bit codes in groups of 64, against the
 // prefill kernel on whole K: 48 rows of 4096 x 14336 104 -> 22 us, 17 rows of
 // 4096 x 4096 35 -> 12, 48 rows of 14336 x 4096 37 -> 22; float16 activations and
-// tables, 77 rows of 4096 x 4096 46 -> 21.  Of the 22 us about 10 are fixed (launch, first
+// tables, 77 rows of 4096 x 4096 46 -> 21 -> 14.8 without terms.  Of the 22 us about 10 are fixed (launch, first
 // data, the sums' second launch); a step takes 0.76 us and 0.14 more per row
 // block, the vector ALU's instructions about half of it.
 //
@@ -42,6 +42,7 @@
 // float16 / float32 activations are exact sums of two / three bf16 terms; each
 // term is a row block of its own on the same weight fragments and the terms'
 // float32 sums are added in the epilogue, so the weight is still streamed once.
+// float16 ones with float16 tables need no terms (short_terms).
 #include <type_traits>
 #include <utility>
 
@@ -120,9 +121,11 @@ struct ShortShape {
 };
 
 // TAB: QMM_BF16, QMM_F16 or QMM_F32 tables (MXFP4: QMM_BF16, its scales are widened to that).
-template <int MODE, int BITS, int TAB, int MB>
+// HALF: float16 rows times float16 tables as they are, weights rounded to float16.
+template <int MODE, int BITS, int TAB, int MB, bool HALF>
 __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   using S = ShortShape<MODE, BITS, MB>;
+  static_assert(!HALF || (MODE == 0 && TAB == QMM_F16), "float16 weights come from float16 tables");
   constexpr int D = S::kDepth;
   constexpr int SUB = S::kStep / 4;              // codes of a wavefront's quarter: 64 | 32
   constexpr int STEPS = SUB / 32;                // MFMA steps: 2 | 1
@@ -336,6 +339,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
         bi = __uint_as_float(o.t0[c] & 0xFFFF0000u);
       }
       const uint32_t q[2] = {o.q[c][BITS == 4 ? j : 0], o.q[c][1]};
+      if constexpr (HALF) {
+        const float s24 = sc * (float)(1 << (24 + g2::kF16Shift)), bs = bi * (float)(1 << g2::kF16Shift);
+        if constexpr (BITS == 4) return __builtin_bit_cast(bf16x8, g2::dequant_nibbles_f16(q[0], s24, s24 * 0x1p-4f, bs));
+        const u32x2 lo = g2::dequant_bytes_f16(q[0], s24, bs), hi = g2::dequant_bytes_f16(q[1], s24, bs);
+        return __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+      }
       return __builtin_bit_cast(bf16x8, g2::dequant_piece<0, BITS>(q, 0, sc, bi));
     }
   };
@@ -347,7 +356,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
       bf16x8 wn8 = wq;
       if constexpr (b + 1 < NB) wn8 = widen(o, std::integral_constant<int, b + 1>{});
 #pragma unroll
-      for (int i = 0; i < MB; ++i) acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.xa[j][i], wq, acc[c][i], 0, 0, 0);
+      for (int i = 0; i < MB; ++i) {
+        if constexpr (HALF)
+          acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, o.xa[j][i]), __builtin_bit_cast(f16x8, wq), acc[c][i], 0, 0, 0);
+        else
+          acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.xa[j][i], wq, acc[c][i], 0, 0, 0);
+      }
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // one MFMA,
@@ -431,8 +445,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   if constexpr (MB == 3) {
     if (a.terms == 3) r[0] += r[1] + r[2];
   }
+  if constexpr (HALF) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) r[i] *= 1.f / (1 << g2::kF16Shift);
+  }
   const int n = n0 + 64 * wn + 4 * r16;
-  if constexpr (MODE == 0 && TAB != QMM_F16) {
+  if constexpr (MODE == 0 && (TAB != QMM_F16 || HALF)) {
     // a scale too large for the short form of the dequantization: its column's results
     // are not finite, in rows of zeros either
     float probe = 0.f;
@@ -456,7 +474,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
         if (n + j >= a.N) break;
         if (fin >> j & 1) continue;
         const g2::LongRow<BITS> row(a.w, a.s, a.b, e, n + j, a.N, a.K, a.gshift, TAB);
-        if (!row.large(k0, k1)) continue;        // an activation, or a sum that is out of range
+        if (!(HALF ? row.large_f16(k0, k1) : row.large(k0, k1))) continue;       // an activation, or a sum that is out of range
 #pragma nounroll
         for (int i = 0; i < a.blocks; ++i) {
           const int m = m0 + i * 16 + 4 * kg + wk;
@@ -466,8 +484,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
 #pragma nounroll
             for (int t = 0; t < a.terms; ++t)
 #pragma nounroll
-              for (int k = k0; k < k1; ++k)
-                sum = fma((double)bf16_bits_to_f32(static_cast<const uint16_t*>(a.x)[((int64_t)t * a.x_rows + src) * a.K + k]), row.weight(k), sum);
+              for (int k = k0; k < k1; ++k) {
+                const uint32_t x = static_cast<const uint16_t*>(a.x)[((int64_t)t * a.x_rows + src) * a.K + k];
+                if constexpr (HALF) sum = fma((double)f16_bits_to_f32(x), (double)row.unrounded(k), sum);
+                else sum = fma((double)bf16_bits_to_f32(x), row.weight(k), sum);
+              }
           reinterpret_cast<float*>(own + i * 4 * 64)[j] = (float)sum;
         }
       }
@@ -581,26 +602,27 @@ ShortPlan short_plan(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int m
   return p;
 }
 
-template <int MODE, int BITS, int TAB, int MB>
+template <int MODE, int BITS, int TAB, int MB, bool HALF>
 void launch_mb(const ShortArgs& a, hipStream_t st) {
   constexpr size_t lds = ShortShape<MODE, BITS, MB>::kLds;
-  constexpr auto kern = short_kernel<MODE, BITS, TAB, MB>;
+  constexpr auto kern = short_kernel<MODE, BITS, TAB, MB, HALF>;
   if (!lds_limit<kern>(lds)) return;
   const int64_t total = ceil_div((int64_t)a.n_tiles * a.m_tiles * a.splits, 8) * 8;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * kWaves), lds, st, a);
 }
 
-template <int MODE, int BITS, int TAB>
+template <int MODE, int BITS, int TAB, bool HALF = false>
 void launch_short(const ShortArgs& a, int mb, hipStream_t st) {
-  if (mb == 1) launch_mb<MODE, BITS, TAB, 1>(a, st);
-  else if (mb == 2) launch_mb<MODE, BITS, TAB, 2>(a, st);
-  else if (mb == 3) launch_mb<MODE, BITS, TAB, 3>(a, st);
-  else launch_mb<MODE, BITS, TAB, 4>(a, st);
+  if (mb == 1) launch_mb<MODE, BITS, TAB, 1, HALF>(a, st);
+  else if (mb == 2) launch_mb<MODE, BITS, TAB, 2, HALF>(a, st);
+  else if (mb == 3) launch_mb<MODE, BITS, TAB, 3, HALF>(a, st);
+  else launch_mb<MODE, BITS, TAB, 4, HALF>(a, st);
 }
 
 template <int BITS>
-void launch_affine(const ShortArgs& a, int tab, int mb, hipStream_t st) {
-  if (tab == QMM_BF16) launch_short<0, BITS, QMM_BF16>(a, mb, st);
+void launch_affine(const ShortArgs& a, int tab, int mb, bool half, hipStream_t st) {
+  if (half) launch_short<0, BITS, QMM_F16, true>(a, mb, st);
+  else if (tab == QMM_BF16) launch_short<0, BITS, QMM_BF16>(a, mb, st);
   else if (tab == QMM_F16) launch_short<0, BITS, QMM_F16>(a, mb, st);
   else launch_short<0, BITS, QMM_F32>(a, mb, st);
 }
@@ -623,7 +645,18 @@ bool short_supported(int64_t R, int64_t E, int64_t N, int64_t K, int gs, int bit
   return terms * R * K < (1ll << 30);
 }
 
-// The activations' terms (none for bf16), without the splits' sums.
+// The terms that this kernel multiplies activations as: one for bf16, and for
+// float16 ones whose tables are float16 too -- they go to the matrix cores as they
+// are, with weights rounded to float16 (11 significant bits instead of the bf16
+// tile's 8).  77 rows of 4096 x 4096 in groups of 128: 21.7 us
+// in two terms (a launch for them, tiles of 32 rows), 14.8 like this (tiles of 48).
+// (Groups of 32 keep the bf16 tile, which their products are compared with.)
+int short_terms(int x_dtype, int tab, int gs, int mode) {
+  if (x_dtype == QMM_F16) return mode == QMM_MODE_AFFINE && tab == QMM_F16 && gs >= 64 ? 1 : 2;
+  return x_dtype == QMM_F32 ? 3 : 1;
+}
+
+// The activations' terms (none where there is one), without the splits' sums.
 size_t short_prep_bytes(int64_t R, int64_t K, int terms) {
   return terms == 1 ? 0 : ((size_t)terms * R * K * 2 + 255) / 256 * 256;
 }
@@ -650,7 +683,7 @@ void short_dispatch(const void* x, int x_dtype, const void* w, const void* s, co
                     int y_dtype, const int32_t* row_offsets, const int32_t* src_row, const int32_t* out_idx, int64_t R,
                     int64_t x_rows, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, void* workspace,
                     size_t workspace_bytes, hipStream_t st) {
-  const int terms = x_dtype == QMM_F32 ? 3 : x_dtype == QMM_F16 ? 2 : 1;
+  const int terms = short_terms(x_dtype, tab, gs, mode);
   const size_t prep = short_prep_bytes(R, K, terms);
   const ShortPlan p = short_plan(R, row_offsets ? E : 1, N, K, bits, mode, terms, workspace_bytes - prep);
   ShortArgs a;
@@ -681,8 +714,8 @@ void short_dispatch(const void* x, int x_dtype, const void* w, const void* s, co
     a.x_rows = (int)R;
   }
   if (mode == QMM_MODE_MXFP4) launch_short<1, 4, QMM_BF16>(a, p.mb, st);
-  else if (bits == 4) launch_affine<4>(a, tab, p.mb, st);
-  else launch_affine<8>(a, tab, p.mb, st);
+  else if (bits == 4) launch_affine<4>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
+  else launch_affine<8>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
   if (p.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, p.splits, row_offsets, E, out_idx, st);
 }
 
