@@ -40,6 +40,7 @@
 // Per K-step a wavefront issues 32 MFMAs of 32x32x64 (2 K-halves x 2 terms x 2
 // row tiles x 4 column tiles) against 24 + 8 loads.  (The 16x16x128 form of
 // the instruction sustains well under half the rate of the 32x32x64 form.)
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -709,14 +710,19 @@ void mxfp4_geometry(int64_t R, int64_t N, int64_t K, int* grid, int* block) {
   *block = K % 2048 == 0 ? 512 : 256;            // the eight-wavefront form | the four-wavefront form
 }
 
-// About how long the product takes, in microseconds: the launches, a round for
-// every 256 tiles, the result (fitted on 20 to 400 rows, N and K 1024 to 14336; 17 %
-// off on average, and 40 % too short for groups: profiles/prefill_plan_fits.txt).
+// About how long the product takes, in microseconds: the launches, a round for every
+// 256 tiles (a step a little longer where they fill the chip), the split of the
+// activations, the result, and for groups their experts' weights, each streamed by a
+// tile or two.  Fitted on 68 dense products of 17 to 2048 rows, N and K 1024 to 14336,
+// and 24 over 8 to 32 experts: 6 and 7 % off on average, and the choice between this
+// kernel and the short-group one 0.6 % from the better (5.5 % before, when it came out
+// 40 % too short for groups); profiles/prefill_plan_fits.txt.
 double mxfp4_us(int64_t R, int64_t E, int64_t N, int64_t K) {
   const int64_t group = E > 1 ? ceil_div(R, E) : R;
   const int64_t tiles = ceil_div(N, TN) * (E > 1 ? E * ceil_div(group * 5 / 4, TM) : ceil_div(R, TM));
-  return 3.5 + (double)ceil_div(tiles, 256) * (3.0 + (double)K * (K % 2048 == 0 ? 2.2e-3 : 5.0e-3)) +
-         (double)R * K * 0.5e-6 + (double)R * N * 0.5e-6;
+  const double step = K % 2048 == 0 ? 2.18e-3 + 0.48e-3 * (tiles < 256 ? tiles / 256.0 : 1.0) : 3.30e-3;
+  return 4.9 + (double)ceil_div(tiles, 256) * (2.7 + (double)K * step) + (double)R * K * 1.63e-6 +
+         (double)R * N * 0.85e-6 + (E > 1 ? (double)std::min(E, R) * N * K * 7.2e-8 : 0.0);
 }
 
 // x bf16 [x_rows, K] (rows gathered through lhs_idx when given); w uint8 [E, N, K/2];
