@@ -429,6 +429,8 @@ bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products)
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
                               int64_t products);
 void skinny2_ragged_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int tab, hipStream_t st);
+bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b, int64_t products);
+void skinny2_g32_dispatch(const GemvArgs& a0, int64_t batch, int bits, int tab, hipStream_t st);
 void skinny2_mx_dispatch(const GemvArgs& a0, int64_t batch, hipStream_t st);
 
 // Tile / slice / unroll choice; QMM_GEMV_T, QMM_GEMV_WAVES and QMM_GEMV_U
@@ -495,6 +497,8 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
   const int64_t weights = std::max(batch, n_experts);
   if (!no_skinny && mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, weights))
     return skinny2_ragged_dispatch(a, batch, gs, bits, tab, st);
+  if (!no_skinny && mode == QMM_MODE_AFFINE && skinny2_g32_supported(N, K, gs, bits, tab, s, b, weights))
+    return skinny2_g32_dispatch(a, batch, bits, tab, st);
   Geometry g;
   gemv_geometry(M, N, K, &g.t, &g.waves);
   g.u = env_u ? env_u : 8;
@@ -521,7 +525,9 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
 bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b,
                        int64_t products) {
   if (skinny_supported(N, K, gs, bits, mode, tab, s, b)) return false;
-  if (mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, products)) return false;
+  if (mode == QMM_MODE_AFFINE && (skinny2_ragged_supported(N, K, gs, bits, tab, s, b, products) ||
+                                  skinny2_g32_supported(N, K, gs, bits, tab, s, b, products)))
+    return false;
   if ((tab == QMM_F16 || tab == QMM_F32) && K * bits / 8 / 256 >= 8 &&
       skinny_supported(N, K, gs, bits, mode, QMM_BF16, s, b))
     return false;

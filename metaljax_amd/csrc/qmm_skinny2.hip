@@ -199,8 +199,12 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // float32 tables with groups of 64 (eight 4-byte entries: 32 bytes, WIDE).
   // From 7 on K is any multiple of 64 (a RAGGED last slice): 7 = MXFP4, 8 + kind
   // = the affine kinds above.
+  // G32: 24 / 25 = groups of 32 with bf16 / float16 tables, K any multiple of 64, whole
+  // slices too.  A chunk's two entries are one dword, so that a row's share of a slice
+  // is fetched and staged as that of float32 tables with groups of 64 (kind 5).
   constexpr bool RAG = GSHIFT >= 7;
-  constexpr int GK = GSHIFT >= 8 ? GSHIFT - 8 : GSHIFT;
+  constexpr bool G32 = GSHIFT >= 24;
+  constexpr int GK = G32 ? 5 : GSHIFT >= 8 ? GSHIFT - 8 : GSHIFT;
   constexpr bool WIDE = GK == 5;
   constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (WIDE ? 2 : 1);   // scale rows | bias rows of one tile
   constexpr int kTab = 2 * kTabKind;
@@ -314,7 +318,8 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   const int slices = RAG ? (a.K + KS - 1) / KS : a.K / KS;
   const int passes = (slices + CW - 1) / CW;
   const int tail_codes = RAG ? a.K % KS : 0;                   // codes of a ragged last slice (0: it is whole)
-  const int tailp = tail_codes * BITS / 128, tailc = tail_codes / 64;  // its 16-byte pieces | its 64-code chunks
+  const int tailp = tail_codes * BITS / 128;                   // its 16-byte pieces
+  const int tailc = G32 && tail_codes == 0 ? CPS : tail_codes / 64;    // its 64-code chunks
   const uint32_t spitch = (uint32_t)(ng * ES);                 // bytes of a table row
 
   int64_t xz = !GRP && a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
@@ -632,7 +637,10 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
       return sr < xrows ? sr : -1;
     };
     const int64_t xr0 = xrow(r);
-    const uint32_t xlane = xr0 >= 0 ? (uint32_t)(xr0 * a.K * 2) + (uint32_t)kg * 32u : kOutOfRange;
+    // (lane quarter kg takes the 16-byte pieces 2 kg and 2 kg + 1 of a chunk's eight; in
+    // groups of 32 pieces kg and 4 + kg, so that an MFMA step stays inside a group)
+    constexpr uint32_t XL = G32 ? 16u : 32u, XJ = G32 ? 64u : 16u;
+    const uint32_t xlane = xr0 >= 0 ? (uint32_t)(xr0 * a.K * 2) + (uint32_t)kg * XL : kOutOfRange;
     int sl_cur[NI], sl_nxt[NI], prev_last = 0;     // the loaders' slot bookkeeping, mirrored
 #pragma unroll
     for (int k = 0; k < NI; ++k) sl_cur[k] = sl_nxt[k] = 0;
@@ -680,9 +688,9 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     // variant with start values in registers, 15.0 against 15.6).
     constexpr int NT = F32T ? 3 : F16T ? 2 : 1;     // bf16 terms per table entry
     constexpr bool SCALE_TERM = BITS == 4 && XD != 1 && !RAG && NT == 1;
-    constexpr int NG = BITS == 4 ? (SCALE_TERM ? 2 : 1) * NT * 3 : 0;
+    constexpr int NG = BITS == 4 && !G32 ? (SCALE_TERM ? 2 : 1) * NT * 3 : 0;
     constexpr int NA = (NG + 3) / 4;
-    constexpr bool XC_REG = BITS == 8 || XD == 1 || (XD == 0 && !WIDE && !SCALE_TERM);
+    constexpr bool XC_REG = !G32 && (BITS == 8 || XD == 1 || (XD == 0 && !WIDE && !SCALE_TERM));
     constexpr bool XC_LDS = !XC_REG && !WIDE && !SCALE_TERM;
     static_assert(!XC_LDS || XD != 0, "the ring variant has no patches");
     bf16x8 ax[NA ? NA : 1];
@@ -769,6 +777,60 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           if constexpr (MXR) sc = c < nv ? sc : 1.0f;        // past K: zero codes times a finite scale
           at = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][0], widen_e2m1(q[0], sc), at, 0, 0, 0);
           at = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][1], widen_e2m1(q[1], sc), at, 0, 0, 0);
+        }
+        return at;
+      }
+      if constexpr (G32) {
+        // Two groups a chunk, a group an MFMA step.  The sum of the group's activations, in
+        // the layout of the results, is one more step: times -128 it is what four-bit codes'
+        // dot starts from, and times the bias it is added behind the dot.  Kept for the whole
+        // slice these sums take 64 registers: the one-pass loop over the tiles has them, eight
+        // tiles' sums and eight chunks' activations do not leave them (there the operand is
+        // made new for every tile, or the compiler keeps them all the same: 254 registers spill,
+        // 8192 x 8192 at one row 59 us).
+        f32x4 at = acc_in;
+        uint32_t xg = xf, sz = swz;
+        if constexpr (XD == 2) {
+          xg = pin_vgpr(xg);
+          sz = pin_vgpr(sz);                     // (nor sixteen LDS addresses)
+        }
+        u32x4 s0, s1, b0, b1;
+        if constexpr (XD == 1) {
+          s0 = *reinterpret_cast<const u32x4*>(tb); b0 = *reinterpret_cast<const u32x4*>(tb + kTabKind);
+          s1 = *reinterpret_cast<const u32x4*>(tb + 1024); b1 = *reinterpret_cast<const u32x4*>(tb + kTabKind + 1024);
+        }
+        auto entry = [&](uint32_t v, int j) __attribute__((always_inline)) {
+          if constexpr (GSHIFT == 25) return f16_bits_to_f32(j ? v >> 16 : v & 0xFFFFu);
+          else return __uint_as_float(j ? v & 0xFFFF0000u : v << 16);
+        };
+#pragma unroll
+        for (int c = 0; c < CPS; ++c) {
+          uint32_t se, be;
+          if constexpr (XD == 1) {
+            se = c < 4 ? s0[c & 3] : s1[c & 3];
+            be = c < 4 ? b0[c & 3] : b1[c & 3];
+          } else {                               // (nor sixteen entries)
+            const unsigned char* te = tb + (c >> 2) * 1024 + (c & 3) * 4;
+            se = *reinterpret_cast<const uint32_t*>(te);
+            be = *reinterpret_cast<const uint32_t*>(te + kTabKind);
+          }
+          se = c < nv ? se : 0u;                 // past K: the next row's
+          be = c < nv ? be : 0u;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const f32x4 from = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][j], as_bf16x8(xg, xg, xg, xg), zero, 0, 0, 0);
+            f32x4 d;
+            if constexpr (BITS == 4) {
+              const uint32_t q = *reinterpret_cast<const uint32_t*>(base + (((uint32_t)(2 * c + j) ^ sz) << 4) + kg * 4);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][j], widen_int4(q, nib, magic), from, 0, 0, 0);
+            } else {
+              const u32x2 q = *reinterpret_cast<const u32x2*>(base + (((uint32_t)(4 * c + 2 * j + (kg >> 1)) ^ sz) << 4) + (kg & 1) * 8);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[c][j], widen_int8(q[0], q[1]), zero, 0, 0, 0);
+            }
+            const float sc = entry(se, j), bi = BITS == 4 ? entry(be, j) * (-1.f / 128.f) : entry(be, j);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) at[e] = fmaf(bi, from[e], fmaf(sc, d[e], at[e]));
+          }
         }
         return at;
       }
@@ -917,7 +979,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 #pragma unroll
           for (int j = 0; j < 2; ++j)
             raw[c][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                rxc, active && (!RAG || c < nv) ? lane_off + (uint32_t)(c * 128 + j * 16) : kOutOfRange, so, 0);
+                rxc, active && (!RAG || c < nv) ? lane_off + (uint32_t)c * 128u + (uint32_t)j * XJ : kOutOfRange, so, 0);
 #pragma unroll
         for (int c = 0; c < CPS; ++c)
 #pragma unroll
@@ -925,7 +987,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
             if constexpr (BITS == 4 && !MX) xa[c][j] = pair_stride4(raw[c][j]);
             else xa[c][j] = __builtin_bit_cast(bf16x8, raw[c][j]);
           }
-        if constexpr (!MX) {
+        if constexpr (!MX && !G32) {
           if (active) chunk_sums();
         }
       };
@@ -995,7 +1057,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
           }
-        if constexpr (!MX) {
+        if constexpr (!MX && !G32) {
           if (active) chunk_sums();
         }
       };
@@ -1054,7 +1116,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        if constexpr (!MX) {
+        if constexpr (!MX && !G32) {
           if (active) chunk_sums();
         }
       };
@@ -1100,7 +1162,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
           }
         }
-        if constexpr (!MX) {
+        if constexpr (!MX && !G32) {
           if (active) chunk_sums();
         }
       };
@@ -1148,7 +1210,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
           // the last slice read zeros)
           const int q = r / PK, m = r - q * PK;
           const int64_t xr = q * CW + wave < slices ? xrow(m) : -1;
-          const uint32_t off = xr >= 0 ? (uint32_t)(xr * a.K * 2) + (uint32_t)kg * 32u + (uint32_t)(q * CW * KS) * 2u
+          const uint32_t off = xr >= 0 ? (uint32_t)(xr * a.K * 2) + (uint32_t)kg * XL + (uint32_t)(q * CW * KS) * 2u
                                        : kOutOfRange;
           // more than eight live operand rows: whole-line loads through the
           // patch, as in the one-pass variant (the direct fetch asks for a
@@ -1252,11 +1314,11 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 
 template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD, bool GRP = false>
 void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int pair_wgs = 0) {
-  if constexpr (XD != 0 && !GRP && GSHIFT != 5 && GSHIFT != 13) {
+  if constexpr (XD != 0 && !GRP && GSHIFT != 5 && GSHIFT != 13 && GSHIFT < 24) {
     if (pair_wgs) return launch_one<BITS, CW, NL, TMAX, GSHIFT, XD, true>(a, batch, rows_per_wg, st, pair_wgs);
   }
   dim3 grid(GRP ? (unsigned)pair_wgs : (unsigned)ceil_div(a.N, rows_per_wg), (unsigned)batch);
-  constexpr bool wide = GSHIFT == 5 || GSHIFT == 13;
+  constexpr bool wide = GSHIFT == 5 || GSHIFT == 13 || GSHIFT >= 24;
   constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (wide ? 2 : 1);
   constexpr int XR = XD ? 0 : 2048 / BITS / 128;
   // (direct variants: plus a 1 KB patch a compute wavefront for staging activations)
@@ -1284,6 +1346,8 @@ void launch_k(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st,
       case 12: return launch_one<BITS, CW, NL, TMAX, 12, XD>(a, batch, rows_per_wg, st, pair_wgs);
       case 13: return launch_one<BITS, CW, NL, TMAX, 13, XD>(a, batch, rows_per_wg, st, pair_wgs);
       case 14: return launch_one<BITS, CW, NL, TMAX, 14, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 24: return launch_one<BITS, CW, NL, TMAX, 24, XD>(a, batch, rows_per_wg, st, pair_wgs);
+      case 25: return launch_one<BITS, CW, NL, TMAX, 25, XD>(a, batch, rows_per_wg, st, pair_wgs);
       default: break;
     }
   }
@@ -1398,6 +1462,8 @@ static int affine_kind(int gs, int tab) {
   return (gs == 128 ? 1 : 0) + (tab == QMM_F16 ? 3 : tab == QMM_F32 ? 5 : 0);
 }
 
+static int g32_kind(int tab) { return tab == QMM_F16 ? 25 : 24; }
+
 // tab: QMM_BF16 or QMM_F16 tables; force_direct: a direct variant even where
 // the ring variant or the self-loading kernel would be chosen
 void skinny2_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int rows, hipStream_t st,
@@ -1436,11 +1502,14 @@ bool skinny_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
 bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products);
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
                               int64_t products);
+bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b, int64_t products);
 static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products);
 
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                                const void* s, const void* b, int64_t E, int64_t least_slices) {
-  if (mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, gs, bits, tab, s, b, E)) return true;
+  if (mode == QMM_MODE_AFFINE && (skinny2_ragged_supported(N, K, gs, bits, tab, s, b, E) ||
+                                  skinny2_g32_supported(N, K, gs, bits, tab, s, b, E)))
+    return true;
   // (MXFP4 whose K is no whole number of slices has no other staged kernel to go to: its ragged
   // one-pass form takes the grouped decode from three slices on)
   if (mode == QMM_MODE_MXFP4) return (K / 512 >= least_slices || K % 512 != 0) && skinny2_mx_supported(N, K, s, E);
@@ -1464,7 +1533,7 @@ void skinny2_grouped_dispatch(const void* x, const void* w, const void* s, const
   a.M = 1; a.N = (int)N; a.K = (int)K;
   const bool ragged = K * bits / 8 % 256 != 0;
   const bool sorted_here = rhs_idx != nullptr;
-  a.gshift = mode == QMM_MODE_MXFP4 ? (ragged ? 7 : 2) : (ragged ? 8 : 0) + affine_kind(gs, tab);
+  a.gshift = mode == QMM_MODE_MXFP4 ? (ragged ? 7 : 2) : gs == 32 ? g32_kind(tab) : (ragged ? 8 : 0) + affine_kind(gs, tab);
   a.y_dtype = y_dtype;
   a.lhs_idx = lhs_idx;
   a.rhs_idx = rhs_idx;
@@ -1566,6 +1635,36 @@ bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, c
   const int64_t tbytes = N * (K / gs) * (tab == QMM_F32 ? 4 : 2);
   if (products > 1 && tbytes % 4) return false;
   return N * (K * bits / 8) < 0x7FFFFFFFll && tbytes < 0x7FFFFFFCll;   // 32-bit lane offsets
+}
+
+// Affine decode in groups of 32 with 16-bit tables, K any multiple of 64: the direct
+// variants (us a launch against the general kernel, 1 / 5 / 16 rows, four-bit codes:
+// 4096 x 4096 6.3 / 6.6 / 8.4 against 7.8 / 8.4 / 10.5, 14336 x 4096 11.3 / 12.0 /
+// 14.4 against 23.9 / 26.9 / 29.7, 8192 x 8192 12.9 / 13.5 / 18.9 against 24.4 / 27.7 /
+// 29.7, 4096 x 14336 11.9 / 16.2 / 23.0 against 22.3 / 25.3 / 32.0; eight-bit 14336 x
+// 4096 16.4 / 17.0 / 19.2 against 24.9 / 27.6 / 32.8; groups of 64 take 8.8 / 9.0 / 9.7
+// of 14336 x 4096: half the table entries, and room for their activations' patches).
+// Up to K = 1024 the general kernel's shorter start wins (4096 x 768 4.6 / 4.7 / 5.1
+// against 5.2 / 5.0 / 5.2, eight-bit 4096 x 576 4.0 / 4.0 / 4.3 against 5.2 / 4.7 / 4.7;
+// from 1024 x 1088 on, 5.4 / 5.5 / 6.0, it is 5.2 / 5.0 / 5.1 here).
+bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b, int64_t products) {
+  if (gs != 32 || (bits != 4 && bits != 8) || tab == QMM_F32 || K % 64 || K <= 1024) return false;
+  if ((reinterpret_cast<uintptr_t>(s) & 3u) || (reinterpret_cast<uintptr_t>(b) & 3u)) return false;
+  (void)products;                                 // (a weight's table is whole dwords: K / 32 is even)
+  return N * (K * bits / 8) < 0x7FFFFFFFll && N * (K / 16) < 0x7FFFFFFCll;       // 32-bit lane offsets
+}
+
+void skinny2_g32_dispatch(const GemvArgs& a0, int64_t batch, int bits, int tab, hipStream_t st) {
+  GemvArgs a = a0;
+  a.gshift = g32_kind(tab);
+  const int rows = (int)mx_rows_per_wg(a.N, a.K, batch);
+  if (a.K * bits / 8 <= 2048) {
+    if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, batch, rows, st);
+    else launch_k<8, 8, 4, 4, 1>(a, batch, rows, st);
+  } else {
+    if (bits == 4) launch_k<4, 8, 4, 8, 2>(a, batch, rows, st);
+    else launch_k<8, 8, 4, 8, 2>(a, batch, rows, st);
+  }
 }
 
 int64_t skinny2_ragged_rows(int64_t N, int64_t K, int64_t products) { return mx_rows_per_wg(N, K, products); }
