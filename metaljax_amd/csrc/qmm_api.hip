@@ -345,6 +345,11 @@ bool grouped_decode_pairs(int64_t P, int64_t E) {
 bool grouped_decode_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                            const void* s, const void* b, size_t workspace_bytes) {
   static const bool off = experiment_env("QMM_NO_GROUPED_DECODE") != nullptr;
+  // Groups of 32 decode more slowly: past 64 pairs, with more than ten an expert, the
+  // row-group kernels are ahead (us, here / there: 100 pairs over 8 experts of 4096 x 4096
+  // 38.5 / 34.2, 500 over 32 of 1024 x 4096 43.9 / 34.9, 256 over 16 of 4096 x 2048 46.5 / 40.7;
+  // 300 over 32 of 2048 x 2048 33.3 / 37.4, 128 over 32 32.4 / 35.9).
+  if (mode == QMM_MODE_AFFINE && gs == 32 && P > kGatherGemvMaxPairs && P > 10 * E) return false;
   return grouped_decode_pairs(P, E) && !off && workspace_bytes >= route_bytes_segments(P, E) &&
          skinny2_grouped_supported(N, K, gs, bits, mode, tab, s, b, E, 8);
 }
