@@ -21,8 +21,19 @@ _DT = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 _MODE = {"affine": MODE_AFFINE, "mxfp4": MODE_MXFP4}
 
 
+# The current stream's handle without a Stream object made for it (what torch's own
+# generated code calls): 0.1 instead of 1.1 us, 2.7 where the device is looked up too.
+# A decode launch lasts five.
+_raw_stream, _this_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device.index).cuda_stream
+    return _raw_stream(t.device.index)
+
+
+def _stream_here() -> int:
+    """The current stream of the current device."""
+    return _raw_stream(_this_device())
 
 
 # One scratch allocation per (device, stream), grown to the largest request seen:
@@ -98,7 +109,7 @@ def quantized_matmul(x, w, scales, biases=None, transpose=True, group_size=64, b
         for d in xlead:
             mrows *= d
     out_dtype = out_dtype or x.dtype
-    y = torch.empty(xlead + (m, n), dtype=out_dtype, device=x.device)
+    y = x.new_empty(xlead + (m, n), dtype=out_dtype)
     w, scales = w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
     tab = _dt(scales.dtype) if mode == "affine" else BF16
@@ -176,7 +187,7 @@ def gather_qmm(x, w, scales, biases=None, lhs_indices=None, rhs_indices=None, tr
     t = x.shape[0]
     p = rhs.numel()
     out_dtype = out_dtype or x.dtype
-    y = torch.empty((p, n), dtype=out_dtype, device=x.device)
+    y = x.new_empty((p, n), dtype=out_dtype)
     x, w, scales = x.contiguous(), w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
     act, stream = _dt(x.dtype), _stream(x)
@@ -290,7 +301,7 @@ class BoundQmm:
         self.y = y
 
     def launch(self, stream=None):
-        st = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+        st = stream if stream is not None else _stream_here()
         rc = self._lib.qmm_quantized_matmul(*self._args, st)
         if rc:
             _lib.check(rc)
@@ -323,7 +334,7 @@ class BoundGrouped:
         self.y = y
 
     def launch(self, stream=None):
-        st = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+        st = stream if stream is not None else _stream_here()
         rc = self._lib.qmm_grouped_qmm(*self._args, st)
         if rc:
             _lib.check(rc)
@@ -358,7 +369,7 @@ class BoundGather:
         self.y = y
 
     def launch(self, stream=None):
-        st = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+        st = stream if stream is not None else _stream_here()
         rc = self._lib.qmm_gather_qmm(*self._args, st)
         if rc:
             _lib.check(rc)

@@ -662,7 +662,7 @@ class Launches:
 
     def run(self, interp, env):
         import torch
-        from . import moe, qmm
+        from . import kernels, moe, qmm
         g, r = self.g, self.g.router
         inputs = {}                                     # of this call: value -> tensor (kept until its launches are out)
 
@@ -674,7 +674,7 @@ class Launches:
         if self.rows is not None:
             values = [at(v) for v, _ in self.row_leaves] + ([at(self.row_dot[1]), at(self.row_dot[2])] if self.row_dot else [])
             device = values[0].device
-            stream = torch.cuda.current_stream(device.index).cuda_stream if device.type == "cuda" else 0
+            stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
             experts = torch.empty(g.P, dtype=torch.int32, device=device)
             weights = torch.empty(g.P, dtype=qmm._torch_dtype(elem(r.weights)), device=device)
             p = _copy(self.rows)
@@ -688,7 +688,7 @@ class Launches:
             experts = moe.pair_experts(env, r)
             weights = qmm.to_device(env[r.weights]).contiguous()
             device = experts.device
-            stream = torch.cuda.current_stream(device.index).cuda_stream if device.type == "cuda" else 0
+            stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
         results = []
 
         def launch(built, program, y, summed=None):
