@@ -26,7 +26,6 @@ from . import ir
 from .packing import f32_to_bf16_bits
 
 REGISTRY = {}
-_SKIP = object()
 
 
 def register(*names):
@@ -184,37 +183,33 @@ class Interpreter:
     def invalidate_plans(self):
         self._plans = {}
 
-    # -- rewrite plan: op -> _SKIP | (emit, match)
+    # -- rewrite plan: the ops that run, each with None or (emit, match) in its
+    # place (what a fused root absorbed never runs and is not in it)
     def _rewrite_plan(self, block):
         plan = self._plans.get(block)
         if plan is not None:
             return plan
-        plan = {}
+        plan = []
         st = self._qmm
-        if st is not None and st.active:
+        fused = st is not None and st.active
+        if fused:
             from . import qmm
-            for op in block.ops:
-                key = op.results[0] if op.results else None
-                if key is None:
-                    continue
-                m = st.roots.get(key)
-                if m is not None:
-                    plan[op] = (qmm.emit, m, qmm.emit_reads(m))
-                elif key in st.skip:
-                    plan[op] = _SKIP
+        for op in block.ops:
+            key = op.results[0] if fused and op.results else None
+            m = st.roots.get(key) if key is not None else None
+            if m is not None:
+                plan.append((op, (qmm.emit, m)))
+            elif key is None or key not in st.skip:
+                plan.append((op, None))
         self._plans[block] = plan
         return plan
 
     def run_block(self, block, env):
-        plan = self._rewrite_plan(block)
-        for op in block.ops:
+        for op, entry in self._rewrite_plan(block):
             if op.name == "return":
                 return [env[v] for v in op.operands]
-            entry = plan.get(op)
-            if entry is _SKIP:
-                continue                       # absorbed into a fused root: never runs
             if entry is not None:
-                fuse, match, _ = entry
+                fuse, match = entry
                 out = fuse(self, match, env)
             else:
                 handler = REGISTRY.get(op.name)

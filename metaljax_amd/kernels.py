@@ -12,6 +12,8 @@ literal chain, as the reference does on any packing or launch failure).
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -55,6 +57,17 @@ def _scratch(need: int, like: torch.Tensor, stream=None):
     return ws
 
 
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(*shape) -> int:
+    """What the library asks for a product of this shape (a function of the shape alone)."""
+    return int(_lib.load().qmm_workspace_bytes(*shape))
+
+
+@functools.lru_cache(maxsize=4096)
+def _gather_workspace_bytes(*shape) -> int:
+    return int(_lib.load().qmm_gather_workspace_bytes(*shape))
+
+
 def _need_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -77,7 +90,8 @@ def _weight_dims(w: torch.Tensor, bits: int, mode: str):
     per = (8 // bits) if w.dtype == torch.uint8 else (32 // bits)
     if mode == "mxfp4":
         per = 2 if w.dtype == torch.uint8 else 8
-    return tuple(w.shape[:-2]), w.shape[-2], w.shape[-1] * per
+    *lead, n, words = w.shape
+    return tuple(lead), n, words * per
 
 
 def quantized_matmul(x, w, scales, biases=None, transpose=True, group_size=64, bits=4,
@@ -93,33 +107,34 @@ def quantized_matmul(x, w, scales, biases=None, transpose=True, group_size=64, b
     _need_cuda(x, w, scales, biases)
     lib = _lib.load()
     lead, n, k = _weight_dims(w, bits, mode)
-    if x.shape[-1] != k:
-        raise _lib.QmmError(2, f"x K={x.shape[-1]} vs weight K={k}")
-    m = x.shape[-2]
-    xlead = tuple(x.shape[:-2])
-    if lead and xlead != lead:
-        raise _lib.QmmError(2, f"batch dims {xlead} vs {lead}")
-    batch = 1
-    for d in lead:
-        batch *= d
-    x2 = x.contiguous()
-    mrows = m
-    if not lead:
+    *xlead, m, xk = x.shape
+    if xk != k:
+        raise _lib.QmmError(2, f"x K={xk} vs weight K={k}")
+    batch, mrows = 1, m
+    if lead:
+        if tuple(xlead) != lead:
+            raise _lib.QmmError(2, f"batch dims {tuple(xlead)} vs {lead}")
+        for d in lead:
+            batch *= d
+    else:
         # unbatched weight: leading activation dims fold into M
         for d in xlead:
             mrows *= d
-    out_dtype = out_dtype or x.dtype
-    y = x.new_empty(xlead + (m, n), dtype=out_dtype)
+    x2 = x.contiguous()
+    act = _dt(x2.dtype)
+    out, out_dtype = (act, x.dtype) if out_dtype is None or out_dtype == x.dtype else (_dt(out_dtype), out_dtype)
+    y = x.new_empty((*xlead, m, n), dtype=out_dtype)
     w, scales = w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
-    tab = _dt(scales.dtype) if mode == "affine" else BF16
+    tab, mode = _dt(scales.dtype) if mode == "affine" else BF16, _MODE[mode]
     stream = _stream(x)
-    need = lib.qmm_workspace_bytes(batch, mrows, n, k, group_size, bits, _MODE[mode], _dt(x2.dtype))
+    need = _workspace_bytes(batch, mrows, n, k, group_size, bits, mode, act)
     ws = _scratch(need, x, stream)
     rc = lib.qmm_quantized_matmul(
-        _ptr(x2), _dt(x2.dtype), _ptr(w), _ptr(scales), _ptr(biases), tab, _ptr(y), _dt(out_dtype),
-        batch, mrows, n, k, group_size, bits, _MODE[mode], _ptr(ws), need, stream)
-    _lib.check(rc)
+        x2.data_ptr(), act, w.data_ptr(), scales.data_ptr(), _ptr(biases), tab, y.data_ptr(), out,
+        batch, mrows, n, k, group_size, bits, mode, _ptr(ws), need, stream)
+    if rc:
+        _lib.check(rc)
     return y
 
 
@@ -191,7 +206,7 @@ def gather_qmm(x, w, scales, biases=None, lhs_indices=None, rhs_indices=None, tr
     x, w, scales = x.contiguous(), w.contiguous(), scales.contiguous()
     biases = None if biases is None else biases.contiguous()
     act, stream = _dt(x.dtype), _stream(x)
-    nbytes = lib.qmm_gather_workspace_bytes(p, e, n, k, act)
+    nbytes = _gather_workspace_bytes(p, e, n, k, act)
     ws = _scratch(nbytes, x, stream)
     tab = _dt(scales.dtype) if mode == "affine" else BF16
     rc = lib.qmm_gather_qmm(_ptr(x), act, _ptr(w), _ptr(scales), _ptr(biases), tab,

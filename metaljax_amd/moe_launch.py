@@ -35,6 +35,8 @@ from .recognize import count, dims_of, elem, op_key
 
 ELS = {"f32": 0, "bf16": 1, "f16": 2, "i1": 3, "i32": 4}           # QMM_EL_*
 FLOATS = ("f32", "bf16", "f16")
+SIZE = {"f32": 4, "bf16": 2, "f16": 2, "i32": 4}
+_DT = {"f32": _lib.F32, "bf16": _lib.BF16, "f16": _lib.F16}
 _OPS = ("copy add subtract multiply divide maximum minimum power abs negate exponential log logistic tanh sqrt rsqrt "
         "ceil floor round_nearest_even sign EQ NE LT LE GT GE and or xor not select clamp imm sum rowmax rowmin slice "
         "top_k").split()
@@ -91,6 +93,23 @@ def _copy(struct):
 
 def run_map(program, stream):
     rc = _lib.load().qmm_pair_map_run(ctypes.byref(program), stream)
+    if rc:
+        _lib.check(rc)
+
+
+def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n, k, like, stream):
+    """y [pairs, n] = row lhs[p] of x [rows, k] (row p without lhs) times expert
+    rhs[p] of a match's packed weight; x, lhs, rhs and y are addresses.  `like`: a
+    tensor of the device."""
+    from . import kernels
+    lib = _lib.load()
+    affine = match.mode == "affine"
+    arrays = [a if a.is_contiguous() else a.contiguous() for a in arrays[:3 if affine else 2]]
+    nbytes = kernels._gather_workspace_bytes(pairs, experts, n, k, _DT[el])
+    ws = kernels._scratch(nbytes, like, stream)
+    rc = lib.qmm_gather_qmm(x, _DT[el], arrays[0].data_ptr(), arrays[1].data_ptr(), arrays[2].data_ptr() if affine else None,
+                            kernels._dt(arrays[1].dtype) if affine else _lib.BF16, y, _DT[y_el], lhs, rhs, pairs, rows, experts,
+                            n, k, match.gs, match.bits, kernels._MODE[match.mode], None if ws is None else ws.data_ptr(), nbytes, stream)
     if rc:
         _lib.check(rc)
 
@@ -574,6 +593,7 @@ class Launches:
 
     def __init__(self, interp, g, block):
         self.interp, self.g = interp, g
+        self.modules = None              # what a call needs of this package, looked up once
         self.reads = []
         self.dots, self._dot_of = [], {}
         r = g.router
@@ -612,6 +632,8 @@ class Launches:
             d.strides[axis] = count(info.nshape[pos + 1:])
         data = info.data
         dshape = dims_of(data)
+        if elem(data) not in FLOATS:
+            raise Reject("activations of other than floats")
         if info.direct:
             if info.t_dim != 0 or [i for i in range(1, len(dshape)) if dshape[i] != 1] != [i for i in info.contract if dshape[i] != 1]:
                 raise Reject("activations that would have to be re-laid")
@@ -623,8 +645,6 @@ class Launches:
             for j, i in enumerate(info.contract):
                 index[i] = feed.coordinate(j)
             el = elem(data)
-            if el not in FLOATS:
-                raise Reject("activations of other than floats")
             result = feed.pull(data, info.data_e, info.t_dim, index)
             d.feed = (feed, feed.finish(result, el), el)
         d.number = len(self.dots)
@@ -651,73 +671,84 @@ class Launches:
 
     # -- a call
 
-    def _tensor(self, value):
-        import torch
-        from . import moe, qmm
-        if isinstance(value, torch.Tensor):
-            t = value if value.device.type == qmm.DEVICE else value.to(qmm.DEVICE)
-        else:
-            t = moe.dev(value).t
-        return t if t.is_contiguous() else t.contiguous()
+    def _layout(self):
+        """Where a call's intermediate results lie in its one buffer."""
+        g = self.g
+        self.buffer = 0
+
+        def place(n, el):
+            at, self.buffer = self.buffer, (self.buffer + n * SIZE[el] + 255) // 256 * 256
+            return at
+        self.at_experts, self.at_weights = place(g.P, "i32"), place(g.P, elem(g.router.weights))
+        self.at_feed = [place(g.P * d.info.k, d.feed[2]) if d.feed else None for d in self.dots]
+        self.at_dot = [place(g.P * d.n, d.out_el) for d in self.dots]
 
     def run(self, interp, env):
-        import torch
-        from . import kernels, moe, qmm
+        if self.modules is None:
+            import torch
+            from . import kernels, moe, qmm
+            self.modules = torch, kernels, moe, qmm
+            self._layout()
+        torch, kernels, moe, qmm = self.modules
         g, r = self.g, self.g.router
         inputs = {}                                     # of this call: value -> tensor (kept until its launches are out)
 
         def at(v):
-            if v not in inputs:
-                inputs[v] = self._tensor(env[v])
-            return inputs[v]
+            t = inputs.get(v)
+            if t is None:
+                t = env[v]
+                if not isinstance(t, torch.Tensor):
+                    t = moe.dev(t).t
+                elif t.device.type != qmm.DEVICE:
+                    t = t.to(qmm.DEVICE)
+                inputs[v] = t = t if t.is_contiguous() else t.contiguous()
+            return t
 
+        if self.rows is None:
+            inputs[r.indices] = moe.pair_experts(env, r)
+            inputs[r.weights] = at(r.weights)
+        device = at(self.reads[0]).device
+        stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
+        buffer = torch.empty(self.buffer, dtype=torch.uint8, device=device)
+        base = buffer.data_ptr()
         if self.rows is not None:
-            values = [at(v) for v, _ in self.row_leaves] + ([at(self.row_dot[1]), at(self.row_dot[2])] if self.row_dot else [])
-            device = values[0].device
-            stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
-            experts = torch.empty(g.P, dtype=torch.int32, device=device)
-            weights = torch.empty(g.P, dtype=qmm._torch_dtype(elem(r.weights)), device=device)
+            experts, weights = base + self.at_experts, base + self.at_weights
             p = _copy(self.rows)
             for i, (v, _) in enumerate(self.row_leaves):
                 p.leaf[i].p = at(v).data_ptr()
             if self.row_dot:
                 p.dot_x, p.dot_w = at(self.row_dot[1]).data_ptr(), at(self.row_dot[2]).data_ptr()
-            p.out[0].p, p.out[1].p = experts.data_ptr(), weights.data_ptr()
+            p.out[0].p, p.out[1].p = experts, weights
             run_rows(p, stream)
         else:
-            experts = moe.pair_experts(env, r)
-            weights = qmm.to_device(env[r.weights]).contiguous()
-            device = experts.device
-            stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
-        results = []
+            experts, weights = inputs[r.indices].data_ptr(), inputs[r.weights].data_ptr()
 
         def launch(built, program, y, summed=None):
             m = _copy(program)
             for i, (source, _) in enumerate(built.leaves):
-                m.leaf[i].p = (at(source[1]) if source[0] == "env" else results[source[1]]).data_ptr()
-            m.y, m.experts_of, m.pairs, m.experts = y.data_ptr(), experts.data_ptr(), g.P, g.E
+                m.leaf[i].p = at(source[1]).data_ptr() if source[0] == "env" else base + self.at_dot[source[1]]
+            m.y, m.experts_of, m.pairs, m.experts = y, experts, g.P, g.E
             if summed is not None:
-                m.weights, m.weights_el = summed.data_ptr(), ELS[elem(r.weights)]
+                m.weights, m.weights_el = summed, ELS[elem(r.weights)]
             run_map(m, stream)
-            return y
 
-        tokens = None
-        for d in self.dots:
+        for d, feed, y in zip(self.dots, self.at_feed, self.at_dot):
             info = d.info
+            arrays = qmm.pack_arrays(interp, info.match)
             if d.feed is None:
-                x = at(info.data).reshape(g.T, info.k)
-                if tokens is None:
-                    tokens = g.pair_tokens(device)[0]
-                lhs = tokens
+                rows, el, lhs = g.T, elem(info.data), g.pair_tokens(device)[0].data_ptr()
+                x = at(info.data).data_ptr()
             else:
-                built, program, el = d.feed
-                x = launch(built, program, torch.empty((g.P, info.k), dtype=qmm._torch_dtype(el), device=device))
-                lhs = None
-            results.append(moe.emit_dot(x, qmm.pack_arrays(interp, info.match), info.match.mode, info.match.gs,
-                                        info.match.bits, lhs, experts, g.E, out_dtype=qmm._torch_dtype(d.out_el),
-                                        has_perm=info.match.has_perm))
+                rows, el, lhs, x = g.P, d.feed[2], None, base + feed
+                launch(d.feed[0], d.feed[1], x)
+            if info.match.has_perm:
+                whole = at(info.data) if d.feed is None else buffer[feed:feed + rows * info.k * SIZE[el]].view(qmm._torch_dtype(el))
+                taken = inputs[d] = kernels.take_k(whole.reshape(rows, info.k), arrays[-1])
+                x = taken.data_ptr()
+            run_product(x, el, rows, arrays, info.match, lhs, experts, base + y, d.out_el, g.P, g.E, d.n, info.k, buffer, stream)
+            moe.STATS["gather_qmm"] += 1
         total = torch.empty([g.T] + self.rest, dtype=qmm._torch_dtype(g.out_el), device=device)
-        launch(self.final_map, self.final, total, weights)
+        launch(self.final_map, self.final, total.data_ptr(), weights)
         return total
 
 

@@ -98,6 +98,17 @@ def run_rows(r, _stream):
                 store(o.p, t * o.n + i, regs[o.src + (0 if o.srcn == 1 else i)], o.el)
 
 
+def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n, k, like, _stream):
+    from oracle import qmm_oracle as O
+    assert match.mode == "mxfp4"
+    a = np.array([[load(x, i * k + j, ML.ELS[el]) for j in range(k)] for i in range(rows)], np.float32)
+    index = [np.array([ctypes.c_int32.from_address(p + 4 * i).value for i in range(pairs)]) if p else np.arange(pairs) for p in (lhs, rhs)]
+    w, scales = moe.split_experts([np.asarray(arrays[0]), np.asarray(arrays[1])], experts)
+    out = O.gather_qmm(a, w, scales, None, *index, match.gs, match.bits, match.mode)
+    for i, v in enumerate(out.reshape(-1)):
+        store(y, i, v, ML.ELS[y_el])
+
+
 def both(text, args, monkeypatch):
     """(launches, results as launches, results as array operations)"""
     monkeypatch.setattr(qmm, "DEVICE", "cpu")
@@ -106,6 +117,7 @@ def both(text, args, monkeypatch):
     monkeypatch.setattr(ML, "available", lambda: True)
     monkeypatch.setattr(ML, "run_map", run_map)
     monkeypatch.setattr(ML, "run_rows", run_rows)
+    monkeypatch.setattr(ML, "run_product", run_product)
     moe.reset_stats()
     ex = engine.compile_program(text)
     out = [I.host(b.data).a for b in engine.execute(ex, args)]
