@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // eight entries of a slice then end in the dword after its sixteen bytes: that
   // is the first one of the next slice's, which for a pass's last slice is
   // fetched apart (XD = 1: that slice is the ragged one and does not need it).
-  constexpr bool EXTRA = XD == 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11);
+  constexpr bool EXTRA = XD >= 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11);
   constexpr int LX = QI, LT = QI + QT + (EXTRA ? 1 : 0);      // loads per loader wavefront: activation item | tile item
   typedef Sched<XR, TMAX, LX, LT> S;
   static_assert(!EXTRA || NL == 4, "four requests of eight rows");
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
     if (segs == 0) return;
     // Workgroups a segment: as many as fill whole rounds of the compute units,
     // with at least those that the tiles a workgroup may hold ask for.
-    const int tiles = (a.N + 15) / 16, least = XD == 2 ? (tiles + TMAX - 1) / TMAX : 1;
+    const int tiles = (a.N + 15) / 16, least = XD >= 2 ? (tiles + TMAX - 1) / TMAX : 1;
     const int round = rows_per_wg, rounds = (segs * least + round - 1) / round;
     int wgs = rounds * round / segs;
     if (wgs > tiles) wgs = tiles;
@@ -356,7 +356,11 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
   // passes.  A tile of pass p then yields meaningful sums only in row block p
   // (the other blocks multiply another pass's activations with this pass's
   // weights and are masked off), and the blocks are added up at the end.
-  const int PK = XD != 2 ? 0 : (passes <= 2 && M <= 8) ? 8 : (passes <= 4 && M <= 4) ? 4 : 0;
+  // XD = 3: three passes of five rows, in blocks of five.  A form of its own: those rows
+  // lie across lanes, and as one more case of the other the masks cost every row count 2 to
+  // 4 % (4096 x 11008 at one row 9.2 -> 9.4 us; as a branch they spill, 11.7).
+  constexpr bool FIVES = XD == 3;
+  const int PK = FIVES ? 5 : XD != 2 ? 0 : (passes <= 2 && M <= 8) ? 8 : (passes <= 4 && M <= 4) ? 4 : 0;
 
   if (wave >= CW) {
     // ------------------------------------------------------------ loaders ----
@@ -484,7 +488,17 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         float v = 0.f;
 #pragma unroll
         for (int wv = 0; wv < CW; ++wv) v += part[wv * 1024 + e * kWave + lane];
-        if constexpr (XD == 2) {
+        if constexpr (FIVES) {                      // rows m, 5 + m and 10 + m: other lanes', and other elements
+          const int m5 = 4 * (lane >> 4) + e;
+          if (m5 < 5) {
+#pragma unroll
+            for (int q = 1; q < 3; ++q) {
+              const int row = 5 * q + m5;
+#pragma unroll
+              for (int wv = 0; wv < CW; ++wv) v += part[wv * 1024 + (row & 3) * kWave + (row >> 2) * 16 + (lane & 15)];
+            }
+          }
+        } else if constexpr (XD == 2) {
           if (PK != 0) {                            // row blocks of the passes -> rows [0, PK)
             v += __shfl_xor(v, 32);
             if (PK == 4) v += __shfl_xor(v, 16);
@@ -1019,7 +1033,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
             xr = active ? xrow(rr) : -1;
             nv[h] = chunks_of(p * CW + sw);
           } else {
-            const int q = pk == 8 ? rr >> 3 : rr >> 2, m = rr - q * pk;
+            const int q = FIVES ? rr / 5 : pk == 8 ? rr >> 3 : rr >> 2, m = rr - q * pk;
             xr = active && q * CW + wave < slices ? xrow(m) : -1;
             pass_off = (uint32_t)(q * CW * KS) * 2u;
             nv[h] = chunks_of(q * CW + wave);
@@ -1228,7 +1242,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
         QMM_STAMP(2);
         for (int p = 0; p < passes; ++p) {
           const bool active = p * CW + wave < slices;   // uniform
-          if (PK == 0) {
+          if (!FIVES && PK == 0) {
             if constexpr (!WIDE && (MX || BITS == 8)) fetch_x_halves(p, active);
             else fetch_x(p, active, xlane, chunks_of(p * CW + sw));
           }
@@ -1243,7 +1257,7 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
                                           chunks_of(p * CW + wave), slot);
                 const bool mine = PK == 0 || my_pass == p;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[t][e] += mine ? d[e] : 0.f;
+                for (int e = 0; e < 4; ++e) acc[t][e] += (FIVES ? (uint32_t)(4 * kg + e - 5 * p) < 5u : mine) ? d[e] : 0.f;
               }
               if (p == passes - 1) {
                 float* part = reinterpret_cast<float*>(ring + slot * kItem + wave * 4096);
@@ -1314,7 +1328,16 @@ __global__ __launch_bounds__(kWave*(CW + NL)) void skinny2_kernel(GemvArgs a, in
 
 template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD, bool GRP = false>
 void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int pair_wgs = 0) {
-  if constexpr (XD != 0 && !GRP && GSHIFT != 5 && GSHIFT != 13 && GSHIFT < 24) {
+  // Three passes of five rows: all of them fit the operand's sixteen rows, as three of four do,
+  // and nothing is fetched between passes (us, from where a pass's rows are fetched when it
+  // begins: 4096 x 11008 13.4 -> 9.7, 14336 x 11008 25.5 -> 21.2, eight-bit 4096 x 5504 9.6 ->
+  // 8.0; six rows, which do not fit, 13.9).  Tables that fill the LDS, and pairs, keep that.
+  if constexpr (XD == 2 && !GRP && GSHIFT != 5 && GSHIFT != 13 && GSHIFT < 24) {
+    const int64_t slices = ceil_div((int64_t)a.K * BITS / 8, 256);
+    if (a.M == 5 && !a.segments && !pair_wgs && slices > 2 * CW && slices <= 3 * CW)
+      return launch_one<BITS, CW, NL, TMAX, GSHIFT, 3>(a, batch, rows_per_wg, st);
+  }
+  if constexpr (XD != 0 && XD != 3 && !GRP && GSHIFT != 5 && GSHIFT != 13 && GSHIFT < 24) {
     if (pair_wgs) return launch_one<BITS, CW, NL, TMAX, GSHIFT, XD, true>(a, batch, rows_per_wg, st, pair_wgs);
   }
   dim3 grid(GRP ? (unsigned)pair_wgs : (unsigned)ceil_div(a.N, rows_per_wg), (unsigned)batch);
@@ -1324,7 +1347,7 @@ void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t s
   // (direct variants: plus a 1 KB patch a compute wavefront for staging activations)
   const size_t lds = (size_t)(XD || XR + TMAX >= 4 ? 4 : XR + TMAX) * (CW * 4096 + 2 * kTabKind) +
                      (XD != 0 && !wide ? (size_t)CW * 1024 : 0) + (GRP ? (CW + NL) * 128 + 512 : 0) +
-                     (XD == 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11) ? 2048 : 0);      // (the kernel's EXTRA)
+                     (XD >= 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11) ? 2048 : 0);      // (the kernel's EXTRA)
   constexpr auto kern = skinny2_kernel<BITS, CW, NL, TMAX, GSHIFT, XD, GRP>;
   if (!lds_limit<kern>(lds)) return;
   hipLaunchKernelGGL(kern, grid, dim3(kWave * (CW + NL)), lds, st, a, rows_per_wg);
