@@ -37,6 +37,11 @@ void gemm_dispatch(const void* x, const void* w, const void* s, const void* b, i
 int64_t gemm_row_tile(int64_t R, int64_t E);
 bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b,
                        int64_t products);
+bool gemv_terms_supported(const void* x, int64_t N, int64_t K, int mode, const void* s, int64_t products);
+void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
+                         int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
+                         const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,
+                         int64_t x_rows, hipStream_t st);
 void gemv_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                            int y_dtype, const int32_t* segments, const int32_t* src_row,
                            const int32_t* out_row, int64_t max_segments, int64_t x_rows, int64_t N,
@@ -868,8 +873,17 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
                 xs + ps + inner, workspace ? workspace_bytes : (size_t)0);
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc;
+  if (terms * M <= kGemvMaxM && batch <= 65535 && N <= INT32_MAX && y && gemv_terms_supported(x, N, K, mode, scales, batch)) {
+    // (the general MXFP4 decode kernel splits them itself)
+    rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
+    if (rc) return rc;
+    gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, batch, M, N, K, nullptr, nullptr, nullptr, nullptr, nullptr,
+                        0, 0, st);
+    return check_launch("gemv launch");
+  }
   split_terms_dispatch(x, x_dtype, ws, batch, M, K, nullptr, -1, st);
-  int rc = check_launch("activation split launch");
+  rc = check_launch("activation split launch");
   if (rc) return rc;
   rc = dense_bf16(ws, QMM_BF16, w, scales, biases, table_dtype, ws + xs, QMM_F32, batch, terms * M, N, K,
                   group_size, bits, mode, inner ? ws + xs + ps : nullptr, workspace_bytes - xs - ps, stream, true);
@@ -992,6 +1006,31 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   if (terms * P * K >= (1ll << 30)) return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // What the general MXFP4 decode kernel serves: it splits the rows itself.  One launch
+  // instead of three for pairs of their own, two instead of eight for sorted ones.
+  if (P <= kGatherGemvMaxPairs && E <= 65535 && N <= INT32_MAX && K <= INT32_MAX &&
+      gemv_terms_supported(x, N, K, mode, scales, std::max(P, E)) &&
+      !sorted_here_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases) &&
+      !grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
+    int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
+    if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);
+    if (rc) return rc;
+    if (!grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
+      gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, P, 1, N, K, lhs_idx, rhs_idx, nullptr, nullptr, nullptr, E, T, st);
+      return check_launch("gather gemv launch");
+    }
+    int32_t* ro = reinterpret_cast<int32_t*>(ws);
+    int32_t* cursor = ro + E + 1;
+    int32_t* src_row = cursor + E;
+    int32_t* out_row = src_row + P;
+    int32_t* segments = out_row + P;
+    route(lhs_idx, rhs_idx, P, E, ro, cursor, src_row, out_row, segments, st);
+    rc = check_launch("route launch");
+    if (rc) return rc;
+    gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, skinny2_max_segments(P, E), 16, N, K, nullptr, nullptr, segments,
+                        src_row, out_row, E, T, st);
+    return check_launch("grouped gemv launch");
+  }
   // Pairs that are decode products of their own: the terms are the rows of one (terms
   // <= 16: a pair's weight is streamed once, in one launch instead of one a term).
   if (P <= kGatherGemvMaxPairs && E <= 65535 && N <= INT32_MAX && K <= INT32_MAX &&

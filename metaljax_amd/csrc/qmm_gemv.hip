@@ -233,15 +233,74 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
   }
 }
 
+// Eight activations as TERMS bf16 operands: bf16 as they are, float16 / float32 cut off
+// term by term (exact; inf and NaN stay in the first term, a NaN stays one).  The upper
+// halves of what is left are the terms as they are, five instructions a value; where any
+// of the eight is not finite the last remainder is a NaN and they are done one by one
+// (24 instructions a value; all of them so, and with four chunks in flight of which a
+// wavefront had two, 6 pairs over 8 experts of 1024 x 1024 took 18.0 us instead of 7.4).
+template <int TERMS>
+__device__ __forceinline__ void operand_terms(const u32x4* raw, bf16x8* out) {
+  if constexpr (TERMS == 1) {
+    out[0] = __builtin_bit_cast(bf16x8, raw[0]);
+  } else {
+    float v[8], left[8];
+    uint32_t hi[TERMS][8];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (TERMS == 3) v[e] = __uint_as_float(raw[e >> 2][e & 3]);
+      else v[e] = f16_bits_to_f32((uint16_t)(e & 1 ? raw[0][e >> 1] >> 16 : raw[0][e >> 1] & 0xFFFFu));
+      left[e] = v[e];
+#pragma unroll
+      for (int term = 0; term < TERMS; ++term) {
+        hi[term][e] = __float_as_uint(left[e]);
+        if (term + 1 < TERMS) left[e] -= __uint_as_float(hi[term][e] & 0xFFFF0000u);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) finite = finite && !__builtin_isunordered(left[e], left[e + 1]);
+    if (!finite) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+#pragma unroll
+        for (int term = 0; term < TERMS; ++term) {
+          hi[term][e] = __float_as_uint(v[e]);
+          if (v[e] != v[e]) hi[term][e] |= 0x00400000u;
+          const uint32_t cut = hi[term][e] & 0xFFFF0000u;
+          v[e] = (cut & 0x7F800000u) == 0x7F800000u ? 0.f : v[e] - __uint_as_float(cut);
+        }
+      }
+    }
+#pragma unroll
+    for (int term = 0; term < TERMS; ++term) {
+      const uint32_t* h = hi[term];                // (the upper halves of two)
+      out[term] = as_bf16x8(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u), __builtin_amdgcn_perm(h[3], h[2], 0x07060302u),
+                            __builtin_amdgcn_perm(h[5], h[4], 0x07060302u), __builtin_amdgcn_perm(h[7], h[6], 0x07060302u));
+    }
+  }
+}
+
 // MXFP4 kernel.  A lane's 16-byte load is exactly one 32-element MX block, so
 // the block's power-of-two scale rides along in the hardware fp4 -> bf16
 // conversion (exact: an E2M1 value has one mantissa bit) and the products need
 // no rescaling afterwards.  One macro chunk = 128 k = four MFMA steps.
-template <int T, int WAVES, int U>
+//
+// TERMS: 1 for bf16 rows of x; float16 (2) and float32 (3) ones are split into that
+// many bf16 terms as they arrive (what split_terms_kernel writes), a weight operand
+// meets a term after the other, each with its own accumulator, and the terms' sums are
+// added largest first.  A product of a few rows is bound by its launches, and the split
+// and the sum were two of three (sorted pairs: five of eight; us a call, float32 /
+// float16, before -> now: 6 pairs over 8 experts of 1024 x 1024 12.5 / 12.1 -> 8.3 / 7.9,
+// 24 pairs 29.7 / 21.3 -> 10.9 / 10.7, 64 over 8 of 2048 x 512 34.0 / 24.0 -> 12.3 / 11.1,
+// 4 rows of 16384 x 1024 13.4 / 13.4 -> 8.8 / 8.2).  The kernel takes 7.4 us for the
+// first of these, 6.5 over bf16 terms.
+template <int T, int WAVES, int U, int TERMS>
 __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
   load_args_now(a);
   constexpr int ROWS = 16 * T;
-  __shared__ float red[WAVES][T][4][kWave];
+  constexpr int XW = TERMS == 3 ? 2 : 1;           // 16-byte pieces of eight activations
+  __shared__ float red[TERMS][WAVES][T][4][kWave];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -265,7 +324,7 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
     if (wz < 0 || wz >= a.n_experts) return;        // uniform, before any barrier
     if (xz < 0 || xz >= a.n_xrows) { xz = 0; x_ok = false; }
   }
-  const uint16_t* xb = a.x + xz * a.M * (int64_t)a.K;
+  const uint16_t* xb = a.x + xz * a.M * (int64_t)a.K * XW;
   const uint32_t* wb = a.w + wz * a.N * wpr;
   const uint8_t* sb = static_cast<const uint8_t*>(a.s) + wz * a.N * (int64_t)nblk;
 
@@ -283,21 +342,23 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
     srow[t] = sb + n * nblk;
   }
   bool xvalid = r < M && x_ok;
-  const uint16_t* xrow = xb + (int64_t)(xvalid ? r : 0) * a.K;
+  const uint16_t* xrow = xb + (int64_t)(xvalid ? r : 0) * a.K * XW;
   if (a.segments) {                                 // row r of the segment is row src_row[first + r] of x
     const int64_t src = r < M ? (int64_t)a.src_row[seg_lo + r] : -1;
     xvalid = src >= 0 && src < a.x_rows;
-    xrow = a.x + (xvalid ? src : 0) * a.K;
+    xrow = a.x + (xvalid ? src : 0) * a.K * XW;
   }
 
-  f32x4 acc[T];
+  f32x4 acc[TERMS][T];
 #pragma unroll
-  for (int t = 0; t < T; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int term = 0; term < TERMS; ++term)
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[term][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (int cb = c0; cb < c1; cb += U) {
     u32x4 q[U][T];
     uint8_t sraw[U][T];
-    u32x4 xr[U][4];
+    u32x4 xr[U][4][XW];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       int blk = (cb + u) * 4 + kg;
@@ -318,36 +379,51 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
       const int blk = (cb + u) * 4 + kg;
       const bool live = cb + u < c1 && blk < nblk;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        xr[u][j] = u32x4{0u, 0u, 0u, 0u};
-        if (xvalid && live)
-          xr[u][j] = *reinterpret_cast<const u32x4*>(xrow + (int64_t)blk * 32 + j * 8);
-      }
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < XW; ++h) {
+          xr[u][j][h] = u32x4{0u, 0u, 0u, 0u};
+          if (xvalid && live)
+            xr[u][j][h] = *reinterpret_cast<const u32x4*>(xrow + ((int64_t)blk * 32 + j * 8) * XW + h * 8);
+        }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      float sc[T];
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const float sc = e8m0_to_f32(sraw[u][t]);
+      for (int t = 0; t < T; ++t) sc[t] = e8m0_to_f32(sraw[u][t]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bf16x8 xa = __builtin_bit_cast(bf16x8, xr[u][j]);   // zero where not live
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, widen_e2m1(q[u][t][j], sc), acc[t], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        bf16x8 xa[TERMS];                                          // zero where not live
+        operand_terms<TERMS>(xr[u][j], xa);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const bf16x8 wq = widen_e2m1(q[u][t][j], sc[t]);
+#pragma unroll
+          for (int term = 0; term < TERMS; ++term)
+            acc[term][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[term], wq, acc[term][t], 0, 0, 0);
         }
       }
     }
   }
 
 #pragma unroll
-  for (int t = 0; t < T; ++t)
+  for (int term = 0; term < TERMS; ++term)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][t][i][lane] = acc[t][i];
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[term][wave][t][i][lane] = acc[term][t][i];
   __syncthreads();
   for (int e = threadIdx.x; e < T * 4 * kWave; e += kWave * WAVES) {
     const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
     float v = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv) v += red[wv][t][i][l];
+    for (int term = 0; term < TERMS; ++term) {
+      float part = 0.f;
+#pragma unroll
+      for (int wv = 0; wv < WAVES; ++wv) part += red[term][wv][t][i][l];
+      v = term ? v + part : part;
+    }
     const int m = 4 * (l >> 4) + i;
     const int64_t n = n0 + t * 16 + (l & 15);
     if (m < M && n < a.N) {
@@ -395,10 +471,16 @@ void launch_affine(const GemvArgs& a, int64_t batch, int tab, Geometry g, hipStr
   else launch_affine_g<BITS, CH, QMM_F16>(a, batch, g, st);
 }
 
-template <int T, int WAVES, int U>
+template <int T, int WAVES, int U, int TERMS = 1>
 void launch_mxfp4_k(const GemvArgs& a, int64_t batch, hipStream_t st) {
   dim3 grid((unsigned)ceil_div(a.N, 16 * T), (unsigned)batch);
-  hipLaunchKernelGGL((gemv_mxfp4_kernel<T, WAVES, U>), grid, dim3(kWave * WAVES), 0, st, a);
+  hipLaunchKernelGGL((gemv_mxfp4_kernel<T, WAVES, U, TERMS>), grid, dim3(kWave * WAVES), 0, st, a);
+}
+
+template <int TERMS>
+void launch_mxfp4_terms(const GemvArgs& a, int64_t batch, int t, int waves, hipStream_t st) {
+  if (t == 2) waves == 8 ? launch_mxfp4_k<2, 8, 2, TERMS>(a, batch, st) : launch_mxfp4_k<2, 4, 2, TERMS>(a, batch, st);
+  else waves == 8 ? launch_mxfp4_k<1, 8, 2, TERMS>(a, batch, st) : launch_mxfp4_k<1, 4, 2, TERMS>(a, batch, st);
 }
 
 void launch_mxfp4(const GemvArgs& a, int64_t batch, Geometry g, hipStream_t st) {
@@ -533,6 +615,43 @@ bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab
     return false;
   if (mode == QMM_MODE_MXFP4 && skinny2_mx_supported(N, K, s, products)) return false;
   return true;
+}
+
+// float16 / float32 rows that the MXFP4 kernel above takes as they are: 16-byte loads,
+// and no staged kernel for the shape (those read bf16 terms).
+bool gemv_terms_supported(const void* x, int64_t N, int64_t K, int mode, const void* s, int64_t products) {
+  return mode == QMM_MODE_MXFP4 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && !skinny2_mx_supported(N, K, s, products);
+}
+
+// ... dense (rhs_idx null), a pair a batch entry, or the sorted pairs of `segments`.
+void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
+                         int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
+                         const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,
+                         int64_t x_rows, hipStream_t st) {
+  GemvArgs a;
+  a.x = static_cast<const uint16_t*>(x);
+  a.w = static_cast<const uint32_t*>(w);
+  a.s = s;
+  a.b = nullptr;
+  a.y = y;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.gshift = 0;
+  a.y_dtype = y_dtype;
+  a.lhs_idx = lhs_idx;
+  a.rhs_idx = rhs_idx;
+  a.n_experts = (int)n_experts;
+  a.n_xrows = (int)x_rows;
+  a.segments = segments;
+  a.src_row = src_row;
+  a.out_row = out_row;
+  a.x_rows = (int)x_rows;
+  int t, waves;
+  // (as wide as the terms' rows would be: the sums then meet as they did)
+  gemv_geometry(segments ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
+  if (x_dtype == QMM_F32) launch_mxfp4_terms<3>(a, batch, t, waves, st);
+  else launch_mxfp4_terms<2>(a, batch, t, waves, st);
 }
 
 // Expert-indexed pairs sorted by expert (segments / src_row / out_row as the
