@@ -37,7 +37,6 @@ void gemm_dispatch(const void* x, const void* w, const void* s, const void* b, i
 int64_t gemm_row_tile(int64_t R, int64_t E);
 bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab, const void* s, const void* b,
                        int64_t products);
-bool gemv_terms_supported(const void* x, int64_t N, int64_t K, int mode, const void* s, int64_t products);
 void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
                          int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
                          const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,
@@ -376,10 +375,13 @@ bool sorted_here_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int 
 // 110, 64 pairs 109 against 216; on 128 experts: 32 pairs 128 against 110,
 // 64 pairs 194 against 217; 8 experts of [4096, 11008] with four-bit
 // codes: 16 pairs 108 against 206 us, 32 pairs 110 against 397.)
+bool sorts_general(int64_t P, int64_t E, size_t workspace_bytes) {
+  return P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace_bytes >= route_bytes_segments(P, E);
+}
+
 bool grouped_general_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                             const void* s, const void* b, size_t workspace_bytes) {
-  return P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace_bytes >= route_bytes_segments(P, E) &&
-         gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E) && !experiment_env("QMM_NO_GROUPED_GEMV");
+  return sorts_general(P, E, workspace_bytes) && gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E) && !experiment_env("QMM_NO_GROUPED_GEMV");
 }
 
 // ---- float16 / float32 activations ---------------------------------------------
@@ -390,6 +392,37 @@ bool grouped_general_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, 
 // output type.  In the dense decode case the terms ride as extra rows of the
 // same launch (terms x M <= 16: the weight is still streamed once).
 int act_terms(int x_dtype) { return x_dtype == QMM_F32 ? 3 : x_dtype == QMM_F16 ? 2 : 1; }
+
+// The general MXFP4 decode kernel splits the rows itself, one launch where the
+// loader-wavefront kernel needs the split and the sum round it (three, and one or two a
+// term for pairs that it sorts); but it reads the weight more slowly.  By the bytes that
+// it would stream, then (us, float32, here / there):
+//   rows, pairs of their own: 4096 x 4096 9.3 / 13.2, two pairs of it 14.2 / 14.0, 8 of
+//   1024 x 2048 9.7 / 14.0, 32 of 16 experts of it (19 MB) 17.7 / 15.5, 4096 x 11008 21.3 / 13.9;
+//   64 pairs of 16 experts of 1024 x 2048 (21 MB, a third of what pairs of their own
+//   stream) 19.2 / 32.7;
+//   sorted pairs: 8 of 32 experts of 2880 x 2880 (33 MB) 26.4 / 35.6, 64 of 8 of 2880 x
+//   1088 22.0 / 36.8, 8 of 8 of 4096 x 4096 (67 MB) 45.4 / 39.0;
+//   past 64 pairs, against the row-group kernels: 78 of 8 of 1024 x 1024 (6.3 MB) 11.7 /
+//   15.4 (float16 11.0 / 14.3), 128 of it (8.4) 15.5 / 15.7 (11.4 / 16.3), 78 of 8 of 2880 x
+//   1088 (19) 23.5 / 17.5; a K that is no multiple of 64 has only a product a term there:
+//   128 of 8 of 512 x 288 11.3 / 66.3.
+constexpr int64_t kTermsBytes = 12 << 20, kTermsBytesMost = 34 << 20, kTermsBytesManyPairs = 18 << 20;
+
+bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
+                     const void* s, const void* b, size_t workspace_bytes) {
+  if (mode != QMM_MODE_MXFP4 || !aligned16(x) || P <= 0 || E > 65535 || N > INT32_MAX || K > INT32_MAX || N * K >= (1ll << 40))
+    return false;
+  const bool sorted = sorts_general(P, E, workspace_bytes);
+  if (P > kGatherGemvMaxPairs && !sorted) return false;
+  const int64_t bytes = (sorted ? skinny2_max_segments(P, E) : P) * (N * K / 2);
+  if (P > kGatherGemvMaxPairs) return terms * bytes <= kTermsBytesManyPairs || (K % 64 && bytes <= kTermsBytesMost);
+  if (gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E)) return true;
+  if (sorted_here_serves(P, E, N, K, gs, bits, mode, tab, s, b) ||
+      grouped_decode_serves(P, E, N, K, gs, bits, mode, tab, s, b, workspace_bytes))
+    return bytes <= kTermsBytesMost;
+  return bytes <= kTermsBytes || (bytes <= kTermsBytesMost && P * (N * K / 2) >= 3 * bytes);
+}
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
@@ -874,7 +907,8 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc;
-  if (terms * M <= kGemvMaxM && batch <= 65535 && N <= INT32_MAX && y && gemv_terms_supported(x, N, K, mode, scales, batch)) {
+  if (terms * M <= kGemvMaxM && batch <= 65535 && N <= INT32_MAX && y && mode == QMM_MODE_MXFP4 &&
+      (gemv_runs_general(N, K, group_size, bits, mode, table_dtype, scales, biases, batch) || N * K / 2 <= kTermsBytes / batch)) {
     // (the general MXFP4 decode kernel splits them itself)
     rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (rc) return rc;
@@ -973,10 +1007,12 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   // 1.6e-3 from the product of the exact weights, 128 pairs over 8 experts of 1024 x
   // 4096, eight-bit codes; four-bit ones 4e-7).  MXFP4 weights are exact in both.
   const int own = short_terms(x_dtype, table_dtype, group_size, mode);
+  const size_t inner = gather_scratch(P, E, N, K, true);
+  const bool in_kernel = terms_in_kernel(x, terms, P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner);
   const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
-  if (!exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
+  if (!in_kernel && !exact_decode && P > kGatherGemvMaxPairs && P <= INT32_MAX / 2 && E > 0 && E <= 65535 && workspace && aligned16(workspace) &&
       workspace_bytes >= route_bytes(P, E) + short_prep_bytes(P, K, own) &&
       workspace_bytes >= term_bytes(terms, P, N, K) + gather_scratch(P, E, N, K, true) &&
       short_wins(P, E, N, K, bits, mode, terms, own, true, workspace_bytes - route_bytes(P, E)) &&
@@ -999,23 +1035,19 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   // the pairs' rows are gathered while they are split; every term is then a
   // gathered product over rows already in pair order
   const size_t xs = align256((size_t)(terms * P * K) * 2), ps = align256((size_t)(terms * P * N) * 4);
-  const size_t inner = gather_scratch(P, E, N, K, true);
   if (!workspace || workspace_bytes < xs + ps + inner || !aligned16(workspace))
     return fail(QMM_ERR_WORKSPACE, "float16 / float32 activations need %zu aligned workspace bytes, got %zu",
                 xs + ps + inner, workspace ? workspace_bytes : (size_t)0);
   if (terms * P * K >= (1ll << 30)) return fail(QMM_ERR_BAD_SHAPE, "shape exceeds kernel index range");
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // What the general MXFP4 decode kernel serves: it splits the rows itself.  One launch
-  // instead of three for pairs of their own, two instead of eight for sorted ones.
-  if (P <= kGatherGemvMaxPairs && E <= 65535 && N <= INT32_MAX && K <= INT32_MAX &&
-      gemv_terms_supported(x, N, K, mode, scales, std::max(P, E)) &&
-      !sorted_here_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases) &&
-      !grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
+  // The general MXFP4 decode kernel splits the rows itself: one launch for pairs of their
+  // own, two for sorted ones.
+  if (in_kernel) {
     int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);
     if (rc) return rc;
-    if (!grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
+    if (!sorts_general(P, E, inner)) {
       gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, P, 1, N, K, lhs_idx, rhs_idx, nullptr, nullptr, nullptr, E, T, st);
       return check_launch("gather gemv launch");
     }

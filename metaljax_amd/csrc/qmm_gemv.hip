@@ -289,7 +289,7 @@ __device__ __forceinline__ void operand_terms(const u32x4* raw, bf16x8* out) {
 // TERMS: 1 for bf16 rows of x; float16 (2) and float32 (3) ones are split into that
 // many bf16 terms as they arrive (what split_terms_kernel writes), a weight operand
 // meets a term after the other, each with its own accumulator, and the terms' sums are
-// added largest first.  A product of a few rows is bound by its launches, and the split
+// added smallest first.  A product of a few rows is bound by its launches, and the split
 // and the sum were two of three (sorted pairs: five of eight; us a call, float32 /
 // float16, before -> now: 6 pairs over 8 experts of 1024 x 1024 12.5 / 12.1 -> 8.3 / 7.9,
 // 24 pairs 29.7 / 21.3 -> 10.9 / 10.7, 64 over 8 of 2048 x 512 34.0 / 24.0 -> 12.3 / 11.1,
@@ -418,11 +418,15 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
     const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
     float v = 0.f;
 #pragma unroll
-    for (int term = 0; term < TERMS; ++term) {
-      float part = 0.f;
+    for (int term = TERMS - 1; term >= 0; --term) {              // (smallest first: one rounding at full size)
+      float part[WAVES];                                           // (in pairs: fewer roundings in a row)
 #pragma unroll
-      for (int wv = 0; wv < WAVES; ++wv) part += red[term][wv][t][i][l];
-      v = term ? v + part : part;
+      for (int wv = 0; wv < WAVES; ++wv) part[wv] = red[term][wv][t][i][l];
+#pragma unroll
+      for (int d = 1; d < WAVES; d *= 2)
+#pragma unroll
+        for (int wv = 0; wv < WAVES; wv += 2 * d) part[wv] += part[wv + d];
+      v = term == TERMS - 1 ? part[0] : v + part[0];
     }
     const int m = 4 * (l >> 4) + i;
     const int64_t n = n0 + t * 16 + (l & 15);
@@ -617,13 +621,7 @@ bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab
   return true;
 }
 
-// float16 / float32 rows that the MXFP4 kernel above takes as they are: 16-byte loads,
-// and no staged kernel for the shape (those read bf16 terms).
-bool gemv_terms_supported(const void* x, int64_t N, int64_t K, int mode, const void* s, int64_t products) {
-  return mode == QMM_MODE_MXFP4 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && !skinny2_mx_supported(N, K, s, products);
-}
-
-// ... dense (rhs_idx null), a pair a batch entry, or the sorted pairs of `segments`.
+// float16 / float32 rows on a 16-byte address, as the MXFP4 kernel above takes them: dense (rhs_idx null), a pair a batch entry, or the sorted pairs of `segments`.
 void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
                          int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
                          const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,

@@ -1,10 +1,11 @@
 """float16 / float32 rows that the general MXFP4 decode kernel splits into bf16 terms as
 they arrive: the same numbers, bit for bit, as the terms multiplied one by one and added
-largest first (every sum meets in the same order), for products of a few rows, batches,
+smallest first (every sum meets in the same order), for products of a few rows, batches,
 pairs of their own and sorted ones; contractions of less than a chunk of 128 to several a
 wavefront, columns that end inside a tile, rows and experts that are out of range, rows
 that hold infinities, NaNs and the smallest values.  Rows that start between two 16-byte
-addresses take the split as a launch of its own and give the same."""
+addresses take the split as a launch of its own and give the same but for the order of
+three terms' sums."""
 
 import pytest
 import torch
@@ -45,7 +46,7 @@ def bf16_terms(x):
 
 def total(parts):
     y = None
-    for p in parts:
+    for p in reversed(list(parts)):
         y = p if y is None else y + p
     return y
 
@@ -75,11 +76,36 @@ def test_pairs(pairs, e, n, k, act):
     half = K.gather_qmm(x, w, s, None, lhs, rhs, out_dtype=torch.float16, **HOW)
     assert same(half[live], got[live].half())
     apart = torch.empty(x.numel() + 2, dtype=x.dtype, device=DEV)[2:].view(x.shape).copy_(x)
-    assert same(K.gather_qmm(apart, w, s, None, lhs, rhs, out_dtype=torch.float32, **HOW)[live], got[live])
+    apart = K.gather_qmm(apart, w, s, None, lhs, rhs, out_dtype=torch.float32, **HOW)[live]
+    sound = got[live].isfinite()
+    assert same(apart.masked_fill(sound, 0), got[live].masked_fill(sound, 0))
+    apart, there = apart[sound].double(), got[live][sound].double()
+    assert (apart - there).norm() <= 2.0 ** -23 * there.norm()           # (two roundings each)
     few = min(pairs, 11)
     own = K.gather_qmm(x[:few], w, s, None, None, rhs[:few], out_dtype=torch.float32, **HOW)
     want = total(K.gather_qmm(t, w, s, None, None, rhs[:few], out_dtype=torch.float32, **HOW) for t in bf16_terms(x[:few]))
     assert same(own[live[:few]], want[live[:few]])
+
+
+# where the general kernel is the faster one although a staged one serves the shape: sizes on both sides of the rules
+@pytest.mark.parametrize("act", ["f16", "f32"])
+@pytest.mark.parametrize("pairs,e,n,k", [(1, 2, 4096, 4096), (3, 2, 4096, 4096), (5, 4, 352, 1216), (20, 4, 352, 1216), (30, 8, 2880, 1088),
+                                         (40, 16, 1024, 2048), (64, 16, 1024, 2048), (8, 9, 2880, 2880), (9, 9, 2880, 2880),
+                                         # past 64 pairs
+                                         (65, 8, 512, 288), (78, 8, 384, 576), (128, 8, 600, 288), (129, 8, 600, 288), (200, 16, 1024, 1024)])
+def test_pairs_of_staged_shapes(pairs, e, n, k, act):
+    g = torch.Generator(device=DEV).manual_seed(pairs + k)
+    w, s = weight(g, (e,), n, k)
+    s[:, 0, 0] = 120
+    x = torch.randn((pairs, k), device=DEV, generator=g).to(ACT[act])
+    rhs = torch.randint(0, e, (pairs,), device=DEV, generator=g, dtype=torch.int32)
+    y = K.gather_qmm(x, w, s, None, None, rhs, out_dtype=torch.float32, **HOW)
+    want = torch.empty((pairs, n), dtype=torch.float64, device=DEV)
+    for i in range(e):
+        want[rhs == i] = x[rhs == i].double() @ K.dequantize(w[i], s[i], None, out_dtype=torch.float32, **HOW).double().T
+    # exact products, a rounding (or cut) of 2^-23 at most an instruction of 32 products, a wavefront and a term
+    err = ((y.double() - want).norm() / want.norm()).item()
+    assert err <= 2.0 ** -23 * (k / 32 + 11) ** 0.5, err
 
 
 @pytest.mark.parametrize("act", ["f16", "f32"])
