@@ -40,10 +40,11 @@ bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab
 void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
                          int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
                          const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,
-                         int64_t x_rows, hipStream_t st);
+                         int64_t x_rows, int pairs_here, hipStream_t st);
 void gemv_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                            int y_dtype, const int32_t* segments, const int32_t* src_row,
-                           const int32_t* out_row, int64_t max_segments, int64_t x_rows, int64_t N,
+                           const int32_t* out_row, const int32_t* lhs_idx, const int32_t* rhs_idx, int64_t pairs,
+                           int64_t n_experts, int64_t max_segments, int64_t x_rows, int64_t N,
                            int64_t K, int gs, int bits, int mode, hipStream_t st);
 bool gemm2_supported(int64_t R, int64_t N, int64_t K);
 size_t gemm2_workspace_bytes(int64_t R, int64_t K);
@@ -377,6 +378,16 @@ bool sorted_here_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int 
 // codes: 16 pairs 108 against 206 us, 32 pairs 110 against 397.)
 bool sorts_general(int64_t P, int64_t E, size_t workspace_bytes) {
   return P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace_bytes >= route_bytes_segments(P, E);
+}
+
+// The general kernels sort up to 64 pairs themselves: a few instructions an expert that
+// occurs, in every workgroup, against a launch ahead of the product.  By how many there
+// are of both (us, here / behind the launch: 64 pairs over 8 experts of 1024 x 1024, 9200,
+// 8.4 / 11.5, over 8 of 6528 x 1024, 58750, 27.3 / 29.2, 16 over 32 of 2048 x 992, 37000, 12.0 / 13.8,
+// 24 of it, 80000, 15.8 / 15.8, 32 of it, 148000, 21.6 / 19.1; MXFP4, bf16 activations).
+bool sorts_itself(int64_t P, int64_t E, int64_t N) {
+  const int64_t segments = skinny2_max_segments(P, E);
+  return P <= kGatherGemvMaxPairs && segments * segments * ((N + 15) / 16) <= (1 << 16);
 }
 
 bool grouped_general_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
@@ -816,6 +827,11 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
   }
   if (P <= kGatherGemvMaxPairs) {
     if (workspace && grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, workspace_bytes)) {
+      if (sorts_itself(P, E, N)) {
+        gemv_grouped_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, nullptr, nullptr, nullptr, lhs_idx, rhs_idx, P, E,
+                              skinny2_max_segments(P, E), T, N, K, group_size, bits, mode, st);
+        return check_launch("grouped gemv launch");
+      }
       int32_t* ro = static_cast<int32_t*>(workspace);
       int32_t* cursor = ro + E + 1;
       int32_t* src_row = cursor + E;
@@ -824,7 +840,7 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
       route(lhs_idx, rhs_idx, P, E, ro, cursor, src_row, out_row, segments, st);
       rc = check_launch("route launch");
       if (rc) return rc;
-      gemv_grouped_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, segments, src_row, out_row,
+      gemv_grouped_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, segments, src_row, out_row, nullptr, nullptr, 0, E,
                             skinny2_max_segments(P, E), T, N, K, group_size, bits, mode, st);
       return check_launch("grouped gemv launch");
     }
@@ -913,7 +929,7 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
     rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (rc) return rc;
     gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, batch, M, N, K, nullptr, nullptr, nullptr, nullptr, nullptr,
-                        0, 0, st);
+                        0, 0, 0, st);
     return check_launch("gemv launch");
   }
   split_terms_dispatch(x, x_dtype, ws, batch, M, K, nullptr, -1, st);
@@ -1048,8 +1064,13 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
     if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);
     if (rc) return rc;
     if (!sorts_general(P, E, inner)) {
-      gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, P, 1, N, K, lhs_idx, rhs_idx, nullptr, nullptr, nullptr, E, T, st);
+      gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, P, 1, N, K, lhs_idx, rhs_idx, nullptr, nullptr, nullptr, E, T, 0, st);
       return check_launch("gather gemv launch");
+    }
+    if (sorts_itself(P, E, N)) {
+      gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, skinny2_max_segments(P, E), 16, N, K, lhs_idx, rhs_idx, nullptr,
+                          nullptr, nullptr, E, T, (int)P, st);
+      return check_launch("grouped gemv launch");
     }
     int32_t* ro = reinterpret_cast<int32_t*>(ws);
     int32_t* cursor = ro + E + 1;
@@ -1060,7 +1081,7 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
     rc = check_launch("route launch");
     if (rc) return rc;
     gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, skinny2_max_segments(P, E), 16, N, K, nullptr, nullptr, segments,
-                        src_row, out_row, E, T, st);
+                        src_row, out_row, E, T, 0, st);
     return check_launch("grouped gemv launch");
   }
   // Pairs that are decode products of their own: the terms are the rows of one (terms

@@ -35,6 +35,37 @@ namespace qmm {
 
 namespace {
 
+// The rows of a workgroup, for up to 64 pairs that nobody has sorted: every wavefront
+// holds the pairs' experts, one a lane, and goes through those that occur in order of
+// their first pair; each takes a row of workgroups per sixteen of its pairs.  Leaves the
+// pairs of segment z in rows[wave][] and returns how many there are (0: no such segment;
+// the same for the whole workgroup).  A few instructions an expert; the sort is a launch
+// of its own otherwise: 64 pairs over 8 experts of 1024 x 1024 11.5 -> 8.4 us, four-bit or
+// eight-bit codes or MXFP4 (the host takes 8 a call), the three terms of float32 rows
+// over affine codes 33 -> 24.
+__device__ __forceinline__ int take_segment(const GemvArgs& a, int z, int lane, int* rows, int64_t& expert) {
+  int e = -1;
+  if (lane < a.x_rows) e = a.rhs_idx[lane];
+  uint64_t left = __ballot(e >= 0 && e < a.n_experts);
+  while (left) {
+    const int of = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+    const uint64_t same = __ballot(e == of);
+    const int n = __popcll(same), segments = (n + 15) / 16;
+    if (z < segments) {
+      const int at = __popcll(same & ((1ull << lane) - 1)) - 16 * z;
+      if (e == of && at >= 0 && at < 16) rows[at] = lane;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      expert = of;
+      return n - 16 * z < 16 ? n - 16 * z : 16;
+    }
+    z -= segments;
+    left &= ~same;
+  }
+  return 0;
+}
+
 // Affine kernel.  BITS: 4 or 8.  CH: K-chunk per scale application (64, or 32
 // for group size 32).  T: 16-row tiles per wavefront.  WAVES: K slices per
 // workgroup.  U: chunks whose loads are all issued before any is consumed --
@@ -57,6 +88,7 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
   constexpr int ROWS = 16 * T;
   constexpr int TABSZ = (TAB == QMM_F32) ? 4 : 2;
   __shared__ float red[WAVES][T][4][kWave];
+  __shared__ int taken[WAVES][16];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -66,8 +98,9 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
   const int64_t wpr = (int64_t)a.K * BITS / 32;             // words per weight row
   const int64_t ng = (int64_t)((a.K / CH) >> a.gshift);     // table entries per row
 
-  int64_t xz = a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
-  int64_t wz = a.rhs_idx ? (int64_t)a.rhs_idx[bz] : bz;
+  const bool here = !a.segments && a.x_rows;        // x_rows pairs, sorted by this kernel
+  int64_t xz = a.lhs_idx && !here ? (int64_t)a.lhs_idx[bz] : bz;
+  int64_t wz = a.rhs_idx && !here ? (int64_t)a.rhs_idx[bz] : bz;
   bool x_ok = true;
   int M = a.M, seg_lo = 0;
   if (a.segments) {                                 // grouped form: up to 16 sorted pairs of one expert
@@ -76,11 +109,16 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
     seg_lo = a.segments[2 + 3 * bz];
     M = a.segments[3 + 3 * bz];
     xz = 0;
+  } else if (here) {
+    M = take_segment(a, (int)bz, lane, taken[wave], wz);
+    if (M == 0) return;                             // uniform, before any barrier
+    xz = 0;
   } else if (a.rhs_idx) {                           // gather form: indices are data
     if (wz < 0 || wz >= a.n_experts) return;        // uniform, before any barrier
     if (xz < 0 || xz >= a.n_xrows) { xz = 0; x_ok = false; }
   }
   const auto rx = a.segments ? make_rsrc(a.x, (int64_t)a.x_rows * a.K * 2)
+                  : here     ? make_rsrc(a.x, (int64_t)a.n_xrows * a.K * 2)
                              : make_rsrc(a.x + xz * a.M * (int64_t)a.K, x_ok ? (int64_t)a.M * a.K * 2 : 0);
   const auto rw = make_rsrc(a.w + wz * a.N * wpr, a.N * wpr * 4);
   const auto rs = make_rsrc(static_cast<const char*>(a.s) + wz * a.N * ng * TABSZ, a.N * ng * TABSZ);
@@ -102,6 +140,10 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
   if (a.segments && r < M) {                        // row r of the segment is row src_row[first + r] of x
     const int64_t src = a.src_row[seg_lo + r];
     xoff = src >= 0 && src < a.x_rows ? (uint32_t)((src * a.K + kg * (CH / 4)) * 2) : kOutOfRange;
+  }
+  if (here && r < M) {
+    const int64_t pair = taken[wave][r], src = a.lhs_idx ? (int64_t)a.lhs_idx[pair] : pair;
+    xoff = src >= 0 && src < a.n_xrows ? (uint32_t)((src * a.K + kg * (CH / 4)) * 2) : kOutOfRange;
   }
 
   f32x4 acc[T];
@@ -228,6 +270,7 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_affine_kernel(GemvArgs a) {
     if (m < M && n < a.N) {
       int64_t orow = bz * a.M + m;
       if (a.segments) orow = a.out_row[seg_lo + m];
+      else if (here) orow = taken[wave][m];
       if (orow >= 0) store_out(a.y, orow * (int64_t)a.N + n, v, a.y_dtype);
     }
   }
@@ -301,6 +344,7 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
   constexpr int ROWS = 16 * T;
   constexpr int XW = TERMS == 3 ? 2 : 1;           // 16-byte pieces of eight activations
   __shared__ float red[TERMS][WAVES][T][4][kWave];
+  __shared__ int taken[WAVES][16];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -310,8 +354,9 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
   const int64_t wpr = (int64_t)a.K / 8;
   const int nblk = a.K / 32;                       // MX blocks per row
 
-  int64_t xz = a.lhs_idx ? (int64_t)a.lhs_idx[bz] : bz;
-  int64_t wz = a.rhs_idx ? (int64_t)a.rhs_idx[bz] : bz;
+  const bool here = !a.segments && a.x_rows;        // x_rows pairs, sorted by this kernel
+  int64_t xz = a.lhs_idx && !here ? (int64_t)a.lhs_idx[bz] : bz;
+  int64_t wz = a.rhs_idx && !here ? (int64_t)a.rhs_idx[bz] : bz;
   bool x_ok = true;
   int M = a.M, seg_lo = 0;
   if (a.segments) {                                 // grouped form: up to 16 sorted pairs of one expert
@@ -319,6 +364,10 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
     wz = a.segments[1 + 3 * bz];
     seg_lo = a.segments[2 + 3 * bz];
     M = a.segments[3 + 3 * bz];
+    xz = 0;
+  } else if (here) {
+    M = take_segment(a, (int)bz, lane, taken[wave], wz);
+    if (M == 0) return;                             // uniform, before any barrier
     xz = 0;
   } else if (a.rhs_idx) {                           // gather form: indices are data
     if (wz < 0 || wz >= a.n_experts) return;        // uniform, before any barrier
@@ -346,6 +395,11 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
   if (a.segments) {                                 // row r of the segment is row src_row[first + r] of x
     const int64_t src = r < M ? (int64_t)a.src_row[seg_lo + r] : -1;
     xvalid = src >= 0 && src < a.x_rows;
+    xrow = a.x + (xvalid ? src : 0) * a.K * XW;
+  }
+  if (here) {
+    const int64_t pair = r < M ? taken[wave][r] : -1, src = pair < 0 ? -1 : a.lhs_idx ? (int64_t)a.lhs_idx[pair] : pair;
+    xvalid = src >= 0 && src < a.n_xrows;
     xrow = a.x + (xvalid ? src : 0) * a.K * XW;
   }
 
@@ -433,6 +487,7 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_mxfp4_kernel(GemvArgs a) {
     if (m < M && n < a.N) {
       int64_t orow = bz * a.M + m;
       if (a.segments) orow = a.out_row[seg_lo + m];
+      else if (here) orow = taken[wave][m];
       if (orow >= 0) store_out(a.y, orow * (int64_t)a.N + n, v, a.y_dtype);
     }
   }
@@ -621,11 +676,12 @@ bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab
   return true;
 }
 
-// float16 / float32 rows on a 16-byte address, as the MXFP4 kernel above takes them: dense (rhs_idx null), a pair a batch entry, or the sorted pairs of `segments`.
+// float16 / float32 rows on a 16-byte address, as the MXFP4 kernel above takes them: dense (rhs_idx null), a pair a batch
+// entry, the sorted pairs of `segments`, or `pairs_here` pairs that the kernel sorts.
 void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
                          int64_t M, int64_t N, int64_t K, const int32_t* lhs_idx, const int32_t* rhs_idx,
                          const int32_t* segments, const int32_t* src_row, const int32_t* out_row, int64_t n_experts,
-                         int64_t x_rows, hipStream_t st) {
+                         int64_t x_rows, int pairs_here, hipStream_t st) {
   GemvArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.w = static_cast<const uint32_t*>(w);
@@ -644,22 +700,23 @@ void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* 
   a.segments = segments;
   a.src_row = src_row;
   a.out_row = out_row;
-  a.x_rows = (int)x_rows;
+  a.x_rows = segments ? (int)x_rows : pairs_here;
   int t, waves;
   // (as wide as the terms' rows would be: the sums then meet as they did)
-  gemv_geometry(segments ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
+  gemv_geometry(segments || pairs_here ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
   if (x_dtype == QMM_F32) launch_mxfp4_terms<3>(a, batch, t, waves, st);
   else launch_mxfp4_terms<2>(a, batch, t, waves, st);
 }
 
 // Expert-indexed pairs sorted by expert (segments / src_row / out_row as the
-// routing pass writes them) on the general kernels: one decode product per
+// routing pass writes them; null: up to 64 `pairs` that the kernel sorts) on the general kernels: one decode product per
 // expert and sixteen pairs, so that an expert's weights are read once for all
 // of its pairs instead of once per pair.  `max_segments` rows of workgroups
 // are launched; the ones past the list's count exit at once.
 void gemv_grouped_dispatch(const void* x, const void* w, const void* s, const void* b, int tab, void* y,
                            int y_dtype, const int32_t* segments, const int32_t* src_row,
-                           const int32_t* out_row, int64_t max_segments, int64_t x_rows, int64_t N,
+                           const int32_t* out_row, const int32_t* lhs_idx, const int32_t* rhs_idx, int64_t pairs,
+                           int64_t n_experts, int64_t max_segments, int64_t x_rows, int64_t N,
                            int64_t K, int gs, int bits, int mode, hipStream_t st) {
   GemvArgs a;
   a.x = static_cast<const uint16_t*>(x);
@@ -671,12 +728,14 @@ void gemv_grouped_dispatch(const void* x, const void* w, const void* s, const vo
   a.N = (int)N;
   a.K = (int)K;
   a.y_dtype = y_dtype;
-  a.lhs_idx = nullptr;
-  a.rhs_idx = nullptr;
+  a.lhs_idx = segments ? nullptr : lhs_idx;
+  a.rhs_idx = segments ? nullptr : rhs_idx;
   a.segments = segments;
   a.src_row = src_row;
   a.out_row = out_row;
-  a.x_rows = (int)x_rows;
+  a.n_experts = (int)n_experts;
+  a.n_xrows = (int)x_rows;
+  a.x_rows = (int)(segments ? x_rows : pairs);
   Geometry g;
   gemv_geometry(16, N, K, &g.t, &g.waves);
   if (mode == QMM_MODE_MXFP4) {

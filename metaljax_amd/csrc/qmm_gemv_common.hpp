@@ -66,7 +66,8 @@ struct GemvArgs {
   // blockIdx.y takes segment y of `segments` ([0] = count, then (expert, first
   // sorted position, rows <= 16) triples): it multiplies the rows
   // x[src_row[first + r]] by w[expert] and stores row r at y[out_row[first + r]];
-  // x has x_rows rows
+  // x has x_rows rows.  (General kernels, no segments: x_rows > 0 is the number of
+  // pairs, at most 64, that the kernel sorts by itself.)
   const int32_t* segments = nullptr;
   const int32_t* src_row = nullptr;
   const int32_t* out_row = nullptr;
