@@ -380,6 +380,20 @@ bool sorts_general(int64_t P, int64_t E, size_t workspace_bytes) {
   return P >= 16 && 2 * P >= E && grouped_decode_pairs(P, E) && workspace_bytes >= route_bytes_segments(P, E);
 }
 
+// More pairs whose K is no multiple of 64 (groups of 32): neither the re-laying kernels
+// nor the short-group one takes them, and the row-group kernel that does walks K in a
+// workgroup a tile.  The general decode kernels behind a sort's launch read an expert's
+// weight once for sixteen of its pairs (us, here / on row groups; 8 experts of 4096 x 992,
+// four-bit affine codes: 65 pairs 22 / 53, 256 46 / 61, 512 80 / 69, 16 of 1024 x 480:
+// 512 pairs 23.9 / 23.4; MXFP4: 65 17 / 76, 512 60 / 93, 1024 109 / 129, float32 rows in one
+// launch instead of one a term and more 23 / 233, 102 / 299, 189 / 423).
+constexpr int64_t kOddPairs = 2048;
+
+bool sorts_odd(int64_t P, int64_t E, int64_t N, int64_t K, int mode, size_t workspace_bytes) {
+  return P > kGatherGemvMaxPairs && P <= kOddPairs && P <= (mode == QMM_MODE_MXFP4 ? 64 : 24) * E && K % 64 != 0 && E <= 65535 &&
+         N <= INT32_MAX && K <= INT32_MAX && workspace_bytes >= route_bytes_segments(P, E);
+}
+
 // The general kernels sort up to 64 pairs themselves: a few instructions an expert that
 // occurs, in every workgroup, against a launch ahead of the product.  By how many there
 // are of both (us, here / behind the launch: 64 pairs over 8 experts of 1024 x 1024, 9200,
@@ -416,8 +430,7 @@ int act_terms(int x_dtype) { return x_dtype == QMM_F32 ? 3 : x_dtype == QMM_F16 
 //   1088 22.0 / 36.8, 8 of 8 of 4096 x 4096 (67 MB) 45.4 / 39.0;
 //   past 64 pairs, against the row-group kernels: 78 of 8 of 1024 x 1024 (6.3 MB) 11.7 /
 //   15.4 (float16 11.0 / 14.3), 128 of it (8.4) 15.5 / 15.7 (11.4 / 16.3), 78 of 8 of 2880 x
-//   1088 (19) 23.5 / 17.5; a K that is no multiple of 64 has only a product a term there:
-//   128 of 8 of 512 x 288 11.3 / 66.3.
+//   1088 (19) 23.5 / 17.5 (a K that is no multiple of 64: sorts_odd).
 constexpr int64_t kTermsBytes = 12 << 20, kTermsBytesMost = 34 << 20, kTermsBytesManyPairs = 18 << 20;
 
 bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
@@ -427,7 +440,7 @@ bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, 
   const bool sorted = sorts_general(P, E, workspace_bytes);
   if (P > kGatherGemvMaxPairs && !sorted) return false;
   const int64_t bytes = (sorted ? skinny2_max_segments(P, E) : P) * (N * K / 2);
-  if (P > kGatherGemvMaxPairs) return terms * bytes <= kTermsBytesManyPairs || (K % 64 && bytes <= kTermsBytesMost);
+  if (P > kGatherGemvMaxPairs) return terms * bytes <= kTermsBytesManyPairs;
   if (gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E)) return true;
   if (sorted_here_serves(P, E, N, K, gs, bits, mode, tab, s, b) ||
       grouped_decode_serves(P, E, N, K, gs, bits, mode, tab, s, b, workspace_bytes))
@@ -576,8 +589,9 @@ size_t qmm_gather_workspace_bytes(int64_t P, int64_t E, int64_t N, int64_t K, in
   const size_t least = gather_minimum(P, E, N, K, x_dtype);
   if (P <= kGatherGemvMaxPairs) return least;
   const int terms = act_terms(x_dtype);
-  const size_t sums = route_bytes(P, E) + std::max(short_scratch(P, N, K, 4, QMM_MODE_AFFINE, terms),
-                                                   short_scratch(P, N, K, 8, QMM_MODE_AFFINE, terms));
+  size_t sums = route_bytes(P, E) + std::max(short_scratch(P, N, K, 4, QMM_MODE_AFFINE, terms),
+                                             short_scratch(P, N, K, 8, QMM_MODE_AFFINE, terms));
+  if (K % 64 != 0 && P <= kOddPairs) sums = std::max(sums, route_bytes_segments(P, E));
   return std::max(least, std::min(sums, (size_t)QMM_STATIC_SCRATCH_BYTES));
 }
 
@@ -848,6 +862,19 @@ static int gather_bf16(const void* x, int x_dtype, const void* w, const void* sc
                   mode, lhs_idx, rhs_idx, E, T, st);
     return check_launch("gather gemv launch");
   }
+  if (workspace && sorts_odd(P, E, N, K, mode, workspace_bytes)) {
+    int32_t* ro = static_cast<int32_t*>(workspace);
+    int32_t* cursor = ro + E + 1;
+    int32_t* src_row = cursor + E;
+    int32_t* out_row = src_row + P;
+    int32_t* segments = out_row + P;
+    route(lhs_idx, rhs_idx, P, E, ro, cursor, src_row, out_row, segments, st);
+    rc = check_launch("route launch");
+    if (rc) return rc;
+    gemv_grouped_dispatch(x, w, scales, biases, table_dtype, y, y_dtype, segments, src_row, out_row, nullptr, nullptr, 0, E,
+                          skinny2_max_segments(P, E), T, N, K, group_size, bits, mode, st);
+    return check_launch("grouped gemv launch");
+  }
   const size_t need = route_bytes(P, E);
   if (!workspace || workspace_bytes < need)
     return fail(QMM_ERR_WORKSPACE, "gather_qmm needs %zu workspace bytes, got %zu", need,
@@ -1024,7 +1051,9 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   // 4096, eight-bit codes; four-bit ones 4e-7).  MXFP4 weights are exact in both.
   const int own = short_terms(x_dtype, table_dtype, group_size, mode);
   const size_t inner = gather_scratch(P, E, N, K, true);
-  const bool in_kernel = terms_in_kernel(x, terms, P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner);
+  // (what follows needs the workspace for more than the sort)
+  const bool odd = workspace && aligned16(x) && mode == QMM_MODE_MXFP4 && sorts_odd(P, E, N, K, mode, workspace_bytes);
+  const bool in_kernel = odd || terms_in_kernel(x, terms, P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner);
   const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);
@@ -1063,7 +1092,7 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
     int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);
     if (rc) return rc;
-    if (!sorts_general(P, E, inner)) {
+    if (!odd && !sorts_general(P, E, inner)) {
       gemv_terms_dispatch(x, x_dtype, w, scales, y, y_dtype, P, 1, N, K, lhs_idx, rhs_idx, nullptr, nullptr, nullptr, E, T, 0, st);
       return check_launch("gather gemv launch");
     }

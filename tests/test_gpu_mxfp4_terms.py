@@ -92,7 +92,7 @@ def test_pairs(pairs, e, n, k, act):
 @pytest.mark.parametrize("pairs,e,n,k", [(1, 2, 4096, 4096), (3, 2, 4096, 4096), (5, 4, 352, 1216), (20, 4, 352, 1216), (30, 8, 2880, 1088),
                                          (40, 16, 1024, 2048), (64, 16, 1024, 2048), (8, 9, 2880, 2880), (9, 9, 2880, 2880),
                                          # past 64 pairs
-                                         (65, 8, 512, 288), (78, 8, 384, 576), (128, 8, 600, 288), (129, 8, 600, 288), (200, 16, 1024, 1024)])
+                                         (65, 8, 512, 288), (78, 8, 384, 576), (128, 8, 600, 288), (129, 8, 600, 288), (200, 16, 1024, 1024), (257, 4, 200, 352), (260, 3, 40, 96)])
 def test_pairs_of_staged_shapes(pairs, e, n, k, act):
     g = torch.Generator(device=DEV).manual_seed(pairs + k)
     w, s = weight(g, (e,), n, k)
