@@ -1526,7 +1526,7 @@ bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products)
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
                               int64_t products);
 bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b, int64_t products);
-static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products);
+static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products, int64_t least = 16);
 
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
                                const void* s, const void* b, int64_t E, int64_t least_slices) {
@@ -1621,13 +1621,13 @@ bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products)
 // once per product (grouped, four-bit codes, us against a share of all compute units for every
 // segment: 128 pairs over 8 experts of 4096 x 4096 38.6 / 66.8, over 32 of 2048 x 4096 40.8 / 81.7; 256
 // over 32 of 2048 x 4096 44.0 / 96.9).  For the ragged form a multiple of eight (see above).
-static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products) {
+static int64_t mx_rows_per_wg(int64_t N, int64_t K, int64_t products, int64_t least) {
   const int64_t cus = device_cus();
   if (products < 1) products = 1;
   const int64_t wgs = products >= cus ? 1 : cus / products;      // workgroups a product
   int64_t rows = ceil_div(N, wgs);
   if (rows > 128) rows = ceil_div(N, ceil_div(N, (int64_t)128));
-  if (rows < 16) rows = 16;
+  if (rows < least) rows = least;
   if (K % 512) rows = ceil_div(rows, (int64_t)8) * 8;
   return rows;
 }
@@ -1680,7 +1680,13 @@ bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, cons
 void skinny2_g32_dispatch(const GemvArgs& a0, int64_t batch, int bits, int tab, hipStream_t st) {
   GemvArgs a = a0;
   a.gshift = g32_kind(tab);
-  const int rows = (int)mx_rows_per_wg(a.N, a.K, batch);
+  // Half tiles where whole ones leave compute units without one: a tile's rows, their
+  // tables and the sums are what a workgroup waits for, and half of them are half of that
+  // (us, 16 / 8 rows at least, 1 / 6 / 16 rows of x: eight-bit 1504 x 10304 13.7 / 14.7 / 19.2
+  // -> 12.1 / 13.1 / 17.4, 2000 x 7168 8.8 / 10.6 / 13.4 -> 8.4 / 9.9 / 12.8, four-bit 3072 x 8192
+  // 9.0 / 10.1 / 14.4 -> 8.5 / 9.5 / 13.6, 2560 x 9728 9.7 / 12.5 / 16.9 -> 9.4 / 12.2 / 16.5; four
+  // rows at least the same.  Groups of 64 and 128 and MXFP4 lie within 3 % either way.)
+  const int rows = (int)mx_rows_per_wg(a.N, a.K, batch, 8);
   if (a.K * bits / 8 <= 2048) {
     if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, batch, rows, st);
     else launch_k<8, 8, 4, 4, 1>(a, batch, rows, st);
