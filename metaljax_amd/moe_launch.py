@@ -430,6 +430,13 @@ class _Rows:
                     self.memo[at] = self._leaf(v, t, c)
         return self.memo[at]
 
+    def _whole(self, v, t, axis):
+        """`lower` with a float an element: a repeated value (a broadcast, a splat)
+        is one float for the whole row, which instructions that go through the row's
+        elements cannot read."""
+        reg, n = self.lower(v, t, axis), dims_of(v)[axis]
+        return reg if reg[1] == n else self._emit(OP["copy"], n, reg)
+
     def _leaf(self, v, t, c):
         if elem(v) not in FLOATS + ("i1",):
             raise Reject(f"a router input of {elem(v)}")
@@ -451,7 +458,7 @@ class _Rows:
             last = len(shape) - 1
             if c not in (None, last) or top_k_width(op) != shape[last] or dims_of(x)[last] > MAX_ROW:
                 raise Reject("a top-k along another axis")
-            src = self.lower(x, t, last)
+            src = self._whole(x, t, last)
             vals, idx = self._row(shape[last]), self._row(shape[last])
             self._emit(OP["top_k"], shape[last], src, src, idx, dst=vals)
             for i, reg in ((0, vals), (1, idx)):
@@ -491,7 +498,7 @@ class _Rows:
             axis = axes[0]
             if len(axes) != 1 or axis == t or (c is not None and axis != c) or s[axis] < 1:
                 raise Reject("a slice of a router's rows")
-            reg, n = self.lower(x, t, axis), shape[axis]
+            reg, n = self._whole(x, t, axis), shape[axis]
             return self._emit(OP["slice"], n, reg, (b[axis], 0), (s[axis], 0))
         if name == "stablehlo.reduce":
             if len(op.operands) != 2 or len(op.attrs["dimensions"]) != 1:
@@ -507,8 +514,7 @@ class _Rows:
                 raise Reject("a reduction a row program does not model")
             axis = op.attrs["dimensions"][0]
             st = None if t is None else t + (1 if axis <= t else 0)
-            src = self.lower(x, st, axis)
-            return self._emit(OP[how[0]], 1, src, rnd=_round_el(op))
+            return self._emit(OP[how[0]], 1, self._whole(x, st, axis), rnd=_round_el(op))
         if name == "stablehlo.dot_general":
             return self._product(v, op, shape, t, c)
         code, operands = _elementwise(op)

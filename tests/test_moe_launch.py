@@ -167,6 +167,40 @@ def test_blocks_before_and_inside_a_loop(monkeypatch):
         np.testing.assert_allclose(a, b, rtol=2e-5, atol=1e-6)
 
 
+def repeated(what, Tk, E, K):
+    """(old, new) lines of moe_block_mxfp4: a sum, a slice, a top-k over a value that is repeated along the row"""
+    tk, tok, te = f"tensor<{Tk}x{K}xf32>", f"tensor<{Tk}xf32>", f"tensor<{Tk}x{E}xf32>"
+    down = f"applies stablehlo.add across dimensions = [1] : ({tk}, tensor<f32>) -> {tok}"
+    if what == "sum of a broadcast":
+        return f"%sm = stablehlo.reduce(%ex init: %z32) {down}", f"%sm = stablehlo.reduce(%mxb init: %z32) {down}"
+    if what == "sum of a constant":
+        return (f"%sm = stablehlo.reduce(%ex init: %z32) {down}",
+                f"%twos = stablehlo.constant dense<2.0> : {tk}\n    %sm = stablehlo.reduce(%twos init: %z32) {down}")
+    if what == "slice of a broadcast":
+        one = f"tensor<{Tk}x1xf32>"
+        return (f"%smb = stablehlo.broadcast_in_dim %sm, dims = [0] : ({tok}) -> {tk}",
+                f"%smw = stablehlo.broadcast_in_dim %sm, dims = [0] : ({tok}) -> {tk}\n"
+                f"    %sm1 = stablehlo.slice %smw [0:{Tk}, 1:2] : ({tk}) -> {one}\n"
+                f"    %smb = stablehlo.broadcast_in_dim %sm1, dims = [0, 1] : ({one}) -> {tk}")
+    return (f"%logits = stablehlo.add %lg, %brb : {te}",
+            f"%raised = stablehlo.add %lg, %brb : {te}\n"
+            f"    %least = stablehlo.reduce(%raised init: %ninf) applies stablehlo.maximum across dimensions = [1] : ({te}, tensor<f32>) -> {tok}\n"
+            f"    %logits = stablehlo.broadcast_in_dim %least, dims = [0] : ({tok}) -> {te}")
+
+
+@_without_a_gpu
+@pytest.mark.parametrize("what", ["sum of a broadcast", "sum of a constant", "slice of a broadcast", "top-k of a broadcast"])
+def test_instructions_over_repeated_values(what, monkeypatch):
+    E, Tk, H, Ii, K = 4, 3, 32, 32, 2
+    old, new = repeated(what, Tk, E, K)
+    text = T.moe_block_mxfp4(E, Tk, H, Ii, K)
+    assert old in text
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    (g,), (out,), (plain,) = both(text.replace(old, new), [I.from_numpy(a) for a in raw], monkeypatch)
+    assert g is not None and g.rows is not None
+    np.testing.assert_allclose(out, plain, rtol=2e-5, atol=1e-6 * np.abs(plain).max())
+
+
 @_without_a_gpu
 def test_a_router_that_is_read_elsewhere_stays_with_the_program(monkeypatch):
     """The weights are a result of the program too: the router runs as it did,
