@@ -599,7 +599,6 @@ class Launches:
 
     def __init__(self, interp, g, block):
         self.interp, self.g = interp, g
-        self.modules = None              # what a call needs of this package, looked up once
         self.reads = []
         self.dots, self._dot_of = [], {}
         r = g.router
@@ -620,6 +619,7 @@ class Launches:
             self._route(block)
         except Reject:
             self.rows = None
+        self._layout()
 
     def dot(self, v, e, t) -> _Dot:
         at = (v, e, t)
@@ -675,10 +675,13 @@ class Launches:
         self.rows, self.row_leaves, self.row_dot = rows.finish(idx, weights), rows.leaves, rows.dot
         self.skip_keys = frozenset(skip)
 
-    # -- a call
-
     def _layout(self):
-        """Where a call's intermediate results lie in its one buffer."""
+        """Where a call's intermediate results lie in its one buffer, and the modules
+        a call needs: looked up once, and ahead of any call -- several threads may make
+        the first one, and none of them changes what the others read."""
+        import torch
+        from . import kernels, moe, qmm
+        self.modules = torch, kernels, moe, qmm
         g = self.g
         self.buffer = 0
 
@@ -689,12 +692,9 @@ class Launches:
         self.at_feed = [place(g.P * d.info.k, d.feed[2]) if d.feed else None for d in self.dots]
         self.at_dot = [place(g.P * d.n, d.out_el) for d in self.dots]
 
+    # -- a call
+
     def run(self, interp, env):
-        if self.modules is None:
-            import torch
-            from . import kernels, moe, qmm
-            self.modules = torch, kernels, moe, qmm
-            self._layout()
         torch, kernels, moe, qmm = self.modules
         g, r = self.g, self.g.router
         inputs = {}                                     # of this call: value -> tensor (kept until its launches are out)

@@ -167,6 +167,17 @@ def test_blocks_before_and_inside_a_loop(monkeypatch):
         np.testing.assert_allclose(a, b, rtol=2e-5, atol=1e-6)
 
 
+@_without_a_gpu
+def test_a_call_changes_nothing_that_another_one_reads(monkeypatch):
+    """Threads share a dispatch's launches: what a call reads of them is there when
+    the program is compiled, the size of its buffer first of all."""
+    seen, run = [], ML.Launches.run
+    monkeypatch.setattr(ML.Launches, "run", lambda self, *a: (seen.append(dict(vars(self))), run(self, *a))[1])
+    raw, _ = _moe_inputs(4, 3, 32, 32)
+    (g,), _, _ = both(T.moe_block_mxfp4(4, 3, 32, 32, 2), [I.from_numpy(a) for a in raw], monkeypatch)
+    assert seen and seen[0] == vars(g)
+
+
 def repeated(what, Tk, E, K):
     """(old, new) lines of moe_block_mxfp4: a sum, a slice, a top-k over a value that is repeated along the row"""
     tk, tok, te = f"tensor<{Tk}x{K}xf32>", f"tensor<{Tk}xf32>", f"tensor<{Tk}x{E}xf32>"
