@@ -593,6 +593,17 @@ class _Dot:
     __slots__ = ("number", "info", "feed", "strides", "n", "out_el")
 
 
+def _producers(values):
+    """The ops that compute `values`, all the way up."""
+    ops, todo = set(), list(values)
+    while todo:
+        v = todo.pop()
+        if not v.is_block_arg and v.op not in ops:
+            ops.add(v.op)
+            todo += v.op.operands
+    return ops
+
+
 class Launches:
     """The launches of one dispatch.  `skip_keys`: ops besides the dispatch's
     own that need not run (the router's)."""
@@ -619,6 +630,8 @@ class Launches:
             self._route(block)
         except Reject:
             self.rows = None
+        if any(op_key(op) in g.skip_keys for op in _producers(self.reads)):
+            raise Reject("the launches read what the dispatch replaces")
         self._layout()
 
     def dot(self, v, e, t) -> _Dot:
@@ -664,9 +677,11 @@ class Launches:
         rows = _Rows(self.interp, r, block)
         idx = rows.lower(r.indices, 0, 1)
         weights = rows.lower(r.weights, 0, 1)
+        keep = self.reads + [v for v, _ in rows.leaves] + ([rows.dot[1], rows.dot[2]] if rows.dot else [])
+        for op in _producers(keep):      # what the launches still read is computed as before, whoever else does so
+            rows.ops.pop(op_key(op), None)
         if not any(moe.is_top_k(op) for op in rows.ops.values()):
             raise Reject("the top-k is not part of the program")
-        keep = self.reads + [v for v, _ in rows.leaves] + ([rows.dot[1], rows.dot[2]] if rows.dot else [])
         skip = moe.sweep_dead(block, set(g.skip_keys) | set(rows.ops), g, keep)
         for key, op in rows.ops.items():
             for res in op.results:

@@ -168,6 +168,30 @@ def test_blocks_before_and_inside_a_loop(monkeypatch):
 
 
 @_without_a_gpu
+@pytest.mark.parametrize("shared", ["a conversion", "the largest logit"])
+def test_what_router_and_experts_share_is_computed(shared, monkeypatch):
+    """A value that the row program computes for itself and that the launches read
+    as well: the activations' conversion, and a router's value that the experts' results
+    are multiplied by (the program computes the router then)."""
+    E, Tk, H, Ii, K = 4, 3, 64, 32, 2
+    text, th, eth = T.moe_block_mxfp4(E, Tk, H, Ii, K), f"tensor<{Tk}x{H}xf32>", f"tensor<{E}x{Tk}x{H}xf32>"
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    args = [I.from_numpy(a) for a in raw]
+    if shared == "a conversion":
+        half = f"tensor<{Tk}x{H}xbf16>"
+        new = text.replace(f"%x: {th}", f"%xh: {half}", 1).replace("    %gu0 =", f"    %x = stablehlo.convert %xh : ({half}) -> {th}\n    %gu0 =")
+        args[0] = I.from_numpy(raw[0], "bf16")
+    else:
+        new = text.replace("    %ys = stablehlo.multiply %y, ", f"""    %lb = stablehlo.broadcast_in_dim %mx, dims = [1] : (tensor<{Tk}xf32>) -> {eth}
+    %yl = stablehlo.multiply %y, %lb : {eth}
+    %ys = stablehlo.multiply %yl, """)
+    assert new != text
+    (g,), (out,), (plain,) = both(new, args, monkeypatch)
+    assert g is not None and (g.rows is not None) == (shared == "a conversion")
+    np.testing.assert_allclose(out, plain, rtol=2e-5, atol=1e-6 * np.abs(plain).max())
+
+
+@_without_a_gpu
 def test_a_call_changes_nothing_that_another_one_reads(monkeypatch):
     """Threads share a dispatch's launches: what a call reads of them is there when
     the program is compiled, the size of its buffer first of all."""
