@@ -124,14 +124,15 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
   else if (threadIdx.x >= 64 && (int)threadIdx.x - 64 < a.leaves) leaves[threadIdx.x - 64] = a.leaf[threadIdx.x - 64];
   __syncthreads();
   const int i = (int)blockIdx.x * kThreads + (int)threadIdx.x;
-  if (i >= (int)a.inner) return;
+  const int per = a.weights ? a.per_token : 1;
+  const int64_t row = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;         // of y: a pair, a token
+  if (i >= (int)a.inner || row * per >= a.pairs) return;
   int c[3] = {0, 0, i};
   if (a.rank > 1) { c[1] = i / (int)a.dims[2]; c[2] = i - c[1] * (int)a.dims[2]; }
   if (a.rank > 2) { c[0] = c[1] / (int)a.dims[1]; c[1] -= c[0] * (int)a.dims[1]; }
-  const int per = a.weights ? a.per_token : 1;
   float total = 0.f;
   for (int k = 0; k < per; ++k) {
-    const int p = (int)blockIdx.y * per + k, t = p / a.per_token;
+    const int p = (int)row * per + k, t = p / a.per_token;
     const int e0 = __builtin_amdgcn_readfirstlane(a.experts_of[p]);
     const int e = e0 < 0 ? 0 : e0 >= a.experts ? a.experts - 1 : e0;
     Raw raw[QMM_MAP_LEAVES];
@@ -140,8 +141,8 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
     for (int j = 0; j < QMM_MAP_LEAVES; ++j) {
       if (j < a.leaves) {
         const qmm_map_leaf l = uniform(leaves[j]);
-        const int64_t row = l.base + (int64_t)p * l.pair + (int64_t)e * l.expert + (int64_t)t * l.token;
-        raw[j] = load_raw(l.p, row + (int64_t)c[0] * l.coef[0] + (int64_t)c[1] * l.coef[1] + (int64_t)c[2] * l.coef[2], l.el);
+        const int64_t at = l.base + (int64_t)p * l.pair + (int64_t)e * l.expert + (int64_t)t * l.token;
+        raw[j] = load_raw(l.p, at + (int64_t)c[0] * l.coef[0] + (int64_t)c[1] * l.coef[1] + (int64_t)c[2] * l.coef[2], l.el);
         el[j] = l.el;
       }
     }
@@ -155,12 +156,12 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
     }
     const float v = r[a.result * kThreads];
     if (!a.weights) {
-      store_el(a.y, (int64_t)blockIdx.y * a.inner + i, v, a.y_el);
+      store_el(a.y, row * a.inner + i, v, a.y_el);
       return;
     }
     total += round_to(v, a.sum_el) * widen_raw(load_raw(a.weights, p, a.weights_el), a.weights_el);
   }
-  store_el(a.y, (int64_t)blockIdx.y * a.inner + i, total, a.y_el);
+  store_el(a.y, row * a.inner + i, total, a.y_el);
 }
 
 constexpr int kRowThreads = 1024;
@@ -274,7 +275,7 @@ int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
     return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: shape");
   if (a->pairs == 0 || a->inner == 0) return QMM_OK;
   const int64_t rows = a->weights ? a->pairs / a->per_token : a->pairs;
-  if (rows > 65535 || a->inner > INT32_MAX - kThreads) return moe_fail(QMM_ERR_BAD_SHAPE, "pair map: more pairs than a grid takes");
+  if (a->inner > INT32_MAX - kThreads) return moe_fail(QMM_ERR_BAD_SHAPE, "pair map: a larger result than a grid takes");
   int64_t n = 1;
   for (int i = 0; i < a->rank; ++i) {
     if (a->dims[2 - i] < 1) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: dimensions");
@@ -292,7 +293,9 @@ int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
     if (!map_op(q.op) || q.dst >= a->registers || q.a >= a->registers || q.b >= a->registers || q.c >= a->registers || !float_el(q.el))
       return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: instruction");
   }
-  const dim3 grid((unsigned)ceil_div(a->inner, kThreads), (unsigned)rows);
+  // (a grid's second axis ends at 65535; with more rows than that the third takes part)
+  const int64_t planes = ceil_div(rows, 65535);
+  const dim3 grid((unsigned)ceil_div(a->inner, kThreads), (unsigned)ceil_div(rows, planes), (unsigned)planes);
   const size_t lds = (size_t)a->registers * kThreads * 4 + sizeof(a->code) + sizeof(a->leaf);
   hipLaunchKernelGGL(pair_map_kernel, grid, dim3(kThreads), lds, static_cast<hipStream_t>(stream), *a);
   return moe_launched("pair map launch");

@@ -90,3 +90,33 @@ def test_an_elementwise_instruction(op, fn):
     want = fn(v.double().cpu().numpy().transpose(1, 0, 2))
     for half in y.cpu().numpy():
         np.testing.assert_allclose(half, want, rtol=4e-7, atol=1e-30)
+
+
+@pytest.mark.parametrize("pairs,per", [(65535, 1), (65536, 1), (131071, 1), (3 * 65536, 3), (140000, 2)])
+@pytest.mark.parametrize("summed", [False, True])
+def test_more_pairs_than_a_grid_axis(pairs, per, summed):
+    """y[p] = 2 x[p], and its weighted sum over a token's pairs, past the 65535 rows
+    that a grid's second axis takes: exact in float32 for small integers."""
+    from metaljax_amd.kernels import _stream
+    g = torch.Generator(device="cuda").manual_seed(pairs)
+    x = torch.randint(-8, 8, (pairs, 3), device="cuda", generator=g).float()
+    w = torch.randint(-8, 8, (pairs,), device="cuda", generator=g).float()
+    experts = torch.zeros(pairs, dtype=torch.int32, device="cuda")
+    y = torch.full((pairs // per if summed else pairs, 3), -99.0, device="cuda")
+    m = ML.PairMap(y=y.data_ptr(), experts_of=experts.data_ptr(), pairs=pairs, inner=3, dims=(1, 1, 3), per_token=per, experts=1,
+                   rank=1, leaves=1, instructions=1, registers=2, result=1, weights=w.data_ptr() if summed else None)
+    m.leaf[0] = ML.MapLeaf(x.data_ptr(), 0, 3, 0, 0, (0, 0, 1), 0)
+    m.code[0] = ML.Instruction(ML.OP["add"], 1, 0, 0, 0, 0, 0.0)
+    ML.run_map(m, _stream(y))
+    want = 2 * x if not summed else (2 * x * w[:, None]).reshape(pairs // per, per, 3).sum(1)
+    assert torch.equal(y, want)
+
+
+def test_a_long_prompt(monkeypatch):
+    """65600 pairs of 32800 tokens: as launches what it is as array operations."""
+    E, Tk, H, Ii, K = 4, 32800, 32, 32, 2
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    (g,), (out,), (plain,) = both(T.moe_block_mxfp4(E, Tk, H, Ii, K), [I.from_numpy(a) for a in raw], monkeypatch)
+    assert g is not None
+    same = np.abs(out - plain).max(1) <= 2e-5 * np.abs(plain).max()     # (a logit's last place may choose another expert)
+    assert same.mean() >= 0.999
