@@ -44,6 +44,7 @@ OP = {name: i for i, name in enumerate(_OPS)}                      # QMM_OP_*, i
 LEAVES, CODE, REGISTERS = 8, 40, 32                                # QMM_MAP_*
 ROW_LEAVES, ROW_CODE, ROW_OUTS, ROW_FLOATS = 8, 48, 2, 8192        # QMM_ROW_*
 MAX_ROW = 256                   # elements of a row register: a top-k counts, for each, those ahead of it
+MAX_DEPTH = 2 * ROW_CODE        # operations followed up from a value (the recursion's depth): shape ops have no instruction
 # Products up to this many multiplications ride in the row program, whose workgroups (one a token) each read the
 # whole router weight; larger ones stay a library product.
 MAX_ROUTER_MACS = 1 << 23
@@ -375,7 +376,13 @@ class _Rows:
         self.ops = {}                    # key -> op the program replaces
         self.floats = 0
         self.dot = None
-        self._below = {}
+        self.depth = 0
+        self.below = {router.top_k}      # the ops that depend on the router's top-k
+        todo = [router.top_k]
+        while todo:
+            for user in [u for res in todo.pop().results for u in res.uses if u not in self.below]:
+                self.below.add(user)
+                todo.append(user)
 
     def _row(self, n):
         at, self.floats = self.floats, self.floats + n
@@ -390,15 +397,6 @@ class _Rows:
         a, b, c = a or dst, b or a or dst, c or a or dst
         self.code.append(RowInstruction(op, rnd, dst[0], n, a[0], a[1], b[0], b[1], c[0], c[1], imm))
         return dst
-
-    def _after_top_k(self, v):
-        """Does `v` depend on the router's top-k?"""
-        op = None if v.is_block_arg else v.op
-        if op is None:
-            return False
-        if op not in self._below:
-            self._below[op] = op is self.router.top_k or any(self._after_top_k(x) for x in op.operands)
-        return self._below[op]
 
     def lower(self, v, t, c):
         """The register holding, for a token, `v` along axis `c` at the token
@@ -418,7 +416,7 @@ class _Rows:
                 self.memo[at] = self._emit(OP["imm"], 1, None, imm=splat)
             elif op is None or op not in self.inside:
                 self.memo[at] = self._leaf(v, t, c)
-            elif self._after_top_k(v):
+            elif op in self.below:
                 self.memo[at] = self._op(v, op, t, c)
             else:
                 was = len(self.code), len(self.leaves), self.floats, self.dot, dict(self.ops), dict(self.memo)
@@ -450,6 +448,15 @@ class _Rows:
         return reg
 
     def _op(self, v, op, t, c):
+        if self.depth == MAX_DEPTH:
+            raise Reject("a chain of more operations than a row program follows")
+        self.depth += 1
+        try:
+            return self._followed(v, op, t, c)
+        finally:
+            self.depth -= 1
+
+    def _followed(self, v, op, t, c):
         shape = dims_of(v)
         name = op.name
         from .moe import _splat_value, is_top_k, top_k_width
@@ -777,7 +784,7 @@ def compile_dispatch(interp, g, block):
     """The dispatch's launches, None where it runs as array operations."""
     try:
         return Launches(interp, g, block)
-    except Reject as why:
+    except (Reject, RecursionError) as why:
         from .moe import _debug
         _debug(f"{g.name}: array operations ({why})")
         return None

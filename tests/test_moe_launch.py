@@ -192,6 +192,26 @@ def test_what_router_and_experts_share_is_computed(shared, monkeypatch):
 
 
 @_without_a_gpu
+@pytest.mark.parametrize("behind", ["the activations", "the logits"])
+def test_a_long_program_ahead_of_the_router(behind, monkeypatch):
+    """What lies ahead of a block may be a whole model: it is not walked by recursion."""
+    E, Tk, H, Ii, K, n = 4, 3, 32, 32, 2, 1500
+    text = T.moe_block_mxfp4(E, Tk, H, Ii, K)
+    if behind == "the activations":
+        ty, first, last, before = f"tensor<{Tk}x{H}xf32>", "%x0", "%x", "    %gu0 ="
+        text = text.replace(f"%x: {ty}", f"%x0: {ty}", 1)
+    else:
+        ty, first, last, before = f"tensor<{Tk}x{E}xf32>", "%raised", "%logits", "    %vals, %idx ="
+        text = text.replace("%logits =", "%raised =", 1)
+    names = [first] + [f"%neg{i}" for i in range(n - 1)] + [last]
+    chain = "".join(f"    {b} = stablehlo.negate {a} : {ty}\n" for a, b in zip(names, names[1:]))
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    (g,), (out,), (plain,) = both(text.replace(before, chain + before), [I.from_numpy(a) for a in raw], monkeypatch)
+    assert g is not None and (g.rows is not None or behind == "the logits")     # (a chain may leave no room for the rest)
+    np.testing.assert_allclose(out, plain, rtol=2e-5, atol=1e-6 * np.abs(plain).max())
+
+
+@_without_a_gpu
 def test_a_call_changes_nothing_that_another_one_reads(monkeypatch):
     """Threads share a dispatch's launches: what a call reads of them is there when
     the program is compiled, the size of its buffer first of all."""
