@@ -20,6 +20,7 @@ bool skinny2_plan(int64_t M, int64_t N, int64_t K, int bits, int* rows_per_wg);
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
                               int64_t products);
 int64_t skinny2_ragged_rows(int64_t N, int64_t K, int64_t products);
+int64_t skinny2_g32_rows(int64_t N, int64_t K, int64_t products);
 bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b, int64_t products);
 bool skinny2_mx_plan(int64_t N, int64_t K, int* rows_per_wg);
 bool skinny2_grouped_supported(int64_t N, int64_t K, int gs, int bits, int mode, int tab,
@@ -637,10 +638,10 @@ int qmm_plan(int64_t M, int64_t N, int64_t K, int group_size, int bits, int mode
     if (block) *block = loaders ? 64 * 12 : 64 * waves;
     return QMM_OK;
   }
-  if (M <= kGemvMaxM && mode == QMM_MODE_AFFINE && (skinny2_ragged_supported(N, K, group_size, bits, QMM_BF16, nullptr, nullptr, 1) ||
-                                                    skinny2_g32_supported(N, K, group_size, bits, QMM_BF16, nullptr, nullptr, 1))) {
+  const bool ragged = M <= kGemvMaxM && mode == QMM_MODE_AFFINE && skinny2_ragged_supported(N, K, group_size, bits, QMM_BF16, nullptr, nullptr, 1);
+  if (ragged || (M <= kGemvMaxM && mode == QMM_MODE_AFFINE && skinny2_g32_supported(N, K, group_size, bits, QMM_BF16, nullptr, nullptr, 1))) {
     if (kernel) *kernel = QMM_KERNEL_GEMV;
-    if (grid) *grid = (int)ceil_div(N, skinny2_ragged_rows(N, K, 1));
+    if (grid) *grid = (int)ceil_div(N, ragged ? skinny2_ragged_rows(N, K, 1) : skinny2_g32_rows(N, K, 1));
     if (block) *block = 64 * 12;
     return QMM_OK;
   }

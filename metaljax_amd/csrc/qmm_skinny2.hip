@@ -1677,16 +1677,18 @@ bool skinny2_g32_supported(int64_t N, int64_t K, int gs, int bits, int tab, cons
   return N * (K * bits / 8) < 0x7FFFFFFFll && N * (K / 16) < 0x7FFFFFFCll;       // 32-bit lane offsets
 }
 
+// Half tiles where whole ones leave compute units without one: a tile's rows, their
+// tables and the sums are what a workgroup waits for, and half of them are half of that
+// (us, 16 / 8 rows at least, 1 / 6 / 16 rows of x: eight-bit 1504 x 10304 13.7 / 14.7 / 19.2
+// -> 12.1 / 13.1 / 17.4, 2000 x 7168 8.8 / 10.6 / 13.4 -> 8.4 / 9.9 / 12.8, four-bit 3072 x 8192
+// 9.0 / 10.1 / 14.4 -> 8.5 / 9.5 / 13.6, 2560 x 9728 9.7 / 12.5 / 16.9 -> 9.4 / 12.2 / 16.5; four
+// rows at least the same.  Groups of 64 and 128 and MXFP4 lie within 3 % either way.)
+int64_t skinny2_g32_rows(int64_t N, int64_t K, int64_t products) { return mx_rows_per_wg(N, K, products, 8); }
+
 void skinny2_g32_dispatch(const GemvArgs& a0, int64_t batch, int bits, int tab, hipStream_t st) {
   GemvArgs a = a0;
   a.gshift = g32_kind(tab);
-  // Half tiles where whole ones leave compute units without one: a tile's rows, their
-  // tables and the sums are what a workgroup waits for, and half of them are half of that
-  // (us, 16 / 8 rows at least, 1 / 6 / 16 rows of x: eight-bit 1504 x 10304 13.7 / 14.7 / 19.2
-  // -> 12.1 / 13.1 / 17.4, 2000 x 7168 8.8 / 10.6 / 13.4 -> 8.4 / 9.9 / 12.8, four-bit 3072 x 8192
-  // 9.0 / 10.1 / 14.4 -> 8.5 / 9.5 / 13.6, 2560 x 9728 9.7 / 12.5 / 16.9 -> 9.4 / 12.2 / 16.5; four
-  // rows at least the same.  Groups of 64 and 128 and MXFP4 lie within 3 % either way.)
-  const int rows = (int)mx_rows_per_wg(a.N, a.K, batch, 8);
+  const int rows = (int)skinny2_g32_rows(a.N, a.K, batch);
   if (a.K * bits / 8 <= 2048) {
     if (bits == 4) launch_k<4, 8, 4, 4, 1>(a, batch, rows, st);
     else launch_k<8, 8, 4, 4, 1>(a, batch, rows, st);

@@ -90,6 +90,17 @@ def test_plan_of_the_decode_variants(lib):
     assert b.value == 768
 
 
+def test_plan_of_the_decode_in_groups_of_32(lib):
+    """Eight rows a workgroup at least, where groups of 64 keep sixteen: fewer than
+    4096 weight rows still give every compute unit (256 assumed) a workgroup."""
+    k, g, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    for n, kk, bits, grid in ((1504, 10304, 8, 188), (2000, 7168, 8, 250), (3072, 8192, 4, 256), (14336, 4096, 4, 256)):
+        assert lib.qmm_plan(4, n, kk, 32, bits, 0, k, g, b) == 0
+        assert (k.value, g.value, b.value) == (_lib.KERNEL_GEMV, grid, 768), (n, kk)
+    assert lib.qmm_plan(4, 1504, 10304, 64, 8, 0, k, g, b) == 0
+    assert (g.value, b.value) == (94, 768)
+
+
 def test_plan_of_the_mxfp4_kernels(lib):
     """MXFP4 prefill: the eight-wavefront block-scaled kernel (512 threads, a
     64 x 128 tile a workgroup) when K is a whole number of 2048-code stages,
