@@ -26,7 +26,8 @@ _MODE = {"affine": MODE_AFFINE, "mxfp4": MODE_MXFP4}
 # The current stream's handle without a Stream object made for it (what torch's own
 # generated code calls): 0.1 instead of 1.1 us, 2.7 where the device is looked up too.
 # A decode launch lasts five.
-_raw_stream, _this_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+# (Names that a torch without GPU support lacks; nothing here is launched on one.)
+_raw_stream, _this_device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream(t: torch.Tensor) -> int:

@@ -219,3 +219,17 @@ def test_the_gather_query_tells_what_the_static_entry_takes(lib, act):
         rc = lib.qmm_gather_qmm_static(at, act, at, at, at, _lib.BF16, at, _lib.BF16, at, at, p, p, e, n, k, 64, 4, 0, None)
         want = 4 if lib.qmm_gather_workspace_bytes(p, e, n, k, act) > _lib.STATIC_SCRATCH_BYTES else 5
         assert rc == want, (p, e, n, k)
+
+
+def test_the_wrappers_import_without_a_gpu_build_of_torch(monkeypatch):
+    """torch's stream queries are not there in a build for the CPU alone; packing,
+    the interpreter and the recognizer import the wrappers all the same."""
+    import importlib.util
+
+    import torch
+
+    from metaljax_amd import kernels
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        monkeypatch.delattr(torch._C, name, raising=False)
+    spec = importlib.util.spec_from_file_location("metaljax_amd.kernels_without_a_gpu", kernels.__file__)
+    spec.loader.exec_module(importlib.util.module_from_spec(spec))
