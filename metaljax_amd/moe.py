@@ -1032,7 +1032,10 @@ def prologue(interp, st) -> bool:
 
 def emit_reads(g):
     """Everything `emit` reads out of env: what the plan gathers on the way
-    into the region, and the router's two tensors."""
+    into the region, and the router's two tensors -- or, where a row program
+    stands for the router, what that reads."""
+    if g.launches is not None:
+        return tuple(dict.fromkeys(g.launches.env_reads))
     return tuple(g.reads) + (g.router.indices, g.router.weights)
 
 

@@ -613,7 +613,8 @@ def _producers(values):
 
 class Launches:
     """The launches of one dispatch.  `skip_keys`: ops besides the dispatch's
-    own that need not run (the router's)."""
+    own that need not run (the router's); `env_reads`: the program's values that a
+    call reads."""
 
     def __init__(self, interp, g, block):
         self.interp, self.g = interp, g
@@ -633,6 +634,7 @@ class Launches:
         self.rest = rest
         self.rows = None
         self.skip_keys = frozenset()
+        self.env_reads = self.reads + [r.indices, r.weights]
         try:
             self._route(block)
         except Reject:
@@ -695,7 +697,7 @@ class Launches:
                 if any(op_key(u) is not g.key and op_key(u) not in skip for u in res.uses):
                     raise Reject(f"{op.name} of the router is read elsewhere")
         self.rows, self.row_leaves, self.row_dot = rows.finish(idx, weights), rows.leaves, rows.dot
-        self.skip_keys = frozenset(skip)
+        self.skip_keys, self.env_reads = frozenset(skip), keep
 
     def _layout(self):
         """Where a call's intermediate results lie in its one buffer, and the modules

@@ -222,6 +222,31 @@ def test_a_call_changes_nothing_that_another_one_reads(monkeypatch):
     assert seen and seen[0] == vars(g)
 
 
+@_without_a_gpu
+@pytest.mark.parametrize("elsewhere", [False, True])
+def test_emit_reads_names_what_a_call_reads(elsewhere, monkeypatch):
+    """Exactly the values that the launches look up, with the router as a row
+    program and, where its weights are read elsewhere, with the program's router."""
+    E, Tk, H, Ii, K = 4, 3, 32, 32, 2
+    text = T.moe_block_mxfp4(E, Tk, H, Ii, K)
+    if elsewhere:
+        text = text.replace(f"return %out : tensor<{Tk}x{H}xf32>", f"return %out, %w : tensor<{Tk}x{H}xf32>, tensor<{Tk}x{K}xf32>")
+        text = text.replace(f"-> tensor<{Tk}x{H}xf32> {{\n", f"-> (tensor<{Tk}x{H}xf32>, tensor<{Tk}x{K}xf32>) {{\n", 1)
+    seen, run = set(), ML.Launches.run
+
+    class Looked:
+        def __init__(self, env):
+            self.env = env
+
+        def __getitem__(self, v):
+            seen.add(v)
+            return self.env[v]
+    monkeypatch.setattr(ML.Launches, "run", lambda self, interp, env: run(self, interp, Looked(env)))
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    (g,), _, _ = both(text, [I.from_numpy(a) for a in raw], monkeypatch)
+    assert (g.rows is None) == elsewhere and set(qmm.emit_reads(g.g)) == seen
+
+
 def repeated(what, Tk, E, K):
     """(old, new) lines of moe_block_mxfp4: a sum, a slice, a top-k over a value that is repeated along the row"""
     tk, tok, te = f"tensor<{Tk}x{K}xf32>", f"tensor<{Tk}xf32>", f"tensor<{Tk}x{E}xf32>"
