@@ -716,11 +716,15 @@ void mxfp4_geometry(int64_t R, int64_t N, int64_t K, int* grid, int* block) {
 // tile or two.  Fitted on 68 dense products of 17 to 2048 rows, N and K 1024 to 14336,
 // and 24 over 8 to 32 experts: 6 and 7 % off on average, and the choice between this
 // kernel and the short-group one 0.6 % from the better (5.5 % before, when it came out
-// 40 % too short for groups); profiles/prefill_plan_fits.txt.
+// 40 % too short for groups); profiles/prefill_plan_fits.txt.  The four-wavefront form's
+// step was fitted at 3.30e-3; it is counted as 5.0e-3, so that the short-group kernel,
+// whose products are exact (bf16 activations are split more narrowly here: 3.4e-4
+// against 1.6e-7 from 64 bits in float32 results), keeps what it is at most some per
+// cent slower at (468 rows of 2184 x 7680 38.4 / 36.1 us).
 double mxfp4_us(int64_t R, int64_t E, int64_t N, int64_t K) {
   const int64_t group = E > 1 ? ceil_div(R, E) : R;
   const int64_t tiles = ceil_div(N, TN) * (E > 1 ? E * ceil_div(group * 5 / 4, TM) : ceil_div(R, TM));
-  const double step = K % 2048 == 0 ? 2.18e-3 + 0.48e-3 * (tiles < 256 ? tiles / 256.0 : 1.0) : 3.30e-3;
+  const double step = K % 2048 == 0 ? 2.18e-3 + 0.48e-3 * (tiles < 256 ? tiles / 256.0 : 1.0) : 5.0e-3;
   return 4.9 + (double)ceil_div(tiles, 256) * (2.7 + (double)K * step) + (double)R * K * 1.63e-6 +
          (double)R * N * 0.85e-6 + (E > 1 ? (double)std::min(E, R) * N * K * 7.2e-8 : 0.0);
 }

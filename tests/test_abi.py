@@ -129,6 +129,18 @@ def test_plan_of_the_mxfp4_kernels(lib):
     assert b.value < 768
 
 
+def test_plan_keeps_exact_mxfp4_products(lib):
+    """K a multiple of 512 but not of 2048: where the short-group kernel served, whose
+    products are exact, the four-wavefront form (a narrower split of bf16 activations)
+    is not taken for the few per cent that it is ahead."""
+    k, g, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    for m, n, kk in ((227, 13264, 1536), (468, 2184, 7680), (820, 3088, 3072), (1821, 8128, 2560), (75, 13272, 5632), (430, 9328, 11264)):
+        assert lib.qmm_plan(m, n, kk, 32, 4, 1, k, g, b) == 0
+        assert k.value == _lib.KERNEL_GEMM, (m, n, kk)
+    assert lib.qmm_plan(256, 8192, 8192, 32, 4, 1, k, g, b) == 0
+    assert k.value == _lib.KERNEL_MXFP4_MFMA
+
+
 def test_gather_workspace_covers_the_grouped_decode(lib):
     """From four pairs up to sixteen an expert the workspace holds the expert
     sort and the segment list; below four pairs nothing is needed."""
