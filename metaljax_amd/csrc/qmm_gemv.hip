@@ -702,8 +702,8 @@ void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* 
   a.out_row = out_row;
   a.x_rows = segments ? (int)x_rows : pairs_here;
   int t, waves;
-  // (as wide as the terms' rows would be: the sums then meet as they did)
   gemv_geometry(segments || pairs_here ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
+  if (K > 2048) waves = 8;                         // (512 codes a wavefront up to 4096: see kTermsCodes)
   if (x_dtype == QMM_F32) launch_mxfp4_terms<3>(a, batch, t, waves, st);
   else launch_mxfp4_terms<2>(a, batch, t, waves, st);
 }

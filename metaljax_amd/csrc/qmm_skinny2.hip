@@ -1384,6 +1384,8 @@ void launch_k(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st,
   }
 }
 
+}  // namespace
+
 int device_cus() {
   static const int cus = [] {
     int dev = 0, n = 256;
@@ -1395,6 +1397,8 @@ int device_cus() {
   }();
   return cus;
 }
+
+namespace {
 
 // One pass (K is exactly the eight slices of the compute wavefronts) and few
 // rows of activations: the variant whose compute wavefronts fetch their own
