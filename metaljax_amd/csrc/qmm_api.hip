@@ -431,8 +431,10 @@ int act_terms(int x_dtype) { return x_dtype == QMM_F32 ? 3 : x_dtype == QMM_F16 
 //   sorted pairs: 8 of 32 experts of 2880 x 2880 (33 MB) 26.4 / 35.6, 64 of 8 of 2880 x
 //   1088 22.0 / 36.8, 8 of 8 of 4096 x 4096 (67 MB) 45.4 / 39.0;
 //   past 64 pairs, against the row-group kernels: 78 of 8 of 1024 x 1024 (6.3 MB) 11.7 /
-//   15.4 (float16 11.0 / 14.3), 128 of it (8.4) 15.5 / 15.7 (11.4 / 16.3), 78 of 8 of 2880 x
-//   1088 (19) 23.5 / 17.5 (a K that is no multiple of 64: sorts_odd).
+//   15.4 (float16 11.0 / 14.3), 128 of it (8.4) 15.5 / 15.7 (11.4 / 16.3) (a K that is no
+//   multiple of 64: sorts_odd) -- into 16-bit results: those kernels' sums over parts of K
+//   are the more exact ones (float32 results, 96 pairs of 280 x 1024 6.9e-8 / 6.1e-8 from
+//   64 bits, 134 of 352 x 1408 7.8e-8 / 6.6e-8).
 constexpr int64_t kTermsBytes = 12 << 20, kTermsBytesMost = 34 << 20, kTermsBytesManyPairs = 18 << 20;
 
 // A wavefront adds up its share of K in one accumulator a term: up to 4096 codes in
@@ -455,13 +457,13 @@ bool terms_dense(int terms, int64_t batch, int64_t N, int64_t K) {
 }
 
 bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
-                     const void* s, const void* b, size_t workspace_bytes) {
+                     const void* s, const void* b, int y_dtype, size_t workspace_bytes) {
   if (mode != QMM_MODE_MXFP4 || !aligned16(x) || P <= 0 || E > 65535 || N > INT32_MAX || K > INT32_MAX || N * K >= (1ll << 40))
     return false;
   const bool sorted = sorts_general(P, E, workspace_bytes);
   if (P > kGatherGemvMaxPairs && !sorted) return false;
   const int64_t bytes = (sorted ? skinny2_max_segments(P, E) : P) * (N * K / 2);
-  if (P > kGatherGemvMaxPairs) return terms * bytes <= kTermsBytesManyPairs;
+  if (P > kGatherGemvMaxPairs) return y_dtype != QMM_F32 && terms * bytes <= (K < 512 ? kTermsBytes : kTermsBytesManyPairs);
   if (gemv_runs_general(N, K, gs, bits, mode, tab, s, b, E)) return sorted || K <= kTermsCodesGeneral;
   if (K > kTermsCodes) return false;
   if (sorted_here_serves(P, E, N, K, gs, bits, mode, tab, s, b) ||
@@ -1076,7 +1078,7 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   const size_t inner = gather_scratch(P, E, N, K, true);
   // (what follows needs the workspace for more than the sort)
   const bool odd = workspace && aligned16(x) && mode == QMM_MODE_MXFP4 && sorts_odd(P, E, N, K, mode, workspace_bytes);
-  const bool in_kernel = odd || terms_in_kernel(x, terms, P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner);
+  const bool in_kernel = odd || terms_in_kernel(x, terms, P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, y_dtype, inner);
   const bool exact_decode = mode == QMM_MODE_AFFINE && (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) &&
                             K % group_size == 0 &&
                             grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, ~(size_t)0);

@@ -152,3 +152,11 @@ def pairs_off(pairs, e, n, k, act):
 @pytest.mark.parametrize("pairs,e,n,k", [(52, 16, 456, 3968), (12, 8, 552, 3584), (3, 4, 992, 3776), (5, 2, 400, 8192)])
 def test_pairs_of_long_rows_are_no_less_exact(pairs, e, n, k):
     assert pairs_off(pairs, e, n, k, "f32") <= 1.1e-7
+
+
+# Past 64 pairs the row-group kernels' sums over parts of K measure 4.6e-8 to 7.0e-8 in float32
+# results, the general kernel's 5.0e-8 to 8.2e-8: it serves 16-bit results alone.
+@pytest.mark.parametrize("act", ["f16", "f32"])
+@pytest.mark.parametrize("pairs,e,n,k,most", [(134, 16, 352, 1408, 7.1e-8), (126, 8, 664, 1216, 6.9e-8), (188, 16, 424, 1600, 7.5e-8)])
+def test_many_pairs_are_no_less_exact(pairs, e, n, k, most, act):
+    assert pairs_off(pairs, e, n, k, act) <= most
