@@ -357,6 +357,11 @@ bool grouped_decode_serves(int64_t P, int64_t E, int64_t N, int64_t K, int gs, i
   // 38.5 / 34.2, 500 over 32 of 1024 x 4096 43.9 / 34.9, 256 over 16 of 4096 x 2048 46.5 / 40.7;
   // 300 over 32 of 2048 x 2048 33.3 / 37.4, 128 over 32 32.4 / 35.9).
   if (mode == QMM_MODE_AFFINE && gs == 32 && P > kGatherGemvMaxPairs && P > 10 * E) return false;
+  // Fewer than sixteen stay decode products of their own until what these would stream is
+  // worth the sort's launch (us, here / there: 13 pairs over 4 experts of 296 x 3072, 6 MB, 8.8 /
+  // 7.8, 15 of 472 x 5376, 19 MB, 11.7 / 12.5, 13 of 1312 x 2624, 22 MB, 10.8 / 13.0, 12 over 16 of 2792 x
+  // 1152, 19 MB, 16.6 / 24.3).
+  if (mode == QMM_MODE_AFFINE && gs == 32 && P < 16 && P * (N * K * bits / 8) <= (16 << 20)) return false;
   return grouped_decode_pairs(P, E) && !off && workspace_bytes >= route_bytes_segments(P, E) &&
          skinny2_grouped_supported(N, K, gs, bits, mode, tab, s, b, E, 8);
 }
@@ -1140,9 +1145,14 @@ int qmm_gather_qmm(const void* x, int x_dtype, const void* w, const void* scales
   }
   // Pairs that are decode products of their own: the terms are the rows of one (terms
   // <= 16: a pair's weight is streamed once, in one launch instead of one a term).
+  // In groups of 32 fewer than sixteen pairs are, unless the experts are so few that once a
+  // term each is less than once a pair (us, as rows / sorted once a term: float32, 4 pairs over 64
+  // experts of 440 x 1472 10.3 / 27.6, 8 of 11880 x 2816 over 8 69 / 207, 15 of 4744 x 8768 over 4 124 / 106,
+  // float16, 14 of 4160 x 8000 over 8 73 / 116, 12 of 7280 x 4160 over 4 82 / 66).
+  const bool rows_win = mode == QMM_MODE_AFFINE && group_size == 32 && P < 16 && terms * E >= P;
   if (P <= kGatherGemvMaxPairs && E <= 65535 && N <= INT32_MAX && K <= INT32_MAX &&
       !sorted_here_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases) &&
-      !grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner) &&
+      (!grouped_decode_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner) || rows_win) &&
       !grouped_general_serves(P, E, N, K, group_size, bits, mode, table_dtype, scales, biases, inner)) {
     int rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (!rc) rc = check_io(ws, QMM_BF16, ws + xs, QMM_F32);

@@ -68,6 +68,25 @@ def test_pairs(pairs, e, n, k, bits):
     assert off(y, want) <= ERR
 
 
+# fewer than sixteen pairs: products of their own up to 16 MB of streamed weights, sorted past that; wider rows as
+# the rows of one product a pair, or once a term where the experts are fewer than the pairs
+@pytest.mark.parametrize("act", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("pairs,e,n,k,bits", [(13, 4, 296, 3072, 4), (15, 4, 496, 5376, 4), (4, 16, 712, 2048, 4), (15, 4, 2400, 2240, 8),
+                                              (12, 4, 2400, 2240, 8), (15, 7, 520, 4160, 8), (16, 4, 296, 3072, 4)])
+def test_few_pairs(pairs, e, n, k, bits, act):
+    g = torch.Generator(device=DEV).manual_seed(pairs + n)
+    w, s, b = weight(g, (e,), n, k, bits, "bf16")
+    x = torch.randn((7, k), device=DEV, generator=g).to({"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[act])
+    lhs = torch.randint(0, 7, (pairs,), device=DEV, generator=g, dtype=torch.int32)
+    rhs = torch.randint(0, e, (pairs,), device=DEV, generator=g, dtype=torch.int32)
+    lhs[0], rhs[1] = 7, e                                 # no such row: zeros; no such expert: nothing is written
+    y = K.gather_qmm(x, w, s, b, lhs, rhs, out_dtype=torch.float32, group_size=32, bits=bits)
+    w64, x64 = exact(w, s, b, bits), x.double()
+    live = [p for p in range(2, pairs)]
+    want = torch.stack([w64[rhs[p]] @ x64[lhs[p]] for p in live])
+    assert off(y[live], want) <= ERR and not y[0].any()
+
+
 def test_a_batch_of_weights():
     g = torch.Generator(device=DEV).manual_seed(3)
     w, s, b = weight(g, (3,), 130, 1600, 4, "bf16")
