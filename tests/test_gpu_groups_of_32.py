@@ -36,7 +36,9 @@ def off(y, want):
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("tab", ["bf16", "f16"])
-@pytest.mark.parametrize("n,k", [(16, 1088), (72, 1536), (4104, 2112), (33, 4096), (300, 4160), (1000, 8192), (520, 11008), (9000, 1152)])
+@pytest.mark.parametrize("n,k", [(16, 1088), (72, 1536), (4104, 2112), (33, 4096), (300, 4160), (1000, 8192), (520, 11008), (9000, 1152),
+                                 # 9, 12 and 10 rows a workgroup (K whole slices), 16 where they are dealt by eights
+                                 (2100, 1536), (3070, 4096), (2530, 8192), (2100, 4160)])
 def test_dense(n, k, bits, tab):
     g = torch.Generator(device=DEV).manual_seed(n + k)
     w, s, b = weight(g, (), n, k, bits, tab)

@@ -109,14 +109,14 @@ def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n
         store(y, i, v, ML.ELS[y_el])
 
 
-def both(text, args, monkeypatch):
+def both(text, args, monkeypatch, rows=run_rows):
     """(launches, results as launches, results as array operations)"""
     monkeypatch.setattr(qmm, "DEVICE", "cpu")
     monkeypatch.setattr(moe, "emit_dot", _oracle_expert_product([]))
     plain = [I.host(b.data).a for b in engine.execute(engine.compile_program(text), args)]
     monkeypatch.setattr(ML, "available", lambda: True)
     monkeypatch.setattr(ML, "run_map", run_map)
-    monkeypatch.setattr(ML, "run_rows", run_rows)
+    monkeypatch.setattr(ML, "run_rows", rows)
     monkeypatch.setattr(ML, "run_product", run_product)
     moe.reset_stats()
     ex = engine.compile_program(text)
@@ -209,6 +209,42 @@ def test_a_long_program_ahead_of_the_router(behind, monkeypatch):
     (g,), (out,), (plain,) = both(text.replace(before, chain + before), [I.from_numpy(a) for a in raw], monkeypatch)
     assert g is not None and (g.rows is not None or behind == "the logits")     # (a chain may leave no room for the rest)
     np.testing.assert_allclose(out, plain, rtol=2e-5, atol=1e-6 * np.abs(plain).max())
+
+
+@_without_a_gpu
+@pytest.mark.parametrize("draw", [0, 1, 2])
+@pytest.mark.parametrize("block", ["gpt-oss", "gpt-oss composite", "gemma4", "sum of a broadcast", "sum of a constant", "slice of a broadcast",
+                                   "top-k of a broadcast"])
+def test_a_row_program_is_the_programs_router(block, draw, monkeypatch):
+    """The compiled router's experts and weights against the program's own evaluation
+    of them, on drawn inputs; from the second draw on coarse ones, whose logits tie."""
+    from metaljax_amd.packs import evaluate
+    E, Tk, H, Ii, K = 6, 5, 32, 32, 3
+    rng = np.random.default_rng(draw)
+    if block == "gemma4":
+        text, args = T.moe_block_gemma4_mxfp4(E, Tk, H, Ii, K), gemma_inputs(E, Tk, H, Ii, "f32")
+        drawn = [0, 1]
+    else:
+        text = T.moe_block_mxfp4(E, Tk, H, Ii, K, composite=block.endswith("composite"))
+        if not block.startswith("gpt-oss"):
+            old, new = repeated(block, Tk, E, K)
+            assert old in text
+            text = text.replace(old, new)
+        args, drawn = [I.from_numpy(a) for a in _moe_inputs(E, Tk, H, Ii)[0]], [0, 1, 2]
+    for i in drawn:
+        a = rng.standard_normal(I.host(args[i]).a.shape).astype(np.float32)
+        args[i] = I.from_numpy(np.round(2 * a) / 2 if draw else a)
+    out = []
+
+    def kept(r, stream):
+        run_rows(r, stream)
+        out.append([[load(o.p, i, o.el) for i in range(r.tokens * o.n)] for o in r.out[:2]])
+    (g,), _, _ = both(text, args, monkeypatch, rows=kept)
+    assert len(out) == 1 and g.rows is not None
+    env = dict(zip(g.interp._main_block().args, [I.host(a) for a in args]))
+    router = g.g.router
+    assert out[0][0] == list(I.host(evaluate(g.interp, router.indices, env)).a.reshape(-1))
+    np.testing.assert_allclose(out[0][1], I.host(evaluate(g.interp, router.weights, env)).a.reshape(-1), rtol=2e-6, atol=1e-7)
 
 
 @_without_a_gpu
