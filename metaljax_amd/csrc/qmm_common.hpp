@@ -166,8 +166,8 @@ __device__ __forceinline__ RowTile find_row_tile(const int32_t* offsets, int E, 
 // workgroups beside those that re-lay the activations, or by a launch of its own
 // where a product has no such launch.  (Every row was zeroed ahead of the product
 // before, none of which stayed: a launch of 7.3 us for 1024 x 14336 bf16 results,
-// whose product over eight experts takes 172 us with it and 170 without -- the
-// matrix cores, short of power, run a little slower for not having had the pause.)
+// whose product over eight experts takes 172 us with it and 170 without: most of
+// the pause comes back as a slower product.)
 struct ClearArgs {
   void* y;                      // [R][N], null: nothing is cleared
   const int32_t* row_offsets;   // [E+1]

@@ -11,7 +11,10 @@
 // an empty launch is 2.7).  As array operations a block of 3 tokens over 8 experts
 // of 1024 x 1024 was some thirty launches with their host work and three round
 // trips to the host, 430 us; now it is these three launches and the two products,
-// 45 us, 37 of them the device's.
+// 45 us, 37 of them the device's.  They stay ahead as blocks grow and the products
+// take over (us, launches / array operations, 8 experts of 1024 x 1024, top 2: 256 tokens
+// 93 / 439, 2048 tokens 364 / 815; 32 experts of 2880 x 2880, top 4: 64 tokens 286 / 533, 2048
+// tokens 3476 / 4536).
 //
 // Both kernels interpret a short program that the planner wrote once: the same
 // instruction for every lane, operands in LDS (column of a lane: its own, so that no

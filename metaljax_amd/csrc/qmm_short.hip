@@ -650,7 +650,8 @@ bool short_supported(int64_t R, int64_t E, int64_t N, int64_t K, int gs, int bit
 // are, with weights rounded to float16 (11 significant bits instead of the bf16
 // tile's 8).  77 rows of 4096 x 4096 in groups of 128: 21.7 us
 // in two terms (a launch for them, tiles of 32 rows), 14.8 like this (tiles of 48).
-// (Groups of 32 keep the bf16 tile, which their products are compared with.)
+// (Groups of 32 keep the two terms and the bf16 tile.  Nothing in the kernel asks for
+// that; what they would gain has not been measured.)
 int short_terms(int x_dtype, int tab, int gs, int mode) {
   if (x_dtype == QMM_F16) return mode == QMM_MODE_AFFINE && tab == QMM_F16 && gs >= 64 ? 1 : 2;
   return x_dtype == QMM_F32 ? 3 : 1;

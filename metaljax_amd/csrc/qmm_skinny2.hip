@@ -1330,8 +1330,11 @@ template <int BITS, int CW, int NL, int TMAX, int GSHIFT, int XD, bool GRP = fal
 void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t st, int pair_wgs = 0) {
   // Three passes of five rows: all of them fit the operand's sixteen rows, as three of four do,
   // and nothing is fetched between passes (us, from where a pass's rows are fetched when it
-  // begins: 4096 x 11008 13.4 -> 9.7, 14336 x 11008 25.5 -> 21.2, eight-bit 4096 x 5504 9.6 ->
-  // 8.0; six rows, which do not fit, 13.9).  Tables that fill the LDS, and pairs, keep that.
+  // begins: 4096 x 11008 13.4 -> 9.7, 14336 x 11008 25.5 -> 22.0, eight-bit 4096 x 5504 9.6 ->
+  // 8.0; six rows, which do not fit, 13.9).  Up to four passes five rows over three are the only
+  // ones that fit and are in no packed form; one to three rows over five to seven passes
+  // (eight-bit codes of K past 8192) fit too, for which no form is built.  Tables that fill the
+  // LDS, and pairs, keep the fetch between passes.
   if constexpr (XD == 2 && !GRP && GSHIFT != 5 && GSHIFT != 13 && GSHIFT < 24) {
     const int64_t slices = ceil_div((int64_t)a.K * BITS / 8, 256);
     if (a.M == 5 && !a.segments && !pair_wgs && slices > 2 * CW && slices <= 3 * CW)
