@@ -442,23 +442,24 @@ int act_terms(int x_dtype) { return x_dtype == QMM_F32 ? 3 : x_dtype == QMM_F16 
 //   64 bits, 134 of 352 x 1408 7.8e-8 / 6.6e-8).
 constexpr int64_t kTermsBytes = 12 << 20, kTermsBytesMost = 34 << 20, kTermsBytesManyPairs = 18 << 20;
 
-// A wavefront adds up its share of K in one accumulator a term: up to 4096 codes in
-// eight wavefronts that is as many matrix steps as in the loader-wavefront kernel's,
-// beyond it more, and the sums come out less exact (float32 rows, distance from 64 bits,
-// here / there: 0.98e-7 / 0.98e-7 up to K = 4096, 1.25e-7 / 1.04e-7 at 8192, 1.55e-7 /
-// 1.06e-7 at 13312) and later.  Against its own launches round the general kernel, whose
-// sums are the same, it holds to 6144 (us: 1744 x 6048 13.4 / 14.1, 1416 x 7136 14.9 / 13.7,
+// A wavefront adds up its share of K in one accumulator a term.  Eight of them to about 5120
+// codes are as exact as the loader-wavefront kernel, beyond it their sums come out less
+// exact and later (float32 rows, distance from 64 bits, here / there: 0.98e-7 / 0.98e-7 up to K =
+// 4096, within 8 % either way by the rows up to 5120, 1.16e-7 / 1.04e-7 at 6464, 1.25e-7 / 1.04e-7
+// at 8192, 1.55e-7 / 1.06e-7 at 13312).  Against its own launches round the general kernel,
+// whose sums are the same, it holds to 6144 (us: 1744 x 6048 13.4 / 14.1, 1416 x 7136 14.9 / 13.7,
 // 784 x 11424 20.5 / 15.8, float16 4040 x 6112 10.7 / 12.8, 2216 x 8672 15.2 / 14.3).
-constexpr int64_t kTermsCodes = 4096, kTermsCodesGeneral = 6144;
+constexpr int64_t kTermsCodes = 5120, kTermsCodesGeneral = 6144;
 
 // Dense rows split in the kernel, where the loader-wavefront kernel serves the shape too
-// (us a call, here / there): while the workgroups are one round (float32 3904 x 4032 9.2 /
-// 12.3, 2296 x 3648 9.7 / 12.9; 4408 x 4032 15.1 / 13.1, 9416 x 2432 18.4 / 11.9), and with
-// two of them a compute unit -- half the wavefronts -- by the bytes (12688 x 1472 float16
-// 10.4 / 11.8, float32 8232 x 1216 9.7 / 11.6, 12992 x 1920 12.8 / 10.9).
-bool terms_dense(int terms, int64_t batch, int64_t N, int64_t K) {
-  if (K > kTermsCodes) return false;
-  return batch * ceil_div(N, 16) <= device_cus() || (K <= 2048 && terms * (N * K / 2) <= (24ll << 20) / batch);
+// (us a call, here / there): with two workgroups a compute unit, half the wavefronts each, by
+// the bytes (12688 x 1472 float16 10.4 / 11.8, float32 8232 x 1216 9.7 / 11.6, 13800 x 1216 10.4 /
+// 11.8, 12992 x 1920 12.8 / 10.9, but 0.73e-7 from 64 bits against 0.85e-7), past 2048 codes while
+// the workgroups are one round (float32 3904 x 4032 9.2 / 12.3, 2296 x 3648 9.7 / 12.9; 4408 x
+// 4032 15.1 / 13.1, 9416 x 2432 18.4 / 11.9).
+bool terms_dense(int64_t batch, int64_t N, int64_t K) {
+  if (K <= 2048) return N * K / 2 <= kTermsBytes / batch;
+  return K <= kTermsCodes && batch * ceil_div(N, 16) <= device_cus();
 }
 
 bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, int64_t K, int gs, int bits, int mode, int tab,
@@ -981,7 +982,7 @@ int qmm_quantized_matmul(const void* x, int x_dtype, const void* w, const void* 
   int rc;
   if (terms * M <= kGemvMaxM && batch <= 65535 && N <= INT32_MAX && y && mode == QMM_MODE_MXFP4 &&
       (gemv_runs_general(N, K, group_size, bits, mode, table_dtype, scales, biases, batch) ? K <= kTermsCodesGeneral
-                                                                                           : terms_dense(terms, batch, N, K))) {
+                                                                                           : terms_dense(batch, N, K))) {
     // (the general MXFP4 decode kernel splits them itself)
     rc = check_quant(N, K, group_size, bits, mode, table_dtype, w, scales, biases);
     if (rc) return rc;

@@ -567,6 +567,7 @@ void skinny2_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int r
                       int tab, bool force_direct);
 int skinny2_direct_rows(int64_t N);
 bool skinny2_mx_supported(int64_t N, int64_t K, const void* s, int64_t products);
+int device_cus();
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
                               int64_t products);
 void skinny2_ragged_dispatch(const GemvArgs& a0, int64_t batch, int gs, int bits, int tab, hipStream_t st);
@@ -703,7 +704,12 @@ void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* 
   a.x_rows = segments ? (int)x_rows : pairs_here;
   int t, waves;
   gemv_geometry(segments || pairs_here ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
-  if (K > 2048) waves = 8;                         // (512 codes a wavefront up to 4096: see kTermsCodes)
+  // Past 2048 codes eight wavefronts: the sums of four are the less exact ones (1.16e-7 from 64
+  // bits at 3968 against 0.98e-7), and a call of one round is slower with them (one float32 row
+  // of 1936 x 3840 12.7 us with four, of 1880 x 3072 8.9 with eight).  Shapes that no staged kernel serves summed in four before, and keep
+  // them where the workgroups are several rounds (205 pairs over 64 of 1792 x 3168 94 / 120).
+  const bool staged = !gemv_runs_general(N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, rhs_idx || segments ? n_experts : batch);
+  if (K > 2048 && (staged || batch * ceil_div(N, 16 * t) <= device_cus())) waves = 8;
   if (x_dtype == QMM_F32) launch_mxfp4_terms<3>(a, batch, t, waves, st);
   else launch_mxfp4_terms<2>(a, batch, t, waves, st);
 }
