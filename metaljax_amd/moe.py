@@ -776,11 +776,12 @@ class Dispatch:
         self.launches = None            # moe_launch.Launches where a GPU is visible and it serves the plan
 
     def pair_tokens(self, device):
-        """Token of pair p, p // K, as int32 and int64: the same every call."""
+        """Token of pair p, p // K, as int32 and int64: the same every call.  Uploaded
+        from the host, which waits: the next call may come from another stream."""
         import torch
         if self._tidx is None:
-            t32 = torch.arange(self.T, dtype=torch.int32, device=device).repeat_interleave(self.K)
-            self._tidx = (t32, t32.long())
+            tokens = np.repeat(np.arange(self.T, dtype=np.int64), self.K)
+            self._tidx = tuple(torch.from_numpy(t).to(device) for t in (tokens.astype(np.int32), tokens))
         return self._tidx
 
     def run(self, interp, env):

@@ -120,3 +120,21 @@ def test_a_long_prompt(monkeypatch):
     assert g is not None
     same = np.abs(out - plain).max(1) <= 2e-5 * np.abs(plain).max()     # (a logit's last place may choose another expert)
     assert same.mean() >= 0.999
+
+
+def test_pair_tokens_are_there_for_another_stream():
+    """Made by the first call, on whatever stream it runs, behind whatever that
+    stream still has to do; the next call's launches may be on another one."""
+    g = moe.Dispatch()
+    g.T, g.K = 3000, 7
+    a, stream = torch.randn((4096, 4096), device="cuda"), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            a = a @ a * 1e-2
+        t32, t64 = g.pair_tokens("cuda")
+    seen = t32.clone(), t64.clone()
+    want = torch.arange(3000).repeat_interleave(7)
+    assert seen[0].dtype == torch.int32 and seen[1].dtype == torch.int64
+    assert torch.equal(seen[0].cpu().long(), want) and torch.equal(seen[1].cpu(), want)
+    stream.synchronize()
