@@ -221,6 +221,23 @@ typedef struct {
  * expert index outside [0, experts) reads the nearest expert's data. */
 int qmm_pair_map_run(const qmm_pair_map* map, void* stream);
 
+/* A product of MXFP4 experts and the pair map that alone reads it, as one launch:
+ * pair p multiplies row p / x_per of x [x_rows, k] by expert experts_of[p] of w
+ * [experts, n, k / 8 words] with block scales s, rounded to product_el; leaf
+ * col_leaf[t] of the map (whose p is null) is column col_base[t] + col_step[t] *
+ * element of that.  UNSUPPORTED where a product and a map are the better launches
+ * (by the sizes, the types and the alignment alone).  `sorted` is the library's. */
+typedef struct {
+  const void *x, *w, *s;
+  int64_t x_rows, n, k;
+  int32_t x_el, x_per, product_el, tiles, col_leaf[2], col_base[2], col_step[2], sorted;
+  qmm_pair_map map;
+} qmm_pair_product;
+
+/* One pair product launch (the per-expert product of reference
+ * src/metaljax/moe.py:1283-1340 and what follows it there, :1425-1461). */
+int qmm_pair_product_run(const qmm_pair_product* product, void* stream);
+
 #define QMM_ROW_LEAVES 8
 #define QMM_ROW_CODE 48
 #define QMM_ROW_OUTS 2

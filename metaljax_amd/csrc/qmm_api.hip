@@ -478,6 +478,24 @@ bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, 
   return bytes <= kTermsBytes || (bytes <= kTermsBytesMost && P * (N * K / 2) >= 3 * bytes);
 }
 
+}  // namespace
+
+// How the general MXFP4 decode kernel would take these pairs: 1 each a product of its
+// own, 2 sorted by the kernel itself, 0 not at all (another kernel, or the sort's launch).
+int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype) {
+  if (P <= 0 || P > kGatherGemvMaxPairs || !aligned16(x)) return 0;
+  const int terms = act_terms(x_dtype);
+  const size_t any = ~(size_t)0 / 4;               // (the route of a call with all the scratch it asks for)
+  if (terms > 1 ? !terms_in_kernel(x, terms, P, E, N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, y_dtype, any)
+                : E > 65535 || N > INT32_MAX || K > INT32_MAX || N * K >= (1ll << 40) ||
+                      !gemv_runs_general(N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, E))
+    return 0;
+  if (!sorts_general(P, E, any)) return 1;
+  return sorts_itself(P, E, N) ? 2 : 0;
+}
+
+namespace {
+
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Scratch of the bf16 dense / grouped product over `rows` rows.  `exact`: the

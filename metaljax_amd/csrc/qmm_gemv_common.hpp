@@ -107,4 +107,83 @@ __device__ __forceinline__ void load_args_now(const GemvArgs& a) {
                "s"(a.n_xrows), "s"(a.segments), "s"(a.src_row), "s"(a.out_row), "s"(a.x_rows));
 }
 
+// The rows of a workgroup, for up to 64 pairs that nobody has sorted: every wavefront
+// holds the pairs' experts, one a lane, and goes through those that occur in order of
+// their first pair; each takes a row of workgroups per sixteen of its pairs.  Leaves the
+// pairs of segment z in rows[wave][] and returns how many there are (0: no such segment;
+// the same for the whole workgroup).  A few instructions an expert; the sort is a launch
+// of its own otherwise: 64 pairs over 8 experts of 1024 x 1024 11.5 -> 8.4 us, four-bit or
+// eight-bit codes or MXFP4 (the host takes 8 a call), the three terms of float32 rows
+// over affine codes 33 -> 24.
+__device__ __forceinline__ int take_segment(const int32_t* experts_of, int pairs, int n_experts, int z, int lane, int* rows, int64_t& expert) {
+  int e = -1;
+  if (lane < pairs) e = experts_of[lane];
+  uint64_t left = __ballot(e >= 0 && e < n_experts);
+  while (left) {
+    const int of = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+    const uint64_t same = __ballot(e == of);
+    const int n = __popcll(same), segments = (n + 15) / 16;
+    if (z < segments) {
+      const int at = __popcll(same & ((1ull << lane) - 1)) - 16 * z;
+      if (e == of && at >= 0 && at < 16) rows[at] = lane;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      expert = of;
+      return n - 16 * z < 16 ? n - 16 * z : 16;
+    }
+    z -= segments;
+    left &= ~same;
+  }
+  return 0;
+}
+
+// Eight activations as TERMS bf16 operands: bf16 as they are, float16 / float32 cut off
+// term by term (exact; inf and NaN stay in the first term, a NaN stays one).  The upper
+// halves of what is left are the terms as they are, five instructions a value; where any
+// of the eight is not finite the last remainder is a NaN and they are done one by one
+// (24 instructions a value; all of them so, and with four chunks in flight of which a
+// wavefront had two, 6 pairs over 8 experts of 1024 x 1024 took 18.0 us instead of 7.4).
+template <int TERMS>
+__device__ __forceinline__ void operand_terms(const u32x4* raw, bf16x8* out) {
+  if constexpr (TERMS == 1) {
+    out[0] = __builtin_bit_cast(bf16x8, raw[0]);
+  } else {
+    float v[8], left[8];
+    uint32_t hi[TERMS][8];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (TERMS == 3) v[e] = __uint_as_float(raw[e >> 2][e & 3]);
+      else v[e] = f16_bits_to_f32((uint16_t)(e & 1 ? raw[0][e >> 1] >> 16 : raw[0][e >> 1] & 0xFFFFu));
+      left[e] = v[e];
+#pragma unroll
+      for (int term = 0; term < TERMS; ++term) {
+        hi[term][e] = __float_as_uint(left[e]);
+        if (term + 1 < TERMS) left[e] -= __uint_as_float(hi[term][e] & 0xFFFF0000u);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) finite = finite && !__builtin_isunordered(left[e], left[e + 1]);
+    if (!finite) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+#pragma unroll
+        for (int term = 0; term < TERMS; ++term) {
+          hi[term][e] = __float_as_uint(v[e]);
+          if (v[e] != v[e]) hi[term][e] |= 0x00400000u;
+          const uint32_t cut = hi[term][e] & 0xFFFF0000u;
+          v[e] = (cut & 0x7F800000u) == 0x7F800000u ? 0.f : v[e] - __uint_as_float(cut);
+        }
+      }
+    }
+#pragma unroll
+    for (int term = 0; term < TERMS; ++term) {
+      const uint32_t* h = hi[term];                // (the upper halves of two)
+      out[term] = as_bf16x8(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u), __builtin_amdgcn_perm(h[3], h[2], 0x07060302u),
+                            __builtin_amdgcn_perm(h[5], h[4], 0x07060302u), __builtin_amdgcn_perm(h[7], h[6], 0x07060302u));
+    }
+  }
+}
+
 }  // namespace qmm

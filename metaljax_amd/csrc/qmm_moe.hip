@@ -21,12 +21,14 @@
 // barrier is needed between instructions), arithmetic in float32, one rounding to the
 // value's element type an instruction -- what an array operation of that type does.
 #include "../../include/qmm_hip.h"
-#include "qmm_common.hpp"
+#include "qmm_gemv_common.hpp"
 
 namespace qmm {
 
 int moe_fail(int code, const char* what);        // qmm_api.hip: sets qmm_last_error
 int moe_launched(const char* what);
+int64_t skinny2_max_segments(int64_t P, int64_t E);
+int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype);
 
 namespace {
 
@@ -115,6 +117,19 @@ __device__ __forceinline__ T uniform(const T& in) {
 }
 
 constexpr int kThreads = 256;
+// The sum over a token's pairs reads an expert's weight for each of them, where sorted
+// pairs share it: while that is no more than the last-level caches deliver in the time of
+// the launch that it spares.
+constexpr int64_t kSumBytes = 16 << 20;
+
+// A pair map's program over a lane's column of the register file.
+__device__ __forceinline__ void run_map(const qmm_instruction* code, int instructions, float* r) {
+  for (int n = 0; n < instructions; ++n) {
+    const qmm_instruction q = uniform(code[n]);
+    const float v = q.op == QMM_OP_IMM ? q.imm : apply(q.op, r[q.a * kThreads], r[q.b * kThreads], r[q.c * kThreads]);
+    r[q.dst * kThreads] = round_to(v, q.el);
+  }
+}
 
 // One output element a thread: its leaves are requested together (one round trip
 // for all of them), then the program runs over its column of the register file.
@@ -152,11 +167,7 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
 #pragma unroll
     for (int j = 0; j < QMM_MAP_LEAVES; ++j)
       if (j < a.leaves) r[j * kThreads] = widen_raw(raw[j], el[j]);
-    for (int n = 0; n < a.instructions; ++n) {
-      const qmm_instruction q = uniform(code[n]);
-      const float v = q.op == QMM_OP_IMM ? q.imm : apply(q.op, r[q.a * kThreads], r[q.b * kThreads], r[q.c * kThreads]);
-      r[q.dst * kThreads] = round_to(v, q.el);
-    }
+    run_map(code, a.instructions, r);
     const float v = r[a.result * kThreads];
     if (!a.weights) {
       store_el(a.y, row * a.inner + i, v, a.y_el);
@@ -165,6 +176,184 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
     total += round_to(v, a.sum_el) * widen_raw(load_raw(a.weights, p, a.weights_el), a.weights_el);
   }
   store_el(a.y, row * a.inner + i, total, a.y_el);
+}
+
+// A product of MXFP4 experts and the pair map behind it, one launch.  A workgroup takes
+// sixteen output elements of a pair (HERE: of up to sixteen pairs of one expert; SUM: of a
+// token, WAVES wavefronts a pair, THREADS at most) and multiplies the weight rows that these read: tile t's
+// row r is column col_base[t] + col_step[t] * element of the product.  The multiplication
+// is the general decode kernel's (gemv_mxfp4_kernel: the same operands, sums and order);
+// its sums meet in LDS, where the map finds them as leaves.
+//
+// What bounds it: one round trip after the other -- arguments, the pair's expert, the
+// weight -- with the map's memory leaves requested ahead of the weight: 6 pairs over 8
+// experts of 2048 x 1024 and a map of two columns 10.8 us, of 1024 x 1024 and the sum of
+// a token's two pairs 8.2.  As two launches each took 7.7 + 5.3 and the gap between them.
+template <int T, int WAVES, int TERMS, int THREADS>
+__global__ __launch_bounds__(THREADS ? THREADS : kWave* WAVES) void pair_product_kernel(qmm_pair_product a) {
+  constexpr bool SUM = THREADS > 0;
+  constexpr int XW = TERMS == 3 ? 2 : 1;           // 16-byte pieces of eight activations
+  constexpr int U = THREADS == 1024 ? 1 : 2;       // macro chunks of 128 k whose loads are under way together (as registers allow)
+  extern __shared__ float smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slice = wave % WAVES, group = wave / WAVES;
+  const int r = lane & 15, kg = lane >> 4;
+  const int all = SUM ? a.map.per_token * WAVES : WAVES;
+  float* const red = smem;                         // [TERMS][all][T][4][64]
+  float* const regs = red + TERMS * all * T * 4 * kWave;
+  qmm_instruction* const code = reinterpret_cast<qmm_instruction*>(regs + a.map.registers * kThreads);
+  int* const taken = reinterpret_cast<int*>(code + QMM_MAP_CODE) + wave * 16;
+  float* const addends = reinterpret_cast<float*>(reinterpret_cast<int*>(code + QMM_MAP_CODE) + 16 * 16);    // [2][256]
+  if ((int)threadIdx.x < a.map.instructions) code[threadIdx.x] = a.map.code[threadIdx.x];
+
+  // ---- the pairs of this workgroup and the expert of this wavefront's
+  const int z = (int)blockIdx.y, last = a.map.experts - 1;
+  auto expert_of = [&](int p) __attribute__((always_inline)) {
+    const int e = a.map.experts_of[p];
+    return e < 0 ? 0 : e > last ? last : e;
+  };
+  int rows = SUM ? a.map.per_token : 1;
+  int64_t e;
+  if (!SUM && a.sorted) {
+    rows = take_segment(a.map.experts_of, (int)a.map.pairs, a.map.experts, z, lane, taken, e);
+    if (rows == 0) return;                         // uniform, before any barrier
+  } else {
+    e = __builtin_amdgcn_readfirstlane(expert_of(SUM ? z * a.map.per_token + group : z));
+  }
+  // row m of the workgroup is pair ...
+  auto pair_of = [&](int m) __attribute__((always_inline)) { return SUM ? z * a.map.per_token + m : a.sorted ? taken[m] : z; };
+
+  // ---- the element of this thread (the first 256) and what its map reads from memory
+  const int em = (threadIdx.x & 255) >> 4, er = threadIdx.x & 15;
+  const int inner = (int)a.map.inner, element = (int)blockIdx.x * 16 + er;
+  const bool mine = threadIdx.x < 256 && em < rows && element < inner;
+  const int ep = mine ? pair_of(em) : 0;
+  Raw raw[QMM_MAP_LEAVES], weight{0u, 0u};
+  if (mine) {
+    const int ee = SUM ? expert_of(ep) : (int)e, et = ep / a.map.per_token;
+#pragma unroll
+    for (int j = 0; j < QMM_MAP_LEAVES; ++j) {
+      if (j < a.map.leaves && a.map.leaf[j].p) {
+        const qmm_map_leaf& l = a.map.leaf[j];
+        raw[j] = load_raw(l.p, l.base + (int64_t)ep * l.pair + (int64_t)ee * l.expert + (int64_t)et * l.token + (int64_t)element * l.coef[2], l.el);
+      }
+    }
+    if constexpr (SUM) weight = load_raw(a.map.weights, ep, a.map.weights_el);
+  }
+
+  // ---- the product
+  const int64_t wpr = a.k / 8;
+  const int nblk = (int)(a.k / 32), chunks = (nblk + 3) / 4;
+  const int c0 = (int)((int64_t)chunks * slice / WAVES), c1 = (int)((int64_t)chunks * (slice + 1) / WAVES);
+  const uint32_t* wrow[T];
+  const uint8_t* srow[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    int i = (int)blockIdx.x * 16 + r;
+    if (i >= inner) i = inner - 1;
+    const int64_t n = e * a.n + a.col_base[t] + (int64_t)i * a.col_step[t];
+    wrow[t] = static_cast<const uint32_t*>(a.w) + n * wpr;
+    srow[t] = static_cast<const uint8_t*>(a.s) + n * nblk;
+  }
+  int64_t src = -1;
+  if (SUM ? r == 0 : r < rows) src = pair_of(SUM ? group : r) / a.x_per;
+  const bool xvalid = src >= 0 && src < a.x_rows;
+  const uint16_t* xrow = static_cast<const uint16_t*>(a.x) + (xvalid ? src : 0) * a.k * XW;
+  f32x4 acc[TERMS][T];
+#pragma unroll
+  for (int term = 0; term < TERMS; ++term)
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[term][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int cb = c0; cb < c1; cb += U) {
+    u32x4 q[U][T];
+    uint8_t sraw[U][T];
+    u32x4 xr[U][4][XW];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int blk = (cb + u) * 4 + kg;
+      const bool live = cb + u < c1 && blk < nblk;
+      if (!live) blk = nblk - 1;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        q[u][t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[t] + (int64_t)blk * 4));
+        sraw[u][t] = srow[t][blk];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < XW; ++h) {
+          xr[u][j][h] = u32x4{0u, 0u, 0u, 0u};
+          if (xvalid && live) xr[u][j][h] = *reinterpret_cast<const u32x4*>(xrow + ((int64_t)blk * 32 + j * 8) * XW + h * 8);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float sc[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) sc[t] = e8m0_to_f32(sraw[u][t]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        bf16x8 xa[TERMS];                          // (zero where not live)
+        operand_terms<TERMS>(xr[u][j], xa);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const bf16x8 wq = widen_e2m1(q[u][t][j], sc[t]);
+#pragma unroll
+          for (int term = 0; term < TERMS; ++term)
+            acc[term][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[term], wq, acc[term][t], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int term = 0; term < TERMS; ++term)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[(((term * all + wave) * T + t) * 4 + i) * kWave + lane] = acc[term][t][i];
+  __syncthreads();
+
+  // ---- the map
+  float* const file = regs + (threadIdx.x & 255);
+  float v = 0.f;
+  if (mine) {
+#pragma unroll
+    for (int j = 0; j < QMM_MAP_LEAVES; ++j)
+      if (j < a.map.leaves && a.map.leaf[j].p) file[j * kThreads] = widen_raw(raw[j], a.map.leaf[j].el);
+    // (SUM: a pair's row is the first of its wavefronts' sixteen)
+    const int first = SUM ? em * WAVES : 0, l = SUM ? er : 16 * (em >> 2) + er, i = SUM ? 0 : em & 3;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      float total = 0.f;
+#pragma unroll
+      for (int term = TERMS - 1; term >= 0; --term) {            // smallest first, in pairs: as gemv_mxfp4_kernel
+        float part[WAVES];
+#pragma unroll
+        for (int wv = 0; wv < WAVES; ++wv) part[wv] = red[(((term * all + first + wv) * T + t) * 4 + i) * kWave + l];
+#pragma unroll
+        for (int d = 1; d < WAVES; d *= 2)
+#pragma unroll
+          for (int wv = 0; wv < WAVES; wv += 2 * d) part[wv] += part[wv + d];
+        total = term == TERMS - 1 ? part[0] : total + part[0];
+      }
+      file[a.col_leaf[t] * kThreads] = round_to(total, a.product_el);
+    }
+    run_map(code, a.map.instructions, file);
+    v = file[a.map.result * kThreads];
+    if constexpr (!SUM) store_el(a.map.y, (int64_t)ep * inner + element, v, a.map.y_el);
+  }
+  if constexpr (SUM) {
+    if (mine) {
+      addends[threadIdx.x] = round_to(v, a.map.sum_el);
+      addends[256 + threadIdx.x] = widen_raw(weight, a.map.weights_el);
+    }
+    __syncthreads();
+    if (threadIdx.x >= 16 || element >= inner) return;
+    float total = 0.f;
+    for (int k = 0; k < rows; ++k) total += addends[k * 16 + er] * addends[256 + k * 16 + er];
+    store_el(a.map.y, (int64_t)z * inner + element, total, a.map.y_el);
+  }
 }
 
 constexpr int kRowThreads = 1024;
@@ -263,21 +452,12 @@ __global__ __launch_bounds__(kRowThreads) void row_program_kernel(qmm_row_progra
 bool float_el(int el) { return el == QMM_EL_F32 || el == QMM_EL_BF16 || el == QMM_EL_F16; }
 bool map_op(int op) { return op >= QMM_OP_COPY && op <= QMM_OP_IMM; }
 
-}  // namespace
-}  // namespace qmm
-
-using namespace qmm;
-
-extern "C" {
-
 // Every index that the program holds is checked here: what the kernel computes from
 // it then stays inside the register file; addresses are the caller's shapes.
-int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
-  if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
+int check_map(const qmm_pair_map* a, bool product) {
   if (a->pairs < 0 || a->inner < 0 || a->per_token < 1 || a->pairs % a->per_token || a->experts < 1 || a->rank < 1 || a->rank > 3)
     return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: shape");
   if (a->pairs == 0 || a->inner == 0) return QMM_OK;
-  const int64_t rows = a->weights ? a->pairs / a->per_token : a->pairs;
   if (a->inner > INT32_MAX - kThreads) return moe_fail(QMM_ERR_BAD_SHAPE, "pair map: a larger result than a grid takes");
   int64_t n = 1;
   for (int i = 0; i < a->rank; ++i) {
@@ -290,18 +470,90 @@ int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
       a->registers < 1 || a->registers > QMM_MAP_REGISTERS || a->leaves > a->registers || a->result < 0 || a->result >= a->registers)
     return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: program size");
   for (int i = 0; i < a->leaves; ++i)
-    if (!a->leaf[i].p || a->leaf[i].el < 0 || a->leaf[i].el > QMM_EL_BOOL) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: leaf");
+    if ((!a->leaf[i].p && !product) || a->leaf[i].el < 0 || a->leaf[i].el > QMM_EL_BOOL) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: leaf");
   for (int i = 0; i < a->instructions; ++i) {
     const qmm_instruction& q = a->code[i];
     if (!map_op(q.op) || q.dst >= a->registers || q.a >= a->registers || q.b >= a->registers || q.c >= a->registers || !float_el(q.el))
       return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair map: instruction");
   }
+  return QMM_OK;
+}
+
+template <int T, int WAVES, int TERMS>
+void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t rest, hipStream_t st) {
+  const int all = a.map.weights ? a.map.per_token * WAVES : WAVES;
+  const size_t lds = (size_t)TERMS * all * T * 4 * kWave * 4 + rest;
+  if constexpr (T == 1) {
+    if (a.map.weights) {
+      if (all <= 8) hipLaunchKernelGGL((pair_product_kernel<T, WAVES, TERMS, 512>), grid, dim3(kWave * all), lds, st, a);
+      else hipLaunchKernelGGL((pair_product_kernel<T, WAVES, TERMS, 1024>), grid, dim3(kWave * all), lds, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((pair_product_kernel<T, WAVES, TERMS, 0>), grid, dim3(kWave * all), lds, st, a);
+}
+
+template <int T, int WAVES>
+void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t rest, hipStream_t st) {
+  if (a.x_el == QMM_EL_F32) launch_pair_product<T, WAVES, 3>(a, grid, rest, st);
+  else if (a.x_el == QMM_EL_F16) launch_pair_product<T, WAVES, 2>(a, grid, rest, st);
+  else launch_pair_product<T, WAVES, 1>(a, grid, rest, st);
+}
+
+}  // namespace
+}  // namespace qmm
+
+using namespace qmm;
+
+extern "C" {
+
+int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
+  if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
+  const int rc = check_map(a, false);
+  if (rc || a->pairs == 0 || a->inner == 0) return rc;
+  const int64_t rows = a->weights ? a->pairs / a->per_token : a->pairs;
   // (a grid's second axis ends at 65535; with more rows than that the third takes part)
   const int64_t planes = ceil_div(rows, 65535);
   const dim3 grid((unsigned)ceil_div(a->inner, kThreads), (unsigned)ceil_div(rows, planes), (unsigned)planes);
   const size_t lds = (size_t)a->registers * kThreads * 4 + sizeof(a->code) + sizeof(a->leaf);
   hipLaunchKernelGGL(pair_map_kernel, grid, dim3(kThreads), lds, static_cast<hipStream_t>(stream), *a);
   return moe_launched("pair map launch");
+}
+
+int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
+  if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
+  const int rc = check_map(&a->map, true);
+  if (rc) return rc;
+  const qmm_pair_map& m = a->map;
+  if (!a->x || !a->w || !a->s || !float_el(a->x_el) || !float_el(a->product_el) || a->x_rows < 0 || a->x_per < 1 || a->n < 1 || a->k < 1 || a->k % 32)
+    return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: operands");
+  if (a->tiles < 1 || a->tiles > 2) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: tiles");
+  if (m.pairs == 0 || m.inner == 0) return QMM_OK;
+  uint32_t from_product = 0;
+  for (int t = 0; t < a->tiles; ++t) {
+    if (a->col_leaf[t] < 0 || a->col_leaf[t] >= m.leaves || a->col_base[t] < 0 || a->col_step[t] < 0 ||
+        a->col_base[t] + (m.inner - 1) * (int64_t)a->col_step[t] >= a->n)
+      return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: columns");
+    from_product |= 1u << a->col_leaf[t];
+  }
+  for (int i = 0; i < m.leaves; ++i)
+    if (!m.leaf[i].p != (from_product >> i & 1)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: leaf");
+  if (m.rank != 1) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: a result of several axes a pair");
+  int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el);
+  const int waves = a->k > 2048 ? 8 : 4;           // (more than 2048 codes: gemv_terms_dispatch)
+  if (m.weights && (a->tiles > 1 || m.per_token * waves > 16 || (route == 2 && m.pairs * (a->n * a->k / 2) > kSumBytes))) route = 0;
+  if (!route || (reinterpret_cast<uintptr_t>(a->w) & 15u)) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: two launches are better");
+  const int64_t segments = m.weights ? m.pairs / m.per_token : route == 2 ? skinny2_max_segments(m.pairs, m.experts) : m.pairs;
+  qmm_pair_product p = *a;
+  p.sorted = route == 2;
+  const dim3 grid((unsigned)ceil_div(m.inner, 16), (unsigned)segments);
+  const size_t rest = (size_t)m.registers * kThreads * 4 + sizeof(m.code) + 16 * 16 * 4 + 2 * 256 * 4;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a->tiles == 1 && waves == 4) launch_pair_product<1, 4>(p, grid, rest, st);
+  else if (a->tiles == 1) launch_pair_product<1, 8>(p, grid, rest, st);
+  else if (waves == 4) launch_pair_product<2, 4>(p, grid, rest, st);
+  else launch_pair_product<2, 8>(p, grid, rest, st);
+  return moe_launched("pair product launch");
 }
 
 int qmm_row_program_run(const qmm_row_program* a, void* stream) {

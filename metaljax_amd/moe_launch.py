@@ -49,6 +49,7 @@ MAX_DEPTH = 2 * ROW_CODE        # operations followed up from a value (the recur
 # whole router weight; larger ones stay a library product.
 MAX_ROUTER_MACS = 1 << 23
 
+_UNSUPPORTED = 3
 _i32, _i64, _vp, _u8 = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p, ctypes.c_uint8
 
 
@@ -66,6 +67,12 @@ class PairMap(ctypes.Structure):
                [(n, _i32) for n in ("per_token", "experts", "rank", "y_el", "sum_el", "weights_el", "leaves",
                                     "instructions", "registers", "result")] + \
                [("leaf", MapLeaf * LEAVES), ("code", Instruction * CODE)]
+
+
+class PairProduct(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("x", "w", "s")] + [(n, _i64) for n in ("x_rows", "n", "k")] + \
+               [(n, _i32) for n in ("x_el", "x_per", "product_el", "tiles")] + \
+               [(n, _i32 * 2) for n in ("col_leaf", "col_base", "col_step")] + [("sorted", _i32), ("map", PairMap)]
 
 
 class RowInstruction(ctypes.Structure):
@@ -113,6 +120,16 @@ def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n
                             n, k, match.gs, match.bits, kernels._MODE[match.mode], None if ws is None else ws.data_ptr(), nbytes, stream)
     if rc:
         _lib.check(rc)
+
+
+def run_pair_product(program, stream) -> bool:
+    """False: not where this library takes a product and its map as two launches."""
+    rc = _lib.load().qmm_pair_product_run(ctypes.byref(program), stream)
+    if rc == _UNSUPPORTED:
+        return False
+    if rc:
+        _lib.check(rc)
+    return True
 
 
 def run_rows(program, stream):
@@ -712,9 +729,30 @@ class Launches:
         def place(n, el):
             at, self.buffer = self.buffer, (self.buffer + n * SIZE[el] + 255) // 256 * 256
             return at
+        self.fused = [self._fused(d) for d in self.dots]
         self.at_experts, self.at_weights = place(g.P, "i32"), place(g.P, elem(g.router.weights))
         self.at_feed = [place(g.P * d.info.k, d.feed[2]) if d.feed else None for d in self.dots]
         self.at_dot = [place(g.P * d.n, d.out_el) for d in self.dots]
+
+    def _fused(self, d):
+        """A product with the one map that reads it, the next product's activations or
+        the result: the launch's program without its addresses.  None: two launches."""
+        behind = self.dots[d.number + 1:d.number + 2]
+        if behind and behind[0].feed is None:
+            return None
+        built, program = behind[0].feed[:2] if behind else (self.final_map, self.final)
+        maps = [other.feed[0] for other in self.dots if other.feed] + [self.final_map]
+        if any(source == ("dot", d.number) for m in maps if m is not built for source, _ in m.leaves):
+            return None
+        mine = [(i, leaf) for i, (source, leaf) in enumerate(built.leaves) if source[0] == "dot"]
+        if not 1 <= len(mine) <= 2 or any(built.leaves[i][0][1] != d.number for i, _ in mine) or program.rank != 1:
+            return None
+        p = PairProduct(n=d.n, k=d.info.k, product_el=ELS[d.out_el], tiles=len(mine))
+        for t, (i, leaf) in enumerate(mine):
+            p.col_leaf[t], p.col_base[t], p.col_step[t] = i, leaf.base, leaf.coef[2]
+        p.map = program
+        p.map.pairs, p.map.experts = self.g.P, self.g.E
+        return p
 
     # -- a call
 
@@ -753,32 +791,61 @@ class Launches:
         else:
             experts, weights = inputs[r.indices].data_ptr(), inputs[r.weights].data_ptr()
 
-        def launch(built, program, y, summed=None):
-            m = _copy(program)
+        def fill(m, built, y, summed, fused=False):
             for i, (source, _) in enumerate(built.leaves):
-                m.leaf[i].p = at(source[1]).data_ptr() if source[0] == "env" else base + self.at_dot[source[1]]
+                if source[0] == "env":
+                    m.leaf[i].p = at(source[1]).data_ptr()
+                elif not fused:
+                    m.leaf[i].p = base + self.at_dot[source[1]]
             m.y, m.experts_of, m.pairs, m.experts = y, experts, g.P, g.E
             if summed is not None:
                 m.weights, m.weights_el = summed, ELS[elem(r.weights)]
+
+        def launch(built, program, y, summed=None):
+            m = _copy(program)
+            fill(m, built, y, summed)
             run_map(m, stream)
 
+        total = torch.empty([g.T] + self.rest, dtype=qmm._torch_dtype(g.out_el), device=device)
+        done = False                                    # is the map ahead of the next product's, or the last one, launched?
         for d, feed, y in zip(self.dots, self.at_feed, self.at_dot):
             info = d.info
             arrays = qmm.pack_arrays(interp, info.match)
+            fused, behind = self.fused[d.number], d.number + 1 < len(self.dots)
+            if fused is not None and device.type == "cuda" and info.match.mode == "mxfp4" and not info.match.has_perm:
+                if d.feed is not None and not done:
+                    launch(d.feed[0], d.feed[1], base + feed)
+                done = True
+                p = _copy(fused)
+                if d.feed is None:
+                    p.x, p.x_rows, p.x_el, p.x_per = at(info.data).data_ptr(), g.T, ELS[elem(info.data)], g.K
+                else:
+                    p.x, p.x_rows, p.x_el, p.x_per = base + feed, g.P, ELS[d.feed[2]], 1
+                arrays = inputs[d] = [a if a.is_contiguous() else a.contiguous() for a in arrays[:2]]
+                p.w, p.s = arrays[0].data_ptr(), arrays[1].data_ptr()
+                if behind:
+                    fill(p.map, self.dots[d.number + 1].feed[0], base + self.at_feed[d.number + 1], None, True)
+                else:
+                    fill(p.map, self.final_map, total.data_ptr(), weights, True)
+                if run_pair_product(p, stream):
+                    moe.STATS["gather_qmm"] += 1
+                    continue
             if d.feed is None:
                 rows, el, lhs = g.T, elem(info.data), g.pair_tokens(device)[0].data_ptr()
                 x = at(info.data).data_ptr()
             else:
                 rows, el, lhs, x = g.P, d.feed[2], None, base + feed
-                launch(d.feed[0], d.feed[1], x)
+                if not done:
+                    launch(d.feed[0], d.feed[1], x)
+            done = False
             if info.match.has_perm:
                 whole = at(info.data) if d.feed is None else buffer[feed:feed + rows * info.k * SIZE[el]].view(qmm._torch_dtype(el))
                 taken = inputs[d] = kernels.take_k(whole.reshape(rows, info.k), arrays[-1])
                 x = taken.data_ptr()
             run_product(x, el, rows, arrays, info.match, lhs, experts, base + y, d.out_el, g.P, g.E, d.n, info.k, buffer, stream)
             moe.STATS["gather_qmm"] += 1
-        total = torch.empty([g.T] + self.rest, dtype=qmm._torch_dtype(g.out_el), device=device)
-        launch(self.final_map, self.final, total.data_ptr(), weights)
+        if not done:
+            launch(self.final_map, self.final, total.data_ptr(), weights)
         return total
 
 

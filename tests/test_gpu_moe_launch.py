@@ -138,3 +138,28 @@ def test_pair_tokens_are_there_for_another_stream():
     assert seen[0].dtype == torch.int32 and seen[1].dtype == torch.int64
     assert torch.equal(seen[0].cpu().long(), want) and torch.equal(seen[1].cpu(), want)
     stream.synchronize()
+
+
+@pytest.mark.parametrize("el", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("E,Tk,H,Ii,K,fused", [
+    (1, 1, 32, 32, 1, 2), (4, 1, 160, 96, 4, 2), (8, 3, 1024, 1024, 2, 2), (8, 5, 96, 2080, 2, 2), (8, 7, 4160, 32, 1, 2),
+    (4, 32, 512, 96, 2, 2), (8, 64, 288, 64, 1, 2), (8, 33, 64, 64, 2, 0), (3, 11, 1056, 544, 3, 2), (5, 2, 64, 32, 5, 1)])
+def test_a_product_and_its_map_in_one_launch(E, Tk, H, Ii, K, fused, el, monkeypatch):
+    """Pairs of their own, pairs sorted by the kernel, the sum over a token's pairs in two
+    to sixteen wavefronts, K of a part of a chunk and of more than 2048: what two launches
+    give.  The sums are the same ones in the same order, but for sixteen-bit rows of more
+    than 2048 codes, which take twice the wavefronts here (and a bf16 place)."""
+    raw, _ = _moe_inputs(E, Tk, H, Ii)
+    args = [I.from_numpy(a, el) if a.dtype == np.float32 else I.from_numpy(a) for a in raw]
+    alone, took, out = ML.run_pair_product, [], []
+    for on in (True, False):
+        monkeypatch.setattr(ML, "run_pair_product", lambda p, st, on=on: on and (took.append(alone(p, st)) or took[-1]))
+        ex = engine.compile_program(T.moe_block_mxfp4(E, Tk, H, Ii, K, el=el))
+        (buf,) = engine.execute(ex, args)
+        assert ex.interp._qmm.moe[0].launches is not None
+        out.append(engine.to_numpy(buf)[0])
+    assert took.count(True) == fused or el != "f32"
+    if max(H, Ii) <= 2048 or el == "f32":
+        assert np.array_equal(*out)
+    else:
+        close(*out, "bf16")
