@@ -226,10 +226,10 @@ int qmm_pair_map_run(const qmm_pair_map* map, void* stream);
  * [experts, n, k / 8 words] with block scales s, rounded to product_el; leaf
  * col_leaf[t] of the map (whose p is null) is column col_base[t] + col_step[t] *
  * element of that.  UNSUPPORTED where a product and a map are the better launches
- * (by the sizes, the types and the alignment alone).  `sorted` is the library's. */
+ * (by the mode, the sizes, the types and the alignment alone).  `sorted` is the library's. */
 typedef struct {
   const void *x, *w, *s;
-  int64_t x_rows, n, k;
+  int64_t x_rows, n, k, mode;
   int32_t x_el, x_per, product_el, tiles, col_leaf[2], col_base[2], col_step[2], sorted;
   qmm_pair_map map;
 } qmm_pair_product;
@@ -261,6 +261,31 @@ typedef struct {
 /* One row program launch: a router from its logits to the selected experts and
  * their weights (the graph of reference src/metaljax/moe.py:335-442). */
 int qmm_row_program_run(const qmm_row_program* program, void* stream);
+
+/* The arguments of qmm_gather_qmm. */
+typedef struct {
+  const void *x, *w, *scales, *biases;
+  void* y;
+  const int32_t *lhs_idx, *rhs_idx;
+  void* workspace;
+  int64_t workspace_bytes, table_dtype, group_size, bits, mode, pairs, rows, experts, n, k;
+  int32_t x_dtype, y_dtype;
+} qmm_pair_gather;
+
+/* A call of a compiled dispatch, launch after launch: step i's program, with the
+ * eight bytes at every patch's `at` replaced by values[value] + add, goes to the
+ * entry point that its kind names.  A pair product that is served skips the `skip`
+ * steps behind it, the launches it stands for; one that is not is passed over.  The
+ * programs are only read: several threads may run the same steps.  Stands for the
+ * host side of reference src/metaljax/moe.py:1425-1461. */
+enum { QMM_STEP_ROWS, QMM_STEP_PAIR_PRODUCT, QMM_STEP_MAP, QMM_STEP_GATHER };
+typedef struct { int32_t at, value; int64_t add; } qmm_patch;
+typedef struct {
+  int32_t kind, bytes, patches, skip;
+  const void* program;
+  const qmm_patch* patch;
+} qmm_step;
+int qmm_steps_run(const qmm_step* steps, int64_t n, const uint64_t* values, int64_t n_values, void* stream);
 
 #ifdef __cplusplus
 }

@@ -26,7 +26,7 @@ SYMBOLS = (
     "qmm_abi_version", "qmm_last_error", "qmm_quantized_matmul", "qmm_workspace_bytes",
     "qmm_gather_workspace_bytes", "qmm_plan", "qmm_gather_qmm", "qmm_grouped_qmm",
     "qmm_grouped_qmm_zeroed", "qmm_gather_qmm_static", "qmm_dequantize", "qmm_unpack_codes", "qmm_pack_codes", "qmm_take_k",
-    "qmm_pair_map_run", "qmm_pair_product_run", "qmm_row_program_run",
+    "qmm_pair_map_run", "qmm_pair_product_run", "qmm_row_program_run", "qmm_steps_run",
 )
 
 
@@ -85,6 +85,7 @@ def load():
     lib.qmm_pair_map_run.argtypes = [vp, vp]
     lib.qmm_pair_product_run.argtypes = [vp, vp]
     lib.qmm_row_program_run.argtypes = [vp, vp]
+    lib.qmm_steps_run.argtypes = [vp, i64, vp, i64, vp]
     for name in SYMBOLS:
         getattr(lib, name)
     if lib.qmm_abi_version() != ABI_VERSION:

@@ -20,6 +20,8 @@
 // instruction for every lane, operands in LDS (column of a lane: its own, so that no
 // barrier is needed between instructions), arithmetic in float32, one rounding to the
 // value's element type an instruction -- what an array operation of that type does.
+#include <cstring>
+
 #include "../../include/qmm_hip.h"
 #include "qmm_gemv_common.hpp"
 
@@ -538,7 +540,7 @@ int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
   }
   for (int i = 0; i < m.leaves; ++i)
     if (!m.leaf[i].p != (from_product >> i & 1)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: leaf");
-  if (m.rank != 1) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: a result of several axes a pair");
+  if (m.rank != 1 || a->mode != QMM_MODE_MXFP4) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: a result of several axes a pair, or affine experts");
   int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el);
   const int waves = a->k > 2048 ? 8 : 4;           // (more than 2048 codes: gemv_terms_dispatch)
   if (m.weights && (a->tiles > 1 || m.per_token * waves > 16 || (route == 2 && m.pairs * (a->n * a->k / 2) > kSumBytes))) route = 0;
@@ -588,6 +590,41 @@ int qmm_row_program_run(const qmm_row_program* a, void* stream) {
   const size_t lds = ((size_t)a->reg_floats + (a->dot_x ? kRowThreads : 0)) * 4 + sizeof(a->code);
   hipLaunchKernelGGL(row_program_kernel, dim3((unsigned)a->tokens), dim3(kRowThreads), lds, static_cast<hipStream_t>(stream), *a);
   return moe_launched("row program launch");
+}
+
+int qmm_steps_run(const qmm_step* steps, int64_t n, const uint64_t* values, int64_t n_values, void* stream) {
+  if (n < 0 || (n && !steps) || (n_values && !values)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null steps");
+  union { qmm_row_program rows; qmm_pair_product product; qmm_pair_map map; qmm_pair_gather gather; } u;
+  constexpr size_t sizes[] = {sizeof(u.rows), sizeof(u.product), sizeof(u.map), sizeof(u.gather)};
+  for (int64_t i = 0; i < n; ++i) {
+    const qmm_step& s = steps[i];
+    if (s.kind < QMM_STEP_ROWS || s.kind > QMM_STEP_GATHER || s.bytes < 0 || (size_t)s.bytes != sizes[s.kind] || s.skip < 0 || !s.program || (s.patches && !s.patch))
+      return moe_fail(QMM_ERR_BAD_ARGUMENT, "step");
+    memcpy(&u, s.program, (size_t)s.bytes);
+    for (int j = 0; j < s.patches; ++j) {
+      const qmm_patch& q = s.patch[j];
+      if (q.at < 0 || q.at > s.bytes - 8 || q.value < 0 || q.value >= n_values) return moe_fail(QMM_ERR_BAD_ARGUMENT, "step: patch");
+      const uint64_t v = values[q.value] + (uint64_t)q.add;
+      memcpy(reinterpret_cast<char*>(&u) + q.at, &v, 8);
+    }
+    int rc;
+    if (s.kind == QMM_STEP_PAIR_PRODUCT) {
+      rc = qmm_pair_product_run(&u.product, stream);
+      if (rc == QMM_OK) i += s.skip;
+      if (rc == QMM_ERR_UNSUPPORTED) rc = QMM_OK;
+    } else if (s.kind == QMM_STEP_ROWS) {
+      rc = qmm_row_program_run(&u.rows, stream);
+    } else if (s.kind == QMM_STEP_MAP) {
+      rc = qmm_pair_map_run(&u.map, stream);
+    } else {
+      const qmm_pair_gather& g = u.gather;
+      rc = qmm_gather_qmm(g.x, g.x_dtype, g.w, g.scales, g.biases, (int)g.table_dtype, g.y, g.y_dtype, g.lhs_idx, g.rhs_idx, g.pairs,
+                          g.rows, g.experts, g.n, g.k, (int)g.group_size, (int)g.bits, (int)g.mode, g.workspace,
+                          (size_t)g.workspace_bytes, stream);
+    }
+    if (rc) return rc;
+  }
+  return QMM_OK;
 }
 
 }  // extern "C"

@@ -55,6 +55,7 @@ _ENUM_EL = {
     _ENUM["BF16"]: ("bf16", np.uint16),          # host bytes are the 16-bit patterns
 }
 _EL_ENUM = {el: k for k, (el, _) in _ENUM_EL.items()}
+_ENUM_SIZE = {k: np.dtype(dt).itemsize for k, (_, dt) in _ENUM_EL.items()}
 
 
 class Buffer:
@@ -70,7 +71,7 @@ class Buffer:
         n = 1
         for d in self.dims:
             n *= d
-        self.nbytes = n * np.dtype(_ENUM_EL[self.type_enum][1]).itemsize
+        self.nbytes = n * _ENUM_SIZE[self.type_enum]
 
 
 def buffer_from_host(data, type_enum: int, dims, byte_strides=None, offset: int = 0) -> Buffer:

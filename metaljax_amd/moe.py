@@ -45,8 +45,8 @@ import os
 
 import numpy as np
 
-from . import ir
-from .interpreter import REGISTRY, HostArray, host, settle
+from . import ir, qmm
+from .interpreter import HOST_COPIES, REGISTRY, HostArray, host, settle
 from .packing import Reject
 from .recognize import OPAQUE_OPS, count, dims_of, elem, op_key
 
@@ -788,9 +788,6 @@ class Dispatch:
         """The closure list on the device, then the routing-weighted sum over
         each token's K pairs.  The only host data read are the router's indices
         when the program computed them on the host (an upload, no copy back)."""
-        import torch
-        from . import qmm
-        from .interpreter import HOST_COPIES
         copies = HOST_COPIES[0]
         if self.launches is not None:
             return self._finish(self.launches.run(interp, env), copies)
@@ -814,11 +811,8 @@ class Dispatch:
         return self._finish(combine(yd, wd), copies)
 
     def _finish(self, total, copies):
-        import torch
-        from . import qmm
-        from .interpreter import HOST_COPIES
         if self.out_axis:
-            total = torch.movedim(total, 0, self.out_axis)
+            total = total.movedim(0, self.out_axis)
         if list(total.shape) != self.out_shape:
             raise RuntimeError(f"expert dispatch produced {list(total.shape)}, expected {self.out_shape}")
         STATS["dispatches"] += 1
@@ -829,7 +823,6 @@ class Dispatch:
 def pair_experts(env, router):
     """The expert of every pair, int32 on the device, from the program's indices."""
     import torch
-    from . import qmm
     iv = env[router.indices]
     if hasattr(iv, "type_enum") and hasattr(iv, "data"):
         iv = iv.data

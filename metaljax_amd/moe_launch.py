@@ -49,7 +49,6 @@ MAX_DEPTH = 2 * ROW_CODE        # operations followed up from a value (the recur
 # whole router weight; larger ones stay a library product.
 MAX_ROUTER_MACS = 1 << 23
 
-_UNSUPPORTED = 3
 _i32, _i64, _vp, _u8 = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p, ctypes.c_uint8
 
 
@@ -70,9 +69,23 @@ class PairMap(ctypes.Structure):
 
 
 class PairProduct(ctypes.Structure):
-    _fields_ = [(n, _vp) for n in ("x", "w", "s")] + [(n, _i64) for n in ("x_rows", "n", "k")] + \
+    _fields_ = [(n, _vp) for n in ("x", "w", "s")] + [(n, _i64) for n in ("x_rows", "n", "k", "mode")] + \
                [(n, _i32) for n in ("x_el", "x_per", "product_el", "tiles")] + \
                [(n, _i32 * 2) for n in ("col_leaf", "col_base", "col_step")] + [("sorted", _i32), ("map", PairMap)]
+
+
+class PairGather(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("x", "w", "scales", "biases", "y", "lhs_idx", "rhs_idx", "workspace")] + \
+               [(n, _i64) for n in ("workspace_bytes", "table_dtype", "group_size", "bits", "mode", "pairs", "rows", "experts", "n", "k")] + \
+               [(n, _i32) for n in ("x_dtype", "y_dtype")]
+
+
+class Patch(ctypes.Structure):
+    _fields_ = [("at", _i32), ("value", _i32), ("add", _i64)]
+
+
+class Step(ctypes.Structure):
+    _fields_ = [(n, _i32) for n in ("kind", "bytes", "patches", "skip")] + [("program", _vp), ("patch", ctypes.POINTER(Patch))]
 
 
 class RowInstruction(ctypes.Structure):
@@ -105,6 +118,15 @@ def run_map(program, stream):
         _lib.check(rc)
 
 
+STEPS = ROWS, PRODUCT, MAP, GATHER = range(4)                      # QMM_STEP_*
+
+
+def run_steps(steps, values, stream):
+    rc = _lib.load().qmm_steps_run(steps, len(steps), (ctypes.c_uint64 * len(values))(*values), len(values), stream)
+    if rc:
+        _lib.check(rc)
+
+
 def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n, k, like, stream):
     """y [pairs, n] = row lhs[p] of x [rows, k] (row p without lhs) times expert
     rhs[p] of a match's packed weight; x, lhs, rhs and y are addresses.  `like`: a
@@ -120,16 +142,6 @@ def run_product(x, el, rows, arrays, match, lhs, rhs, y, y_el, pairs, experts, n
                             n, k, match.gs, match.bits, kernels._MODE[match.mode], None if ws is None else ws.data_ptr(), nbytes, stream)
     if rc:
         _lib.check(rc)
-
-
-def run_pair_product(program, stream) -> bool:
-    """False: not where this library takes a product and its map as two launches."""
-    rc = _lib.load().qmm_pair_product_run(ctypes.byref(program), stream)
-    if rc == _UNSUPPORTED:
-        return False
-    if rc:
-        _lib.check(rc)
-    return True
 
 
 def run_rows(program, stream):
@@ -648,7 +660,9 @@ class Launches:
         if g.out_el not in FLOATS or g.sum_el not in FLOATS or elem(r.weights) not in FLOATS:
             raise Reject("a dispatch of other than floats")
         self.final, self.final_map = final.finish(result, g.out_el, g.sum_el), final
-        self.rest = rest
+        import torch
+        self.result = [g.T] + rest
+        self.result_type = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[g.out_el]
         self.rows = None
         self.skip_keys = frozenset()
         self.env_reads = self.reads + [r.indices, r.weights]
@@ -717,22 +731,117 @@ class Launches:
         self.skip_keys, self.env_reads = frozenset(skip), keep
 
     def _layout(self):
-        """Where a call's intermediate results lie in its one buffer, and the modules
-        a call needs: looked up once, and ahead of any call -- several threads may make
-        the first one, and none of them changes what the others read."""
+        """Where a call's intermediate results lie in its one buffer, its steps, and the
+        modules it needs: looked up once, and ahead of any call -- several threads may
+        make the first one, and none of them changes what the others read."""
         import torch
         from . import kernels, moe, qmm
         self.modules = torch, kernels, moe, qmm
-        g = self.g
+        g, r = self.g, self.g.router
         self.buffer = 0
 
         def place(n, el):
-            at, self.buffer = self.buffer, (self.buffer + n * SIZE[el] + 255) // 256 * 256
+            return place_bytes(n * SIZE[el])
+
+        def place_bytes(n):
+            at, self.buffer = self.buffer, (self.buffer + n + 255) // 256 * 256
             return at
-        self.fused = [self._fused(d) for d in self.dots]
-        self.at_experts, self.at_weights = place(g.P, "i32"), place(g.P, elem(g.router.weights))
+        self.at_experts, self.at_weights = place(g.P, "i32"), place(g.P, elem(r.weights))
         self.at_feed = [place(g.P * d.info.k, d.feed[2]) if d.feed else None for d in self.dots]
         self.at_dot = [place(g.P * d.n, d.out_el) for d in self.dots]
+        self.workspace = max([kernels._gather_workspace_bytes(g.P, g.E, d.n, d.info.k, _DT[self._rows_of(d)[0]]) for d in self.dots])
+        self.at_workspace = place_bytes(self.workspace)
+        self.inputs = list(dict.fromkeys(v for v in self.env_reads if self.rows is not None or v is not r.indices))
+        self.lhs = any(d.feed is None for d in self.dots)
+        self._steps()
+
+    def _rows_of(self, d):
+        """(element type, number of rows) of what a product multiplies."""
+        return (elem(d.info.data), self.g.T) if d.feed is None else (d.feed[2], self.g.P)
+
+    # A call's values, in this order: its buffer, its result, the pairs' experts,
+    # weights and tokens, the inputs, and of every product the packed weight's
+    # w, scales, biases, table type, group size, bits and mode.
+    BUFFER, RESULT, EXPERTS, WEIGHTS, TOKENS, INPUTS = range(6)
+    OF_PRODUCT = 7
+
+    def _steps(self):
+        """A call as the library's steps: every launch's program and where a call's
+        values go in it.  A product and its map are a step and, behind it, the two
+        that take their place where the library says so."""
+        g, r = self.g, self.g.router
+        steps = []
+
+        def add(kind, program, patches, skip=0, about=None):
+            where = (Patch * len(patches))(*[Patch(*p) for p in patches])
+            steps.append((kind, program, where, skip, about))
+
+        def of(v):
+            return self.INPUTS + self.inputs.index(v)
+
+        def leaf(kind, i):
+            struct = MapLeaf if kind is PairMap else RowLeaf
+            return kind.leaf.offset + i * ctypes.sizeof(struct) + struct.p.offset
+
+        def map_patches(built, summed, y, fused=False):
+            patches = [(PairMap.y.offset, *y), (PairMap.experts_of.offset, self.EXPERTS, 0)]
+            if summed:
+                patches.append((PairMap.weights.offset, self.WEIGHTS, 0))
+            for i, (source, _) in enumerate(built.leaves):
+                if source[0] == "env":
+                    patches.append((leaf(PairMap, i), of(source[1]), 0))
+                elif not fused:
+                    patches.append((leaf(PairMap, i), self.BUFFER, self.at_dot[source[1]]))
+            return patches
+
+        if self.rows is not None:
+            patches = [(leaf(RowProgram, i), of(v), 0) for i, (v, _) in enumerate(self.row_leaves)]
+            if self.row_dot:
+                patches += [(RowProgram.dot_x.offset, of(self.row_dot[1]), 0), (RowProgram.dot_w.offset, of(self.row_dot[2]), 0)]
+            for i, value in enumerate((self.EXPERTS, self.WEIGHTS)):
+                patches.append((RowProgram.out.offset + i * ctypes.sizeof(RowOut) + RowOut.p.offset, value, 0))
+            add(ROWS, self.rows, patches)
+        for m in [d.feed[1] for d in self.dots if d.feed] + [self.final]:
+            m.pairs, m.experts = g.P, g.E
+        self.final.weights_el = ELS[elem(r.weights)]
+        for d in self.dots:                             # (a map ahead of a product is a step of the product before it)
+            at = d.number
+            behind = self.dots[at + 1] if at + 1 < len(self.dots) else None
+            el, rows = self._rows_of(d)
+            x = (of(d.info.data), 0) if d.feed is None else (self.BUFFER, self.at_feed[at])
+            packed = self.INPUTS + len(self.inputs) + self.OF_PRODUCT * at
+            if at == 0 and d.feed is not None:
+                add(MAP, d.feed[1], map_patches(d.feed[0], False, x))
+            if behind is None:
+                after = self.final, map_patches(self.final_map, True, (self.RESULT, 0))
+            elif behind.feed is not None:
+                after = behind.feed[1], map_patches(behind.feed[0], False, (self.BUFFER, self.at_feed[at + 1]))
+            else:
+                after = None
+            fused = self._fused(d)
+            if fused is not None:
+                fused.x_rows, fused.x_el, fused.x_per = rows, ELS[el], g.K if d.feed is None else 1
+                built = behind.feed[0] if behind else self.final_map
+                y = (self.BUFFER, self.at_feed[at + 1]) if behind else (self.RESULT, 0)
+                patches = [(PairProduct.map.offset + o, v, plus) for o, v, plus in map_patches(built, behind is None, y, True)]
+                patches += [(PairProduct.x.offset, *x), (PairProduct.w.offset, packed, 0), (PairProduct.s.offset, packed + 1, 0),
+                            (PairProduct.mode.offset, packed + 6, 0)]
+                add(PRODUCT, fused, patches, 2, d)
+            p = PairGather(workspace_bytes=self.workspace, pairs=g.P, rows=rows, experts=g.E, n=d.n, k=d.info.k,
+                           x_dtype=_DT[el], y_dtype=_DT[d.out_el])
+            patches = [(PairGather.x.offset, *x), (PairGather.y.offset, self.BUFFER, self.at_dot[at]),
+                       (PairGather.rhs_idx.offset, self.EXPERTS, 0), (PairGather.workspace.offset, self.BUFFER, self.at_workspace)]
+            if d.feed is None:
+                patches.append((PairGather.lhs_idx.offset, self.TOKENS, 0))
+            for i, name in enumerate(("w", "scales", "biases", "table_dtype", "group_size", "bits", "mode")):
+                patches.append((getattr(PairGather, name).offset, packed + i, 0))
+            add(GATHER, p, patches, 0, d)
+            if after is not None:
+                add(MAP, *after)
+        self.programs = steps                           # (what the library's steps point at)
+        self.steps = (Step * len(steps))(*[
+            Step(kind, ctypes.sizeof(program), len(where), skip, ctypes.addressof(program), where)
+            for kind, program, where, skip, _ in steps])
 
     def _fused(self, d):
         """A product with the one map that reads it, the next product's activations or
@@ -751,7 +860,6 @@ class Launches:
         for t, (i, leaf) in enumerate(mine):
             p.col_leaf[t], p.col_base[t], p.col_step[t] = i, leaf.base, leaf.coef[2]
         p.map = program
-        p.map.pairs, p.map.experts = self.g.P, self.g.E
         return p
 
     # -- a call
@@ -759,94 +867,71 @@ class Launches:
     def run(self, interp, env):
         torch, kernels, moe, qmm = self.modules
         g, r = self.g, self.g.router
-        inputs = {}                                     # of this call: value -> tensor (kept until its launches are out)
-
-        def at(v):
-            t = inputs.get(v)
-            if t is None:
-                t = env[v]
-                if not isinstance(t, torch.Tensor):
-                    t = moe.dev(t).t
-                elif t.device.type != qmm.DEVICE:
-                    t = t.to(qmm.DEVICE)
-                inputs[v] = t = t if t.is_contiguous() else t.contiguous()
-            return t
-
-        if self.rows is None:
-            inputs[r.indices] = moe.pair_experts(env, r)
-            inputs[r.weights] = at(r.weights)
-        device = at(self.reads[0]).device
-        stream = kernels._raw_stream(device.index) if device.type == "cuda" else 0
+        values, keep = [0] * self.INPUTS, []            # of this call (kept until its launches are out)
+        for v in self.inputs:
+            t = env[v]
+            if not isinstance(t, torch.Tensor):
+                t = moe.dev(t).t
+            elif t.device.type != qmm.DEVICE:
+                t = t.to(qmm.DEVICE)
+            if not t.is_contiguous():
+                t = t.contiguous()
+            keep.append(t)
+            values.append(t.data_ptr())
+        device = keep[0].device
         buffer = torch.empty(self.buffer, dtype=torch.uint8, device=device)
+        total = torch.empty(self.result, dtype=self.result_type, device=device)
         base = buffer.data_ptr()
-        if self.rows is not None:
-            experts, weights = base + self.at_experts, base + self.at_weights
-            p = _copy(self.rows)
-            for i, (v, _) in enumerate(self.row_leaves):
-                p.leaf[i].p = at(v).data_ptr()
-            if self.row_dot:
-                p.dot_x, p.dot_w = at(self.row_dot[1]).data_ptr(), at(self.row_dot[2]).data_ptr()
-            p.out[0].p, p.out[1].p = experts, weights
-            run_rows(p, stream)
+        values[self.BUFFER], values[self.RESULT] = base, total.data_ptr()
+        if self.rows is None:
+            experts = moe.pair_experts(env, r)
+            values[self.EXPERTS], values[self.WEIGHTS] = experts.data_ptr(), keep[self.inputs.index(r.weights)].data_ptr()
         else:
-            experts, weights = inputs[r.indices].data_ptr(), inputs[r.weights].data_ptr()
-
-        def fill(m, built, y, summed, fused=False):
-            for i, (source, _) in enumerate(built.leaves):
-                if source[0] == "env":
-                    m.leaf[i].p = at(source[1]).data_ptr()
-                elif not fused:
-                    m.leaf[i].p = base + self.at_dot[source[1]]
-            m.y, m.experts_of, m.pairs, m.experts = y, experts, g.P, g.E
-            if summed is not None:
-                m.weights, m.weights_el = summed, ELS[elem(r.weights)]
-
-        def launch(built, program, y, summed=None):
-            m = _copy(program)
-            fill(m, built, y, summed)
-            run_map(m, stream)
-
-        total = torch.empty([g.T] + self.rest, dtype=qmm._torch_dtype(g.out_el), device=device)
-        done = False                                    # is the map ahead of the next product's, or the last one, launched?
-        for d, feed, y in zip(self.dots, self.at_feed, self.at_dot):
-            info = d.info
-            arrays = qmm.pack_arrays(interp, info.match)
-            fused, behind = self.fused[d.number], d.number + 1 < len(self.dots)
-            if fused is not None and device.type == "cuda" and info.match.mode == "mxfp4" and not info.match.has_perm:
-                if d.feed is not None and not done:
-                    launch(d.feed[0], d.feed[1], base + feed)
-                done = True
-                p = _copy(fused)
-                if d.feed is None:
-                    p.x, p.x_rows, p.x_el, p.x_per = at(info.data).data_ptr(), g.T, ELS[elem(info.data)], g.K
-                else:
-                    p.x, p.x_rows, p.x_el, p.x_per = base + feed, g.P, ELS[d.feed[2]], 1
-                arrays = inputs[d] = [a if a.is_contiguous() else a.contiguous() for a in arrays[:2]]
-                p.w, p.s = arrays[0].data_ptr(), arrays[1].data_ptr()
-                if behind:
-                    fill(p.map, self.dots[d.number + 1].feed[0], base + self.at_feed[d.number + 1], None, True)
-                else:
-                    fill(p.map, self.final_map, total.data_ptr(), weights, True)
-                if run_pair_product(p, stream):
-                    moe.STATS["gather_qmm"] += 1
-                    continue
-            if d.feed is None:
-                rows, el, lhs = g.T, elem(info.data), g.pair_tokens(device)[0].data_ptr()
-                x = at(info.data).data_ptr()
+            values[self.EXPERTS], values[self.WEIGHTS] = base + self.at_experts, base + self.at_weights
+        if self.lhs:
+            values[self.TOKENS] = g.pair_tokens(device)[0].data_ptr()
+        moe.STATS["gather_qmm"] += len(self.dots)
+        if device.type != "cuda" or any(d.info.match.has_perm for d in self.dots):
+            self._one_by_one(interp, values, buffer, keep)
+            return total
+        for d in self.dots:
+            match = d.info.match
+            arrays = [a if a.is_contiguous() else a.contiguous() for a in qmm.pack_arrays(interp, match)]
+            keep += arrays
+            w, scales = arrays[:2]
+            if match.mode == "affine":
+                values += (w.data_ptr(), scales.data_ptr(), arrays[2].data_ptr(), kernels._dt(scales.dtype), match.gs, match.bits, _lib.MODE_AFFINE)
             else:
-                rows, el, lhs, x = g.P, d.feed[2], None, base + feed
-                if not done:
-                    launch(d.feed[0], d.feed[1], x)
-            done = False
-            if info.match.has_perm:
-                whole = at(info.data) if d.feed is None else buffer[feed:feed + rows * info.k * SIZE[el]].view(qmm._torch_dtype(el))
-                taken = inputs[d] = kernels.take_k(whole.reshape(rows, info.k), arrays[-1])
-                x = taken.data_ptr()
-            run_product(x, el, rows, arrays, info.match, lhs, experts, base + y, d.out_el, g.P, g.E, d.n, info.k, buffer, stream)
-            moe.STATS["gather_qmm"] += 1
-        if not done:
-            launch(self.final_map, self.final, total.data_ptr(), weights)
+                values += (w.data_ptr(), scales.data_ptr(), 0, _lib.BF16, match.gs, match.bits, _lib.MODE_MXFP4)
+        run_steps(self.steps, values, kernels._raw_stream(device.index))
         return total
+
+    def _one_by_one(self, interp, values, buffer, keep):
+        """The steps by way of this module's functions: a weight packed with its
+        contraction axis permuted, whose activations are permuted ahead of a product."""
+        _, kernels, _, qmm = self.modules
+        stream = kernels._raw_stream(buffer.device.index) if buffer.device.type == "cuda" else 0
+        for kind, program, where, _, d in self.programs:
+            if kind == PRODUCT:
+                continue
+            p = _copy(program)
+            for q in where:
+                if q.value < len(values):               # (what a packed weight adds goes to run_product)
+                    ctypes.c_uint64.from_address(ctypes.addressof(p) + q.at).value = values[q.value] + q.add
+            if kind == ROWS:
+                run_rows(p, stream)
+            elif kind == MAP:
+                run_map(p, stream)
+            else:
+                el, rows = self._rows_of(d)
+                arrays, x = qmm.pack_arrays(interp, d.info.match), p.x
+                if d.info.match.has_perm:
+                    at, n = self.at_feed[d.number], rows * d.info.k
+                    whole = keep[self.inputs.index(d.info.data)] if at is None else buffer[at:at + n * SIZE[el]].view(qmm._torch_dtype(el))
+                    keep.append(kernels.take_k(whole.reshape(rows, d.info.k), arrays[-1]))
+                    x = keep[-1].data_ptr()
+                run_product(x, el, rows, arrays, d.info.match, p.lhs_idx, p.rhs_idx, p.y, d.out_el, p.pairs, p.experts, p.n, p.k,
+                            buffer, stream)
 
 
 def compile_dispatch(interp, g, block):

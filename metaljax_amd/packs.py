@@ -467,8 +467,12 @@ class Pack:
         return [a for a in (self.w, self.scales, self.biases, self.perm) if a is not None]
 
     def matches(self, leaves) -> bool:
-        return len(leaves) == len(self.sources) and all(
-            ref() is buf and st == _stamp(buf) for ref, st, buf in zip(self.sources, self.stamps, leaves))
+        if len(leaves) != len(self.sources):
+            return False
+        for ref, st, buf in zip(self.sources, self.stamps, leaves):
+            if ref() is not buf or st != _stamp(buf):
+                return False
+        return True
 
     def alias(self, leaves):
         """The same arrays for another set of source buffers."""

@@ -34,6 +34,7 @@ import os
 import numpy as np
 
 from . import ir, packing, packs, recognize
+from ._lib import QmmLibraryError
 from .interpreter import host
 from .packing import Reject
 from .packs import Pack as _Pack                      # noqa: F401  (the reference's name for it)
@@ -165,7 +166,6 @@ def prologue(interp, args) -> bool:
     st = interp._qmm or analyze(interp)
     if not (st.matches or st.moe):
         return False
-    from ._lib import QmmLibraryError
     rewrite_changed = False
     layout = []
     built = since_reclaim = 0
@@ -203,8 +203,7 @@ def prologue(interp, args) -> bool:
         m.slot, m.nvals = len(layout), len(arrays)
         layout += arrays
     if st.moe:
-        from . import moe
-        if moe.prologue(interp, st):            # a dispatch whose weight did not pack, or that fails its check, runs densely
+        if _late()[2].prologue(interp, st):            # a dispatch whose weight did not pack, or that fails its check, runs densely
             rewrite_changed = True
     if rewrite_changed:
         st.rebuild()
@@ -232,6 +231,20 @@ def reclaim():
 # --------------------------------------------------------------------------
 # runtime
 # --------------------------------------------------------------------------
+
+_LATE = None
+
+
+def _late():
+    """torch and the modules that need it or this one, looked up by the first call that
+    runs something: an import statement costs a call up to a microsecond every time."""
+    global _LATE
+    if _LATE is None:
+        import torch
+        from . import kernels, moe
+        _LATE = torch, kernels, moe, {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
+    return _LATE
+
 
 def values(interp):
     """The packed arrays of the last prologue, in slot order: the explicit
@@ -280,8 +293,7 @@ def emit_bytes(m) -> int:
 
 
 def _torch_dtype(el):
-    import torch
-    return {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[el]
+    return _late()[3][el]
 
 
 # Where the tensors of the fused calls and of a running expert dispatch live.
@@ -292,7 +304,7 @@ DEVICE = "cuda"
 
 def to_device(v):
     """A runtime value as a device tensor (bf16 HostArrays become bfloat16)."""
-    import torch
+    torch = _late()[0]
     if isinstance(v, torch.Tensor):
         return v if v.device.type == DEVICE else v.to(DEVICE)
     h = host(v)
@@ -308,10 +320,9 @@ def to_device(v):
 def emit(interp, m, env):
     """One fused quantized matmul in place of the whole dequant-and-dot
     (reference qmm.py:2469-2501)."""
+    _, kernels, moe, _ = _late()
     if not isinstance(m, Match):
-        from . import moe
         return moe.emit(interp, m, env)
-    from . import kernels
     st = interp._qmm
     vals = st.values[m.slot:m.slot + m.nvals]
     w, scales = vals[0], vals[1]

@@ -2,12 +2,14 @@
 GPU: experts past a wavefront, a router wider than a workgroup's share of it, ties
 and NaN among the logits, and the two kernels against float64."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import stablehlo_text as T
 import torch
 
-from metaljax_amd import engine, interpreter as I, moe, moe_launch as ML, qmm
+from metaljax_amd import _lib, engine, interpreter as I, moe, moe_launch as ML, qmm
 from test_moe_launch import gemma_inputs
 from test_recognizer import _moe_inputs
 
@@ -151,15 +153,39 @@ def test_a_product_and_its_map_in_one_launch(E, Tk, H, Ii, K, fused, el, monkeyp
     than 2048 codes, which take twice the wavefronts here (and a bf16 place)."""
     raw, _ = _moe_inputs(E, Tk, H, Ii)
     args = [I.from_numpy(a, el) if a.dtype == np.float32 else I.from_numpy(a) for a in raw]
-    alone, took, out = ML.run_pair_product, [], []
+    out, all_steps, run_steps = [], ML.Launches._steps, ML.run_steps
+
+    def two_launches(self):
+        all_steps(self)
+        for s in self.steps:
+            if s.kind == ML.PRODUCT:
+                s.kind, s.skip = ML.MAP, 0                               # (a map of no pairs: nothing)
+                nothing = ML.PairMap(per_token=1, experts=1, rank=1)
+                s.bytes, s.patches, s.program = ctypes.sizeof(nothing), 0, ctypes.addressof(nothing)
+                self.programs.append(nothing)
+    served = []
+    monkeypatch.setattr(ML, "run_steps", lambda steps, values, stream: (served.append(which(steps, values, stream)), run_steps(steps, values, stream))[1])
     for on in (True, False):
-        monkeypatch.setattr(ML, "run_pair_product", lambda p, st, on=on: on and (took.append(alone(p, st)) or took[-1]))
+        if not on:
+            monkeypatch.setattr(ML.Launches, "_steps", two_launches)
         ex = engine.compile_program(T.moe_block_mxfp4(E, Tk, H, Ii, K, el=el))
         (buf,) = engine.execute(ex, args)
         assert ex.interp._qmm.moe[0].launches is not None
         out.append(engine.to_numpy(buf)[0])
-    assert took.count(True) == fused or el != "f32"
+    assert served[-1] == 0 and (served[0] == fused or el != "f32")
     if max(H, Ii) <= 2048 or el == "f32":
         assert np.array_equal(*out)
     else:
         close(*out, "bf16")
+
+
+def which(steps, values, stream):
+    """How many of the pair products the library serves (each is run once more by the call)."""
+    n = 0
+    for s in steps:
+        if s.kind == ML.PRODUCT:
+            p = ML.PairProduct.from_buffer_copy(ctypes.string_at(s.program, s.bytes))
+            for q in s.patch[:s.patches]:
+                ctypes.c_uint64.from_address(ctypes.addressof(p) + q.at).value = values[q.value] + q.add
+            n += _lib.load().qmm_pair_product_run(ctypes.byref(p), stream) == 0
+    return n
