@@ -20,6 +20,7 @@
 // instruction for every lane, operands in LDS (column of a lane: its own, so that no
 // barrier is needed between instructions), arithmetic in float32, one rounding to the
 // value's element type an instruction -- what an array operation of that type does.
+#include <cstddef>
 #include <cstring>
 
 #include "../../include/qmm_hip.h"
@@ -359,7 +360,9 @@ __global__ __launch_bounds__(THREADS ? THREADS : kWave* WAVES) void pair_product
 }
 
 constexpr int kRowThreads = 1024;
-static_assert(QMM_ROW_CODE * sizeof(qmm_row_instruction) / 4 <= kRowThreads && QMM_MAP_CODE <= kThreads, "the program is copied a word (an instruction) a thread");
+constexpr int kLeafTurns = 4;                      // elements of a leaf a lane holds while they arrive: 256 a leaf
+static_assert(QMM_ROW_CODE <= 64 && QMM_MAP_CODE <= kThreads, "a program is held (copied) an instruction a lane (a thread)");
+static_assert(QMM_ROW_LEAVES <= kRowThreads / 64, "a leaf a wavefront");
 
 __device__ __forceinline__ void wave_lds_fence() {          // one wavefront's LDS accesses, in the order written
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -367,87 +370,223 @@ __device__ __forceinline__ void wave_lds_fence() {          // one wavefront's L
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Kernel arguments from byte FROM to byte TO, brought in together: a line of them that is
+// first asked for where it is used is a round trip there, one line after the other.
+template <int FROM, int TO, class T>
+__device__ __forceinline__ void touch_arguments(const T& a) {
+  constexpr int n = (TO - FROM + 63) / 64;
+  static_assert(TO <= (int)sizeof(T) && FROM % 4 == 0 && n <= 24, "a word of every 64 bytes");
+  const int* p = reinterpret_cast<const int*>(&a) + FROM / 4;
+  int any = 0;
+#pragma unroll
+  for (int i = 0; i < n; ++i) any |= p[16 * i];
+  asm volatile("" ::"s"(any));
+}
+
+template <int EL>
+__device__ __forceinline__ float load_as(const void* p, uint32_t bytes) {
+  const char* at = static_cast<const char*>(p) + bytes;
+  if constexpr (EL == QMM_EL_F32) return *reinterpret_cast<const float*>(at);
+  const uint32_t v = *reinterpret_cast<const uint16_t*>(at);
+  return EL == QMM_EL_BF16 ? __uint_as_float(v << 16) : f16_bits_to_f32(v);
+}
+
+// sum over k = first, first + shares, ... < dot_k of x[t][k] w[k][n], both of type EL and
+// within 2^31 bytes of a token's row and of the weight (the host looks).
+template <int EL>
+__device__ __forceinline__ float dot_share(const qmm_row_program& a, int64_t t, int n, int first, int shift) {
+  constexpr uint32_t size = EL == QMM_EL_F32 ? 4 : 2;
+  constexpr int kTurn = 8;                         // operand pairs under way together
+  const char* x = static_cast<const char*>(a.dot_x) + t * a.dot_x_t * size;
+  const uint32_t xk = (uint32_t)a.dot_x_k * size, wk = (uint32_t)a.dot_w_k * size, shares = 1u << shift;
+  uint32_t xo = (uint32_t)first * xk, wo = (uint32_t)n * (uint32_t)a.dot_w_n * size + (uint32_t)first * wk;
+  const uint32_t dx = shares * xk, dw = shares * wk;
+  int left = ((int)a.dot_k - first + (int)shares - 1) >> shift;
+  float sum = 0.f, xs[kTurn], ws[kTurn];
+  for (; left >= kTurn; left -= kTurn) {
+#pragma unroll
+    for (int j = 0; j < kTurn; ++j, xo += dx, wo += dw) {
+      xs[j] = load_as<EL>(x, xo);
+      ws[j] = load_as<EL>(a.dot_w, wo);
+    }
+#pragma unroll
+    for (int j = 0; j < kTurn; ++j) sum = fmaf(xs[j], ws[j], sum);
+  }
+  if (left > 0) {
+#pragma unroll
+    for (int j = 0; j < kTurn; ++j) {              // (past the last: the last again, not added)
+      xs[j] = load_as<EL>(x, xo);
+      ws[j] = load_as<EL>(a.dot_w, wo);
+      if (j + 1 < left) { xo += dx; wo += dw; }
+    }
+#pragma unroll
+    for (int j = 0; j < kTurn; ++j)
+      if (j < left) sum = fmaf(xs[j], ws[j], sum);
+  }
+  return sum;
+}
+
+// Which form of the product: the element type of both operands, or -1 (as written).
+int dot_form(const qmm_row_program& a) {
+  if (!a.dot_x || a.dot_x_el != a.dot_w_el || a.dot_k > (1 << 28) || a.dot_x_k < 0 || a.dot_w_k < 0 || a.dot_w_n < 0 ||
+      a.dot_x_k > (1 << 28) || a.dot_w_k > (1 << 28) || a.dot_w_n > (1 << 28))
+    return -1;
+  return a.dot_k * a.dot_x_k < (1 << 28) && a.dot_k * a.dot_w_k + a.dot_n * a.dot_w_n < (1 << 28) ? a.dot_x_el : -1;
+}
+
+// Keys that compare as the floats do: equal zeros are equal, every NaN is the same and the least.
+__device__ __forceinline__ uint32_t order_key(float v) {
+  const uint32_t b = __float_as_uint(v + 0.f);
+  return v != v ? 0u : (b >> 31) ? ~b : b | 0x80000000u;
+}
+
 // One workgroup a token.  All sixteen wavefronts add up the logits (a thread a
 // column and a share of the contraction, neighbouring threads along the dimension
 // that is contiguous), the first one runs the program: a register is a row of
 // floats in LDS, a lane takes elements lane, lane + 64, ...
-__global__ __launch_bounds__(kRowThreads) void row_program_kernel(qmm_row_program a) {
+//
+// What bounds it: one wavefront's chain of waits and, as nothing else runs on its
+// SIMD, of single instructions.  3 tokens over 1024 x 8 router weights and seven
+// instructions took 10.2 us from the first wavefront's start: the program and the
+// leaves 1.1, the product's operands behind them 2.2, ten rounds of a barrier for its
+// sums 0.9, the instructions 4.9 (the top-k 1.2, a sum over two elements through six
+// exchanges 0.9, 0.4 for the least), the stores 0.7.  So everything that memory holds
+// is requested at once, sums meet behind one barrier, lane q keeps instruction q in
+// registers, a top-k compares integer keys out of a scalar register and a reduction
+// exchanges among as many lanes as there are elements: 6.4 (the operands 1.5, their sums 1.2, the
+// instructions 3.2), the block of such tokens with 1024 x 1024 experts 29.2 -> 25.2.
+__global__ __launch_bounds__(kRowThreads) void row_program_kernel(qmm_row_program a, int form) {
   extern __shared__ float regs[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t t = blockIdx.x;
-  int* const code = reinterpret_cast<int*>(regs + a.reg_floats + (a.dot_x ? kRowThreads : 0));
+  touch_arguments<0, offsetof(qmm_row_program, code)>(a);
   constexpr int kWords = sizeof(qmm_row_instruction) / 4;
-  if ((int)threadIdx.x < a.instructions * kWords) code[threadIdx.x] = reinterpret_cast<const int*>(a.code)[threadIdx.x];
-  if (wave < a.leaves) {                           // (eight leaves at most, sixteen wavefronts)
-    const qmm_row_leaf l = a.leaf[wave];
-    for (int i = lane; i < l.n; i += 64)
-      regs[l.dst + i] = widen_raw(load_raw(l.p, l.base + t * l.token + (int64_t)i * l.step, l.el), l.el);
+  int code[kWords];                                // (wavefront 0) lane q: instruction q
+#pragma unroll
+  for (int w = 0; w < kWords; ++w) code[w] = 0;
+  if (wave == 0 && lane < a.instructions) {
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) code[w] = reinterpret_cast<const int*>(a.code + lane)[w];
   }
+  Raw leaf[kLeafTurns];
+  const bool leaves = wave < a.leaves;             // (eight leaves at most, sixteen wavefronts)
+  const qmm_row_leaf l = a.leaf[leaves ? wave : 0];
+  if (leaves) {
+#pragma unroll
+    for (int i = 0; i < kLeafTurns; ++i)
+      if (lane + 64 * i < l.n) leaf[i] = load_raw(l.p, l.base + t * l.token + (int64_t)(lane + 64 * i) * l.step, l.el);
+  }
+  float* const part = regs + a.reg_floats;
   if (a.dot_x) {
-    float* const part = regs + a.reg_floats;
-    const int cols = a.dot_cols, shares = kRowThreads / cols;
+    const int cols = a.dot_cols, log = 31 - __builtin_clz(cols), shift = 10 - log, shares = 1 << shift;
     const bool along_k = a.dot_w_k == 1;
-    const int n = along_k ? (int)threadIdx.x / shares : (int)threadIdx.x % cols;
-    const int s = along_k ? (int)threadIdx.x % shares : (int)threadIdx.x / cols;
+    const int n = along_k ? (int)threadIdx.x >> shift : (int)threadIdx.x & (cols - 1);
+    const int s = along_k ? (int)threadIdx.x & (shares - 1) : (int)threadIdx.x >> log;
     float sum = 0.f;
     if (n < a.dot_n) {
-      const int64_t x0 = t * a.dot_x_t, w0 = n * a.dot_w_n;
-#pragma unroll 8
-      for (int64_t k = s; k < a.dot_k; k += shares)
-        sum = fmaf(widen_raw(load_raw(a.dot_x, x0 + k * a.dot_x_k, a.dot_x_el), a.dot_x_el),
-                   widen_raw(load_raw(a.dot_w, w0 + k * a.dot_w_k, a.dot_w_el), a.dot_w_el), sum);
+      if (form == QMM_EL_F32) {
+        sum = dot_share<QMM_EL_F32>(a, t, n, s, shift);
+      } else if (form == QMM_EL_BF16) {
+        sum = dot_share<QMM_EL_BF16>(a, t, n, s, shift);
+      } else if (form == QMM_EL_F16) {
+        sum = dot_share<QMM_EL_F16>(a, t, n, s, shift);
+      } else {
+        const int64_t x0 = t * a.dot_x_t, w0 = n * a.dot_w_n;
+#pragma unroll 4
+        for (int64_t k = s; k < a.dot_k; k += shares)
+          sum = fmaf(widen_raw(load_raw(a.dot_x, x0 + k * a.dot_x_k, a.dot_x_el), a.dot_x_el),
+                     widen_raw(load_raw(a.dot_w, w0 + k * a.dot_w_k, a.dot_w_el), a.dot_w_el), sum);
+      }
     }
     part[s * cols + n] = sum;
-    for (int h = shares / 2; h > 0; h /= 2) {
-      __syncthreads();
-      if (s < h) part[s * cols + n] += part[(s + h) * cols + n];
-    }
-    __syncthreads();
-    if (s == 0 && n < a.dot_n) regs[a.dot_dst + n] = round_to(part[n], a.dot_el);
+  }
+  if (leaves) {
+#pragma unroll
+    for (int i = 0; i < kLeafTurns; ++i)
+      if (lane + 64 * i < l.n) regs[l.dst + lane + 64 * i] = widen_raw(leaf[i], l.el);
+    for (int i = lane + 64 * kLeafTurns; i < l.n; i += 64)
+      regs[l.dst + i] = widen_raw(load_raw(l.p, l.base + t * l.token + (int64_t)i * l.step, l.el), l.el);
   }
   __syncthreads();
   if (wave) return;
+  if (a.dot_x) {
+    // share s of column n is part[s * cols + n]: a lane adds up those that lie a multiple of
+    // max(cols, 64) apart, in pairs, then (fewer than 64 columns) the lanes of a column meet
+    const int cols = a.dot_cols, apart = cols > 64 ? cols : 64, count = kRowThreads / apart;
+    for (int n = lane; n < apart; n += 64) {
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = part[(j & (count - 1)) * apart + n];
+#pragma unroll
+      for (int h = 8; h > 0; h /= 2)
+        if (h < count) {
+#pragma unroll
+          for (int j = 0; j < h; ++j) v[j] += v[j + h];
+        }
+      float sum = v[0];
+      for (int d = 32; d >= cols; d /= 2) sum += __shfl_xor(sum, d, 64);
+      if (n < a.dot_n) regs[a.dot_dst + n] = round_to(sum, a.dot_el);
+    }
+  }
   for (int q0 = 0; q0 < a.instructions; ++q0) {
     wave_lds_fence();
-    const qmm_row_instruction q = uniform(reinterpret_cast<const qmm_row_instruction*>(code)[q0]);
-    if (q.op == QMM_OP_TOPK) {
-      // an element's place is the number of those ahead of it: larger, or equal (NaN last) and of a smaller index
-      for (int i = lane; i < q.an; i += 64) {
-        const float v = regs[q.a + i];
-        int place = 0;
-        for (int j = 0; j < q.an; ++j) {
-          const float u = regs[q.a + j];
-          const bool alike = v == u || (v != v && u != u);
-          place += (alike ? j < i : u > v || (v != v && u == u)) ? 1 : 0;
+    union { qmm_row_instruction q; int w[kWords]; } u;
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) u.w[w] = __builtin_amdgcn_readlane(code[w], q0);
+    const qmm_row_instruction& q = u.q;
+    if (q.op <= QMM_OP_IMM) {
+      const int am = q.an == 1 ? 0 : -1, bm = q.bn == 1 ? 0 : -1, cm = q.cn == 1 ? 0 : -1;
+      for (int i = lane; i < q.n; i += 64) {
+        const float v = q.op == QMM_OP_IMM ? q.imm : apply(q.op, regs[q.a + (i & am)], regs[q.b + (i & bm)], regs[q.c + (i & cm)]);
+        regs[q.dst + i] = round_to(v, q.el);
+      }
+    } else if (q.op <= QMM_OP_ROWMIN) {            // sum, rowmax, rowmin
+      const bool add = q.op == QMM_OP_SUM, most = q.op == QMM_OP_ROWMAX;
+      auto both = [&](float x, float y) __attribute__((always_inline)) {
+        return add ? x + y : either_nan(x, y, most ? fmaxf(x, y) : fminf(x, y));
+      };
+      float v = add ? 0.f : most ? -INFINITY : INFINITY;
+      for (int i = lane; i < q.an; i += 64) v = both(v, regs[q.a + i]);
+      // (lanes past the last element hold what changes nothing: they are met only where elements are)
+      int d = 32;
+      while (d >= q.an && d > 0) d /= 2;
+      for (; d > 0; d /= 2) v = both(v, __shfl_xor(v, d, 64));
+      if (lane == 0) regs[q.dst] = round_to(v, q.el);
+    } else if (q.op == QMM_OP_SLICE) {
+      for (int i = lane; i < q.n; i += 64) regs[q.dst + i] = round_to(regs[q.a + q.b + i * q.c], q.el);
+    } else {
+      // top-k: an element's place is the number of those ahead of it -- larger, or equal (NaN last) and of a
+      // smaller index; key j counts from the element's own key on for j below it, above that from j = it on
+      for (int i0 = 0; i0 < q.an; i0 += 64) {
+        const int i = i0 + lane;
+        const float v = regs[q.a + (i < q.an ? i : 0)];
+        const uint32_t key = order_key(v);
+        uint32_t place = 0;
+        for (int j0 = 0; j0 < q.an; j0 += 64) {
+          const int last = q.an - j0 < 64 ? q.an - j0 : 64;
+          uint32_t others = order_key(regs[q.a + j0 + (lane < last ? lane : 0)]);
+          if (lane >= last) others = 0u;           // (ahead of nobody: their places are past i)
+          for (int j4 = 0; j4 < last; j4 += 4) {
+#pragma unroll
+            for (int j = j4; j < j4 + 4; ++j)
+              place += (uint32_t)__builtin_amdgcn_readlane(others, j) >= key + (j0 + j >= i ? 1u : 0u) ? 1u : 0u;
+          }
         }
-        if (place < q.n) {
+        if ((i < q.an) & ((int)place < q.n)) {
           regs[q.dst + place] = v;
           regs[q.c + place] = (float)i;
         }
       }
-      continue;
-    }
-    if (q.op == QMM_OP_SUM || q.op == QMM_OP_ROWMAX || q.op == QMM_OP_ROWMIN) {
-      const int op = q.op == QMM_OP_SUM ? QMM_OP_ADD : q.op == QMM_OP_ROWMAX ? QMM_OP_MAX : QMM_OP_MIN;
-      float v = q.op == QMM_OP_SUM ? 0.f : q.op == QMM_OP_ROWMAX ? -INFINITY : INFINITY;
-      for (int i = lane; i < q.an; i += 64) v = apply(op, v, regs[q.a + i], 0.f);
-#pragma unroll
-      for (int d = 32; d > 0; d /= 2) v = apply(op, v, __shfl_xor(v, d, 64), 0.f);
-      if (lane == 0) regs[q.dst] = round_to(v, q.el);
-      continue;
-    }
-    for (int i = lane; i < q.n; i += 64) {
-      float v;
-      if (q.op == QMM_OP_IMM) v = q.imm;
-      else if (q.op == QMM_OP_SLICE) v = regs[q.a + q.b + i * q.c];
-      else v = apply(q.op, regs[q.a + (q.an == 1 ? 0 : i)], regs[q.b + (q.bn == 1 ? 0 : i)], regs[q.c + (q.cn == 1 ? 0 : i)]);
-      regs[q.dst + i] = round_to(v, q.el);
     }
   }
   wave_lds_fence();
-  for (int j = 0; j < a.outs; ++j) {
+#pragma unroll
+  for (int j = 0; j < QMM_ROW_OUTS; ++j) {
+    if (j >= a.outs) break;
     const qmm_row_out o = a.out[j];
-    for (int i = lane; i < o.n; i += 64) store_el(o.p, t * o.n + i, regs[o.src + (o.srcn == 1 ? 0 : i)], o.el);
+    const int sm = o.srcn == 1 ? 0 : -1;
+    for (int i = lane; i < o.n; i += 64) store_el(o.p, t * o.n + i, regs[o.src + (i & sm)], o.el);
   }
 }
 
@@ -539,7 +678,7 @@ int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
     from_product |= 1u << a->col_leaf[t];
   }
   for (int i = 0; i < m.leaves; ++i)
-    if (!m.leaf[i].p != (from_product >> i & 1)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: leaf");
+    if ((m.leaf[i].p == nullptr) != ((from_product >> i & 1) != 0)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: leaf");
   if (m.rank != 1 || a->mode != QMM_MODE_MXFP4) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: a result of several axes a pair, or affine experts");
   int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el);
   const int waves = a->k > 2048 ? 8 : 4;           // (more than 2048 codes: gemv_terms_dispatch)
@@ -587,8 +726,8 @@ int qmm_row_program_run(const qmm_row_program* a, void* stream) {
     if (!a->out[i].p || a->out[i].n < 1 || !in(a->out[i].src, a->out[i].srcn) || (a->out[i].srcn != 1 && a->out[i].srcn < a->out[i].n) ||
         !(float_el(a->out[i].el) || a->out[i].el == QMM_EL_I32))
       return moe_fail(QMM_ERR_BAD_ARGUMENT, "row program: output");
-  const size_t lds = ((size_t)a->reg_floats + (a->dot_x ? kRowThreads : 0)) * 4 + sizeof(a->code);
-  hipLaunchKernelGGL(row_program_kernel, dim3((unsigned)a->tokens), dim3(kRowThreads), lds, static_cast<hipStream_t>(stream), *a);
+  const size_t lds = ((size_t)a->reg_floats + (a->dot_x ? kRowThreads : 0)) * 4;
+  hipLaunchKernelGGL(row_program_kernel, dim3((unsigned)a->tokens), dim3(kRowThreads), lds, static_cast<hipStream_t>(stream), *a, dot_form(*a));
   return moe_launched("row program launch");
 }
 

@@ -10,7 +10,7 @@ import stablehlo_text as T
 import torch
 
 from metaljax_amd import _lib, engine, interpreter as I, moe, moe_launch as ML, qmm
-from test_moe_launch import gemma_inputs
+from test_moe_launch import gemma_inputs, run_rows
 from test_recognizer import _moe_inputs
 
 pytestmark = pytest.mark.gpu
@@ -72,6 +72,51 @@ def test_ties_and_nan_among_the_logits(monkeypatch):
     finite = np.isfinite(plain)
     assert np.array_equal(finite, np.isfinite(out)) and finite[:2].all()
     close(out[finite], plain[finite], "f32")
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("xel,wel,k,n,along_k", [
+    ("f32", "f32", 1000, 8, False), ("f32", "f32", 7, 1, True), ("bf16", "bf16", 77, 100, True), ("f16", "f16", 2049, 3, False),
+    ("f32", "bf16", 300, 33, False), ("bf16", "bf16", 16, 64, False), ("f32", "f32", 3, 300, True)])
+def test_a_row_program(xel, wel, k, n, along_k, special):
+    """Products of every operand form, of whole and partial turns, of a wavefront's columns and
+    more; a leaf past the 256 elements that are held; a top-k over several wavefronts' worth of
+    elements, with ties, both zeros, infinities and NaN; reductions over one to 300.  Small
+    integers: the sums are exact in any order."""
+    from metaljax_amd.kernels import _stream
+    types = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+    g, tokens, top = torch.Generator().manual_seed(k), 3, min(n, 6)
+    x = torch.randint(-3, 4, (tokens, k), generator=g).to(types[xel])
+    w = torch.randint(-2, 3, (n, k) if along_k else (k, n), generator=g).to(types[wel])
+    b = torch.randint(-2, 3, (n,), generator=g).float()
+    if special:
+        x.zero_()
+        b[torch.randperm(n, generator=g)[:7]] = torch.tensor([np.nan, np.inf, -0.0, 0.0, -np.inf, np.nan, np.inf])[:min(n, 7)]
+    OP, at = ML.OP, lambda row: 512 * row                # (a row of 512 floats a value)
+    code = [(OP["add"], at(2), n, at(0), n, at(1), n), (OP["top_k"], at(3), top, at(2), n, 0, 1, at(4), top),
+            (OP["sum"], at(5), 1, at(2), n), (OP["rowmax"], at(5) + 1, 1, at(2), n), (OP["rowmin"], at(5) + 2, 1, at(2), n),
+            (OP["sum"], at(5) + 3, 1, at(3), top), (OP["slice"], at(5) + 4, (n + 1) // 2, at(2), n, 0, 1, 2, 1)]
+
+    def program(x, w, b, idx, out):
+        p = ML.RowProgram(dot_x=x.data_ptr(), dot_w=w.data_ptr(), dot_x_t=k, dot_x_k=1, dot_w_n=k if along_k else 1, dot_w_k=1 if along_k else n,
+                          dot_k=k, dot_n=n, dot_cols=1 << (n - 1).bit_length(), dot_dst=at(0), dot_x_el=ML.ELS[xel], dot_w_el=ML.ELS[wel],
+                          dot_el=0, tokens=tokens, reg_floats=at(6), leaves=1, instructions=len(code), outs=2)
+        p.leaf[0] = ML.RowLeaf(b.data_ptr(), 0, 0, 1, 0, at(1), n)
+        for i, (op, dst, m, *rest) in enumerate(code):
+            p.code[i] = ML.RowInstruction(op, 0, dst, m, *(rest + [0, 1] * 3)[:6], 0.0)
+        p.out[0] = ML.RowOut(idx.data_ptr(), ML.ELS["i32"], at(4), top, top)
+        p.out[1] = ML.RowOut(out.data_ptr(), 0, at(5), 4 + (n + 1) // 2, 4 + (n + 1) // 2)
+        return p
+
+    def results(device):
+        return torch.zeros((tokens, top), dtype=torch.int32, device=device), torch.zeros((tokens, 4 + (n + 1) // 2), device=device)
+    want, host = results("cpu"), [a.contiguous() for a in (x, w, b)]
+    with np.errstate(all="ignore"):
+        run_rows(program(*host, *want), None)
+    got, card = results("cuda"), [a.cuda() for a in host]
+    ML.run_rows(program(*card, *got), _stream(got[1]))
+    assert torch.equal(got[0].cpu(), want[0])
+    np.testing.assert_array_equal(got[1].cpu().numpy(), want[1].numpy())
 
 
 @pytest.mark.parametrize("op,fn", [("exponential", np.exp), ("logistic", lambda v: 1 / (1 + np.exp(-v))), ("tanh", np.tanh), ("log", np.log),
