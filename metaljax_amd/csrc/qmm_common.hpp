@@ -66,6 +66,9 @@ __device__ __forceinline__ float load_table_rt(const void* p, int64_t i, int tab
   return load_table<QMM_F16>(p, i);
 }
 
+// Cache policy of a buffer store that does not stay in the L2 of its XCD (sc1).
+constexpr int kWriteThrough = 16;
+
 __device__ __forceinline__ void store_out(void* y, int64_t i, float v, int yd) {
   if (yd == QMM_BF16) {
     static_cast<uint16_t*>(y)[i] = (uint16_t)f32_to_bf16_bits(v);

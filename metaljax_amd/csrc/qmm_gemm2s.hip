@@ -510,7 +510,9 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
           const int m = m0 + (i == 0 ? wm : (two ? wm + 4 : 4)) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh;
           if (m < m_end && n < a.N) {
             if (a.splits > 1) {
-              a.part[((int64_t)split * a.R + m) * a.N + n] = i == 0 ? acc[j][r] : acc2[j][r];
+              // (written through L2, as short_kernel's)
+              __hip_atomic_store(a.part + ((int64_t)split * a.R + m) * a.N + n, i == 0 ? acc[j][r] : acc2[j][r], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
               continue;
             }
             const int64_t orow = a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m;
