@@ -93,17 +93,25 @@ __device__ __forceinline__ uint32_t block_scale_byte(uint32_t e) {
 // ---------------------------------------------------------------------------
 // x [x_rows, K] bf16 (rows optionally gathered through lhs_idx) -> two FP6
 // terms + scales in matrix-core operand order.
-// One thread = one (row, 32-block); consecutive threads = consecutive rows.
+// One thread = one (row, 32-block).  A workgroup is sixteen rows x a K-quad of sixteen
+// blocks: a wavefront's 64 lanes read whole lines (four neighbouring blocks of a row)
+// and write runs of sixteen rows, and the four bytes of a scale dword, one of each
+// wavefront, meet in LDS.  (With 64 rows a wavefront, half a line of each, and scale
+// bytes written one by one 256 x 8192 ahead of an 8192 x 8192 product took 0.5 us more
+// of 32.0, 300 x 4096 ahead of 4096 x 4096 0.35 of 18.0.)
 __global__ __launch_bounds__(256) void mx_split_kernel(const uint16_t* __restrict__ x,
                                                        const int32_t* __restrict__ lhs_idx,
                                                        u32x4* __restrict__ aq,
-                                                       uint8_t* __restrict__ as, int R, int x_rows,
+                                                       uint32_t* __restrict__ as, int R, int x_rows,
                                                        int K, int Rp) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int row = (int)(idx % Rp);
-  const int blk = (int)(idx / Rp);
-  if (blk >= K / 32 || row >= R) return;
-  const int64_t srow = lhs_idx ? (int64_t)lhs_idx[row] : (int64_t)row;
+  __shared__ uint8_t scales[2][4][16][4];          // term, block of a K-step, row, K-step
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int quad = (int)(blockIdx.z * gridDim.y + blockIdx.y), row0 = (int)blockIdx.x * 16;
+  if (quad * 512 >= K) return;
+  const int row = row0 + (lane >> 2), kb = lane & 3, ks = quad * 4 + wave;
+  const int blk = ks * 4 + kb;
+  int64_t srow = -1;
+  if (row < R) srow = lhs_idx ? (int64_t)lhs_idx[row] : (int64_t)row;
   const bool ok = srow >= 0 && srow < x_rows;      // an index outside x gathers a zero row
   const u32x4* src = reinterpret_cast<const u32x4*>(x + (ok ? srow : 0) * K + blk * 32);
   u32x16 raw;
@@ -140,16 +148,18 @@ __global__ __launch_bounds__(256) void mx_split_kernel(const uint16_t* __restric
   const float scale_lo = __uint_as_float(byte_lo << 23);
   const u32x6 lo6 = __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(__builtin_bit_cast(bf16x32, res), scale_lo);
 
-  const int ks = blk >> 2, kb = blk & 3;
+  scales[0][kb][lane >> 2][wave] = (uint8_t)byte_hi;
+  scales[1][kb][lane >> 2][wave] = (uint8_t)byte_lo;
   const u32x4 planes[3] = {u32x4{hi6[0], hi6[1], hi6[2], hi6[3]}, u32x4{hi6[4], hi6[5], lo6[0], lo6[1]},
                            u32x4{lo6[2], lo6[3], lo6[4], lo6[5]}};
+  if (row < R) {
 #pragma unroll
-  for (int p = 0; p < 3; ++p) aq[(((int64_t)ks * 3 + p) * 4 + kb) * Rp + row] = planes[p];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int64_t so = ((((int64_t)(ks >> 2) * 2 + t) * 4 + kb) * Rp + row) * 4 + (ks & 3);
-    as[so] = (uint8_t)(t ? byte_lo : byte_hi);
+    for (int p = 0; p < 3; ++p) aq[(((int64_t)ks * 3 + p) * 4 + kb) * Rp + row] = planes[p];
   }
+  __syncthreads();
+  const int d = (int)threadIdx.x;                  // scale dword (term, block, row) = d / 64, d / 16 % 4, d % 16
+  if (d < 128 && row0 + (d & 15) < R)
+    as[(((int64_t)quad * 2 + (d >> 6)) * 4 + (d >> 4 & 3)) * Rp + row0 + (d & 15)] = reinterpret_cast<const uint32_t*>(scales)[d];
 }
 
 // ---------------------------------------------------------------------------
@@ -740,10 +750,10 @@ void mxfp4_mfma_dispatch(const void* x, const void* w, const void* s, void* y, i
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   void* aq = ws;
   void* as = ws + rp * K * 3 / 2;
-  const int64_t threads = rp * (K / 32);
-  hipLaunchKernelGGL(mx_split_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0, st,
+  const int64_t quads = K / 512, planes = ceil_div(quads, 65535);       // (a grid's second axis ends at 65535)
+  hipLaunchKernelGGL(mx_split_kernel, dim3((unsigned)ceil_div(R, 16), (unsigned)ceil_div(quads, planes), (unsigned)planes), dim3(256), 0, st,
                      static_cast<const uint16_t*>(x), lhs_idx, static_cast<u32x4*>(aq),
-                     static_cast<uint8_t*>(as), (int)R, (int)x_rows, (int)K, (int)rp);
+                     static_cast<uint32_t*>(as), (int)R, (int)x_rows, (int)K, (int)rp);
   MxArgs a;
   a.aq = aq; a.as = as; a.w = w; a.s = s; a.y = y;
   a.row_offsets = row_offsets; a.out_idx = out_idx;
