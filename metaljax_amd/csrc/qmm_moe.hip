@@ -620,10 +620,17 @@ int check_map(const qmm_pair_map* a, bool product) {
   return QMM_OK;
 }
 
+constexpr size_t kProductLds = 64 << 10;           // what a launch gets without asking for more
+size_t pair_product_lds(const qmm_pair_product& a, int waves) {
+  const qmm_pair_map& m = a.map;
+  const int terms = a.x_el == QMM_EL_F32 ? 3 : a.x_el == QMM_EL_F16 ? 2 : 1;
+  return ((size_t)terms * (m.weights ? m.per_token * waves : waves) * a.tiles * 4 * kWave + (size_t)m.registers * kThreads + 16 * 16 + 2 * 256) * 4 +
+         sizeof(m.code);
+}
+
 template <int T, int WAVES, int TERMS>
-void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t rest, hipStream_t st) {
+void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t lds, hipStream_t st) {
   const int all = a.map.weights ? a.map.per_token * WAVES : WAVES;
-  const size_t lds = (size_t)TERMS * all * T * 4 * kWave * 4 + rest;
   if constexpr (T == 1) {
     if (a.map.weights) {
       if (all <= 8) hipLaunchKernelGGL((pair_product_kernel<T, WAVES, TERMS, 512>), grid, dim3(kWave * all), lds, st, a);
@@ -635,10 +642,10 @@ void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t rest, hipS
 }
 
 template <int T, int WAVES>
-void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t rest, hipStream_t st) {
-  if (a.x_el == QMM_EL_F32) launch_pair_product<T, WAVES, 3>(a, grid, rest, st);
-  else if (a.x_el == QMM_EL_F16) launch_pair_product<T, WAVES, 2>(a, grid, rest, st);
-  else launch_pair_product<T, WAVES, 1>(a, grid, rest, st);
+void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t lds, hipStream_t st) {
+  if (a.x_el == QMM_EL_F32) launch_pair_product<T, WAVES, 3>(a, grid, lds, st);
+  else if (a.x_el == QMM_EL_F16) launch_pair_product<T, WAVES, 2>(a, grid, lds, st);
+  else launch_pair_product<T, WAVES, 1>(a, grid, lds, st);
 }
 
 }  // namespace
@@ -683,17 +690,17 @@ int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
   int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el);
   const int waves = a->k > 2048 ? 8 : 4;           // (more than 2048 codes: gemv_terms_dispatch)
   if (m.weights && (a->tiles > 1 || m.per_token * waves > 16 || (route == 2 && m.pairs * (a->n * a->k / 2) > kSumBytes))) route = 0;
-  if (!route || (reinterpret_cast<uintptr_t>(a->w) & 15u)) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: two launches are better");
+  const size_t lds = pair_product_lds(*a, waves);
+  if (!route || (reinterpret_cast<uintptr_t>(a->w) & 15u) || lds > kProductLds) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: two launches are better");
   const int64_t segments = m.weights ? m.pairs / m.per_token : route == 2 ? skinny2_max_segments(m.pairs, m.experts) : m.pairs;
   qmm_pair_product p = *a;
   p.sorted = route == 2;
   const dim3 grid((unsigned)ceil_div(m.inner, 16), (unsigned)segments);
-  const size_t rest = (size_t)m.registers * kThreads * 4 + sizeof(m.code) + 16 * 16 * 4 + 2 * 256 * 4;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a->tiles == 1 && waves == 4) launch_pair_product<1, 4>(p, grid, rest, st);
-  else if (a->tiles == 1) launch_pair_product<1, 8>(p, grid, rest, st);
-  else if (waves == 4) launch_pair_product<2, 4>(p, grid, rest, st);
-  else launch_pair_product<2, 8>(p, grid, rest, st);
+  if (a->tiles == 1 && waves == 4) launch_pair_product<1, 4>(p, grid, lds, st);
+  else if (a->tiles == 1) launch_pair_product<1, 8>(p, grid, lds, st);
+  else if (waves == 4) launch_pair_product<2, 4>(p, grid, lds, st);
+  else launch_pair_product<2, 8>(p, grid, lds, st);
   return moe_launched("pair product launch");
 }
 

@@ -366,3 +366,14 @@ def test_programs_that_point_outside_their_registers_are_refused():
               (ML.OP["slice"], 0, 0, 4, 4, 4, 1, 0, 1, 0, 0.0)):
         r.code[0] = ML.RowInstruction(*q)
         assert lib.qmm_row_program_run(ctypes.byref(r), None) == 1, q
+
+
+def test_a_map_that_leaves_a_product_no_local_memory_is_two_launches():
+    """Eight wavefronts' sums of two columns in three terms are 48 KB; a file of 32
+    registers besides is more than a launch gets.  Decided on the host, no GPU needed."""
+    at = 4096
+    m = ML.PairMap(y=at, experts_of=at, pairs=2, inner=16, dims=(1, 1, 16), per_token=1, experts=2, rank=1, registers=ML.REGISTERS, leaves=2)
+    p = ML.PairProduct(x=at, w=at, s=at, x_rows=2, n=32, k=2080, mode=_lib.MODE_MXFP4, x_per=1, tiles=2, col_leaf=(0, 1), col_base=(0, 16),
+                       col_step=(1, 1), map=m)
+    assert _lib.load().qmm_pair_product_run(ctypes.byref(p), None) == 3
+    assert b"two launches" in _lib.load().qmm_last_error()
