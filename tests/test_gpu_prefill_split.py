@@ -52,6 +52,22 @@ def test_dense(m, n, k, kind, act):
     close(K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how), x.double() @ tile(w, s, b, how).T)
 
 
+# Row tiles of 256 rows (several rounds of workgroups, or a split K), the last of 188, 76 and
+# 130 rows, dealt row tile first; float32 results and 16-bit ones (one rounding, half a place of eight bits, and the sums).
+@pytest.mark.parametrize("m,n,k", [(700, 11992, 256), (1100, 6240, 1088), (642, 1096, 12800)])
+@pytest.mark.parametrize("kind", [KINDS[0], KINDS[3]])
+def test_tiles_of_256_rows(m, n, k, kind):
+    bits, gs, mode, tab = kind
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    how = dict(group_size=gs, bits=bits, mode=mode)
+    w, s, b = weight(g, (), n, k, bits, gs, mode, tab)
+    x = torch.randn((m, k), device=DEV, generator=g).bfloat16()
+    want = x.double() @ tile(w, s, b, how).T
+    close(K.quantized_matmul(x, w, s, b, out_dtype=torch.float32, **how), want)
+    y = K.quantized_matmul(x, w, s, b, **how).double()
+    assert ((y - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * want.std()).all()
+
+
 @pytest.mark.parametrize("counts", [(0, 1, 16, 0, 17), (22, 0, 3, 31, 17), (40, 0, 3, 70, 64), (90, 129, 0, 161, 300)])
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("act", ["bf16", "f16"])
