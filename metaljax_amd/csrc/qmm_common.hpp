@@ -243,6 +243,6 @@ void clear_rows_dispatch(const ClearArgs& c, hipStream_t st);
 
 // y = the splits' float32 sums [splits][R][N], added in order and rounded once (qmm_util.hip)
 void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,
-                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, hipStream_t st);
+                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, bool wide, hipStream_t st);
 
 }  // namespace qmm

@@ -723,7 +723,7 @@ void short_dispatch(const void* x, int x_dtype, const void* w, const void* s, co
   if (mode == QMM_MODE_MXFP4) launch_short<1, 4, QMM_BF16>(a, p.mb, st);
   else if (bits == 4) launch_affine<4>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
   else launch_affine<8>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
-  if (p.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, p.splits, row_offsets, E, out_idx, st);
+  if (p.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, p.splits, row_offsets, E, out_idx, true, st);
 }
 
 }  // namespace qmm
