@@ -69,6 +69,9 @@ __device__ __forceinline__ float load_table_rt(const void* p, int64_t i, int tab
 // Cache policy of a buffer store that does not stay in the L2 of its XCD (sc1).
 constexpr int kWriteThrough = 16;
 
+// Are the float32 sums [R][N] of a split stored sixteen bytes a lane (32-bit offsets)?
+__host__ __device__ inline bool wide_sums(int64_t R, int64_t N) { return N % 4 == 0 && R * N < (1 << 29); }
+
 __device__ __forceinline__ void store_out(void* y, int64_t i, float v, int yd) {
   if (yd == QMM_BF16) {
     static_cast<uint16_t*>(y)[i] = (uint16_t)f32_to_bf16_bits(v);
@@ -243,6 +246,6 @@ void clear_rows_dispatch(const ClearArgs& c, hipStream_t st);
 
 // y = the splits' float32 sums [splits][R][N], added in order and rounded once (qmm_util.hip)
 void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,
-                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, bool wide, hipStream_t st);
+                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, hipStream_t st);
 
 }  // namespace qmm

@@ -597,7 +597,7 @@ void gemm2_dispatch(const void* x, const void* w, const void* s, const void* b, 
     gemm2s_plan(R, row_offsets ? E : 1, N, K, !row_offsets && workspace_bytes > prep ? workspace_bytes - prep : 0, &a.tile_rows,
                 &a.splits);
     gemm2s_launch(a, mode, bits, st);
-    if (a.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, a.splits, nullptr, 1, nullptr, false, st);
+    if (a.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, a.splits, nullptr, 1, nullptr, st);
     return;
   }
   const int mt = row_tile >= 256 ? 2 : 1;

@@ -507,6 +507,38 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+  } else if (a.splits > 1 && wide_sums(a.R, a.N)) {
+    // a split's float32 sums: the same transposition, sixteen bytes a lane written through
+    // L2 (four bytes a lane as the accumulators lie: 642 rows of 1096 x 12800 40.7 us against
+    // 36.3, 600 of 2048 x 12800 50.5 / 46.8, 900 of 4096 x 8192 73.8 / 69.7, 667 of it x 8064 61.4 / 59.0)
+    float* o32 = reinterpret_cast<float*>(smem) + wave * (32 * BN);
+    const auto rp = make_rsrc(a.part + (int64_t)split * a.R * a.N, (int64_t)a.R * a.N * 4);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (i == 1 && !five && !two) break;
+      const int ncb = (i == 0 || two) ? 4 : 1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j >= ncb) break;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o32[((r & 3) + 8 * (r >> 2) + 4 * kh) * BN + j * 32 + li] = i == 0 ? acc[j][r] : acc2[j][r];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int ppr = ncb * 8;                      // 16-byte pieces per row
+      for (int q = 0; q < (32 * ppr) / 64; ++q) {
+        const int idx = q * 64 + lane, rl = idx / ppr, pc = idx % ppr;
+        const int m = m0 + (i == 0 ? wm : (two ? wm + 4 : 4)) * 32 + rl;
+        const int n = n0 + ((i == 0 || two) ? 0 : wm * 32) + pc * 4;
+        if (m < m_end && n < a.N)
+          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(o32 + rl * BN + pc * 4), rp, (uint32_t)(m * a.N + n) * 4u, 0,
+                                                 kWriteThrough);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -521,9 +553,8 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
           const int m = m0 + (i == 0 ? wm : (two ? wm + 4 : 4)) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh;
           if (m < m_end && n < a.N) {
             if (a.splits > 1) {
-              // (written through L2, as short_kernel's)
               __hip_atomic_store(a.part + ((int64_t)split * a.R + m) * a.N + n, i == 0 ? acc[j][r] : acc2[j][r], __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+                                 __HIP_MEMORY_SCOPE_AGENT);      // (written through L2 as well)
               continue;
             }
             const int64_t orow = a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m;
@@ -568,7 +599,7 @@ void launch_k(const Gemm2Args& a, hipStream_t st) {
   const int64_t m_tiles = ceil_div(a.R, a.tile_rows) + a.E;    // provisioned: a tile never straddles an expert
   int64_t total = ceil_div(ceil_div(a.N, BN), 8) * 8 * m_tiles;
   if (!a.row_offsets) total = ceil_div(ceil_div(a.N, BN) * ceil_div(a.R, a.tile_rows) * a.splits, 8) * 8;
-  const size_t epi = (size_t)4 * 32 * BN * 2;
+  const size_t epi = (size_t)4 * 32 * BN * (a.splits > 1 ? 4 : 2);
   const size_t need = (size_t)(kS * kStage) + (TLDS ? 2 * kTabKind : 0);
   const size_t lds = epi > need ? epi : need;
   constexpr auto kern = gemm2s_kernel<MODE, BITS, TAB, G64, TLDS>;

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void short_kernel(ShortArgs a) {
   // A split's sums are written through L2: left dirty there they are written back when the
   // kernel ends, ahead of the launch that adds them up (48 rows of 4096 x 14336 21.5 -> 20.7 us,
   // float16 77 of 4096 x 4096 14.5 -> 14.1; 6 and 5 MB of sums).
-  const bool through = (int64_t)a.R * a.N < (1 << 29);
+  const bool through = wide_sums(a.R, a.N);
   const auto rp = make_rsrc(a.part + (int64_t)z * a.R * a.N, through ? (int64_t)a.R * a.N * 4 : 0);
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
@@ -723,7 +723,7 @@ void short_dispatch(const void* x, int x_dtype, const void* w, const void* s, co
   if (mode == QMM_MODE_MXFP4) launch_short<1, 4, QMM_BF16>(a, p.mb, st);
   else if (bits == 4) launch_affine<4>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
   else launch_affine<8>(a, tab, p.mb, terms == 1 && x_dtype == QMM_F16, st);
-  if (p.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, p.splits, row_offsets, E, out_idx, true, st);
+  if (p.splits > 1) split_sum_dispatch(a.part, y, y_dtype, R, N, p.splits, row_offsets, E, out_idx, st);
 }
 
 }  // namespace qmm

@@ -176,7 +176,7 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)ceil_div(n, kBlock); }
 // were written through L2 sixteen bytes a lane and whole lines a row (us, kept / read once:
 // 128 rows of 4096 x 4096 17.7 / 15.1, 48 of 4096 x 14336 20.8 / 19.8, float16 77 of 4096 x 4096
 // 14.6 / 13.5, 48 of 14336 x 4096 20.8 / 19.9; of rows that end inside a line float16 17 of
-// 3928 x 2560 13.8 / 14.2, of sums written four bytes a lane 642 of 1096 x 12800 38.4 / 40.6).
+// 3928 x 2560 13.8 / 14.2).
 template <int V, bool ONCE>
 __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ part, void* __restrict__ y,
                                                         int y_dtype, int R, int N, int splits,
@@ -304,10 +304,10 @@ void clear_rows_dispatch(const ClearArgs& c, hipStream_t st) {
 }
 
 void split_sum_dispatch(const float* part, void* y, int y_dtype, int64_t R, int64_t N, int splits,
-                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, bool wide, hipStream_t st) {
+                        const int32_t* row_offsets, int64_t E, const int32_t* out_idx, hipStream_t st) {
   const bool v4 = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
   const dim3 grid((unsigned)ceil_div(R * N, 256 * (v4 ? 4 : 1)));
-  if (v4 && wide && N % 32 == 0) hipLaunchKernelGGL((split_sum_kernel<4, true>), grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
+  if (v4 && wide_sums(R, N) && N % 32 == 0) hipLaunchKernelGGL((split_sum_kernel<4, true>), grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
   else if (v4) hipLaunchKernelGGL((split_sum_kernel<4, false>), grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
   else hipLaunchKernelGGL((split_sum_kernel<1, false>), grid, dim3(256), 0, st, part, y, y_dtype, (int)R, (int)N, splits, row_offsets, (int)E, out_idx);
 }
