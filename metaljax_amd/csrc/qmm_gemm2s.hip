@@ -668,8 +668,10 @@ double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes
       const int64_t tiles = nt * mt * s;
       const double step = (half ? 0.41 : 0.60) + 0.105 * (tiles < 256 ? tiles / 256.0 : 1.0);
       const double us = 5.9 + (double)ceil_div(tiles, 256) * (2.5 + (s == 1 ? kt : 4 * ceil_div(quads, s)) * step) +
-                        (double)R * K * 0.54e-6 + (double)R * N * 0.5e-6 + (s > 1 ? 4.6 + (double)s * R * N * 1.4e-6 : 0.0);
-      double cost = us * (1.0 + 0.01 * s);       // (of two alike the one with fewer splits)
+                        (double)R * K * 0.54e-6 + (double)R * N * 0.5e-6 + (s > 1 ? 4.0 + (double)s * R * N * 0.7e-6 : 0.0);
+      // (of two alike the one with fewer splits, and none that is a second round: 698 rows of
+      // 5432 x 7424 in three parts, 387 tiles, 75.7 us, whole 70.9)
+      double cost = us * (1.0 + 0.01 * s) * (s > 1 && tiles > 256 ? 1.08 : 1.0);
       if (er && E <= 1 && atoi(er) != rows) cost += 1e9;
       if (es && E <= 1 && atoi(es) != s) cost += 1e9;
       if (cost < best) { best = cost; least = us; *tile_rows = rows; *splits = s; }
