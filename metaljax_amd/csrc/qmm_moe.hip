@@ -7,14 +7,15 @@
 //
 // What bounds it: nothing here is more than a few hundred thousand elements, so a
 // launch is its fixed cost and a few dependent loads: a pair map of 6 x 1024 takes
-// 5.4 us, the row program of 3 tokens over 1024 x 8 router weights 11 (both cold;
+// 5.4 us, the row program of 3 tokens over 1024 x 8 router weights 7 (both cold;
 // an empty launch is 2.7).  As array operations a block of 3 tokens over 8 experts
 // of 1024 x 1024 was some thirty launches with their host work and three round
-// trips to the host, 430 us; now it is these three launches and the two products,
-// 45 us, 37 of them the device's.  They stay ahead as blocks grow and the products
-// take over (us, launches / array operations, 8 experts of 1024 x 1024, top 2: 256 tokens
-// 93 / 439, 2048 tokens 364 / 815; 32 experts of 2880 x 2880, top 4: 64 tokens 286 / 533, 2048
-// tokens 3476 / 4536).
+// trips to the host, 430 us; as the row program, two products and two maps it was 45,
+// with each product and its map one launch and all of them issued by one library call
+// it is 25, the host's and the device's alike.  They stay ahead as blocks grow and the
+// products take over (us, launches / array operations, 8 experts of 1024 x 1024, top 2: 256
+// tokens 93 / 439, 2048 tokens 364 / 815; 32 experts of 2880 x 2880, top 4: 64 tokens 286 /
+// 533, 2048 tokens 3476 / 4536).
 //
 // Both kernels interpret a short program that the planner wrote once: the same
 // instruction for every lane, operands in LDS (column of a lane: its own, so that no

@@ -26,10 +26,11 @@
 // weight through that path and sat in issue most of the time.)
 //
 // Measured, bf16 activations and four-bit codes in groups of 64, against the
-// prefill kernel on whole K: 48 rows of 4096 x 14336 104 -> 22 us, 17 rows of
-// 4096 x 4096 35 -> 12, 48 rows of 14336 x 4096 37 -> 22; float16 activations and
-// tables, 77 rows of 4096 x 4096 46 -> 21 -> 14.8 without terms.  Of the 22 us about 10 are fixed (launch, first
-// data, the sums' second launch); a step takes 0.76 us and 0.14 more per row
+// prefill kernel on whole K: 48 rows of 4096 x 14336 104 -> 19.5 us, 17 rows of
+// 4096 x 4096 35 -> 11, 48 rows of 14336 x 4096 37 -> 19.9; float16 activations and
+// tables, 77 rows of 4096 x 4096 46 -> 21 -> 13.5 without terms.  Of the 19.5 us about 8 are
+// fixed (launch, first data, the sums' second launch; 10 before the sums were written
+// through L2 and read once); a step takes 0.76 us and 0.14 more per row
 // block, the vector ALU's instructions about half of it.
 //
 // The dequantized weight never goes through LDS: a lane reads the eight bytes
