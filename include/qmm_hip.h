@@ -225,8 +225,10 @@ int qmm_pair_map_run(const qmm_pair_map* map, void* stream);
  * pair p multiplies row p / x_per of x [x_rows, k] by expert experts_of[p] of w
  * [experts, n, k / 8 words] with block scales s, rounded to product_el; leaf
  * col_leaf[t] of the map (whose p is null) is column col_base[t] + col_step[t] *
- * element of that.  UNSUPPORTED where a product and a map are the better launches
- * (by the mode, the sizes, the types and the alignment alone).  `sorted` is the library's. */
+ * element of that.  An expert index outside [0, experts) multiplies by the nearest
+ * expert, as the map reads that one's data, however the pairs are taken.  UNSUPPORTED
+ * where a product and a map are the better launches (by the mode, the sizes, the types
+ * and the alignment alone).  `sorted` is the library's. */
 typedef struct {
   const void *x, *w, *s;
   int64_t x_rows, n, k, mode;
@@ -275,7 +277,9 @@ typedef struct {
 /* A call of a compiled dispatch, launch after launch: step i's program, with the
  * eight bytes at every patch's `at` replaced by values[value] + add, goes to the
  * entry point that its kind names.  A pair product that is served skips the `skip`
- * steps behind it, the launches it stands for; one that is not is passed over.  The
+ * steps behind it, the launches it stands for; one that is not is passed over.  (The
+ * experts of the pairs are inside the weight, as a top-k's are: qmm_gather_qmm leaves
+ * the row of any other pair alone, where a pair product reads the nearest expert.)  The
  * programs are only read: several threads may run the same steps.  Stands for the
  * host side of reference src/metaljax/moe.py:1425-1461. */
 enum { QMM_STEP_ROWS, QMM_STEP_PAIR_PRODUCT, QMM_STEP_MAP, QMM_STEP_GATHER };

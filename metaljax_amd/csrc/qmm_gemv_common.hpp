@@ -114,10 +114,14 @@ __device__ __forceinline__ void load_args_now(const GemvArgs& a) {
 // the same for the whole workgroup).  A few instructions an expert; the sort is a launch
 // of its own otherwise: 64 pairs over 8 experts of 1024 x 1024 11.5 -> 8.4 us, four-bit or
 // eight-bit codes or MXFP4 (the host takes 8 a call), the three terms of float32 rows
-// over affine codes 33 -> 24.
+// over affine codes 33 -> 24.  A pair whose expert is outside the weight belongs to no
+// segment (NEAREST: to its nearest expert's).
+template <bool NEAREST = false>
 __device__ __forceinline__ int take_segment(const int32_t* experts_of, int pairs, int n_experts, int z, int lane, int* rows, int64_t& expert) {
   int e = -1;
   if (lane < pairs) e = experts_of[lane];
+  if constexpr (NEAREST)
+    if (lane < pairs) e = e < 0 ? 0 : e >= n_experts ? n_experts - 1 : e;
   uint64_t left = __ballot(e >= 0 && e < n_experts);
   while (left) {
     const int of = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));

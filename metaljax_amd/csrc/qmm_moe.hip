@@ -220,7 +220,7 @@ __global__ __launch_bounds__(THREADS ? THREADS : kWave* WAVES) void pair_product
   int rows = SUM ? a.map.per_token : 1;
   int64_t e;
   if (!SUM && a.sorted) {
-    rows = take_segment(a.map.experts_of, (int)a.map.pairs, a.map.experts, z, lane, taken, e);
+    rows = take_segment<true>(a.map.experts_of, (int)a.map.pairs, a.map.experts, z, lane, taken, e);
     if (rows == 0) return;                         // uniform, before any barrier
   } else {
     e = __builtin_amdgcn_readfirstlane(expert_of(SUM ? z * a.map.per_token + group : z));

@@ -234,3 +234,53 @@ def which(steps, values, stream):
                 ctypes.c_uint64.from_address(ctypes.addressof(p) + q.at).value = values[q.value] + q.add
             n += _lib.load().qmm_pair_product_run(ctypes.byref(p), stream) == 0
     return n
+
+
+@pytest.mark.parametrize("el", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("pairs,per,E,n,k,inner,columns,summed", [
+    (5, 1, 8, 17, 96, 17, [(0, 1)], False), (6, 2, 3, 2, 32, 1, [(1, 0)], False), (12, 4, 5, 35, 160, 17, [(0, 2), (1, 2)], False),
+    (3, 3, 2, 24, 1056, 24, [(0, 1), (5, 0)], False), (40, 4, 8, 33, 96, 33, [(0, 1)], False), (64, 1, 3, 34, 288, 17, [(17, 1), (0, 1)], False),
+    (33, 3, 16, 31, 544, 1, [(30, 1), (3, 2)], False), (6, 2, 4, 17, 64, 17, [(0, 1)], True), (4, 4, 8, 40, 96, 20, [(1, 2)], True),
+    (48, 3, 6, 18, 1056, 18, [(0, 1)], True)])
+def test_a_pair_product(pairs, per, E, n, k, inner, columns, summed, el):
+    """The product and its map as one launch against the product, then the map: pairs of their own and (from
+    sixteen on, where two share an expert) sorted by the kernel, and a token's sum; results that end inside a
+    workgroup's sixteen elements, columns that are one, neighbours or every other one; experts outside the
+    weight, whose nearest one is read on every route.  The sums are the same ones in the same order."""
+    from metaljax_amd import kernels
+    types = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+    g = torch.Generator(device="cuda").manual_seed(pairs + k)
+    w = torch.randint(-2**31, 2**31 - 1, (E, n, k // 8), dtype=torch.int32, device="cuda", generator=g)
+    s = torch.randint(120, 128, (E, n, k // 32), dtype=torch.uint8, device="cuda", generator=g)
+    x = torch.randn((pairs // per, k), device="cuda", generator=g).to(types[el])
+    bias, weights = torch.randn((E, inner), device="cuda", generator=g), torch.rand(pairs, device="cuda", generator=g)
+    experts = torch.randint(-2, E + 2, (pairs,), dtype=torch.int32, device="cuda", generator=g)
+    experts[0], experts[pairs - 1] = -1, E
+    rows = pairs // per if summed else pairs
+    token = (torch.arange(pairs, dtype=torch.int32, device="cuda") // per).int()
+    stream = kernels._stream(x)
+
+    def program(y, product):
+        """(columns or their product) + bias of the expert; `product`: the leaves' address, None for the launch that computes it"""
+        m = ML.PairMap(y=y.data_ptr(), experts_of=experts.data_ptr(), pairs=pairs, inner=inner, dims=(1, 1, inner), per_token=per, experts=E,
+                       rank=1, leaves=len(columns) + 1, instructions=2, registers=4, result=3, weights=weights.data_ptr() if summed else None)
+        for i, (base, step) in enumerate(columns):
+            m.leaf[i] = ML.MapLeaf(product, 0, 0, 0, 0, (0, 0, 0), ML.ELS[el]) if product is None else ML.MapLeaf(product, base, n, 0, 0, (0, 0, step), ML.ELS[el])
+        m.leaf[len(columns)] = ML.MapLeaf(bias.data_ptr(), 0, 0, inner, 0, (0, 0, 1), 0)
+        m.code[0] = ML.Instruction(ML.OP["multiply" if len(columns) == 2 else "copy"], 3, 0, 1, 0, 0, 0.0)
+        m.code[1] = ML.Instruction(ML.OP["add"], 3, 3, len(columns), 0, 0, 0.0)
+        return m
+    got, want = (torch.full((rows, inner), float("nan"), device="cuda") for _ in range(2))
+    fused = ML.PairProduct(x=x.data_ptr(), w=w.data_ptr(), s=s.data_ptr(), x_rows=pairs // per, n=n, k=k, mode=_lib.MODE_MXFP4, x_el=ML.ELS[el],
+                           x_per=per, product_el=ML.ELS[el], tiles=len(columns), map=program(got, None))
+    for t, (base, step) in enumerate(columns):
+        fused.col_leaf[t], fused.col_base[t], fused.col_step[t] = t, base, step
+    _lib.check(_lib.load().qmm_pair_product_run(ctypes.byref(fused), stream))
+    nearest = experts.clamp(0, E - 1)
+    y = kernels.gather_qmm(x, w, s, None, token, nearest, group_size=32, bits=4, mode="mxfp4")
+    ML.run_map(program(want, y.data_ptr()), stream)
+    assert torch.equal(got, want)
+    full = kernels.dequantize(w, s, None, group_size=32, bits=4, mode="mxfp4", out_dtype=torch.float32).double().cpu()
+    exact = torch.stack([full[e] @ v for e, v in zip(nearest.tolist(), x.double().cpu()[token.long().cpu()])])
+    tol = 1e-6 if el == "f32" else 2.0 ** -8 if el == "bf16" else 2.0 ** -11      # (one rounding to the product's type)
+    assert ((y.double().cpu() - exact).norm() / exact.norm()).item() <= tol
