@@ -671,13 +671,12 @@ int qmm_pair_map_run(const qmm_pair_map* a, void* stream) {
 
 int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
   if (!a) return moe_fail(QMM_ERR_BAD_ARGUMENT, "null program");
-  const int rc = check_map(&a->map, true);
-  if (rc) return rc;
   const qmm_pair_map& m = a->map;
+  const int rc = check_map(&m, true);
+  if (rc || m.pairs == 0 || m.inner == 0) return rc;
   if (!a->x || !a->w || !a->s || !float_el(a->x_el) || !float_el(a->product_el) || a->x_rows < 0 || a->x_per < 1 || a->n < 1 || a->k < 1 || a->k % 32)
     return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: operands");
   if (a->tiles < 1 || a->tiles > 2) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: tiles");
-  if (m.pairs == 0 || m.inner == 0) return QMM_OK;
   uint32_t from_product = 0;
   for (int t = 0; t < a->tiles; ++t) {
     if (a->col_leaf[t] < 0 || a->col_leaf[t] >= m.leaves || a->col_base[t] < 0 || a->col_step[t] < 0 ||

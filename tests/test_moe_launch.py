@@ -377,3 +377,13 @@ def test_a_map_that_leaves_a_product_no_local_memory_is_two_launches():
                        col_step=(1, 1), map=m)
     assert _lib.load().qmm_pair_product_run(ctypes.byref(p), None) == 3
     assert b"two launches" in _lib.load().qmm_last_error()
+
+
+@pytest.mark.parametrize("pairs,inner", [(0, 4), (3, 0)])
+def test_a_call_without_pairs_or_elements_launches_nothing(pairs, inner):
+    """An array without elements has no address: every step of such a call is taken, not refused."""
+    m = ML.PairMap(per_token=1, experts=2, rank=1, pairs=pairs, inner=inner, registers=1)
+    p = ML.PairProduct(n=16, k=32, mode=_lib.MODE_MXFP4, x_per=1, tiles=1, map=m)
+    lib = _lib.load()
+    assert lib.qmm_pair_map_run(ctypes.byref(m), None) == 0
+    assert lib.qmm_pair_product_run(ctypes.byref(p), None) == 0
