@@ -224,21 +224,17 @@ inline hipError_t& setup_error() {
   return e;
 }
 
-// Raises kernel KERN's dynamic-LDS limit.  The HIP call is made once per
-// process (the initialisation of a function-local static is thread-safe) and
-// its status is kept: every later call reports the same status, so a launch
-// behind a failed set-up is never attempted.  Returns true when the limit is set.
-template <auto KERN>
-inline bool lds_limit(size_t bytes) {
-  static const size_t set_bytes = bytes;
+// Raises kernel KERN's dynamic-LDS limit to MOST, the largest that any launch of it
+// asks for.  The HIP call is made once per process (the initialisation of a
+// function-local static is thread-safe) and its status is kept: every later call
+// reports the same status, so a launch behind a failed set-up is never attempted.
+// Returns true when the limit is set.
+template <auto KERN, size_t MOST>
+inline bool lds_limit() {
   static const hipError_t rc = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  hipError_t r = rc;
-  if (r == hipSuccess && bytes > set_bytes)      // a later call asking for more than the first did
-    r = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (r != hipSuccess) setup_error() = r;
-  return r == hipSuccess;
+      reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST);
+  if (rc != hipSuccess) setup_error() = rc;
+  return rc == hipSuccess;
 }
 
 // zeroes in the rows that no expert covers, in a launch of its own (qmm_util.hip)

@@ -328,9 +328,9 @@ void launch(const GemmArgs& a0, hipStream_t st) {
   a.m_tiles = (int)(a.row_offsets ? ceil_div(a.R, BM) + a.E : ceil_div(a.R, BM));
   const int64_t total = ceil_div(a.N, BN) * a.m_tiles;
   dim3 grid((unsigned)(ceil_div(total, 8) * 8));
-  const size_t lds = 3 * (size_t)(BM + BN) * kRowBytes;
+  constexpr size_t lds = 3 * (size_t)(BM + BN) * kRowBytes;
   constexpr auto kern = gemm_kernel<MODE, BITS, BM>;
-  if (!lds_limit<kern>(lds)) return;
+  if (!lds_limit<kern, lds>()) return;
   hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds, st, a);
 }
 

@@ -499,10 +499,10 @@ void launch2_k(const Gemm2Args& a0, hipStream_t st) {
                                       : ceil_div(ceil_div(a.N, BN) * a.m_tiles, 8) * 8;
   dim3 grid((unsigned)total);
   // three weight stages; the epilogue transposes 32 x NT*32 sixteen-bit results per wavefront there
-  const size_t epi = (size_t)NWAVES * 32 * NT * 32 * 2;
-  const size_t lds = epi > (size_t)(kStages * kStage) ? epi : (size_t)(kStages * kStage);
+  constexpr size_t epi = (size_t)NWAVES * 32 * NT * 32 * 2;
+  constexpr size_t lds = epi > (size_t)(kStages * kStage) ? epi : (size_t)(kStages * kStage);
   constexpr auto kern = gemm2_kernel<MODE, BITS, MT, NT, WMW, NWAVES, RAG, WIN>;
-  if (!lds_limit<kern>(lds)) return;
+  if (!lds_limit<kern, lds>()) return;
   hipLaunchKernelGGL(kern, grid, dim3(64 * NWAVES), lds, st, a);
 }
 

@@ -31,6 +31,7 @@
 // block split by columns, consumer w multiplies it with column block w.  More:
 // consumer w multiplies row blocks w and w + 4 (every weight fragment read
 // from LDS then feeds two MFMAs).  Longer experts take several tiles.
+#include <algorithm>
 #include <type_traits>
 
 #include "qmm_gemm2_common.hpp"
@@ -599,11 +600,12 @@ void launch_k(const Gemm2Args& a, hipStream_t st) {
   const int64_t m_tiles = ceil_div(a.R, a.tile_rows) + a.E;    // provisioned: a tile never straddles an expert
   int64_t total = ceil_div(ceil_div(a.N, BN), 8) * 8 * m_tiles;
   if (!a.row_offsets) total = ceil_div(ceil_div(a.N, BN) * ceil_div(a.R, a.tile_rows) * a.splits, 8) * 8;
-  const size_t epi = (size_t)4 * 32 * BN * (a.splits > 1 ? 4 : 2);
-  const size_t need = (size_t)(kS * kStage) + (TLDS ? 2 * kTabKind : 0);
-  const size_t lds = epi > need ? epi : need;
+  // (a split's results leave as float32 sums, a whole K's as 16-bit ones)
+  constexpr size_t need = (size_t)(kS * kStage) + (TLDS ? 2 * kTabKind : 0), epi = (size_t)4 * 32 * BN * 2;
+  constexpr size_t whole = std::max(need, epi), split = std::max(need, 2 * epi);
   constexpr auto kern = gemm2s_kernel<MODE, BITS, TAB, G64, TLDS>;
-  if (!lds_limit<kern>(lds)) return;
+  if (!lds_limit<kern, split>()) return;
+  const size_t lds = a.splits > 1 ? split : whole;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(512), lds, st, a);
 }
 

@@ -763,11 +763,11 @@ void mxfp4_mfma_dispatch(const void* x, const void* w, const void* s, void* y, i
   a.n_tiles = (int)ceil_div(N, TN);
   const int grid = (int)(ceil_div((int64_t)a.m_tiles * a.n_tiles, 8) * 8), block = 256;
   if (K % 2048 == 0) {
-    if (!lds_limit<mxfp4_mfma8_kernel>(kLds8)) return;
+    if (!lds_limit<mxfp4_mfma8_kernel, kLds8>()) return;
     hipLaunchKernelGGL(mxfp4_mfma8_kernel, dim3(grid), dim3(512), kLds8, st, a);
     return;
   }
-  if (!lds_limit<mxfp4_mfma_kernel>(kLds)) return;
+  if (!lds_limit<mxfp4_mfma_kernel, kLds>()) return;
   hipLaunchKernelGGL(mxfp4_mfma_kernel, dim3(grid), dim3(block), kLds, st, a);
 }
 

@@ -613,7 +613,7 @@ template <int MODE, int BITS, int TAB, int MB, bool HALF>
 void launch_mb(const ShortArgs& a, hipStream_t st) {
   constexpr size_t lds = ShortShape<MODE, BITS, MB>::kLds;
   constexpr auto kern = short_kernel<MODE, BITS, TAB, MB, HALF>;
-  if (!lds_limit<kern>(lds)) return;
+  if (!lds_limit<kern, lds>()) return;
   const int64_t total = ceil_div((int64_t)a.n_tiles * a.m_tiles * a.splits, 8) * 8;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * kWaves), lds, st, a);
 }

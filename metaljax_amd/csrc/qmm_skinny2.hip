@@ -1348,11 +1348,11 @@ void launch_one(const GemvArgs& a, int64_t batch, int rows_per_wg, hipStream_t s
   constexpr int kTabKind = (CW >= 4 ? CW * 256 : 1024) * (wide ? 2 : 1);
   constexpr int XR = XD ? 0 : 2048 / BITS / 128;
   // (direct variants: plus a 1 KB patch a compute wavefront for staging activations)
-  const size_t lds = (size_t)(XD || XR + TMAX >= 4 ? 4 : XR + TMAX) * (CW * 4096 + 2 * kTabKind) +
+  constexpr size_t lds = (size_t)(XD || XR + TMAX >= 4 ? 4 : XR + TMAX) * (CW * 4096 + 2 * kTabKind) +
                      (XD != 0 && !wide ? (size_t)CW * 1024 : 0) + (GRP ? (CW + NL) * 128 + 512 : 0) +
                      (XD >= 2 && BITS == 4 && (GSHIFT == 8 || GSHIFT == 11) ? 2048 : 0);      // (the kernel's EXTRA)
   constexpr auto kern = skinny2_kernel<BITS, CW, NL, TMAX, GSHIFT, XD, GRP>;
-  if (!lds_limit<kern>(lds)) return;
+  if (!lds_limit<kern, lds>()) return;
   hipLaunchKernelGGL(kern, grid, dim3(kWave * (CW + NL)), lds, st, a, rows_per_wg);
 }
 

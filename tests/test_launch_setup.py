@@ -1,0 +1,90 @@
+"""What the host does ahead of its launches, without a GPU: the library runs in a child
+process whose HIP launch calls are recorded and go nowhere (every address it is given is
+made up, and never read)."""
+
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from metaljax_amd import _lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+RECORDER = r"""
+#include <cstddef>
+#include <cstdio>
+struct Dim { unsigned x, y, z; };
+static Dim grid, block;
+static size_t lds;
+extern "C" {
+int __hipPushCallConfiguration(Dim g, Dim b, size_t bytes, void*) { grid = g; block = b; lds = bytes; return 0; }
+int __hipPopCallConfiguration(Dim* g, Dim* b, size_t* bytes, void** stream) { *g = grid; *b = block; *bytes = lds; *stream = nullptr; return 0; }
+int hipLaunchKernel(const void* f, Dim g, Dim b, void**, size_t bytes, void*) {
+  std::printf("launch %zu %u %u %u %zu\n", (size_t)f, g.x, g.y, b.x, bytes);
+  return 0;
+}
+int hipFuncSetAttribute(const void* f, int, int value) { std::printf("limit %zu %d\n", (size_t)f, value); return 0; }
+int hipGetLastError() { return 0; }
+void next_call() { std::printf("call\n"); std::fflush(stdout); }
+}
+"""
+
+CALLS = r"""
+import ctypes, json, sys
+recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)       # ahead of the library: its calls are found first
+sys.path.insert(0, sys.argv[2])
+from metaljax_amd import _lib, moe_launch as ML
+lib, at = _lib.load(), 1 << 20
+SIZE = {_lib.F32: 4, _lib.BF16: 2, _lib.F16: 2}
+
+def dense(m, n, k, bits, x=_lib.BF16):
+    room = lib.qmm_workspace_bytes(1, m, n, k, 64, bits, 0, x)
+    return lib.qmm_quantized_matmul(at, x, at, at, at, _lib.BF16, at, x, 1, m, n, k, 64, bits, 0, at, room, None)
+
+for name, args in json.loads(sys.argv[3]):
+    recorder.next_call()
+    assert globals()[name](*args) == 0, (name, args, lib.qmm_last_error())
+recorder.next_call()
+"""
+
+
+@pytest.fixture(scope="module")
+def record(tmp_path_factory):
+    """calls -> what each did: (kernel, grid x, grid y, threads, bytes of LDS) a launch and (kernel, bytes) a raised limit"""
+    where = tmp_path_factory.mktemp("recorder")
+    (where / "recorder.cc").write_text(RECORDER)
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-o", where / "recorder.so", where / "recorder.cc"], check=True)
+
+    def run(calls):
+        out = subprocess.run([sys.executable, "-c", CALLS, str(where / "recorder.so"), ROOT, json.dumps(calls)], check=True,
+                             capture_output=True, text=True).stdout
+        done = []
+        for line in out.splitlines():
+            what, *numbers = line.split()
+            if what == "call":
+                done.append(([], []))
+            else:
+                done[-1][what == "limit"].append(tuple(int(v) for v in numbers))
+        assert len(done) == len(calls) + 1 and all(launches for launches, _ in done[:-1])
+        return done[:-1]
+    return run
+
+
+def test_a_kernels_limit_is_raised_once(record):
+    """By its first launch, for all that any later one may ask: calls of one kernel with a whole K and
+    with a K that is split need different amounts of local memory, whichever comes first."""
+    calls = [["dense", shape] for shape in ([2048, 4096, 8192, 4], [600, 2048, 12800, 4], [600, 2048, 12800, 4], [2048, 4096, 8192, 4],
+                                            [450, 8192, 8192, 8], [2048, 4096, 8192, 8], [450, 8192, 8192, 8], [48, 4096, 14336, 4], [48, 4096, 14336, 4])]
+    done = record(calls)
+    limits, asked = {}, {}
+    for launches, raised in done:
+        for kernel, value in raised:
+            limits.setdefault(kernel, []).append(value)
+        for kernel, _, _, _, lds in launches:
+            asked.setdefault(kernel, set()).add(lds)
+            assert lds <= max(limits.get(kernel, [65536]))
+    assert any(len(sizes) > 1 for sizes in asked.values())               # (one kernel, two amounts)
+    assert all(len(values) == 1 for values in limits.values()), limits
