@@ -15,6 +15,7 @@ void gemv_dispatch(const void* x, const void* w, const void* s, const void* b, i
                    int mode, const int32_t* lhs_idx, const int32_t* rhs_idx, int64_t n_experts,
                    int64_t n_xrows, hipStream_t st);
 void gemv_geometry(int64_t M, int64_t N, int64_t K, int* t, int* waves);
+void mxfp4_geometry(int terms, int64_t batch, int64_t M, int64_t N, int64_t K, const void* s, int64_t products, int* t, int* waves);
 void skinny_geometry(int64_t N, int64_t K, int bits, int* waves, int* rows_per_wg);
 bool skinny2_plan(int64_t M, int64_t N, int64_t K, int bits, int* rows_per_wg);
 bool skinny2_ragged_supported(int64_t N, int64_t K, int gs, int bits, int tab, const void* s, const void* b,
@@ -482,7 +483,8 @@ bool terms_in_kernel(const void* x, int terms, int64_t P, int64_t E, int64_t N, 
 
 // How the general MXFP4 decode kernel would take these pairs: 1 each a product of its
 // own, 2 sorted by the kernel itself, 0 not at all (another kernel, or the sort's launch).
-int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype) {
+// `waves`: how many wavefronts share the contraction there.
+int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype, int* waves) {
   if (P <= 0 || P > kGatherGemvMaxPairs || !aligned16(x)) return 0;
   const int terms = act_terms(x_dtype);
   const size_t any = ~(size_t)0 / 4;               // (the route of a call with all the scratch it asks for)
@@ -490,8 +492,11 @@ int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t
                 : E > 65535 || N > INT32_MAX || K > INT32_MAX || N * K >= (1ll << 40) ||
                       !gemv_runs_general(N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, E))
     return 0;
-  if (!sorts_general(P, E, any)) return 1;
-  return sorts_itself(P, E, N) ? 2 : 0;
+  const bool sorted = sorts_general(P, E, any);
+  if (sorted && !sorts_itself(P, E, N)) return 0;
+  int t;
+  mxfp4_geometry(terms, sorted ? skinny2_max_segments(P, E) : P, sorted ? 16 : terms, N, K, s, E, &t, waves);
+  return sorted ? 2 : 1;
 }
 
 namespace {

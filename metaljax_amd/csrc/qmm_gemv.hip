@@ -598,6 +598,20 @@ bool gemv_runs_general(int64_t N, int64_t K, int gs, int bits, int mode, int tab
   return true;
 }
 
+// Tile and wavefronts of the general MXFP4 kernel, for `batch` products of M operand rows in
+// `terms` terms by `products` weights (a product fused with its map takes the same: the same
+// sums).  Rows in terms past 2048 codes take eight wavefronts: the sums of four are the less
+// exact ones (1.16e-7 from 64 bits at 3968 against 0.98e-7), and a call of one round is slower
+// with them (one float32 row of 1936 x 3840 12.7 us with four, of 1880 x 3072 8.9 with eight).
+// Shapes that no staged kernel serves summed in four before, and keep them where the
+// workgroups are several rounds (205 pairs over 64 of 1792 x 3168 94 / 120).
+void mxfp4_geometry(int terms, int64_t batch, int64_t M, int64_t N, int64_t K, const void* s, int64_t products, int* t, int* waves) {
+  gemv_geometry(M, N, K, t, waves);
+  if (terms == 1 || K <= 2048) return;
+  const bool staged = !gemv_runs_general(N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, products);
+  if (staged || batch * ceil_div(N, 16 * *t) <= device_cus()) *waves = 8;
+}
+
 // float16 / float32 rows on a 16-byte address, as the MXFP4 kernel above takes them: dense (rhs_idx null), a pair a batch
 // entry, the sorted pairs of `segments`, or `pairs_here` pairs that the kernel sorts.
 void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* s, void* y, int y_dtype, int64_t batch,
@@ -623,14 +637,9 @@ void gemv_terms_dispatch(const void* x, int x_dtype, const void* w, const void* 
   a.src_row = src_row;
   a.out_row = out_row;
   a.x_rows = segments ? (int)x_rows : pairs_here;
+  const int terms = x_dtype == QMM_F32 ? 3 : 2;
   int t, waves;
-  gemv_geometry(segments || pairs_here ? 16 : M * (x_dtype == QMM_F32 ? 3 : 2), N, K, &t, &waves);
-  // Past 2048 codes eight wavefronts: the sums of four are the less exact ones (1.16e-7 from 64
-  // bits at 3968 against 0.98e-7), and a call of one round is slower with them (one float32 row
-  // of 1936 x 3840 12.7 us with four, of 1880 x 3072 8.9 with eight).  Shapes that no staged kernel serves summed in four before, and keep
-  // them where the workgroups are several rounds (205 pairs over 64 of 1792 x 3168 94 / 120).
-  const bool staged = !gemv_runs_general(N, K, 32, 4, QMM_MODE_MXFP4, QMM_BF16, s, nullptr, rhs_idx || segments ? n_experts : batch);
-  if (K > 2048 && (staged || batch * ceil_div(N, 16 * t) <= device_cus())) waves = 8;
+  mxfp4_geometry(terms, batch, segments || pairs_here ? 16 : M * terms, N, K, s, rhs_idx || segments ? n_experts : batch, &t, &waves);
   if (x_dtype == QMM_F32) launch_mxfp4_terms<3>(a, batch, t, waves, st);
   else launch_mxfp4_terms<2>(a, batch, t, waves, st);
 }

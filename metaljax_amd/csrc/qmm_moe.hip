@@ -32,7 +32,7 @@ namespace qmm {
 int moe_fail(int code, const char* what);        // qmm_api.hip: sets qmm_last_error
 int moe_launched(const char* what);
 int64_t skinny2_max_segments(int64_t P, int64_t E);
-int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype);
+int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype, int* waves);
 
 namespace {
 
@@ -687,8 +687,9 @@ int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
   for (int i = 0; i < m.leaves; ++i)
     if ((m.leaf[i].p == nullptr) != ((from_product >> i & 1) != 0)) return moe_fail(QMM_ERR_BAD_ARGUMENT, "pair product: leaf");
   if (m.rank != 1 || a->mode != QMM_MODE_MXFP4) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: a result of several axes a pair, or affine experts");
-  int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el);
-  const int waves = a->k > 2048 ? 8 : 4;           // (more than 2048 codes: gemv_terms_dispatch)
+  int waves = 4;
+  int route = pair_product_route(a->x, a->x_el, m.pairs, m.experts, a->n, a->k, a->s, a->product_el, &waves);
+  waves = waves == 4 ? 4 : 8;                      // (what there are launches of)
   if (m.weights && (a->tiles > 1 || m.per_token * waves > 16 || (route == 2 && m.pairs * (a->n * a->k / 2) > kSumBytes))) route = 0;
   const size_t lds = pair_product_lds(*a, waves);
   if (!route || (reinterpret_cast<uintptr_t>(a->w) & 15u) || lds > kProductLds) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: two launches are better");

@@ -38,11 +38,22 @@ recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)       # ahead of th
 sys.path.insert(0, sys.argv[2])
 from metaljax_amd import _lib, moe_launch as ML
 lib, at = _lib.load(), 1 << 20
-SIZE = {_lib.F32: 4, _lib.BF16: 2, _lib.F16: 2}
 
 def dense(m, n, k, bits, x=_lib.BF16):
     room = lib.qmm_workspace_bytes(1, m, n, k, 64, bits, 0, x)
     return lib.qmm_quantized_matmul(at, x, at, at, at, _lib.BF16, at, x, 1, m, n, k, 64, bits, 0, at, room, None)
+
+def gather(pairs, experts, n, k, x):
+    room = lib.qmm_gather_workspace_bytes(pairs, experts, n, k, x)
+    return lib.qmm_gather_qmm(at, x, at, at, None, _lib.BF16, at, x, at, at, pairs, pairs, experts, n, k, 32, 4, _lib.MODE_MXFP4, at, room, None)
+
+def fused(pairs, experts, n, k, x, per):
+    el = {_lib.F32: 0, _lib.BF16: 1, _lib.F16: 2}[x]
+    m = ML.PairMap(y=at, experts_of=at, pairs=pairs, inner=n, dims=(1, 1, n), per_token=per or 1, experts=experts, rank=1, leaves=1,
+                   registers=1, weights=at if per else None)
+    m.leaf[0] = ML.MapLeaf(None, 0, n, 0, 0, (0, 0, 1), el)
+    p = ML.PairProduct(x=at, w=at, s=at, x_rows=pairs, n=n, k=k, mode=_lib.MODE_MXFP4, x_el=el, x_per=1, product_el=el, tiles=1, col_step=(1, 0), map=m)
+    return lib.qmm_pair_product_run(ctypes.byref(p), None)
 
 for name, args in json.loads(sys.argv[3]):
     recorder.next_call()
@@ -88,3 +99,27 @@ def test_a_kernels_limit_is_raised_once(record):
             assert lds <= max(limits.get(kernel, [65536]))
     assert any(len(sizes) > 1 for sizes in asked.values())               # (one kernel, two amounts)
     assert all(len(values) == 1 for values in limits.values()), limits
+
+
+@pytest.mark.parametrize("pairs,experts,n,k,types", [
+    (4, 8, 64, 2048, "f32 f16"), (4, 8, 64, 2016, "f32 bf16 f16"),
+    (5, 8, 96, 2080, "f32 bf16 f16"), (6, 8, 1792, 3168, "f32 bf16 f16"), (24, 16, 1792, 3168, "f32 bf16 f16"), (24, 16, 96, 3168, "f32 bf16 f16"),
+    (8, 8, 1024, 3072, "f32 f16"), (16, 8, 512, 3072, "f32 f16"), (7, 8, 64, 4160, "f32 bf16 f16"), (40, 8, 96, 4192, "f32 bf16 f16")])
+def test_a_product_and_its_map_share_a_contraction_as_the_product_does(record, pairs, experts, n, k, types):
+    """As many wavefronts, and so the same sums, and a token's pairs as many each: of four
+    and eight, by the contraction, the type and (where the workgroups are several rounds) the
+    columns and the pairs; shapes that a staged kernel would take among them."""
+    calls = []
+    for x in types.split():
+        shape = [pairs, experts, n, k, {"f32": _lib.F32, "bf16": _lib.BF16, "f16": _lib.F16}[x]]
+        calls += [["gather", shape], ["fused", shape + [0]]]
+        if pairs % 2 == 0 and pairs * n * k / 2 <= 16 << 20:
+            calls.append(["fused", shape + [2]])
+    threads = 0
+    for (name, args), (launches, _) in zip(calls, record(calls)):
+        (_, _, rows, lanes, _), = launches
+        if name == "gather":
+            threads, segments = lanes, rows
+        else:
+            assert lanes == threads * (args[5] or 1)
+            assert rows == (pairs // args[5] if args[5] else segments)
