@@ -3,6 +3,7 @@ GPU: experts past a wavefront, a router wider than a workgroup's share of it, ti
 and NaN among the logits, and the two kernels against float64."""
 
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -217,8 +218,42 @@ def test_a_product_and_its_map_in_one_launch(E, Tk, H, Ii, K, fused, el, monkeyp
         (buf,) = engine.execute(ex, args)
         assert ex.interp._qmm.moe[0].launches is not None
         out.append(engine.to_numpy(buf)[0])
-    assert served[-1] == 0 and (served[0] == fused or el != "f32")
+    assert served == [fused, 0]
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("Tk", [3, 12])
+def test_blocks_of_two_threads_on_their_streams(Tk):
+    """The steps of a block are shared by its calls: two threads at once, each on a stream of
+    its own with activations that the work ahead of them there has yet to write, pairs of
+    their own and pairs that the launch sorts; what the calls give one after the other."""
+    E, H, Ii, K, calls = 8, 512, 256, 2, 25
+    args = [I.from_numpy(a) for a in _moe_inputs(E, Tk, H, Ii)[0]]
+    ex = engine.compile_program(T.moe_block_mxfp4(E, Tk, H, Ii, K))
+    xs = torch.randn((2, calls, Tk, H), device="cuda") / 8
+    want = [torch.stack([engine.execute(ex, [x] + args[1:])[0].data.clone() for x in row]) for row in xs]
+    assert ex.interp._qmm.moe[0].launches is not None and not torch.equal(*want)
+    got, errors = [None, None], []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            a, late = torch.randn((2048, 2048), device="cuda"), torch.zeros_like(xs[i])
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                for _ in range(20):
+                    a = a @ a * 1e-2
+                late.copy_(xs[i])
+                got[i] = torch.stack([engine.execute(ex, [x] + args[1:])[0].data for x in late])
+            stream.synchronize()
+        except Exception as e:                           # (the thread's; raised below)
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not errors and all(torch.equal(g, w) for g, w in zip(got, want)), errors
 
 
 def which(steps, values, stream):
