@@ -21,6 +21,7 @@
 // instruction for every lane, operands in LDS (column of a lane: its own, so that no
 // barrier is needed between instructions), arithmetic in float32, one rounding to the
 // value's element type an instruction -- what an array operation of that type does.
+#include <algorithm>
 #include <cstddef>
 #include <cstring>
 
@@ -32,6 +33,7 @@ namespace qmm {
 int moe_fail(int code, const char* what);        // qmm_api.hip: sets qmm_last_error
 int moe_launched(const char* what);
 int64_t skinny2_max_segments(int64_t P, int64_t E);
+int device_cus();
 int pair_product_route(const void* x, int x_dtype, int64_t P, int64_t E, int64_t N, int64_t K, const void* s, int y_dtype, int* waves);
 
 namespace {
@@ -629,6 +631,29 @@ size_t pair_product_lds(const qmm_pair_product& a, int waves) {
          sizeof(m.code);
 }
 
+// Is the sum over a token's pairs better as part of the product, in `groups` workgroups of
+// `all` wavefronts?  Each has its own chain of round trips, so a round of them costs 3 to 8
+// us where the launch that is spared is 3: one round always pays (by 1.1 to 2.2), a second
+// where its workgroups are short (bf16 rows, one term) or the launches it stands for many
+// (three pairs a token and more; long rows of sorted pairs excepted), and for 16-bit rows
+// where the product alone would read an expert for every pair as well (bf16: any number).
+// us, one launch / two, 8 experts: float32 5 and 12 tokens of two pairs over 1024 x 1024 13.4 /
+// 12.3, 19.4 / 12.2, 3 over 8192 x 1024 37.9 / 27.1, 4 of four pairs 9.7 / 14.8, 8 17.5 / 15.0, 8 of
+// K = 256 10.8 / 13.3; bf16 12 of two pairs over 1024 x 1024 9.9 / 11.2, 20 of K = 256 10.3 / 9.6.
+// (10781 drawn products, weights in the caches and not: 0.4 % from the better one's time
+// on average; the fused launch wherever it fits 6.3 %.  Whole blocks of float32, 24 tokens
+// over 16 experts of 768 x 512 44.6 -> 31.6, 40 of one pair over 8 of 1024 x 512 36.1 -> 28.0.)
+bool sum_pays(const qmm_pair_product& a, int all, size_t lds, bool sorted, int64_t groups) {
+  const int terms = a.x_el == QMM_EL_F32 ? 3 : a.x_el == QMM_EL_F16 ? 2 : 1;
+  if (terms == 1 && !sorted) return true;
+  // wavefronts a SIMD holds by the kernels' registers: of 512 threads (142, 104, 88), of 1024 (104, 86, 62)
+  constexpr int kHeld[2][3] = {{5, 4, 3}, {8, 5, 4}};
+  const int64_t held = std::min<int64_t>(kHeld[all > 8][terms - 1] * 4 / all, (160 << 10) / (int64_t)lds);
+  int rounds = terms == 1 || (terms == 2 && !sorted) ? 2 : 1;
+  if (a.map.per_token > 2 && (!sorted || a.k * terms <= 2048)) ++rounds;
+  return groups <= rounds * held * device_cus();
+}
+
 template <int T, int WAVES, int TERMS>
 void launch_pair_product(const qmm_pair_product& a, dim3 grid, size_t lds, hipStream_t st) {
   const int all = a.map.weights ? a.map.per_token * WAVES : WAVES;
@@ -692,6 +717,7 @@ int qmm_pair_product_run(const qmm_pair_product* a, void* stream) {
   waves = waves == 4 ? 4 : 8;                      // (what there are launches of)
   if (m.weights && (a->tiles > 1 || m.per_token * waves > 16 || (route == 2 && m.pairs * (a->n * a->k / 2) > kSumBytes))) route = 0;
   const size_t lds = pair_product_lds(*a, waves);
+  if (m.weights && route && !sum_pays(*a, m.per_token * waves, lds, route == 2, m.pairs / m.per_token * ceil_div(m.inner, 16))) route = 0;
   if (!route || (reinterpret_cast<uintptr_t>(a->w) & 15u) || lds > kProductLds) return moe_fail(QMM_ERR_UNSUPPORTED, "pair product: two launches are better");
   const int64_t segments = m.weights ? m.pairs / m.per_token : route == 2 ? skinny2_max_segments(m.pairs, m.experts) : m.pairs;
   qmm_pair_product p = *a;

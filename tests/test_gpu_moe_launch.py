@@ -190,9 +190,12 @@ def test_pair_tokens_are_there_for_another_stream():
 
 @pytest.mark.parametrize("el", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("E,Tk,H,Ii,K,fused", [
-    (1, 1, 32, 32, 1, 2), (4, 1, 160, 96, 4, 2), (8, 3, 1024, 1024, 2, 2), (8, 5, 96, 2080, 2, 2), (8, 7, 4160, 32, 1, 2),
-    (4, 32, 512, 96, 2, 2), (8, 64, 288, 64, 1, 2), (8, 33, 64, 64, 2, 0), (3, 11, 1056, 544, 3, 2), (5, 2, 64, 32, 5, 1), (16, 24, 3168, 896, 1, 1)])
+    (1, 1, 32, 32, 1, "222"), (4, 1, 160, 96, 4, "222"), (8, 3, 1024, 1024, 2, "222"), (8, 5, 96, 2080, 2, "222"), (8, 7, 4160, 32, 1, "122"),
+    (4, 32, 512, 96, 2, "121"), (8, 64, 288, 64, 1, "121"), (8, 33, 64, 64, 2, "000"), (3, 11, 1056, 544, 3, "121"), (5, 2, 64, 32, 5, "111"),
+    (16, 24, 3168, 896, 1, "111"), (4, 12, 320, 96, 2, "222"), (8, 64, 160, 64, 1, "222"), (3, 11, 224, 544, 3, "222")])
 def test_a_product_and_its_map_in_one_launch(E, Tk, H, Ii, K, fused, el, monkeypatch):
+    # fused: how many of a block's two products are, for float32, bf16 and float16 (the sum over a token's pairs
+    # is where its workgroups are a round or two)
     """Pairs of their own, pairs sorted by the kernel, the sum over a token's pairs in two
     to sixteen wavefronts, K of a part of a chunk and of more than 2048, there in one round of
     workgroups and in several: what two launches give.  The sums are the same ones in the
@@ -218,7 +221,7 @@ def test_a_product_and_its_map_in_one_launch(E, Tk, H, Ii, K, fused, el, monkeyp
         (buf,) = engine.execute(ex, args)
         assert ex.interp._qmm.moe[0].launches is not None
         out.append(engine.to_numpy(buf)[0])
-    assert served == [fused, 0]
+    assert served == [int(fused["f32 bf16 f16".split().index(el)]), 0]
     assert np.array_equal(*out)
 
 

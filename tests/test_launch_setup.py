@@ -55,6 +55,9 @@ def fused(pairs, experts, n, k, x, per):
     p = ML.PairProduct(x=at, w=at, s=at, x_rows=pairs, n=n, k=k, mode=_lib.MODE_MXFP4, x_el=el, x_per=1, product_el=el, tiles=1, col_step=(1, 0), map=m)
     return lib.qmm_pair_product_run(ctypes.byref(p), None)
 
+def refused(*shape):
+    return int(fused(*shape) != 3)                                 # (UNSUPPORTED: two launches)
+
 for name, args in json.loads(sys.argv[3]):
     recorder.next_call()
     assert globals()[name](*args) == 0, (name, args, lib.qmm_last_error())
@@ -79,7 +82,7 @@ def record(tmp_path_factory):
                 done.append(([], []))
             else:
                 done[-1][what == "limit"].append(tuple(int(v) for v in numbers))
-        assert len(done) == len(calls) + 1 and all(launches for launches, _ in done[:-1])
+        assert len(done) == len(calls) + 1 and all(bool(launches) == (name != "refused") for (name, _), (launches, _) in zip(calls, done))
         return done[:-1]
     return run
 
@@ -123,3 +126,20 @@ def test_a_product_and_its_map_share_a_contraction_as_the_product_does(record, p
         else:
             assert lanes == threads * (args[5] or 1)
             assert rows == (pairs // args[5] if args[5] else segments)
+
+
+@pytest.mark.parametrize("tokens,per,experts,n,k,types", [
+    (4, 2, 8, 1024, 1024, "f32 bf16 f16"), (5, 2, 8, 1024, 1024, "bf16 f16"), (7, 2, 8, 1600, 1024, "bf16 f16"), (7, 2, 8, 8192, 256, "bf16"),
+    (8, 2, 8, 512, 512, "f32 bf16 f16"), (12, 2, 8, 512, 512, "bf16 f16"), (20, 2, 8, 512, 512, "bf16"), (32, 2, 8, 1024, 256, ""),
+    (12, 1, 8, 1024, 256, "f32 bf16 f16"), (13, 1, 8, 1024, 256, "bf16 f16"), (64, 1, 8, 256, 256, "bf16 f16"), (64, 1, 8, 512, 256, "bf16"),
+    (4, 4, 8, 1024, 1024, "f32 bf16 f16"), (8, 4, 8, 1024, 1024, "bf16 f16"), (8, 4, 8, 1024, 256, "f32 bf16 f16"), (16, 4, 8, 1024, 256, "bf16"),
+    (2, 4, 8, 4096, 512, "f32 bf16 f16"), (3, 4, 8, 4096, 512, "bf16 f16"), (3, 4, 8, 8192, 256, "bf16")])
+def test_a_tokens_sum_is_part_of_the_product_for_a_round_or_two(record, tokens, per, experts, n, k, types):
+    """On both sides of what a round of the summing workgroups holds, by the type's terms and the pairs a
+    token, sorted by the kernel (16 pairs and more) and not; past it a product and a map are the faster."""
+    calls = [["fused" if x in types.split() else "refused", [tokens * per, experts, n, k, {"f32": _lib.F32, "bf16": _lib.BF16, "f16": _lib.F16}[x], per]]
+             for x in ("f32", "bf16", "f16")]
+    for (name, args), (launches, _) in zip(calls, record(calls)):
+        if name == "fused":
+            (_, columns, rows, lanes, _), = launches
+            assert (columns, rows, lanes) == (-(-n // 16), tokens, 64 * 4 * per)
