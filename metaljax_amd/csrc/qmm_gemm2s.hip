@@ -77,19 +77,23 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
     // one expert of all rows: an eighth of the grid takes a contiguous run of
     // tiles (and the workgroups that share a tile's K come one K range after the
     // other).  Tiles of 128 rows: column tile fastest, so that its workgroups share
-    // few activation rows.  Tiles of 256, where the last row tile may be a short one:
-    // row tile fastest, so that every eighth has its share of the short ones and
+    // few activation rows.  Ten tiles of 256 at most, where the last row tile may be a short
+    // one: row tile fastest, so that every eighth has its share of the short ones and
     // reads a weight once (us, column / row tile fastest: 1106 rows of 6240 x 7424
     // 105.5 / 98.8, eight-bit 380 of 14712 x 1344 27.0 / 25.0 and 563 of 4712 x 13952
     // 104.7 / 100.7, 669 of 13856 x 2176 61.1 / 58.7, whole tiles 2048 of 4096 x 4096
     // 65.2 / 64.8; of 128 rows 500 of 6144 x 4096 37.4 / 38.5, 256 of 9216 x 3072 28.1 / 28.7).
+    // More row tiles than that are more activations than the L2 of an XCD keeps for the next
+    // column tile: 2190 rows of 8070 x 3008 187.7 / 171.9, but 5033 of 3112 x 832 39.7 / 46.0, 8174
+    // of 3552 x 3712 218 / 280, float32 rows in three terms, 2674 of 7600 x 6656, 927 / 1157
+    // (4073 drawn products, 0.2 % from the better order's time on average, row tile fastest in all 1.9 %).
     const int m_tiles = (a.R + a.tile_rows - 1) / a.tile_rows;
     const int tiles = n_tiles * m_tiles, total = tiles * a.splits, per = (total + 7) / 8;
     const int t = xcd * per + l;
     if (l >= per || t >= total) return;
     split = t / tiles;
     const int i = t - split * tiles;
-    const bool by_rows = a.tile_rows == 256;
+    const bool by_rows = a.tile_rows == 256 && m_tiles <= 10;
     tile_m = by_rows ? i % m_tiles : i / n_tiles;
     tile_n = by_rows ? i / m_tiles : i % n_tiles;
     mt_idx = tile_m;

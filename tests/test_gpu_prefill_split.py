@@ -54,8 +54,8 @@ def test_dense(m, n, k, kind, act):
 
 # Row tiles of 256 rows (several rounds of workgroups, or a split K: columns of whole lines,
 # whose sums are stored wide and read once, of whole sixteen bytes and of neither), the last of
-# 188, 76, 130 and 88 rows, dealt row tile first; float32 results and 16-bit ones (one rounding, half a place of eight bits, and the sums).
-@pytest.mark.parametrize("m,n,k", [(700, 11992, 256), (1100, 6240, 1088), (642, 1096, 12800), (600, 2048, 12800), (642, 1090, 12800)])
+# 188, 76, 130 and 88 rows, dealt row tile first, and eleven of them, the last of 140 rows, column tile first; float32 results and 16-bit ones (one rounding, half a place of eight bits, and the sums).
+@pytest.mark.parametrize("m,n,k", [(700, 11992, 256), (1100, 6240, 1088), (642, 1096, 12800), (600, 2048, 12800), (642, 1090, 12800), (2700, 1536, 320)])
 @pytest.mark.parametrize("kind", [KINDS[0], KINDS[3]])
 def test_tiles_of_256_rows(m, n, k, kind):
     bits, gs, mode, tab = kind
