@@ -662,6 +662,7 @@ double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes
   const char* er = experiment_env("QMM_G2S_ROWS");
   const char* es = experiment_env("QMM_G2S_SPLITS");
   const int64_t kt = ceil_div(K, BK), quads = ceil_div(kt, 4), nt = ceil_div(N, BN), group = E > 1 ? ceil_div(R, E) : R;
+  const bool wide = wide_sums(R, N);
   double best = 1e30, least = 1e30;
   *tile_rows = 256;
   *splits = 1;
@@ -673,11 +674,13 @@ double gemm2s_plan(int64_t R, int64_t E, int64_t N, int64_t K, size_t part_bytes
       if (s > 1 && (s > quads || (double)s * R * N * 4 > (double)part_bytes)) break;
       const int64_t tiles = nt * mt * s;
       const double step = (half ? 0.41 : 0.60) + 0.105 * (tiles < 256 ? tiles / 256.0 : 1.0);
+      const double sums = (double)s * R * N;     // (past 64 MB they come back from memory)
       const double us = 5.9 + (double)ceil_div(tiles, 256) * (2.5 + (s == 1 ? kt : 4 * ceil_div(quads, s)) * step) +
-                        (double)R * K * 0.54e-6 + (double)R * N * 0.5e-6 + (s > 1 ? 4.0 + (double)s * R * N * 0.7e-6 : 0.0);
-      // (of two alike the one with fewer splits, and none that is a second round: 698 rows of
-      // 5432 x 7424 in three parts, 387 tiles, 75.7 us, whole 70.9)
-      double cost = us * (1.0 + 0.01 * s) * (s > 1 && tiles > 256 ? 1.08 : 1.0);
+                        (double)R * K * 0.54e-6 + (double)R * N * 0.5e-6 +
+                        (s == 1 ? 0.0 : wide ? 4.0 + (sums + std::max(0.0, sums - (1 << 24))) * 0.7e-6 : 4.6 + sums * 1.4e-6);
+      // (of two alike the one with fewer splits, and none that makes a second round of one: 698
+      // rows of 5432 x 7424 in three parts, 387 tiles, 75.7 us, whole 70.9)
+      double cost = us * (1.0 + 0.01 * s) * (wide && s > 1 && tiles > 256 && nt * mt <= 256 ? 1.08 : 1.0);
       if (er && E <= 1 && atoi(er) != rows) cost += 1e9;
       if (es && E <= 1 && atoi(es) != s) cost += 1e9;
       if (cost < best) { best = cost; least = us; *tile_rows = rows; *splits = s; }

@@ -143,3 +143,13 @@ def test_a_tokens_sum_is_part_of_the_product_for_a_round_or_two(record, tokens, 
         if name == "fused":
             (_, columns, rows, lanes, _), = launches
             assert (columns, rows, lanes) == (-(-n // 16), tokens, 64 * 4 * per)
+
+
+@pytest.mark.parametrize("m,n,k,bits,workgroups", [
+    (698, 5432, 7424, 4, 129), (212, 6896, 5376, 4, 4 * 54),           # (in fours none would be a second round of one, or it is worth it)
+    (635, 2138, 2560, 8, 170), (855, 1458, 2496, 8, 168),              # columns that are no fours, whose sums leave one by one: short groups
+    (6328, 1486, 7552, 8, 2 * 300), (5076, 1920, 7808, 4, 2 * 300),    # more tiles than a round as they are
+    (926, 9576, 14080, 8, 3 * 300)])                                   # more sums than caches hold
+def test_a_split_K_counts_what_its_sums_take(record, m, n, k, bits, workgroups):
+    (launches, _), = record([["dense", [m, n, k, bits]]])
+    assert -(-workgroups // 8) * 8 in [x for _, x, _, lanes, _ in launches if lanes == 512]
