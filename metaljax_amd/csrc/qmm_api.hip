@@ -539,7 +539,7 @@ size_t term_bytes(int64_t terms, int64_t rows, int64_t N, int64_t K) {
 bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, int terms, int own, bool grouped, size_t scratch) {
   if (K % 64 || N <= 0) return false;
   if (const char* env = experiment_env("QMM_SHORT")) return env[0] != '0';
-  double other;
+  double other, ours = 0.0;
   if (mode == QMM_MODE_MXFP4 && terms == 1 && mxfp4_mfma_supported(R, N, K)) {
     if (N < 512) return false;                   // (a few column tiles: not measured, left as it is)
     other = mxfp4_us(R, E, N, K);
@@ -548,9 +548,13 @@ bool short_wins(int64_t R, int64_t E, int64_t N, int64_t K, int bits, int mode, 
     const size_t held = gemm2_workspace_bytes(terms * R, K) + (terms > 1 ? term_bytes(terms, R, N, K) : 0);
     other = grouped ? terms * gemm2_us(R, E, N, K, 0) : gemm2_us(terms * R, 1, N, K, scratch > held ? scratch - held : 0);
     if (terms > 1) other += 5.2 + (double)terms * R * N * 1.4e-6;
+    // (the terms' own launches: float32 rows of 2387 x 11264 83 us ahead of the re-laying, 40 here;
+    // for groups both times are too short by more than that)
+    if (terms > 1 && !grouped) other += (double)R * K * (terms == 3 ? 3.0e-6 : 2.4e-6);
+    if (own > 1 && !grouped) ours = (double)R * K * (own == 3 ? 1.4e-6 : 0.9e-6);
   }
   const size_t prep = short_prep_bytes(R, K, own);
-  return short_us(R, E, N, K, bits, mode, own, scratch > prep ? scratch - prep : 0) < other;
+  return ours + short_us(R, E, N, K, bits, mode, own, scratch > prep ? scratch - prep : 0) < other;
 }
 
 // Scratch that lets a short-group product over R rows run as it would best.

@@ -153,3 +153,13 @@ def test_a_tokens_sum_is_part_of_the_product_for_a_round_or_two(record, tokens, 
 def test_a_split_K_counts_what_its_sums_take(record, m, n, k, bits, workgroups):
     (launches, _), = record([["dense", [m, n, k, bits]]])
     assert -(-workgroups // 8) * 8 in [x for _, x, _, lanes, _ in launches if lanes == 512]
+
+
+@pytest.mark.parametrize("m,n,k,bits,x,short", [
+    (2387, 168, 11264, 4, "f32", True), (2988, 200, 5760, 8, "f32", True), (1048, 264, 12800, 4, "f32", True),
+    (600, 4096, 4096, 4, "f32", False), (2048, 4096, 4096, 4, "f16", False)])
+def test_terms_that_are_launches_of_their_own_count(record, m, n, k, bits, x, short):
+    """Terms, the product and its sums on the kernel of short groups; terms, their re-laying, the product, its
+    sums and the sum over the terms ahead of it on the other, whose terms take twice the time."""
+    (launches, _), = record([["dense", [m, n, k, bits, {"f32": _lib.F32, "f16": _lib.F16}[x]]]])
+    assert (len(launches) <= 3) == short
