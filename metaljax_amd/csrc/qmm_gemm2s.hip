@@ -501,9 +501,9 @@ __global__ __launch_bounds__(512) void gemm2s_kernel(Gemm2Args a) {
         const int n = n0 + ((i == 0 || two) ? 0 : wm * 32) + pc * 8;
         if (m < m_end && n < a.N) {
           const int64_t orow = a.out_idx ? (int64_t)a.out_idx[m] : (int64_t)m;
-          // (not kept in L2, where the activations are read again: 1024 rows over 8 experts of
-          // 14336 x 4096 175.1 -> 174.5 us, 2048 x 4096 x 4096 eight-bit 70.1 -> 68.6, 380 of
-          // 14712 x 1344 27.8 -> 26.6; written through L2 instead it is 2 % slower than plain)
+          // (not kept in L2, where the activations are read again: us, 2048 x 4096 x 4096 eight-bit
+          // 70.1 -> 68.6, 380 of 14712 x 1344 27.8 -> 26.6, 1024 rows over 8 experts of 14336 x 4096
+          // no more than runs differ; written through L2 instead it is 2 % slower than plain)
           __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(o16 + rl * BN + pc * 8),
                                       reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.y) + orow * a.N + n));
         }

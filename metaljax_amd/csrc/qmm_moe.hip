@@ -17,8 +17,8 @@
 // tokens 93 / 439, 2048 tokens 364 / 815; 32 experts of 2880 x 2880, top 4: 64 tokens 286 /
 // 533, 2048 tokens 3476 / 4536).
 //
-// Both kernels interpret a short program that the planner wrote once: the same
-// instruction for every lane, operands in LDS (column of a lane: its own, so that no
+// The kernels interpret a short program that the planner wrote once (a product's, the
+// map's behind it): the same instruction for every lane, operands in LDS (column of a lane: its own, so that no
 // barrier is needed between instructions), arithmetic in float32, one rounding to the
 // value's element type an instruction -- what an array operation of that type does.
 #include <algorithm>
@@ -185,16 +185,18 @@ __global__ __launch_bounds__(kThreads) void pair_map_kernel(qmm_pair_map a) {
 }
 
 // A product of MXFP4 experts and the pair map behind it, one launch.  A workgroup takes
-// sixteen output elements of a pair (HERE: of up to sixteen pairs of one expert; SUM: of a
+// sixteen output elements of a pair (sorted: of up to sixteen pairs of one expert; SUM: of a
 // token, WAVES wavefronts a pair, THREADS at most) and multiplies the weight rows that these read: tile t's
 // row r is column col_base[t] + col_step[t] * element of the product.  The multiplication
-// is the general decode kernel's (gemv_mxfp4_kernel: the same operands, sums and order);
-// its sums meet in LDS, where the map finds them as leaves.
+// is the general decode kernel's (gemv_mxfp4_kernel: the same operands, in as many
+// wavefronts, and so the same sums in the same order: a change to either's loop is one to
+// both); its sums meet in LDS, where the map finds them as leaves.
 //
 // What bounds it: one round trip after the other -- arguments, the pair's expert, the
 // weight -- with the map's memory leaves requested ahead of the weight: 6 pairs over 8
-// experts of 2048 x 1024 and a map of two columns 10.8 us, of 1024 x 1024 and the sum of
-// a token's two pairs 8.2.  As two launches each took 7.7 + 5.3 and the gap between them.
+// experts of 2048 x 1024 and a map of two columns 11.3 us, of 1024 x 1024 and the sum of
+// a token's two pairs 7.8 (a kernel trace of float32 rows); as two launches each 8.0 + 5.2
+// and 6.5 + 5.1, and the gaps between them.
 template <int T, int WAVES, int TERMS, int THREADS>
 __global__ __launch_bounds__(THREADS ? THREADS : kWave* WAVES) void pair_product_kernel(qmm_pair_product a) {
   constexpr bool SUM = THREADS > 0;
